@@ -953,16 +953,17 @@ void engine_flux_update(Engine* e, int RK, int er_slot) {
 }
 
 namespace {
-// Size class of the resident pool: floor(log2(resident cubes)).
-int size_class(const Engine* e) {
-  long n = 0;
+int resident_cubes(const Engine* e) {
+  int n = 0;
   for (const CaseSlot& S : e->cases)
     if (S.active) n += S.tb.n;
-  int c = 0;
-  while (n > 1) {
-    n >>= 1;
-    ++c;
-  }
+  return n;
+}
+
+// Size class of the resident pool: floor(log2(resident cubes)).
+int size_class(const Engine* e) {
+  int n = resident_cubes(e), c = 0;
+  for (; n > 1; n >>= 1) ++c;
   return c;
 }
 }  // namespace
@@ -1042,67 +1043,20 @@ int engine_autotune(Engine* e, int* variant, int* nseg, std::string& err) {
     if (nseg) *nseg = e->mixed_nseg;
     return 0;
   }
-  // Candidates (variant, nseg, fuse): the marching kernel with the RK update
-  // fused in place, and the marching kernel writing the update and face halos
-  // into the other copy of the iterate (fuse 2).  Both reduce the norms over
-  // one partial row per cube, so the norms do not depend on which one wins.
-  // (The plane kernel and the segmented marching kernel, selectable with
-  // set_flux, reduce over per-plane rows and are not candidates.)  Each is
-  // timed as one whole RK stage on the resident cases, as the inner
-  // iterations of a step run it, in three interleaved rounds of which each
-  // keeps its fastest; every array a stage writes is saved first and
-  // restored afterwards.
-  const int cand[2][3] = {{1, 1, 1}, {1, 1, 2}};
-  double* const live[6] = {e->U, e->U2, e->U1p1, e->U1p2, e->Rku, e->Res};
-  struct Saved {
-    double* p[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    ~Saved() {
-      for (double* q : p)
-        if (q) (void)hipFree(q);
-    }
-  } saved;
-  for (int a = 0; a < 6; ++a) {
-    HIP_TRY(hipMalloc((void**)&saved.p[a], pool_bytes(e)));
-    HIP_TRY(hipMemcpyAsync(saved.p[a], live[a], pool_bytes(e), hipMemcpyDeviceToDevice,
-                           e->stream));
-  }
-  const bool full = e->halo_full_next;
-  float fastest[2] = {1e30f, 1e30f};
-  for (int round = 0; round < 3; ++round)
-    for (int c = 0; c < 2; ++c) {
-      const int* cv = cand[c];
-      e->flux_variant = cv[0];
-      e->flux_nseg = cv[1];
-      e->flux_fuse = cv[2] != 0;
-      e->flux_push = cv[2] == 2;
-      e->push_aux = false;
-      engine_stage(e, 2, 0, full);  // warm up
-      HIP_TRY(hipEventRecord(e->ev0, e->stream));
-      for (int r = 0; r < 3; ++r) engine_stage(e, 2, 0, full);
-      HIP_TRY(hipEventRecord(e->ev1, e->stream));
-      e->push_aux = true;
-      HIP_TRY(hipEventSynchronize(e->ev1));
-      float ms = 0;
-      HIP_TRY(hipEventElapsedTime(&ms, e->ev0, e->ev1));
-      e->U = live[0];
-      e->U2 = live[1];
-      for (int a = 0; a < 6; ++a)
-        HIP_TRY(hipMemcpyAsync(live[a], saved.p[a], pool_bytes(e), hipMemcpyDeviceToDevice,
-                               e->stream));
-      fastest[c] = std::min(fastest[c], ms);
-    }
-  HIP_TRY(hipStreamSynchronize(e->stream));
-  const int* win = cand[fastest[1] < fastest[0] ? 1 : 0];
-  const int bv = win[0], bs = win[1];
-  const bool bf = win[2] != 0, bp = win[2] == 2;
-  e->flux_push = bp;
-  e->flux_variant = bv;
-  e->flux_nseg = bs;
-  e->flux_fuse = bf;
+  // FP64: the marching kernel writing the update and face halos into the other
+  // copy of the iterate, whose runs per cube follow the resident cubes
+  // (push_runs).  The in-place kernels stay selectable with set_flux and serve
+  // the stage pieces and drop-ins; as whole stages they are slower at every
+  // size (1,622 against 1,372 us of flux kernel on 2,048 cubes, 230 against
+  // 220 us on 8 with one run each).
+  e->flux_variant = 1;
+  e->flux_nseg = 1;
+  e->flux_fuse = true;
+  e->graph_valid = e->graph_valid && e->flux_push;
+  e->flux_push = true;
   e->flux_tuned = true;
-  e->graph_valid = false;
-  if (variant) *variant = bv;
-  if (nseg) *nseg = bs;
+  if (variant) *variant = 1;
+  if (nseg) *nseg = 1;
   return 0;
 }
 
@@ -1128,10 +1082,11 @@ void engine_flux_push(Engine* e, int RK, int er_slot) {
   }
   launch_flux_push(e->stream, e->U, e->U2, e->halo, e->bc_mask_cube, e->U1, e->U1q, e->fws,
                    e->cube_size, e->Rku, e->Res, e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e,
-                   RK, e->U1p1, e->U1p2, e->partials, e->push_aux ? 1 : 0);
+                   RK, e->U1p1, e->U1p2, e->partials, e->push_aux ? 1 : 0,
+                   push_runs(resident_cubes(e)));
   std::swap(e->U, e->U2);
   if (RK == 3)
-    launch_reduce(e->stream, e->partials, 1, e->case_desc, e->n_active, e->phys_dev,
+    launch_reduce(e->stream, e->partials, PUSH_ROWS_PER_CUBE, e->case_desc, e->n_active, e->phys_dev,
                   er_row(e, er_slot));
 }
 

@@ -238,9 +238,10 @@ int engine_run(Engine* e, int n_steps, int n_inner, double* er_hist, bool use_gr
 int engine_run_converge(Engine* e, int n_steps, int max_inner, double tol, double* E, int* iters,
                         double* er_hist, std::string& err);
 int engine_sync(Engine* e, std::string& err);
-// Times one RK stage for every flux choice on the resident cases (state
-// restored afterwards) and keeps the fastest.  Returns the chosen
-// (variant, nseg) through the pointers.
+// FP64: selects the pushing flux kernel.  Mixed: times one RK stage for every
+// number of runs per cube on the resident cases (state restored afterwards)
+// and keeps the fastest.  Returns the chosen (variant, nseg) through the
+// pointers.
 int engine_autotune(Engine* e, int* variant, int* nseg, std::string& err);
 // Tunes only when no choice was made yet, or (mixed path, choice not pinned
 // with set_flux) when the pool's size class has changed since the last tuning.

@@ -8,6 +8,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace bcm {
 
@@ -180,6 +181,37 @@ __device__ inline void copy_bc_regions(const T* __restrict__ Uin, T* __restrict_
   }
 }
 
+// Sums eight doubles over the 64 lanes of a wave in a fixed order; every lane
+// returns the total of x[lane >> 3].  Halving the values kept at each exchange
+// (lane halves, rows of 16, halves of a row) takes 10 additions where eight
+// separate wave sums would take 48.
+__device__ inline double wave_sum8(double (&x)[8]) {
+  auto both = [](double a, double b, auto swap) {
+    const auto lo = swap((unsigned)__double2loint(a), (unsigned)__double2loint(b));
+    const auto hi = swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b));
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+  };
+  auto half = [](unsigned a, unsigned b) { return __builtin_amdgcn_permlane32_swap(a, b, false, false); };
+  auto row = [](unsigned a, unsigned b) { return __builtin_amdgcn_permlane16_swap(a, b, false, false); };
+#pragma unroll
+  for (int m = 0; m < 4; ++m) x[m] = both(x[m], x[m + 4], half);
+#pragma unroll
+  for (int m = 0; m < 2; ++m) x[m] = both(x[m], x[m + 2], row);
+  auto moved = [](double v, auto ctrl) {
+    constexpr int c = decltype(ctrl)::value;
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), c, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), c, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+  };
+  const bool up = threadIdx.x & 8;
+  double s = up ? x[1] : x[0];
+  s += moved(up ? x[0] : x[1], std::integral_constant<int, 0x128>());   // row_ror 8
+  s += moved(s, std::integral_constant<int, 0x141>());                  // row_half_mirror
+  s += moved(s, std::integral_constant<int, 0xB1>());                   // quad_perm 1,0,3,2
+  s += moved(s, std::integral_constant<int, 0x4E>());                   // quad_perm 2,3,0,1
+  return s;
+}
+
 // Launches cover pool cubes 1..ncube-1; "ncube" is one past the last cube in use.
 // The BC, IB fill and halo kernels exist for an FP64 inner iterate and for the
 // FP32 one of the mixed-precision path, which holds the deviation from the
@@ -227,18 +259,22 @@ void launch_flux_march(hipStream_t s, double* U, const double* U1, const double*
                        const int8_t* fws, const double* cube_size, double* Rku, double* Res,
                        int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int nseg,
                        int RK, int fuse, double* U1p1, double* U1p2, double* partials);
-// Marching kernel with the update written to Uout (one workgroup per cube):
-// every interior cell, and the two layers next to each face with an
+// Marching kernel with the update written to Uout, nseg (1, 2, 4, 8 or 16) runs
+// of 16/nseg planes per cube, one workgroup each, bitwise the same results for
+// every nseg: every interior cell, and the two layers next to each face with an
 // equal-size neighbour (halo[c]) into that neighbour's ghost layers in Uout.
 // With aux != 0 it writes Rku, Res, U1p1 (RK1) and U1p2 (RK2) bitwise as the
 // in-place fused kernel does (nothing reads them back during stages); at RK 3
-// one row of norm partials per cube either way.
+// PUSH_ROWS_PER_CUBE rows of 8 norm partials per cube (one per plane) either way.
 // Ghost regions the domain BCs wrote (cube_mask) are copied from Uin to Uout.
+constexpr int PUSH_ROWS_PER_CUBE = 16;
 void launch_flux_push(hipStream_t s, const double* Uin, double* Uout, const HaloSrc* halo,
                       const uint8_t* cube_mask, const double* U1, const double* U1q,
                       const int8_t* fws, const double* cube_size, double* Rku, double* Res,
                       int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int RK,
-                      double* U1p1, double* U1p2, double* partials, int aux);
+                      double* U1p1, double* U1p2, double* partials, int aux, int nseg);
+// Runs per cube of the pushing FP64 kernel for n resident cubes.
+int push_runs(int n);
 void launch_copy_d(hipStream_t s, const double* src, double* dst, size_t n);
 // Runs n threads of the shared-denominator division against a / b (four
 // quotients each); *mismatches receives the count of differing bit patterns.
@@ -248,8 +284,8 @@ void launch_update(hipStream_t s, int RK, double* U, double* U1p1, double* U1p2,
                    const double* Rku, const double* Res, const int8_t* fws, int ncube,
                    const int* cube_case, double* partials);
 // Norms er[0..7] of each case in cases[0..ncases): rows_per_cube partial rows
-// per cube (1 after the fused FP64 flux kernels, 16 after k_update and the
-// mixed flux kernel; several rows are first summed in row order into each
+// per cube (1 after the fused in-place FP64 kernel, 16 after k_update, the
+// pushing FP64 kernel and the mixed flux kernel; several rows are first summed in row order into each
 // cube's first row); case d writes er[d.slot*8 .. d.slot*8+7].
 void launch_reduce(hipStream_t s, double* partials, int rows_per_cube, const CaseDesc* cases,
                    int ncases, const DevPhys* phys, double* er);

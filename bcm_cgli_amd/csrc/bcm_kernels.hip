@@ -551,7 +551,8 @@ constexpr int NFACE = 17 * 16;      // faces of one axis in one i-plane
 // arithmetic is the reference's, in its order: results are bitwise those of
 // k_flux.
 //
-// PUSH: the update is not done in place but written to Uout, with every
+// PUSH (nseg runs of planes per cube, see push_runs): the update is not done
+// in place but written to Uout, with every
 // interior cell (non-fluid cells unchanged) and, for the two layers next to a
 // face with an equal-size neighbour, into that neighbour's ghost layers: the
 // face part of the post-update exchange.  It uses U for U1p1 (RK2) and U1p2
@@ -565,14 +566,24 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
     double* __restrict__ Rku, double* __restrict__ Res, PhysTab pt, double deltaT,
     double deltaTau, double e, int nseg, int RK, int fuse, double* __restrict__ U1p1,
     double* __restrict__ U1p2, double* __restrict__ partials, double* __restrict__ Uout,
-    const HaloSrc* __restrict__ halo, const uint8_t* __restrict__ cube_mask, int aux) {
+    const HaloSrc* __restrict__ halo, const uint8_t* __restrict__ cube_mask, int aux, int ncube) {
   __shared__ double pr[4][3 * PR_PLANE];   // u, v, w, T = P/(rho R) of 3 planes
   __shared__ double fy[5][NFACE];
   __shared__ double fz[6][NFACE];          // flux + face pressure average
   __shared__ __align__(16) double cpl[5 * 400];   // conserved values of plane i
   __shared__ int8_t fpl[400];              // flags of plane i
-  const int seg = blockIdx.x % nseg;
-  const int c = blockIdx.x / nseg + 1;
+  __shared__ double red[WG / 64][8];       // PUSH, RK 3: the waves' norm sums of a plane
+  int seg, c;
+  if constexpr (PUSH) {
+    // Workgroups go to the 8 XCDs in turn; the runs of one cube share planes
+    // and so go to one XCD's L2.
+    seg = blockIdx.x / 8 % nseg;
+    c = blockIdx.x / (8 * nseg) * 8 + blockIdx.x % 8 + 1;
+    if (c >= ncube) return;
+  } else {
+    seg = blockIdx.x % nseg;
+    c = blockIdx.x / nseg + 1;
+  }
   const int cc = pt.cube_case[c];
   if (cc < 0) return;
   const DevPhys ph = pt.phys[cc];
@@ -1091,6 +1102,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
 #pragma unroll
       for (int v = 0; v < 5; ++v) Rku[b + (size_t)v * PLANE] = out[v];
     }
+    double pn[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // PUSH: the cell's norm and force terms
     if (IF < 1) {
       const double px = pow2 ? -(dPxf - dPxb) * inv : -(dPxf - dPxb) / dx;
       const double pz = pow2 ? -(dPzf - dPzb) * inv : -(dPzf - dPzb) / dz;
@@ -1100,9 +1112,13 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
         Res[b] = r0;
         Res[b + PLANE] = r1;
       }
-      if ((fuse || PUSH) && RK == 3) {
+      if (fuse && RK == 3) {
         acc[5] += r0;
         acc[6] += r1;
+      }
+      if (PUSH) {
+        pn[5] = r0;
+        pn[6] = r1;
       }
     }
     if constexpr (PUSH) {
@@ -1138,11 +1154,11 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
           const double VV = un * un + vn * vn + wn * wn;
           const double P = (nv[4] - 0.5 * r * VV) * KM1;
           const double T = P / r;
-          acc[0] += (P - Po) * (P - Po);
-          acc[1] += (un - uo1) * (un - uo1);
-          acc[2] += (vn - vo1) * (vn - vo1);
-          acc[3] += (wn - wo1) * (wn - wo1);
-          acc[4] += (T - To) * (T - To);
+          pn[0] = (P - Po) * (P - Po);
+          pn[1] = (un - uo1) * (un - uo1);
+          pn[2] = (vn - vo1) * (vn - vo1);
+          pn[3] = (wn - wo1) * (wn - wo1);
+          pn[4] = (T - To) * (T - To);
         }
       }
       const HaloSrc hs = halo[c];
@@ -1160,16 +1176,27 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
         if (ny > 0) Uout[(size_t)ny * CUBE_STRIDE + (size_t)v * PLANE + oy] = nv[v];
         if (nz > 0) Uout[(size_t)nz * CUBE_STRIDE + (size_t)v * PLANE + oz] = nv[v];
       }
+      if (RK == 3) {
+        const double s = wave_sum8(pn);
+        if ((t & 7) == 0) red[t >> 6][(t >> 3) & 7] = s;
+      }
     }
     __syncthreads();
+    // One row of norm partials per plane, so the norms do not depend on the
+    // runs.  (The next plane's sums are written after two more barriers.)
+    if (PUSH && RK == 3 && t < 8) {
+      double s = red[0][t];
+#pragma unroll
+      for (int w = 1; w < WG / 64; ++w) s += red[w][t];
+      partials[((size_t)(c - 1) * PUSH_ROWS_PER_CUBE + (i - 2)) * 8 + t] = s;
+    }
   }
   if constexpr (PUSH) {
     const int bm = cube_mask[c];
-    if (bm) copy_bc_regions(U, Uout, c, bm, 0.0);
+    if (bm && seg == 0) copy_bc_regions(U, Uout, c, bm, 0.0);
   }
-  if (fuse || PUSH) {
-    if (!PUSH)
-      for (int ip = i1 - 3 < i0 ? i0 : i1 - 3; ip <= i1; ++ip) update_plane(ip);
+  if (!PUSH && fuse) {
+    for (int ip = i1 - 3 < i0 ? i0 : i1 - 3; ip <= i1; ++ip) update_plane(ip);
     if (RK == 3) {
       __shared__ double sh[(WG / 64) * 7];
       block_sum<7>(acc, sh);
@@ -2156,18 +2183,31 @@ void launch_flux_march(hipStream_t s, double* U, const double* U1, const double*
   if (ncube > 1)
     hipLaunchKernelGGL(k_flux_march<false>, dim3((ncube - 1) * nseg), dim3(WG), 0, s, U, U1, U1q,
                        fws, cube_size, Rku, Res, pt, deltaT, deltaTau, e, nseg, RK,
-                       fuse && nseg == 1, U1p1, U1p2, partials, nullptr, nullptr, nullptr, 1);
+                       fuse && nseg == 1, U1p1, U1p2, partials, nullptr, nullptr, nullptr, 1, ncube);
 }
 
 void launch_flux_push(hipStream_t s, const double* Uin, double* Uout, const HaloSrc* halo,
                       const uint8_t* cube_mask, const double* U1, const double* U1q,
                       const int8_t* fws, const double* cube_size, double* Rku, double* Res,
                       int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int RK,
-                      double* U1p1, double* U1p2, double* partials, int aux) {
+                      double* U1p1, double* U1p2, double* partials, int aux, int nseg) {
   if (ncube > 1)
-    hipLaunchKernelGGL(k_flux_march<true>, dim3(ncube - 1), dim3(WG), 0, s,
+    hipLaunchKernelGGL(k_flux_march<true>, dim3((ncube + 6) / 8 * 8 * nseg), dim3(WG), 0, s,
                        const_cast<double*>(Uin), U1, U1q, fws, cube_size, Rku, Res, pt, deltaT,
-                       deltaTau, e, 1, RK, 0, U1p1, U1p2, partials, Uout, halo, cube_mask, aux);
+                       deltaTau, e, nseg, RK, 0, U1p1, U1p2, partials, Uout, halo, cube_mask, aux,
+                       ncube);
+}
+
+// Runs per cube of the pushing kernel.  The chip holds 512 of its workgroups
+// (two per CU).  Below 128 cubes the most runs that fit at once are fastest
+// (8 cubes: 28 us in 16 runs, 224 in one; 125 cubes: 98 us in 4 runs, 253 in
+// one).  Above, a run's second x-face pass and ring fill (about one plane's
+// work) stand against the last wave of workgroups being nearly empty: 8 runs
+// to 320 cubes (216 cubes: 168 us, 176 in 4 runs, 262 in one), 4 to 800 (512
+// cubes: 362 us, 401 in one), then 2 (1,000 cubes: 681 us, 704 in one; 2,048:
+// 1,347, 1,351 in one).
+int push_runs(int n) {
+  return n <= 32 ? 16 : n <= 64 ? 8 : n <= 128 ? 4 : n <= 320 ? 8 : n <= 800 ? 4 : 2;
 }
 
 __global__ __launch_bounds__(WG) void k_copy_d(const double* __restrict__ src,

@@ -264,13 +264,14 @@ int bcm_engine_time_part(bcm_engine* e, int part, int RK, int reps, double* ms);
  * lets variant 1 with nseg 1 apply the RK update in the same kernel, in
  * place; fuse 2 (variant 1, nseg 1) writes the update and the face halos into
  * a second copy of the iterate in engine stages, which then open with the
- * edge passes and BCs instead of closing with the halo exchange.  All choices
- * give bitwise the same results.  Setting a choice disables tuning. */
+ * edge passes and BCs instead of closing with the halo exchange (that
+ * kernel's runs per cube follow the number of resident cubes).  All choices
+ * give bitwise the same state arrays.  Setting a choice disables tuning. */
 int bcm_engine_set_flux(bcm_engine* e, int variant, int nseg, int fuse);
-/* Times the flux choices (one whole RK stage each) on the resident cases,
- * restoring the state afterwards, and keeps the fastest; runs automatically
- * before the first bcm_engine_run otherwise.  out3 (may be null) receives
- * {variant, nseg, fuse}. */
+/* Selects the fastest flux choice, as the first bcm_engine_run does otherwise:
+ * FP64 variant 1, fuse 2; mixed the fastest nseg, each timed as one whole RK
+ * stage on the resident cases (the state is restored).  out3 (may be null)
+ * receives {variant, nseg, fuse}. */
 int bcm_engine_autotune(bcm_engine* e, int* out3);
 /* Ghost schedule statistics: entries, cubes with entries, maximum levels. */
 int bcm_engine_ghost_stats(bcm_engine* e, int* stats3);
