@@ -30,38 +30,55 @@ __device__ __forceinline__ int fidx(int c, int i, int j, int k) {
 // max(a,b) of the reference: (((a)>(b))?(a):(b)), NaN falls to b.
 __device__ __forceinline__ double rmax(double a, double b) { return (a > b) ? a : b; }
 
-// Several correctly rounded divisions by one denominator.  a / b compiles for
-// gfx950 to: the denominator scaled (div_scale), its reciprocal refined by
-// two Newton steps, then per quotient the numerator scaled, one product, one
-// correction and the special-case fixup (div_fmas, div_fixup).  DivBy keeps
-// the denominator's part once, scaled as for the numerator 1 (a zero
-// numerator there would give NaN; the quotient's fixup handles zeros);
-// div_sh runs the quotient's part.  The bits are those of a / b whenever the
-// denominator's scaling does not depend on the numerator: for finite
-// operands, unless an exponent difference reaches the scaling thresholds
-// (768) or an operand is subnormal, far outside the solver's values; the
-// self-test below compares against a / b.
+// Correctly rounded division and square root without the range scaling that
+// the compiler's own sequences carry for operands near the ends of the
+// exponent range.
+//
+// A denominator's part (div_by) is its reciprocal r, from the hardware
+// estimate r0 (relative error e0 below 2^-22) by one cubic step,
+// r0 (1 + e0 + e0^2): what is left, e0^3, lies far below the last bit.  A
+// quotient's part (div_sh) is the product a r, its exact remainder, one
+// correction and the fixup that sets zeros, infinities, NaN and signs.
+// Several quotients share one denominator's part.  The bits are those of a / b
+// unless a nonzero numerator is below 2^-969 in magnitude (its remainder is
+// then subnormal) or the denominator's reciprocal is out of range, states no
+// flow reaches; k_div_selftest compares.  Against the scaled form: one
+// instruction less per quotient (4), two less per denominator, no wait
+// between a flag's producer and its consumer (with root below, the pushing
+// flux kernel 1,345 -> 1,252 us on 2,048 cubes).
 struct DivBy {
-  double b, ds, r;   // denominator, as scaled, refined reciprocal of ds
+  double b, r;   // denominator and its reciprocal
 };
 __device__ __forceinline__ DivBy div_by(double b) {
-  bool f;
-  DivBy d;
-  d.b = b;
-  d.ds = __builtin_amdgcn_div_scale(1.0, b, false, &f);
-  const double r0 = __builtin_amdgcn_rcp(d.ds);
-  const double e0 = __builtin_fma(-d.ds, r0, 1.0);
-  const double r1 = __builtin_fma(r0, e0, r0);
-  const double e1 = __builtin_fma(-d.ds, r1, 1.0);
-  d.r = __builtin_fma(r1, e1, r1);
-  return d;
+  const double r0 = __builtin_amdgcn_rcp(b);
+  const double e0 = __builtin_fma(-b, r0, 1.0);
+  return DivBy{b, __builtin_fma(r0, __builtin_fma(e0, e0, e0), r0)};
 }
 __device__ __forceinline__ double div_sh(const DivBy& d, double a) {
-  bool f;
-  const double as = __builtin_amdgcn_div_scale(a, d.b, true, &f);
-  const double q = as * d.r;
-  const double rem = __builtin_fma(-d.ds, q, as);
-  return __builtin_amdgcn_div_fixup(__builtin_amdgcn_div_fmas(rem, d.r, q, f), d.b, a);
+  const double q = a * d.r;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d.b, q, a), d.r, q), d.b, a);
+}
+__device__ __forceinline__ double dvd(double a, double b) { return div_sh(div_by(b), a); }
+// div_by of a value all lanes share, kept in scalar registers.
+__device__ __forceinline__ DivBy div_by_uniform(double b) {
+  const double r = div_by(b).r;
+  return DivBy{b, __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(r)),
+                                   __builtin_amdgcn_readfirstlane(__double2loint(r)))};
+}
+// Square root by Goldschmidt's coupled iteration for sqrt(x) and 1/(2 sqrt(x))
+// from the hardware estimate of 1/sqrt(x), then two corrections by the exact
+// residual x - s^2 (Markstein, "Software division and square root using
+// Goldschmidt's algorithms", 2004).  Correctly rounded for x >= 2^-767; zero
+// and +infinity are returned as they are, a negative x gives NaN.
+__device__ __forceinline__ double root(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double s = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, s, 0.5);
+  s = __builtin_fma(s, r, s);
+  h = __builtin_fma(h, r, h);
+  s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+  s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+  return __builtin_amdgcn_class(x, 0x260) ? x : s;   // -0, +0, +infinity
 }
 
 // Full-state access to an inner iterate.  FP64 storage holds the state
@@ -92,7 +109,6 @@ template <> struct OffOf<float> { using type = RefOff; };
 template <int D>
 __device__ __forceinline__ void roe_flux(const double (&L)[5], const double (&R)[5], double e,
                                          double (&F)[5], double& dP) {
-  // Divisions sharing a denominator go through DivBy (the same bits).
   const double lr = L[0];
   const DivBy dl = div_by(lr);
   const double lq0 = div_sh(dl, L[1]), lq1 = div_sh(dl, L[2]), lq2 = div_sh(dl, L[3]);
@@ -109,8 +125,8 @@ __device__ __forceinline__ void roe_flux(const double (&L)[5], const double (&R)
   const double rC = div_sh(dr, KG * rP);
   const double rH = 0.5 * rVV + div_sh(dk, rC);
 
-  const double t5 = sqrt(lr), t6 = sqrt(rr), t4 = t5 + t6;
-  const double rho = sqrt(lr * rr);
+  const double t5 = root(lr), t6 = root(rr), t4 = t5 + t6;
+  const double rho = root(lr * rr);
   const DivBy d4 = div_by(t4);
   const double q0 = div_sh(d4, t5 * lq0 + t6 * rq0);
   const double q1 = div_sh(d4, t5 * lq1 + t6 * rq1);
@@ -124,8 +140,8 @@ __device__ __forceinline__ void roe_flux(const double (&L)[5], const double (&R)
   const double lun = D == 0 ? lq0 : (D == 1 ? lq1 : lq2);
   const double run = D == 0 ? rq0 : (D == 1 ? rq1 : rq2);
   const double temp = 0.5 * (1 + beta) * un;
-  const double S = 0.5 * sqrt(4 * beta * C + un * un * (1 - beta) * (1 - beta));
-  const double temp1 = div_sh(dC, (rP - lP) / rho / beta);
+  const double S = 0.5 * root(4 * beta * C + un * un * (1 - beta) * (1 - beta));
+  const double temp1 = div_sh(dC, dvd(dvd(rP - lP, rho), beta));
   const DivBy dS = div_by(S);
   const double tS = div_sh(dS, temp);
   const double temp2 = tS * (run - lun);
@@ -251,8 +267,8 @@ __device__ __forceinline__ void visc_face(const Prim (&q)[27], const Prim& me, d
   constexpr int o0 = D == 0 ? SIDE : 0, o1 = D == 1 ? SIDE : 0, o2 = D == 2 ? SIDE : 0;
   const Prim f = q[nslot(o0, o1, o2)];
   const double Tf = 0.5 * (me.T + f.T);
-  const double temp = Tf / T0;
-  const double mu = mu_L * temp * sqrt(temp) * (T0 + 110.) / (Tf + 110.);
+  const double temp = dvd(Tf, T0);
+  const double mu = dvd(mu_L * temp * root(temp) * (T0 + 110.), Tf + 110.);
   double g[3][4];
 #pragma unroll
   for (int t = 0; t < 3; ++t) {
@@ -595,9 +611,11 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
   const double dx = cube_size[c] / 16;
   const double dy = dx, dz = dx;
   const double inv = 1. / dx;
+  const double inv4 = 0.25 * inv;   // (x / 4) inv = x (inv / 4): the scaling by 1/4 is exact
   // x / 2^n equals x * 2^-n exactly: use the multiply when dx is a power of two.
   int ex;
   const bool pow2 = frexp(dx, &ex) == 0.5;
+  const DivBy ddx = div_by_uniform(dx), dT0 = div_by_uniform(ph.T0), d2t = div_by_uniform(2 * deltaT);
 
   // PUSH: the edge ghost cells the viscous stencil reads are not read from
   // memory (no edge pass runs between the stage's face updates and this
@@ -666,7 +684,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
     pr[0][slot * PR_PLANE + n] = u;
     pr[1][slot * PR_PLANE + n] = v;
     pr[2][slot * PR_PLANE + n] = w;
-    pr[3][slot * PR_PLANE + n] = P / (r * RG);
+    pr[3][slot * PR_PLANE + n] = dvd(P, r * RG);
   };
   // The whole 18x18 plane: the 68 cells beyond one per lane go to lanes
   // 188..255, most of which stage no part of the plane.
@@ -702,7 +720,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
     pr[0][slot * PR_PLANE + n] = u;
     pr[1][slot * PR_PLANE + n] = v;
     pr[2][slot * PR_PLANE + n] = w;
-    pr[3][slot * PR_PLANE + n] = P / (r * RG);
+    pr[3][slot * PR_PLANE + n] = dvd(P, r * RG);
   };
   fill_prims(i0 - 1);
   fill_prims(i0);
@@ -737,10 +755,11 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
 #pragma unroll
       for (int v = 0; v < 5; ++v) uo[v] = U[bu + (size_t)v * PLANE];
       const double ro = uo[0];
-      const double uo1 = uo[1] / ro, vo1 = uo[2] / ro, wo1 = uo[3] / ro;
+      const DivBy dro = div_by(ro);
+      const double uo1 = div_sh(dro, uo[1]), vo1 = div_sh(dro, uo[2]), wo1 = div_sh(dro, uo[3]);
       const double VVo = uo1 * uo1 + vo1 * vo1 + wo1 * wo1;
       const double Po = (uo[4] - 0.5 * ro * VVo) * KM1;
-      const double To = Po / ro;
+      const double To = div_sh(dro, Po);
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
         const size_t o = bu + (size_t)v * PLANE;
@@ -748,10 +767,11 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
         U[o] = uo[v];
       }
       const double r = uo[0];
-      const double un = uo[1] / r, vn = uo[2] / r, wn = uo[3] / r;
+      const DivBy dn = div_by(r);
+      const double un = div_sh(dn, uo[1]), vn = div_sh(dn, uo[2]), wn = div_sh(dn, uo[3]);
       const double VV = un * un + vn * vn + wn * wn;
       const double P = (uo[4] - 0.5 * r * VV) * KM1;
-      const double T = P / r;
+      const double T = div_sh(dn, P);
       acc[0] += (P - Po) * (P - Po);
       acc[1] += (un - uo1) * (un - uo1);
       acc[2] += (vn - vo1) * (vn - vo1);
@@ -962,7 +982,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
       for (int v = 0; v < 5; ++v) Rf[v] = -(Rx[v] * inv + Ry[v] * inv + Rz[v] * inv);
     } else {
 #pragma unroll
-      for (int v = 0; v < 5; ++v) Rf[v] = -(Rx[v] / dx + Ry[v] / dy + Rz[v] / dz);
+      for (int v = 0; v < 5; ++v) Rf[v] = -(div_sh(ddx, Rx[v]) + div_sh(ddx, Ry[v]) + div_sh(ddx, Rz[v]));
     }
 
     // ---- viscous (Flux.cpp:1722-2279) from the primitive ring ----
@@ -976,13 +996,16 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
       return pr[m][((i + a) % 3) * PR_PLANE + (j + bb - 1) * 18 + (k + cc - 1)];
     };
     Prim me;
+    const DivBy drho = div_by(rho);
+    double PoR;   // P / rho
     me.u = Q(0, 0, 0, 0);
     me.v = Q(0, 0, 0, 1);
     me.w = Q(0, 0, 0, 2);
     {
       const double VV = me.u * me.u + me.v * me.v + me.w * me.w;
       const double P = (u[4] - 0.5 * rho * VV) * KM1;
-      me.T = P / rho / RG;
+      PoR = div_sh(drho, P);
+      me.T = dvd(PoR, RG);
     }
     double vF[5] = {0, 0, 0, 0, 0};
     double Lb[5], Lf[5];
@@ -997,8 +1020,8 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
         f.w = Q(o0, o1, o2, 2);
         f.T = Q(o0, o1, o2, 3);
         const double Tf = 0.5 * (me.T + f.T);
-        const double temp = Tf / ph.T0;
-        const double mu = ph.mu_L * temp * sqrt(temp) * (ph.T0 + 110.) / (Tf + 110.);
+        const double temp = div_sh(dT0, Tf);
+        const double mu = dvd(ph.mu_L * temp * root(temp) * (ph.T0 + 110.), Tf + 110.);
         double g[3][4];
 #pragma unroll
         for (int tt = 0; tt < 3; ++tt) {
@@ -1019,7 +1042,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
 #pragma unroll
             for (int m = 0; m < 4; ++m)
               g[tt][m] = (Q(p0, p1, p2, m) + Q(p0 + o0, p1 + o1, p2 + o2, m) - Q(-p0, -p1, -p2, m) -
-                          Q(-p0 + o0, -p1 + o1, -p2 + o2, m)) / 4 * inv;
+                          Q(-p0 + o0, -p1 + o1, -p2 + o2, m)) * inv4;
           }
         }
         const double uf = 0.5 * (me.u + f.u), vf = 0.5 * (me.v + f.v), wf = 0.5 * (me.w + f.w);
@@ -1032,7 +1055,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
         L[1] = sg[0];
         L[2] = sg[1];
         L[3] = sg[2];
-        L[4] = uf * sg[0] + vf * sg[1] + wf * sg[2] + mu * CVG * KG * g[d][3] / (PRG);
+        L[4] = uf * sg[0] + vf * sg[1] + wf * sg[2] + dvd(mu * CVG * KG * g[d][3], PRG);
       }
 #pragma unroll
       for (int v = 1; v < 5; ++v) {
@@ -1043,7 +1066,6 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
 
     // ---- residual with the dual-time source, preconditioner, increment ----
     double Rk[5];
-    const DivBy d2t = div_by(2 * deltaT);
     {
       const double uu0 = tu1[0], uq0 = tuq[0];
       Rk[0] = div_sh(d2t, -(3 * u[0] - 4 * uu0 + uq0)) + Rf[0];
@@ -1059,41 +1081,41 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
       const double U_ = me.u, V_ = me.v, W_ = me.w;
       const double VV = U_ * U_ + V_ * V_ + W_ * W_;
       const double P = (u[4] - 0.5 * rho * VV) * KM1;
-      const double C = KG * P / rho;
-      const double T = P / rho;
-      const double H = 0.5 * VV + C / KM1;
-      const double beta = rmax(VV / C, e);
+      const double C = div_sh(drho, KG * P);
+      const double T = PoR;
+      const double H = 0.5 * VV + dvd(C, KM1);
+      const double beta = rmax(dvd(VV, C), e);
       const double temp = KG * T * (2 * deltaT + 3 * deltaTau) * (2 * deltaT + 3 * beta * deltaTau);
       const double temp2 = KM1 * (beta - 1) * deltaT * deltaT;
       const double temp3 = H - H * KG - VV + KG * (T + VV);
+      // The reference's entries; those that differ in sign only (scaling by 4
+      // and negation are exact) are formed once.
       const DivBy dT = div_by(temp);
+      const double U4 = 4 * U_, V4 = 4 * V_, W4 = 4 * W_, H4 = 4 * H;
       const double d11 = div_sh(dT, (2 * deltaT * (-2 * (-KM1 * (H - VV) - temp3 * beta) * deltaT + 3 * KG * T * beta * deltaTau)));
-      const double d12 = div_sh(dT, (-4 * U_ * temp2));
-      const double d13 = div_sh(dT, (-4 * V_ * temp2));
-      const double d14 = div_sh(dT, (-4 * W_ * temp2));
       const double d15 = div_sh(dT, (4 * temp2));
-      out[0] = deltaTau * (d11 * Rk[0] + d12 * Rk[1] + d13 * Rk[2] + d14 * Rk[3] + d15 * Rk[4]);
-      const double d21 = div_sh(dT, (4 * U_ * temp3 * (beta - 1) * deltaT * deltaT));
+      const double d25 = div_sh(dT, (U4 * temp2));   // -d12
+      const double d35 = div_sh(dT, (V4 * temp2));   // -d13
+      const double d45 = div_sh(dT, (W4 * temp2));   // -d14
+      out[0] = deltaTau * (d11 * Rk[0] - d25 * Rk[1] - d35 * Rk[2] - d45 * Rk[3] + d15 * Rk[4]);
+      const double d21 = div_sh(dT, (U4 * temp3 * (beta - 1) * deltaT * deltaT));
       const double d22 = div_sh(dT, (2 * deltaT * (2 * KG * (T - U_ * U_ * (beta - 1)) * deltaT + 2 * U_ * U_ * (beta - 1) * deltaT + 3 * KG * T * beta * deltaTau)));
-      const double d23 = div_sh(dT, (-4 * U_ * V_ * temp2));
-      const double d24 = div_sh(dT, (-4 * U_ * W_ * temp2));
-      const double d25 = div_sh(dT, (4 * U_ * temp2));
-      out[1] = deltaTau * (d21 * Rk[0] + d22 * Rk[1] + d23 * Rk[2] + d24 * Rk[3] + d25 * Rk[4]);
-      const double d31 = div_sh(dT, (4 * V_ * temp3 * (beta - 1) * deltaT * deltaT));
+      const double m23 = div_sh(dT, (U4 * V_ * temp2));
+      const double m24 = div_sh(dT, (U4 * W_ * temp2));
+      out[1] = deltaTau * (d21 * Rk[0] + d22 * Rk[1] - m23 * Rk[2] - m24 * Rk[3] + d25 * Rk[4]);
+      const double d31 = div_sh(dT, (V4 * temp3 * (beta - 1) * deltaT * deltaT));
       const double d33 = div_sh(dT, (2 * deltaT * (2 * KG * (T - V_ * V_ * (beta - 1)) * deltaT + 2 * V_ * V_ * (beta - 1) * deltaT + 3 * KG * T * beta * deltaTau)));
-      const double d34 = div_sh(dT, (-4 * V_ * W_ * temp2));
-      const double d35 = div_sh(dT, (4 * V_ * temp2));
-      out[2] = deltaTau * (d31 * Rk[0] + d23 * Rk[1] + d33 * Rk[2] + d34 * Rk[3] + d35 * Rk[4]);
-      const double d41 = div_sh(dT, (4 * W_ * temp3 * (beta - 1) * deltaT * deltaT));
+      const double m34 = div_sh(dT, (V4 * W_ * temp2));
+      out[2] = deltaTau * (d31 * Rk[0] - m23 * Rk[1] + d33 * Rk[2] - m34 * Rk[3] + d35 * Rk[4]);
+      const double d41 = div_sh(dT, (W4 * temp3 * (beta - 1) * deltaT * deltaT));
       const double d44 = div_sh(dT, (2 * deltaT * (2 * KG * (T - W_ * W_ * (beta - 1)) * deltaT + 2 * W_ * W_ * (beta - 1) * deltaT + 3 * KG * T * beta * deltaTau)));
-      const double d45 = div_sh(dT, (4 * W_ * temp2));
-      out[3] = deltaTau * (d41 * Rk[0] + d24 * Rk[1] + d34 * Rk[2] + d44 * Rk[3] + d45 * Rk[4]);
-      const double d51 = div_sh(dT, (4 * H * temp3 * (beta - 1) * deltaT * deltaT));
-      const double d52 = div_sh(dT, (-4 * H * U_ * temp2));
-      const double d53 = div_sh(dT, (-4 * H * V_ * temp2));
-      const double d54 = div_sh(dT, (-4 * H * W_ * temp2));
+      out[3] = deltaTau * (d41 * Rk[0] - m24 * Rk[1] - m34 * Rk[2] + d44 * Rk[3] + d45 * Rk[4]);
+      const double d51 = div_sh(dT, (H4 * temp3 * (beta - 1) * deltaT * deltaT));
+      const double m52 = div_sh(dT, (H4 * U_ * temp2));
+      const double m53 = div_sh(dT, (H4 * V_ * temp2));
+      const double m54 = div_sh(dT, (H4 * W_ * temp2));
       const double d55 = div_sh(dT, (2 * deltaT * (2 * H * KM1 * (beta - 1) * deltaT + KG * T * (2 * deltaT + 3 * beta * deltaTau))));
-      out[4] = deltaTau * (d51 * Rk[0] + d52 * Rk[1] + d53 * Rk[2] + d54 * Rk[3] + d55 * Rk[4]);
+      out[4] = deltaTau * (d51 * Rk[0] - m52 * Rk[1] - m53 * Rk[2] - m54 * Rk[3] + d55 * Rk[4]);
     }
     // The pushing kernel reads none of Rku1, U1p1, U1p2 and Residual1 back;
     // it stores them only when asked (aux), which the engine does in the
@@ -1104,8 +1126,8 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
     }
     double pn[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // PUSH: the cell's norm and force terms
     if (IF < 1) {
-      const double px = pow2 ? -(dPxf - dPxb) * inv : -(dPxf - dPxb) / dx;
-      const double pz = pow2 ? -(dPzf - dPzb) * inv : -(dPzf - dPzb) / dz;
+      const double px = pow2 ? -(dPxf - dPxb) * inv : div_sh(ddx, -(dPxf - dPxb));
+      const double pz = pow2 ? -(dPzf - dPzb) * inv : div_sh(ddx, -(dPzf - dPzb));
       const double r0 = -(px + vF[1]) * dx * dy * dz;
       const double r1 = -(pz + vF[3]) * dx * dy * dz;
       if (!PUSH || aux) {
@@ -1142,18 +1164,17 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(
             if (aux) U1p2[b + (size_t)v * PLANE] = x;
           }
         } else {
-          const double ro = u[0];
-          const double uo1 = u[1] / ro, vo1 = u[2] / ro, wo1 = u[3] / ro;
-          const double VVo = uo1 * uo1 + vo1 * vo1 + wo1 * wo1;
-          const double Po = (u[4] - 0.5 * ro * VVo) * KM1;
-          const double To = Po / ro;
+          // The cell's primitives before the update are those the fluxes used.
+          const double uo1 = me.u, vo1 = me.v, wo1 = me.w, To = PoR;
+          const double Po = (u[4] - 0.5 * rho * (uo1 * uo1 + vo1 * vo1 + wo1 * wo1)) * KM1;
 #pragma unroll
           for (int v = 0; v < 5; ++v) nv[v] = 1.0 / 3.0 * u[v] + 2.0 / 3.0 * u[v] + 2.0 / 3.0 * out[v];
           const double r = nv[0];
-          const double un = nv[1] / r, vn = nv[2] / r, wn = nv[3] / r;
+          const DivBy dn = div_by(r);
+          const double un = div_sh(dn, nv[1]), vn = div_sh(dn, nv[2]), wn = div_sh(dn, nv[3]);
           const double VV = un * un + vn * vn + wn * wn;
           const double P = (nv[4] - 0.5 * r * VV) * KM1;
-          const double T = P / r;
+          const double T = div_sh(dn, P);
           pn[0] = (P - Po) * (P - Po);
           pn[1] = (un - uo1) * (un - uo1);
           pn[2] = (vn - vo1) * (vn - vo1);
@@ -2217,7 +2238,8 @@ __global__ __launch_bounds__(WG) void k_copy_d(const double* __restrict__ src,
 }
 
 namespace {
-// DivBy/div_sh against a / b: per thread one denominator and four numerators
+// DivBy/div_sh against a / b and root against sqrt: per thread one denominator
+// and four numerators
 // from a seeded hash (random signs, significands and exponents in
 // [-126, 126]; about one numerator in 16 is a signed zero).
 __device__ __forceinline__ unsigned long long mix64(unsigned long long x) {
@@ -2248,6 +2270,7 @@ __global__ __launch_bounds__(WG) void k_div_selftest(unsigned long long seed, in
 #pragma unroll
   for (int k = 0; k < 4; ++k)
     nb += __double_as_longlong(div_sh(d, a[k])) != __double_as_longlong(a[k] / b);
+  nb += __double_as_longlong(root(fabs(a[0]))) != __double_as_longlong(sqrt(fabs(a[0])));
   if (nb) atomicAdd(bad, nb);
 }
 }  // namespace
