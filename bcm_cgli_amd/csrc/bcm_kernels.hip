@@ -9,77 +9,11 @@
 #include <math.h>
 #include <type_traits>
 
+#include "bcm_fp64.h"
 #include "bcm_kernels.h"
 
 namespace bcm {
 namespace {
-
-constexpr double KG = 1.4;          // K
-constexpr double KM1 = 1.4 - 1;     // (K-1), folded exactly as the reference folds it
-constexpr double RG = 287.0;        // R
-constexpr double CVG = 717.5;       // Cv
-constexpr double PRG = 0.72;        // Pr_L
-constexpr int WG = 256;
-
-__device__ __forceinline__ size_t sidx(int c, int v, int i, int j, int k) {
-  return (size_t)c * CUBE_STRIDE + (size_t)v * PLANE + i * 400 + j * 20 + k;
-}
-__device__ __forceinline__ int fidx(int c, int i, int j, int k) {
-  return c * PLANE + i * 400 + j * 20 + k;
-}
-// max(a,b) of the reference: (((a)>(b))?(a):(b)), NaN falls to b.
-__device__ __forceinline__ double rmax(double a, double b) { return (a > b) ? a : b; }
-
-// Correctly rounded division and square root without the range scaling that
-// the compiler's own sequences carry for operands near the ends of the
-// exponent range.
-//
-// A denominator's part (div_by) is its reciprocal r, from the hardware
-// estimate r0 (relative error e0 below 2^-22) by one cubic step,
-// r0 (1 + e0 + e0^2): what is left, e0^3, lies far below the last bit.  A
-// quotient's part (div_sh) is the product a r, its exact remainder, one
-// correction and the fixup that sets zeros, infinities, NaN and signs.
-// Several quotients share one denominator's part.  The bits are those of a / b
-// unless a nonzero numerator is below 2^-969 in magnitude (its remainder is
-// then subnormal) or the denominator's reciprocal is out of range, states no
-// flow reaches; k_div_selftest compares.  Against the scaled form: one
-// instruction less per quotient (4), two less per denominator, no wait
-// between a flag's producer and its consumer (with root below, the pushing
-// flux kernel 1,345 -> 1,252 us on 2,048 cubes).
-struct DivBy {
-  double b, r;   // denominator and its reciprocal
-};
-__device__ __forceinline__ DivBy div_by(double b) {
-  const double r0 = __builtin_amdgcn_rcp(b);
-  const double e0 = __builtin_fma(-b, r0, 1.0);
-  return DivBy{b, __builtin_fma(r0, __builtin_fma(e0, e0, e0), r0)};
-}
-__device__ __forceinline__ double div_sh(const DivBy& d, double a) {
-  const double q = a * d.r;
-  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d.b, q, a), d.r, q), d.b, a);
-}
-__device__ __forceinline__ double dvd(double a, double b) { return div_sh(div_by(b), a); }
-// div_by of a value all lanes share, kept in scalar registers.
-__device__ __forceinline__ DivBy div_by_uniform(double b) {
-  const double r = div_by(b).r;
-  return DivBy{b, __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(r)),
-                                   __builtin_amdgcn_readfirstlane(__double2loint(r)))};
-}
-// Square root by Goldschmidt's coupled iteration for sqrt(x) and 1/(2 sqrt(x))
-// from the hardware estimate of 1/sqrt(x), then two corrections by the exact
-// residual x - s^2 (Markstein, "Software division and square root using
-// Goldschmidt's algorithms", 2004).  Correctly rounded for x >= 2^-767; zero
-// and +infinity are returned as they are, a negative x gives NaN.
-__device__ __forceinline__ double root(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  double s = x * y, h = 0.5 * y;
-  const double r = __builtin_fma(-h, s, 0.5);
-  s = __builtin_fma(s, r, s);
-  h = __builtin_fma(h, r, h);
-  s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
-  s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
-  return __builtin_amdgcn_class(x, 0x260) ? x : s;   // -0, +0, +infinity
-}
 
 // Full-state access to an inner iterate.  FP64 storage holds the state
 // itself; FP32 storage holds its deviation from the case's reference state.
@@ -102,73 +36,6 @@ struct RefOff {
 template <typename T> struct OffOf;
 template <> struct OffOf<double> { using type = NoOff; };
 template <> struct OffOf<float> { using type = RefOff; };
-
-// ---------------------------------------------------------------------------
-// Preconditioned Roe-type flux at one face (Flux.cpp:611-797; X :1061-1247,
-// Y :1520-1695).  D is the face-normal axis.
-template <int D>
-__device__ __forceinline__ void roe_flux(const double (&L)[5], const double (&R)[5], double e,
-                                         double (&F)[5], double& dP) {
-  const double lr = L[0];
-  const DivBy dl = div_by(lr);
-  const double lq0 = div_sh(dl, L[1]), lq1 = div_sh(dl, L[2]), lq2 = div_sh(dl, L[3]);
-  const double lVV = lq0 * lq0 + lq1 * lq1 + lq2 * lq2;
-  const double lP = (L[4] - 0.5 * lr * lVV) * KM1;
-  const double lC = div_sh(dl, KG * lP);
-  const DivBy dk = div_by(KM1);
-  const double lH = 0.5 * lVV + div_sh(dk, lC);
-  const double rr = R[0];
-  const DivBy dr = div_by(rr);
-  const double rq0 = div_sh(dr, R[1]), rq1 = div_sh(dr, R[2]), rq2 = div_sh(dr, R[3]);
-  const double rVV = rq0 * rq0 + rq1 * rq1 + rq2 * rq2;
-  const double rP = (R[4] - 0.5 * rr * rVV) * KM1;
-  const double rC = div_sh(dr, KG * rP);
-  const double rH = 0.5 * rVV + div_sh(dk, rC);
-
-  const double t5 = root(lr), t6 = root(rr), t4 = t5 + t6;
-  const double rho = root(lr * rr);
-  const DivBy d4 = div_by(t4);
-  const double q0 = div_sh(d4, t5 * lq0 + t6 * rq0);
-  const double q1 = div_sh(d4, t5 * lq1 + t6 * rq1);
-  const double q2 = div_sh(d4, t5 * lq2 + t6 * rq2);
-  const double VV = q0 * q0 + q1 * q1 + q2 * q2;
-  const double H = div_sh(d4, t5 * lH + t6 * rH);
-  const double C = (H - 0.5 * VV) * KM1;
-  const DivBy dC = div_by(C);
-  const double beta = rmax(div_sh(dC, VV), e);
-  const double un = D == 0 ? q0 : (D == 1 ? q1 : q2);
-  const double lun = D == 0 ? lq0 : (D == 1 ? lq1 : lq2);
-  const double run = D == 0 ? rq0 : (D == 1 ? rq1 : rq2);
-  const double temp = 0.5 * (1 + beta) * un;
-  const double S = 0.5 * root(4 * beta * C + un * un * (1 - beta) * (1 - beta));
-  const double temp1 = div_sh(dC, dvd(dvd(rP - lP, rho), beta));
-  const DivBy dS = div_by(S);
-  const double tS = div_sh(dS, temp);
-  const double temp2 = tS * (run - lun);
-  const double temp3 = div_sh(dS, 0.5 * (1 - beta) * un * temp);
-  const double an = fabs(un);
-  const double deltaU = (S - temp3 - beta * an) * temp1 + temp2;
-  const double deltaP = tS * (rP - lP) + (S - an + temp3) * rho * (run - lun);
-
-  // Dissipation and the averaged physical flux; Ep = 1 multiplies exactly.
-  const double fav0 = an * (R[0] - L[0]) + deltaU * rho;
-  double fav1 = an * (R[1] - L[1]) + deltaU * rho * q0;
-  double fav2 = an * (R[2] - L[2]) + deltaU * rho * q1;
-  double fav3 = an * (R[3] - L[3]) + deltaU * rho * q2;
-  if (D == 0) fav1 = fav1 + deltaP;
-  if (D == 1) fav2 = fav2 + deltaP;
-  if (D == 2) fav3 = fav3 + deltaP;
-  const double fav4 = an * (R[4] - L[4]) + deltaU * rho * H + deltaP * un;
-  F[0] = 0.5 * ((lr * lun + rr * run) - fav0);
-  F[1] = D == 0 ? 0.5 * ((lr * lq0 * lq0 + lP + rr * rq0 * rq0 + rP) - fav1)
-                : 0.5 * ((lr * lq0 * lun + rr * rq0 * run) - fav1);
-  F[2] = D == 1 ? 0.5 * ((lr * lq1 * lq1 + lP + rr * rq1 * rq1 + rP) - fav2)
-                : 0.5 * ((lr * lq1 * lun + rr * rq1 * run) - fav2);
-  F[3] = D == 2 ? 0.5 * ((lr * lq2 * lq2 + lP + rr * rq2 * rq2 + rP) - fav3)
-                : 0.5 * ((lr * lq2 * lun + rr * rq2 * run) - fav3);
-  F[4] = 0.5 * ((lun * (3.5 * lP + 0.5 * lr * lVV) + run * (3.5 * rP + 0.5 * rr * rVV)) - fav4);
-  dP = 0.5 * (lP + rP);
-}
 
 // Inviscid flux difference of one cell along axis D (Flux.cpp:367-806 for Z):
 // upwind-biased face states of 5th, 3rd or 1st order depending on the cell
@@ -238,9 +105,6 @@ __device__ __forceinline__ void axis_flux(const double* __restrict__ U,
   for (int v = 0; v < 5; ++v) Rf[v] = Ff[v] - Fb[v];
 }
 
-struct Prim {
-  double u, v, w, T;
-};
 
 // Neighbour primitives as the viscous block computes them (T = P/(rho*R)).
 __device__ __forceinline__ Prim nb_prim(const double* __restrict__ U, size_t b) {
@@ -442,789 +306,6 @@ __global__ __launch_bounds__(WG) void k_flux(const double* __restrict__ U,
   if (IF < 1) {
     Res[b] = -(-(dPxf - dPxb) / dx + vF[1]) * dx * dy * dz;
     Res[b + PLANE] = -(-(dPzf - dPzb) / dz + vF[3]) * dx * dy * dz;
-  }
-}
-
-// Block sum of NS doubles per lane in a fixed tree order; lane 0 returns the totals.
-template <int NS>
-__device__ __forceinline__ void block_sum(double (&x)[NS], double* sh) {
-#pragma unroll
-  for (int m = 0; m < NS; ++m)
-    for (int off = 32; off > 0; off >>= 1) x[m] += __shfl_down(x[m], off, 64);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0)
-#pragma unroll
-    for (int m = 0; m < NS; ++m) sh[wave * NS + m] = x[m];
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int nw = blockDim.x >> 6;
-#pragma unroll
-    for (int m = 0; m < NS; ++m) {
-      double s = sh[m];
-      for (int w = 1; w < nw; ++w) s += sh[w * NS + m];
-      x[m] = s;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Face-based formulation of the same flux (used by k_flux_march).
-//
-// The states at the face between cells p and p+1 depend only on the
-// reconstruction order and on the six cells p-2..p+3: the reference's
-// backward-face formulas of cell p+1 and forward-face formulas of cell p are
-// the same expressions (Flux.cpp:499-562).  Only the order choice differs
-// between the two views, so one evaluation serves both cells whenever their
-// orders agree, with bitwise the same result.
-
-// Order of face p+1/2 as cell p sees it (forward face, Flux.cpp:497,533).
-__device__ __forceinline__ int order_fwd(int p, int fm1, int fp1, int fp2) {
-  if (fp1 == 1 && fm1 == 1) return (p == 17 || fp2 != 1) ? 3 : 5;
-  return 1;
-}
-// Order of face q-1/2 as cell q sees it (backward face, Flux.cpp:497,499).
-__device__ __forceinline__ int order_bwd(int q, int fm2, int fm1, int fp1) {
-  if (fp1 == 1 && fm1 == 1) return (q == 2 || fm2 != 1) ? 3 : 5;
-  return 1;
-}
-
-// Flux through the face between p and p+1 along axis D.  b indexes cell p
-// (variable 0) in an array whose variables are VS apart (PLANE in memory, one
-// 20x20 plane in LDS); only the cells the order needs are loaded.
-template <int D, int VS = PLANE>
-__device__ __forceinline__ void face_flux(const double* __restrict__ U, size_t b, int order,
-                                          double e, double (&F)[5], double& dP) {
-  constexpr int st = D == 0 ? 400 : (D == 1 ? 20 : 1);
-  const double c6 = 1. / 6, c60 = 1. / 60;
-  double L[5], R[5];
-  if (order == 5) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      const double* q = U + b + (size_t)v * VS;
-      const double s0 = q[-2 * st], s1 = q[-st], s2 = q[0], s3 = q[st], s4 = q[2 * st], s5 = q[3 * st];
-      L[v] = c60 * (2 * s0 - 13 * s1 + 47 * s2 + 27 * s3 - 3 * s4);
-      R[v] = c60 * (-3 * s1 + 27 * s2 + 47 * s3 - 13 * s4 + 2 * s5);
-    }
-  } else if (order == 3) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      const double* q = U + b + (size_t)v * VS;
-      const double s1 = q[-st], s2 = q[0], s3 = q[st], s4 = q[2 * st];
-      L[v] = c6 * (-s1 + 5 * s2 + 2 * s3);
-      R[v] = c6 * (2 * s2 + 5 * s3 - s4);
-    }
-  } else {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      const double* q = U + b + (size_t)v * VS;
-      L[v] = q[0];
-      R[v] = q[st];
-    }
-  }
-  roe_flux<D>(L, R, e, F, dP);
-}
-
-// face_flux<D> on cells already loaded: s[m][v] is variable v of cell
-// p-2+m.  The same expressions, so the same bits.
-template <int D>
-__device__ __forceinline__ void face_flux_v(const double (&s)[6][5], int order, double e,
-                                            double (&F)[5], double& dP) {
-  const double c6 = 1. / 6, c60 = 1. / 60;
-  double L[5], R[5];
-  if (order == 5) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      L[v] = c60 * (2 * s[0][v] - 13 * s[1][v] + 47 * s[2][v] + 27 * s[3][v] - 3 * s[4][v]);
-      R[v] = c60 * (-3 * s[1][v] + 27 * s[2][v] + 47 * s[3][v] - 13 * s[4][v] + 2 * s[5][v]);
-    }
-  } else if (order == 3) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      L[v] = c6 * (-s[1][v] + 5 * s[2][v] + 2 * s[3][v]);
-      R[v] = c6 * (2 * s[2][v] + 5 * s[3][v] - s[4][v]);
-    }
-  } else {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      L[v] = s[2][v];
-      R[v] = s[3][v];
-    }
-  }
-  roe_flux<D>(L, R, e, F, dP);
-}
-
-// LDS layout of k_flux_march.
-constexpr int PR_PLANE = 18 * 18;   // primitives of j,k in [1,18]
-constexpr int NFACE = 17 * 16;      // faces of one axis in one i-plane
-
-// Flux, residual and stage increment with the work of one cube (or one
-// segment of its i-range) per workgroup, marching along i.  Per plane:
-// primitives of the next plane go into a 3-plane LDS ring (each computed once
-// instead of once per neighbour); the 272 y-faces and 272 z-faces of the plane
-// are evaluated once each into LDS; the x-face i+1/2 is carried in registers to
-// the next plane.  A cell whose backward-face order differs from its
-// neighbour's forward-face order evaluates its own backward face.  All
-// arithmetic is the reference's, in its order: results are bitwise those of
-// k_flux.
-//
-// PUSH (nseg runs of planes per cube, see push_runs): the update is not done
-// in place but written to Uout, with every
-// interior cell (non-fluid cells unchanged) and, for the two layers next to a
-// face with an equal-size neighbour, into that neighbour's ghost layers: the
-// face part of the post-update exchange.  It uses U for U1p1 (RK2) and U1p2
-// (RK3): those equal U1_ bitwise at fluid cells during a stage sequence,
-// since only ghost and non-fluid cells change between stages; both are still
-// written as the reference writes them.
-template <bool PUSH>
-__global__ __launch_bounds__(WG, 2) void k_flux_march(
-    double* __restrict__ U, const double* __restrict__ U1, const double* __restrict__ U1q,
-    const int8_t* __restrict__ fws, const double* __restrict__ cube_size,
-    double* __restrict__ Rku, double* __restrict__ Res, PhysTab pt, double deltaT,
-    double deltaTau, double e, int nseg, int RK, int fuse, double* __restrict__ U1p1,
-    double* __restrict__ U1p2, double* __restrict__ partials, double* __restrict__ Uout,
-    const HaloSrc* __restrict__ halo, const uint8_t* __restrict__ cube_mask, int aux, int ncube) {
-  __shared__ double pr[4][3 * PR_PLANE];   // u, v, w, T = P/(rho R) of 3 planes
-  __shared__ double fy[5][NFACE];
-  __shared__ double fz[6][NFACE];          // flux + face pressure average
-  __shared__ __align__(16) double cpl[5 * 400];   // conserved values of plane i
-  __shared__ int8_t fpl[400];              // flags of plane i
-  __shared__ double red[WG / 64][8];       // PUSH, RK 3: the waves' norm sums of a plane
-  int seg, c;
-  if constexpr (PUSH) {
-    // Workgroups go to the 8 XCDs in turn; the runs of one cube share planes
-    // and so go to one XCD's L2.
-    seg = blockIdx.x / 8 % nseg;
-    c = blockIdx.x / (8 * nseg) * 8 + blockIdx.x % 8 + 1;
-    if (c >= ncube) return;
-  } else {
-    seg = blockIdx.x % nseg;
-    c = blockIdx.x / nseg + 1;
-  }
-  const int cc = pt.cube_case[c];
-  if (cc < 0) return;
-  const DevPhys ph = pt.phys[cc];
-  const int len = 16 / nseg;
-  const int i0 = 2 + seg * len, i1 = i0 + len - 1;
-  // t, j and k are re-formed at the top of every plane iteration (below).
-  int t = threadIdx.x;
-  int j = (t >> 4) + 2, k = (t & 15) + 2;
-  const double dx = cube_size[c] / 16;
-  const double dy = dx, dz = dx;
-  const double inv = 1. / dx;
-  const double inv4 = 0.25 * inv;   // (x / 4) inv = x (inv / 4): the scaling by 1/4 is exact
-  // x / 2^n equals x * 2^-n exactly: use the multiply when dx is a power of two.
-  int ex;
-  const bool pow2 = frexp(dx, &ex) == 0.5;
-  const DivBy ddx = div_by_uniform(dx), dT0 = div_by_uniform(ph.T0), d2t = div_by_uniform(2 * deltaT);
-
-  // PUSH: the edge ghost cells the viscous stencil reads are not read from
-  // memory (no edge pass runs between the stage's face updates and this
-  // kernel) but formed as the pre-flux exchange's edge passes would leave
-  // them, the mean of two face ghost cells.  In the ghost planes 1 and 18
-  // they are the border cells other than the cube corners, formed here (every
-  // other cell is the mean of itself and itself, which is exact).  In the
-  // other planes they are the four corners, read only by the viscous stencil
-  // of their own plane: they are formed from the staged plane during its face
-  // pass (corner_prims below).
-  // ZBC_IN_FLUX faces: the z-ghost cells (k = 0, 1 or 18, 19) of the
-  // interior planes are read as the z-BC sets them, from the cell k = 2 (w
-  // negated) or 17 of the same row.
-  const int zm = PUSH ? cube_mask[c] : 0;
-  const bool zlo = zm & ZBC_IN_FLUX, zhi = zm & (ZBC_IN_FLUX << 1);
-  auto zsrc = [&](int cell, bool& neg) {
-    neg = false;
-    if (!(zlo || zhi)) return cell;
-    const int kk = cell % 20;
-    if (zlo && kk < 2 && cell >= 800 && cell < 7200) {
-      neg = true;
-      return cell - kk + 2;
-    }
-    if (zhi && kk > 17 && cell >= 800 && cell < 7200) return cell - kk + 17;
-    return cell;
-  };
-  // Primitive cell n (j,k = n / 18 + 1, n % 18 + 1) of plane ip: its
-  // conserved values (fill_load), then u, v, w and T into the ring slot
-  // (fill_store).
-  auto fill_load = [&](int ip, int n, double (&q)[5]) {
-    const bool gplane = ip == 1 || ip == 18;
-    const int jj = n / 18 + 1, kk = n % 18 + 1;
-    if (PUSH && gplane) {
-      int ea = 0, eb = 0;
-      if (!edge_sources(ip, jj, kk, ea, eb)) ea = eb = ip * 400 + jj * 20 + kk;
-      bool na, nb;
-      ea = zsrc(ea, na);
-      eb = zsrc(eb, nb);
-      const size_t cb = (size_t)c * CUBE_STRIDE;
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        const double x = U[cb + (size_t)v * PLANE + ea], y = U[cb + (size_t)v * PLANE + eb];
-        q[v] = 0.5 * ((v == 3 && na ? -x : x) + (v == 3 && nb ? -y : y));
-      }
-    } else if (PUSH) {
-      bool na;
-      const int ea = zsrc(ip * 400 + jj * 20 + kk, na);
-      const size_t cb = (size_t)c * CUBE_STRIDE;
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        const double x = U[cb + (size_t)v * PLANE + ea];
-        q[v] = v == 3 && na ? -x : x;
-      }
-    } else {
-      const size_t o = sidx(c, 0, ip, jj, kk);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) q[v] = U[o + (size_t)v * PLANE];
-    }
-  };
-  auto fill_store = [&](int ip, int n, const double (&q)[5]) {
-    const int slot = ip % 3;
-    const double r = q[0];
-    const DivBy dq = div_by(r);
-    const double u = div_sh(dq, q[1]), v = div_sh(dq, q[2]), w = div_sh(dq, q[3]);
-    const double P = (q[4] - 0.5 * r * (u * u + v * v + w * w)) * KM1;
-    pr[0][slot * PR_PLANE + n] = u;
-    pr[1][slot * PR_PLANE + n] = v;
-    pr[2][slot * PR_PLANE + n] = w;
-    pr[3][slot * PR_PLANE + n] = dvd(P, r * RG);
-  };
-  // The whole 18x18 plane: the 68 cells beyond one per lane go to lanes
-  // 188..255, most of which stage no part of the plane.
-  auto fill_prims = [&](int ip) {
-#pragma unroll 1
-    for (int rd = 0; rd < 2; ++rd) {
-      const int n = rd == 0 ? t : WG + t - 188;
-      if (rd == 1 && t < 188) continue;
-      double q[5];
-      fill_load(ip, n, q);
-      fill_store(ip, n, q);
-    }
-  };
-  // PUSH: the four corner cells of interior plane ip, formed from the staged
-  // plane (cpl) and written over the primitive ring's corners by lanes that
-  // have one face fewer to evaluate in the face pass.
-  auto corner_prims = [&](int ip) {
-    const int q4 = t - (WG - 4);
-    if (q4 < 0) return;
-    const int jj = q4 & 2 ? 18 : 1, kk = q4 & 1 ? 18 : 1;
-    int ea, eb;
-    edge_sources(ip, jj, kk, ea, eb);
-    ea %= 400;
-    eb %= 400;
-    double q[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) q[v] = 0.5 * (cpl[v * 400 + ea] + cpl[v * 400 + eb]);
-    const double r = q[0];
-    const DivBy dq = div_by(r);
-    const double u = div_sh(dq, q[1]), v = div_sh(dq, q[2]), w = div_sh(dq, q[3]);
-    const double P = (q[4] - 0.5 * r * (u * u + v * v + w * w)) * KM1;
-    const int n = (jj - 1) * 18 + (kk - 1), slot = ip % 3;
-    pr[0][slot * PR_PLANE + n] = u;
-    pr[1][slot * PR_PLANE + n] = v;
-    pr[2][slot * PR_PLANE + n] = w;
-    pr[3][slot * PR_PLANE + n] = dvd(P, r * RG);
-  };
-  fill_prims(i0 - 1);
-  fill_prims(i0);
-
-  double cF[5], cdP = 0;  // x-face flux carried from the previous plane
-  int corder = -1;
-  // With one workgroup per cube (fuse), the RK update of a plane runs three
-  // planes behind the flux: no later plane's stencil reaches back that far,
-  // and no other workgroup reads this cube.  RK3 norms accumulate per lane.
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-  auto update_plane = [&](int ip) {
-    const size_t bu = sidx(c, 0, ip, j, k);
-    if (fws[fidx(c, ip, j, k)] != 1) return;
-    if (RK == 1) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        const size_t o = bu + (size_t)v * PLANE;
-        const double x = U[o] + Rku[o];
-        U[o] = x;
-        U1p1[o] = x;
-      }
-    } else if (RK == 2) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        const size_t o = bu + (size_t)v * PLANE;
-        const double x = 0.75 * U[o] + 0.25 * U1p1[o] + 0.25 * Rku[o];
-        U[o] = x;
-        U1p2[o] = x;
-      }
-    } else {
-      double uo[5];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) uo[v] = U[bu + (size_t)v * PLANE];
-      const double ro = uo[0];
-      const DivBy dro = div_by(ro);
-      const double uo1 = div_sh(dro, uo[1]), vo1 = div_sh(dro, uo[2]), wo1 = div_sh(dro, uo[3]);
-      const double VVo = uo1 * uo1 + vo1 * vo1 + wo1 * wo1;
-      const double Po = (uo[4] - 0.5 * ro * VVo) * KM1;
-      const double To = div_sh(dro, Po);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        const size_t o = bu + (size_t)v * PLANE;
-        uo[v] = 1.0 / 3.0 * uo[v] + 2.0 / 3.0 * U1p2[o] + 2.0 / 3.0 * Rku[o];
-        U[o] = uo[v];
-      }
-      const double r = uo[0];
-      const DivBy dn = div_by(r);
-      const double un = div_sh(dn, uo[1]), vn = div_sh(dn, uo[2]), wn = div_sh(dn, uo[3]);
-      const double VV = un * un + vn * vn + wn * wn;
-      const double P = (uo[4] - 0.5 * r * VV) * KM1;
-      const double T = div_sh(dn, P);
-      acc[0] += (P - Po) * (P - Po);
-      acc[1] += (un - uo1) * (un - uo1);
-      acc[2] += (vn - vo1) * (vn - vo1);
-      acc[3] += (wn - wo1) * (wn - wo1);
-      acc[4] += (T - To) * (T - To);
-    }
-  };
-#pragma unroll 1
-  for (int i = i0; i <= i1; ++i) {
-    // The lane index passes through an empty asm statement, so every
-    // per-lane quantity derived from it (LDS addresses, face and flag
-    // indices) is computed inside the iteration that uses it rather than
-    // hoisted before the loop and held across it: held, they exceed the
-    // register budget of two waves per SIMD and spill to scratch memory,
-    // whose reloads sit on the plane's critical path.
-    asm volatile("" : "+v"(t));
-    j = (t >> 4) + 2;
-    k = (t & 15) + 2;
-    // Plane i-4 was last read during iteration i-1 (backward-face stencil of
-    // plane i-1 reaches i-4); the barrier that ended that iteration makes its
-    // update safe now.
-    if (!PUSH && fuse && i - 4 >= i0) update_plane(i - 4);
-    {
-      // Plane i's conserved values go from memory straight into the staging
-      // buffer (global_load_lds: lane l of a wave writes the 16 bytes at the
-      // wave's base + 16 l), issued before the primitive fill so that the
-      // fill's loads and arithmetic run while they land; a wait on the
-      // vector memory counter before the barrier completes them.
-      if (t < 200) {
-        const size_t o = sidx(c, 0, i, 0, 0) + 2 * t;
-#pragma unroll
-        for (int v = 0; v < 5; ++v)
-          __builtin_amdgcn_global_load_lds(
-              (const __attribute__((address_space(1))) void*)(U + o + (size_t)v * PLANE),
-              (__attribute__((address_space(3))) void*)(cpl + v * 400 + 2 * (t & ~63)), 16, 0, 0);
-      }
-      // Primitives of plane i+1.  PUSH: the plane's four corners are never
-      // read from the fill (ghost planes are never the current plane, and an
-      // interior plane's corners come from corner_prims), so its 320 other
-      // cells fill the 256 lanes here and wave 3 in the face pass.
-#pragma unroll 1
-      for (int rd = 0; rd < (PUSH ? 1 : 2); ++rd) {
-        const int m = rd == 0 ? t : WG + t - 188;
-        if (rd == 1 && t < 188) continue;
-        const int n = PUSH ? m + 1 + (m >= 16) + (m >= 304) : m;
-        double q[5];
-        fill_load(i + 1, n, q);
-        fill_store(i + 1, n, q);
-      }
-      // ZBC_IN_FLUX faces: the staged plane's z-ghost cells (k = 0, 1 from
-      // k = 2 with w negated; k = 18, 19 from k = 17), 4 per row of 20, are
-      // loaded here and written over the copied plane once every wave's copy
-      // has landed (a barrier of their own).
-      double zq[5];
-      const int zrow = t >> 2, zk = t & 3;
-      const bool zfix = t < 80 && (zk < 2 ? zlo : zhi);
-      const int zdst = zrow * 20 + (zk < 2 ? zk : zk + 16), zs = zrow * 20 + (zk < 2 ? 2 : 17);
-      if (zfix) {
-        const size_t o = sidx(c, 0, i, 0, 0) + zs;
-#pragma unroll
-        for (int v = 0; v < 5; ++v) zq[v] = U[o + (size_t)v * PLANE];
-      }
-      if (t < 200) {
-        const int8_t* fr = fws + fidx(c, i, 0, 0) + 2 * t;
-        fpl[2 * t] = fr[0];
-        fpl[2 * t + 1] = fr[1];
-      }
-      if (zlo || zhi) {
-        __builtin_amdgcn_s_waitcnt(0xF70);   // vmcnt(0)
-        __syncthreads();
-        if (zfix) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) cpl[v * 400 + zdst] = v == 3 && zk < 2 ? -zq[v] : zq[v];
-        }
-      }
-      __builtin_amdgcn_s_waitcnt(0xF70);   // vmcnt(0)
-    }
-    __syncthreads();
-    // y-faces (face f = (p-1)*16 + kk-2 joins j = p and p+1 at k = kk) and
-    // z-faces (g = (jj-2)*17 + p-1 joins k = p and p+1 at j = jj) of plane i.
-    // Round 0: each lane the y-face above its cell; round 1: the z-face
-    // above it (every wave evaluates one face kind at a time); rounds 2 and
-    // 3: the 16 y-faces and 16 z-faces next to the first ghost layers
-    // (p = 1), on lanes of waves 0 and 1.
-    if (PUSH) corner_prims(i);
-#pragma unroll 1
-    for (int r = 0; r < 4; ++r) {
-      const bool bnd = r >= 2;
-      const int l0 = r == 2 ? 0 : 64;
-      if (bnd && (t < l0 || t >= l0 + 16)) continue;
-      if ((r & 1) == 0) {
-        const int p = bnd ? 1 : j, kk = bnd ? t - l0 + 2 : k;
-        const int f = (p - 1) * 16 + (kk - 2);
-        const int8_t* fb = fpl + p * 20 + kk;
-        const int o = p >= 2 ? order_fwd(p, fb[-20], fb[20], fb[40]) : order_bwd(2, fb[-20], fb[0], fb[40]);
-        double F[5], dP;
-        face_flux<1, 400>(cpl, p * 20 + kk, o, e, F, dP);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) fy[v][f] = F[v];
-      } else {
-        const int jj = bnd ? t - l0 + 2 : j, p = bnd ? 1 : k;
-        const int g = (jj - 2) * 17 + (p - 1);
-        const int8_t* fb = fpl + jj * 20 + p;
-        const int o = p >= 2 ? order_fwd(p, fb[-1], fb[1], fb[2]) : order_bwd(2, fb[-1], fb[0], fb[2]);
-        double F[5], dP;
-        face_flux<2, 400>(cpl, jj * 20 + p, o, e, F, dP);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) fz[v][g] = F[v];
-        fz[5][g] = dP;
-      }
-    }
-    // PUSH: the fill's second round (wave 3, which has no boundary faces)
-    // runs in the face pass; plane i+1's primitives are first read after
-    // the next barrier, and its ring slot was last read before the previous
-    // one.
-    if (PUSH && t >= 192) {
-      const int m = WG + t - 192;
-      const int n = m + 1 + (m >= 16) + (m >= 304);
-      double q[5];
-      fill_load(i + 1, n, q);
-      fill_store(i + 1, n, q);
-    }
-    // The x-stencil of the cell's forward face, planes i-2..i+3, and the
-    // flags it needs, loaded before the barrier so that they arrive while the
-    // workgroup gathers.  (Plane i+3 = 20 would lie beyond the cube; the last
-    // interior plane's forward face has order 3 or 1, which does not read
-    // it, so plane 19 stands in.)
-    const int8_t* fc = fws + fidx(c, i, j, k);
-    const int IF = fc[0];
-    const int fm2 = fc[-800], fm1 = fc[-400], fp1 = fc[400], fp2 = fc[800];
-    double xs[6][5];
-#pragma unroll
-    for (int m = 0; m < 6; ++m)
-#pragma unroll
-      for (int v = 0; v < 5; ++v) xs[m][v] = U[sidx(c, v, min(i - 2 + m, 19), j, k)];
-    __syncthreads();
-
-    const size_t b = sidx(c, 0, i, j, k);
-    // ---- inviscid, x: forward face computed, backward face carried ----
-    double Rx[5], Ry[5], Rz[5], dPxb, dPxf, dPzb, dPzf;
-    {
-      const int of = order_fwd(i, fm1, fp1, fp2);
-      double Ff[5];
-      face_flux_v<0>(xs, of, e, Ff, dPxf);
-      const int ob = order_bwd(i, fm2, fm1, fp1);
-      if (i != i0 && ob == corder) {
-        dPxb = cdP;
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Rx[v] = Ff[v] - cF[v];
-      } else {
-        double Fb[5];
-        face_flux<0>(U, b - 400, ob, e, Fb, dPxb);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Rx[v] = Ff[v] - Fb[v];
-      }
-#pragma unroll
-      for (int v = 0; v < 5; ++v) cF[v] = Ff[v];
-      cdP = dPxf;
-      corder = of;
-    }
-    // The cell's time levels, loaded here so that the y-, z- and viscous
-    // terms run while they arrive.
-    double tu1[5], tuq[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      tu1[v] = U1[b + (size_t)v * PLANE];
-      tuq[v] = U1q[b + (size_t)v * PLANE];
-    }
-    // ---- inviscid, y ----
-    {
-      const int8_t* fl = fpl + j * 20 + k;
-      const int fm2 = fl[-40], fm1 = fl[-20], fp1 = fl[20];
-      const int ff = (j - 1) * 16 + (k - 2), fbk = ff - 16;
-      const int ob = order_bwd(j, fm2, fm1, fp1);
-      const bool share = j == 2 || ob == order_fwd(j - 1, fm2, fl[0], fp1);
-      if (share) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Ry[v] = fy[v][ff] - fy[v][fbk];
-      } else {
-        double Fb[5], dPu;
-        face_flux<1, 400>(cpl, j * 20 + k - 20, ob, e, Fb, dPu);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Ry[v] = fy[v][ff] - Fb[v];
-      }
-    }
-    // ---- inviscid, z ----
-    {
-      const int8_t* fl = fpl + j * 20 + k;
-      const int fm2 = fl[-2], fm1 = fl[-1], fp1 = fl[1];
-      const int ff = (j - 2) * 17 + (k - 1), fbk = ff - 1;
-      const int ob = order_bwd(k, fm2, fm1, fp1);
-      const bool share = k == 2 || ob == order_fwd(k - 1, fm2, fl[0], fp1);
-      dPzf = fz[5][ff];
-      if (share) {
-        dPzb = fz[5][fbk];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Rz[v] = fz[v][ff] - fz[v][fbk];
-      } else {
-        double Fb[5];
-        face_flux<2, 400>(cpl, j * 20 + k - 1, ob, e, Fb, dPzb);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Rz[v] = fz[v][ff] - Fb[v];
-      }
-    }
-    double Rf[5];
-    if (pow2) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) Rf[v] = -(Rx[v] * inv + Ry[v] * inv + Rz[v] * inv);
-    } else {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) Rf[v] = -(div_sh(ddx, Rx[v]) + div_sh(ddx, Ry[v]) + div_sh(ddx, Rz[v]));
-    }
-
-    // ---- viscous (Flux.cpp:1722-2279) from the primitive ring ----
-    // The cell's conserved values from the staged plane (interior cells are
-    // staged as they are).
-    double u[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) u[v] = cpl[v * 400 + j * 20 + k];
-    const double rho = u[0];
-    auto Q = [&](int a, int bb, int cc, int m) -> double {
-      return pr[m][((i + a) % 3) * PR_PLANE + (j + bb - 1) * 18 + (k + cc - 1)];
-    };
-    Prim me;
-    const DivBy drho = div_by(rho);
-    double PoR;   // P / rho
-    me.u = Q(0, 0, 0, 0);
-    me.v = Q(0, 0, 0, 1);
-    me.w = Q(0, 0, 0, 2);
-    {
-      const double VV = me.u * me.u + me.v * me.v + me.w * me.w;
-      const double P = (u[4] - 0.5 * rho * VV) * KM1;
-      PoR = div_sh(drho, P);
-      me.T = dvd(PoR, RG);
-    }
-    double vF[5] = {0, 0, 0, 0, 0};
-    double Lb[5], Lf[5];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-#pragma unroll
-      for (int side = -1; side <= 1; side += 2) {
-        const int o0 = d == 0 ? side : 0, o1 = d == 1 ? side : 0, o2 = d == 2 ? side : 0;
-        Prim f;
-        f.u = Q(o0, o1, o2, 0);
-        f.v = Q(o0, o1, o2, 1);
-        f.w = Q(o0, o1, o2, 2);
-        f.T = Q(o0, o1, o2, 3);
-        const double Tf = 0.5 * (me.T + f.T);
-        const double temp = div_sh(dT0, Tf);
-        const double mu = dvd(ph.mu_L * temp * root(temp) * (ph.T0 + 110.), Tf + 110.);
-        double g[3][4];
-#pragma unroll
-        for (int tt = 0; tt < 3; ++tt) {
-          if (tt == d) {
-            if (side < 0) {
-              g[tt][0] = (me.u - f.u) * inv;
-              g[tt][1] = (me.v - f.v) * inv;
-              g[tt][2] = (me.w - f.w) * inv;
-              g[tt][3] = (me.T - f.T) * inv;
-            } else {
-              g[tt][0] = (f.u - me.u) * inv;
-              g[tt][1] = (f.v - me.v) * inv;
-              g[tt][2] = (f.w - me.w) * inv;
-              g[tt][3] = (f.T - me.T) * inv;
-            }
-          } else {
-            const int p0 = tt == 0, p1 = tt == 1, p2 = tt == 2;
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-              g[tt][m] = (Q(p0, p1, p2, m) + Q(p0 + o0, p1 + o1, p2 + o2, m) - Q(-p0, -p1, -p2, m) -
-                          Q(-p0 + o0, -p1 + o1, -p2 + o2, m)) * inv4;
-          }
-        }
-        const double uf = 0.5 * (me.u + f.u), vf = 0.5 * (me.v + f.v), wf = 0.5 * (me.w + f.w);
-        const double div = g[0][0] + g[1][1] + g[2][2];
-        double sg[3];
-#pragma unroll
-        for (int m = 0; m < 3; ++m)
-          sg[m] = (m == d) ? mu * (2 * g[d][d] - 2.0 / 3.0 * div) : mu * (g[m][d] + g[d][m]);
-        double* L = side < 0 ? Lb : Lf;
-        L[1] = sg[0];
-        L[2] = sg[1];
-        L[3] = sg[2];
-        L[4] = uf * sg[0] + vf * sg[1] + wf * sg[2] + dvd(mu * CVG * KG * g[d][3], PRG);
-      }
-#pragma unroll
-      for (int v = 1; v < 5; ++v) {
-        const double term = (Lf[v] - Lb[v]) * inv;
-        vF[v] = d == 0 ? term : vF[v] + term;
-      }
-    }
-
-    // ---- residual with the dual-time source, preconditioner, increment ----
-    double Rk[5];
-    {
-      const double uu0 = tu1[0], uq0 = tuq[0];
-      Rk[0] = div_sh(d2t, -(3 * u[0] - 4 * uu0 + uq0)) + Rf[0];
-    }
-#pragma unroll
-    for (int v = 1; v < 5; ++v) {
-      const double uu = tu1[v], uq = tuq[v];
-      const double Rp = div_sh(d2t, -(3 * u[v] - 4 * uu + uq));
-      Rk[v] = Rp + Rf[v] + vF[v];
-    }
-    double out[5] = {0, 0, 0, 0, 0};
-    if (IF == 1) {
-      const double U_ = me.u, V_ = me.v, W_ = me.w;
-      const double VV = U_ * U_ + V_ * V_ + W_ * W_;
-      const double P = (u[4] - 0.5 * rho * VV) * KM1;
-      const double C = div_sh(drho, KG * P);
-      const double T = PoR;
-      const double H = 0.5 * VV + dvd(C, KM1);
-      const double beta = rmax(dvd(VV, C), e);
-      const double temp = KG * T * (2 * deltaT + 3 * deltaTau) * (2 * deltaT + 3 * beta * deltaTau);
-      const double temp2 = KM1 * (beta - 1) * deltaT * deltaT;
-      const double temp3 = H - H * KG - VV + KG * (T + VV);
-      // The reference's entries; those that differ in sign only (scaling by 4
-      // and negation are exact) are formed once.
-      const DivBy dT = div_by(temp);
-      const double U4 = 4 * U_, V4 = 4 * V_, W4 = 4 * W_, H4 = 4 * H;
-      const double d11 = div_sh(dT, (2 * deltaT * (-2 * (-KM1 * (H - VV) - temp3 * beta) * deltaT + 3 * KG * T * beta * deltaTau)));
-      const double d15 = div_sh(dT, (4 * temp2));
-      const double d25 = div_sh(dT, (U4 * temp2));   // -d12
-      const double d35 = div_sh(dT, (V4 * temp2));   // -d13
-      const double d45 = div_sh(dT, (W4 * temp2));   // -d14
-      out[0] = deltaTau * (d11 * Rk[0] - d25 * Rk[1] - d35 * Rk[2] - d45 * Rk[3] + d15 * Rk[4]);
-      const double d21 = div_sh(dT, (U4 * temp3 * (beta - 1) * deltaT * deltaT));
-      const double d22 = div_sh(dT, (2 * deltaT * (2 * KG * (T - U_ * U_ * (beta - 1)) * deltaT + 2 * U_ * U_ * (beta - 1) * deltaT + 3 * KG * T * beta * deltaTau)));
-      const double m23 = div_sh(dT, (U4 * V_ * temp2));
-      const double m24 = div_sh(dT, (U4 * W_ * temp2));
-      out[1] = deltaTau * (d21 * Rk[0] + d22 * Rk[1] - m23 * Rk[2] - m24 * Rk[3] + d25 * Rk[4]);
-      const double d31 = div_sh(dT, (V4 * temp3 * (beta - 1) * deltaT * deltaT));
-      const double d33 = div_sh(dT, (2 * deltaT * (2 * KG * (T - V_ * V_ * (beta - 1)) * deltaT + 2 * V_ * V_ * (beta - 1) * deltaT + 3 * KG * T * beta * deltaTau)));
-      const double m34 = div_sh(dT, (V4 * W_ * temp2));
-      out[2] = deltaTau * (d31 * Rk[0] - m23 * Rk[1] + d33 * Rk[2] - m34 * Rk[3] + d35 * Rk[4]);
-      const double d41 = div_sh(dT, (W4 * temp3 * (beta - 1) * deltaT * deltaT));
-      const double d44 = div_sh(dT, (2 * deltaT * (2 * KG * (T - W_ * W_ * (beta - 1)) * deltaT + 2 * W_ * W_ * (beta - 1) * deltaT + 3 * KG * T * beta * deltaTau)));
-      out[3] = deltaTau * (d41 * Rk[0] - m24 * Rk[1] - m34 * Rk[2] + d44 * Rk[3] + d45 * Rk[4]);
-      const double d51 = div_sh(dT, (H4 * temp3 * (beta - 1) * deltaT * deltaT));
-      const double m52 = div_sh(dT, (H4 * U_ * temp2));
-      const double m53 = div_sh(dT, (H4 * V_ * temp2));
-      const double m54 = div_sh(dT, (H4 * W_ * temp2));
-      const double d55 = div_sh(dT, (2 * deltaT * (2 * H * KM1 * (beta - 1) * deltaT + KG * T * (2 * deltaT + 3 * beta * deltaTau))));
-      out[4] = deltaTau * (d51 * Rk[0] - m52 * Rk[1] - m53 * Rk[2] - m54 * Rk[3] + d55 * Rk[4]);
-    }
-    // The pushing kernel reads none of Rku1, U1p1, U1p2 and Residual1 back;
-    // it stores them only when asked (aux), which the engine does in the
-    // last inner iteration of a step, so the arrays end as the reference's.
-    if (!PUSH || aux) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) Rku[b + (size_t)v * PLANE] = out[v];
-    }
-    double pn[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // PUSH: the cell's norm and force terms
-    if (IF < 1) {
-      const double px = pow2 ? -(dPxf - dPxb) * inv : div_sh(ddx, -(dPxf - dPxb));
-      const double pz = pow2 ? -(dPzf - dPzb) * inv : div_sh(ddx, -(dPzf - dPzb));
-      const double r0 = -(px + vF[1]) * dx * dy * dz;
-      const double r1 = -(pz + vF[3]) * dx * dy * dz;
-      if (!PUSH || aux) {
-        Res[b] = r0;
-        Res[b + PLANE] = r1;
-      }
-      if (fuse && RK == 3) {
-        acc[5] += r0;
-        acc[6] += r1;
-      }
-      if (PUSH) {
-        pn[5] = r0;
-        pn[6] = r1;
-      }
-    }
-    if constexpr (PUSH) {
-      // The RK update of update_plane with U1p1 = U1p2 = U (see above).
-      double nv[5];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) nv[v] = u[v];
-      if (IF == 1) {
-        if (RK == 1) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) {
-            const double x = u[v] + out[v];
-            nv[v] = x;
-            if (aux) U1p1[b + (size_t)v * PLANE] = x;
-          }
-        } else if (RK == 2) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) {
-            const double x = 0.75 * u[v] + 0.25 * u[v] + 0.25 * out[v];
-            nv[v] = x;
-            if (aux) U1p2[b + (size_t)v * PLANE] = x;
-          }
-        } else {
-          // The cell's primitives before the update are those the fluxes used.
-          const double uo1 = me.u, vo1 = me.v, wo1 = me.w, To = PoR;
-          const double Po = (u[4] - 0.5 * rho * (uo1 * uo1 + vo1 * vo1 + wo1 * wo1)) * KM1;
-#pragma unroll
-          for (int v = 0; v < 5; ++v) nv[v] = 1.0 / 3.0 * u[v] + 2.0 / 3.0 * u[v] + 2.0 / 3.0 * out[v];
-          const double r = nv[0];
-          const DivBy dn = div_by(r);
-          const double un = div_sh(dn, nv[1]), vn = div_sh(dn, nv[2]), wn = div_sh(dn, nv[3]);
-          const double VV = un * un + vn * vn + wn * wn;
-          const double P = (nv[4] - 0.5 * r * VV) * KM1;
-          const double T = div_sh(dn, P);
-          pn[0] = (P - Po) * (P - Po);
-          pn[1] = (un - uo1) * (un - uo1);
-          pn[2] = (vn - vo1) * (vn - vo1);
-          pn[3] = (wn - wo1) * (wn - wo1);
-          pn[4] = (T - To) * (T - To);
-        }
-      }
-      const HaloSrc hs = halo[c];
-      const int o = i * 400 + j * 20 + k;
-      const int nx = i <= 3 ? hs.src[0] : (i >= 16 ? hs.src[1] : 0);
-      const int ny = j <= 3 ? hs.src[2] : (j >= 16 ? hs.src[3] : 0);
-      const int nz = k <= 3 ? hs.src[4] : (k >= 16 ? hs.src[5] : 0);
-      const int ox = o + (i <= 3 ? 16 * 400 : -16 * 400);
-      const int oy = o + (j <= 3 ? 16 * 20 : -16 * 20);
-      const int oz = o + (k <= 3 ? 16 : -16);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        Uout[(size_t)c * CUBE_STRIDE + (size_t)v * PLANE + o] = nv[v];
-        if (nx > 0) Uout[(size_t)nx * CUBE_STRIDE + (size_t)v * PLANE + ox] = nv[v];
-        if (ny > 0) Uout[(size_t)ny * CUBE_STRIDE + (size_t)v * PLANE + oy] = nv[v];
-        if (nz > 0) Uout[(size_t)nz * CUBE_STRIDE + (size_t)v * PLANE + oz] = nv[v];
-      }
-      if (RK == 3) {
-        const double s = wave_sum8(pn);
-        if ((t & 7) == 0) red[t >> 6][(t >> 3) & 7] = s;
-      }
-    }
-    __syncthreads();
-    // One row of norm partials per plane, so the norms do not depend on the
-    // runs.  (The next plane's sums are written after two more barriers.)
-    if (PUSH && RK == 3 && t < 8) {
-      double s = red[0][t];
-#pragma unroll
-      for (int w = 1; w < WG / 64; ++w) s += red[w][t];
-      partials[((size_t)(c - 1) * PUSH_ROWS_PER_CUBE + (i - 2)) * 8 + t] = s;
-    }
-  }
-  if constexpr (PUSH) {
-    const int bm = cube_mask[c];
-    if (bm && seg == 0) copy_bc_regions(U, Uout, c, bm, 0.0);
-  }
-  if (!PUSH && fuse) {
-    for (int ip = i1 - 3 < i0 ? i0 : i1 - 3; ip <= i1; ++ip) update_plane(ip);
-    if (RK == 3) {
-      __shared__ double sh[(WG / 64) * 7];
-      block_sum<7>(acc, sh);
-      if (threadIdx.x == 0)
-#pragma unroll
-        for (int m = 0; m < 7; ++m) partials[(size_t)blockIdx.x * 8 + m] = acc[m];
-    }
   }
 }
 
@@ -2195,40 +1276,6 @@ void launch_flux(hipStream_t s, const double* U, const double* U1, const double*
   if (ncube > 1)
     hipLaunchKernelGGL(k_flux, dim3(16, ncube - 1), dim3(WG), 0, s, U, U1, U1q, fws, cube_size,
                        Rku, Res, pt, deltaT, deltaTau, e);
-}
-
-void launch_flux_march(hipStream_t s, double* U, const double* U1, const double* U1q,
-                       const int8_t* fws, const double* cube_size, double* Rku, double* Res,
-                       int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int nseg,
-                       int RK, int fuse, double* U1p1, double* U1p2, double* partials) {
-  if (ncube > 1)
-    hipLaunchKernelGGL(k_flux_march<false>, dim3((ncube - 1) * nseg), dim3(WG), 0, s, U, U1, U1q,
-                       fws, cube_size, Rku, Res, pt, deltaT, deltaTau, e, nseg, RK,
-                       fuse && nseg == 1, U1p1, U1p2, partials, nullptr, nullptr, nullptr, 1, ncube);
-}
-
-void launch_flux_push(hipStream_t s, const double* Uin, double* Uout, const HaloSrc* halo,
-                      const uint8_t* cube_mask, const double* U1, const double* U1q,
-                      const int8_t* fws, const double* cube_size, double* Rku, double* Res,
-                      int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int RK,
-                      double* U1p1, double* U1p2, double* partials, int aux, int nseg) {
-  if (ncube > 1)
-    hipLaunchKernelGGL(k_flux_march<true>, dim3((ncube + 6) / 8 * 8 * nseg), dim3(WG), 0, s,
-                       const_cast<double*>(Uin), U1, U1q, fws, cube_size, Rku, Res, pt, deltaT,
-                       deltaTau, e, nseg, RK, 0, U1p1, U1p2, partials, Uout, halo, cube_mask, aux,
-                       ncube);
-}
-
-// Runs per cube of the pushing kernel.  The chip holds 512 of its workgroups
-// (two per CU).  Below 128 cubes the most runs that fit at once are fastest
-// (8 cubes: 28 us in 16 runs, 224 in one; 125 cubes: 98 us in 4 runs, 253 in
-// one).  Above, a run's second x-face pass and ring fill (about one plane's
-// work) stand against the last wave of workgroups being nearly empty: 8 runs
-// to 320 cubes (216 cubes: 168 us, 176 in 4 runs, 262 in one), 4 to 800 (512
-// cubes: 362 us, 401 in one), then 2 (1,000 cubes: 681 us, 704 in one; 2,048:
-// 1,347, 1,351 in one).
-int push_runs(int n) {
-  return n <= 32 ? 16 : n <= 64 ? 8 : n <= 128 ? 4 : n <= 320 ? 8 : n <= 800 ? 4 : 2;
 }
 
 __global__ __launch_bounds__(WG) void k_copy_d(const double* __restrict__ src,

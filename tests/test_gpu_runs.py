@@ -9,9 +9,9 @@ from test_gpu_parity import STATE, compare, er_close
 
 pytestmark = pytest.mark.gpu
 
-# (1), 32 | 33, 64 | 65, 128 | 129, 320 | 321, 800 | 801 cubes
-LATTICES = [(1, 1, 1), (8, 4, 1), (11, 3, 1), (4, 4, 4), (13, 5, 1), (8, 4, 4), (43, 1, 3),
-            (8, 8, 5), (107, 1, 3), (10, 10, 8), (89, 3, 3)]
+# 1, 7, 100 | 101, 700 | 701, 1,100 | 1,101 cubes (whole and ragged groups of 8)
+LATTICES = [(1, 1, 1), (7, 1, 1), (5, 5, 4), (101, 1, 1), (10, 10, 7), (701, 1, 1), (11, 10, 10),
+            (367, 3, 1)]
 
 
 @pytest.mark.parametrize("dims", LATTICES, ids=lambda d: str(int(np.prod(d))))
