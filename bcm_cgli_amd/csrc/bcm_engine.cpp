@@ -281,6 +281,7 @@ void engine_destroy(Engine* e) {
   (void)hipSetDevice(e->device);
   if (e->stream) (void)hipStreamSynchronize(e->stream);
   engine_output_free(e);
+  engine_chunks_free(e);
   free_case(e);
   if (e->ev0) (void)hipEventDestroy(e->ev0);
   if (e->ev1) (void)hipEventDestroy(e->ev1);
@@ -796,8 +797,7 @@ int engine_case_state(Engine* e, int slot, int which, double* aos, bool upload,
       launch_soa_to_aos_f(e->stream, dstf, e->staging, (int)n, ref);
     else
       launch_soa_to_aos(e->stream, dst, e->staging, (int)n);
-    HIP_TRY(hipMemcpyAsync(aos + CUBE_STRIDE, e->staging, n * cube_bytes, hipMemcpyDeviceToHost,
-                           e->stream));
+    HIP_TRY(engine_to_host(e, aos + CUBE_STRIDE, e->staging, n * cube_bytes));
     memset(aos, 0, cube_bytes);
   }
   HIP_TRY(hipStreamSynchronize(e->stream));
@@ -825,9 +825,7 @@ int engine_download_state(Engine* e, int which, double* aos) {
   double* d = state_ptr(e, which);
   if (!d) return 1;
   launch_soa_to_aos(e->stream, d, e->staging, e->ncube);
-  if (hipMemcpyAsync(aos, e->staging, pool_bytes(e), hipMemcpyDeviceToHost, e->stream) != hipSuccess)
-    return 1;
-  return hipStreamSynchronize(e->stream) == hipSuccess ? 0 : 1;
+  return engine_to_host(e, aos, e->staging, pool_bytes(e)) == hipSuccess ? 0 : 1;
 }
 
 int engine_upload_flags(Engine* e, const int* fws_aos) {

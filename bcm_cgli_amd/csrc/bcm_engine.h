@@ -70,6 +70,7 @@ struct CaseSlot {
 };
 
 struct OutputQueue;
+struct HostChunks;
 
 struct Engine {
   int device = 0;
@@ -173,6 +174,7 @@ struct Engine {
 
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   OutputQueue* out = nullptr;   // asynchronous output (created on first use)
+  HostChunks* chunks = nullptr; // pinned chunks of large downloads (created on first use)
   bool graph_valid = false;
   hipGraphExec_t graph_exec = nullptr;
   hipGraph_t graph = nullptr;
@@ -206,6 +208,11 @@ int engine_upload_flags(Engine* e, const int* fws_aos);
 // and ignored on upload).
 int engine_case_state(Engine* e, int slot, int which, double* aos, bool upload,
                       std::string& err);
+
+// Copies device memory to (pageable) host memory after the work queued on the
+// engine stream, and waits for it (bcm_download.cpp).
+hipError_t engine_to_host(Engine* e, void* dst, const void* src, size_t bytes);
+void engine_chunks_free(Engine* e);
 
 // Stage pieces (asynchronous on the engine stream).
 void engine_bc(Engine* e);
