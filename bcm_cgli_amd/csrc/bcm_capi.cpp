@@ -402,6 +402,7 @@ int bcm_engine_alloc_pool(bcm_engine* h, int cap_cubes, int max_cases, int preci
   if (engine_alloc(h->e, cap_cubes + 1, max_cases, err, precision)) return fail(err);
   h->e->flux_tuned = false;
   h->e->flux_pinned = false;
+  h->e->tuned_class = -1;
   return 0;
 }
 

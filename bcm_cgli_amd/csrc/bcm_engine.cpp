@@ -747,6 +747,7 @@ int engine_load_case(Engine* e, const Case& cs, std::string& err) {
   if (engine_alloc(e, cs.ncube, 1, err)) return 1;
   e->flux_tuned = false;
   e->flux_pinned = false;
+  e->tuned_class = -1;
   int slot;
   if (engine_add_case(e, cs, &slot, err)) return 1;
   e->halo_full_next = false;
@@ -926,11 +927,34 @@ bool engine_fused(const Engine* e) {
   return e->prec == 1 || (e->flux_variant == 1 && e->flux_nseg == 1 && e->flux_fuse);
 }
 
+namespace {
+int resident_cubes(const Engine* e) {
+  int n = 0;
+  for (const CaseSlot& S : e->cases)
+    if (S.active) n += S.tb.n;
+  return n;
+}
+
+// Size class of the resident pool: floor(log2(resident cubes)).
+int size_class(const Engine* e) {
+  int n = resident_cubes(e), c = 0;
+  for (; n > 1; n >>= 1) ++c;
+  return c;
+}
+
+// Runs per cube of the mixed flux kernel: as pinned, as tuned for this size
+// class, else by rule.
+int mixed_runs_now(const Engine* e) {
+  if (e->flux_pinned || e->tuned_class == size_class(e)) return e->mixed_nseg;
+  return mixed_runs(resident_cubes(e));
+}
+}  // namespace
+
 void engine_flux_update(Engine* e, int RK, int er_slot) {
   if (e->prec == 1) {
     launch_flux_mixed(e->stream, e->Uf, e->Uf2, e->halo, e->bc_mask_cube, e->Bsrc, e->fws,
                       e->cube_size, e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e, RK,
-                      e->partials, e->mixed_nseg);
+                      e->partials, mixed_runs_now(e));
     std::swap(e->Uf, e->Uf2);
     if (RK == 3)
       launch_reduce(e->stream, e->partials, MIXED_ROWS_PER_CUBE, e->case_desc, e->n_active,
@@ -950,27 +974,11 @@ void engine_flux_update(Engine* e, int RK, int er_slot) {
                   er_row(e, er_slot));
 }
 
-namespace {
-int resident_cubes(const Engine* e) {
-  int n = 0;
-  for (const CaseSlot& S : e->cases)
-    if (S.active) n += S.tb.n;
-  return n;
-}
 
-// Size class of the resident pool: floor(log2(resident cubes)).
-int size_class(const Engine* e) {
-  int n = resident_cubes(e), c = 0;
-  for (; n > 1; n >>= 1) ++c;
-  return c;
-}
-}  // namespace
-
-// Tunes the flux kernel choice when it has not been chosen yet, or (mixed
-// path, choice not pinned) when the pool's size class changed since.
+// Before a run: unless a choice was pinned with set_flux, FP64 takes the pushing
+// kernel; the runs per cube follow the resident cubes by rule.
 int engine_maybe_tune(Engine* e, std::string& err) {
-  if (e->flux_tuned && (e->prec == 0 || e->flux_pinned || size_class(e) == e->tuned_class))
-    return 0;
+  if (e->prec == 1 || e->flux_tuned) return 0;
   int v, n;
   return engine_autotune(e, &v, &n, err);
 }
@@ -983,60 +991,56 @@ int engine_autotune(Engine* e, int* variant, int* nseg, std::string& err) {
   }
   if (e->prec == 1) {
     // The mixed flux kernel in 1, 2 or 4 runs per cube (bitwise the same
-    // results), each timed as one whole RK stage on the resident cases, once
-    // per size class of the pool; the iterate the stages write is restored.
-    // The candidates are timed in three interleaved rounds and each keeps its
-    // fastest round, so a clock ramp at the start favours none of them.
-    const int cls = size_class(e);
-    auto known = e->nseg_by_class.find(cls);
-    if (known == e->nseg_by_class.end()) {
-      const size_t bytes = (size_t)e->ncube * CUBE_STRIDE * sizeof(float);
-      struct Saved {
-        float* p[2] = {nullptr, nullptr};
-        ~Saved() {
-          for (float* q : p)
-            if (q) (void)hipFree(q);
-        }
-      } saved;
-      float* const live[2] = {e->Uf, e->Uf2};
-      for (int a = 0; a < 2; ++a) {
-        HIP_TRY(hipMalloc((void**)&saved.p[a], bytes));
-        HIP_TRY(hipMemcpyAsync(saved.p[a], live[a], bytes, hipMemcpyDeviceToDevice, e->stream));
+    // results), each timed as one whole RK stage on the resident cases; the
+    // iterate the stages write is restored.  The candidates are timed in three
+    // interleaved rounds and each keeps its fastest round, so a clock ramp at
+    // the start favours none of them.  The choice holds for this size class of
+    // the pool; a run on another takes the rule's.
+    const size_t bytes = (size_t)e->ncube * CUBE_STRIDE * sizeof(float);
+    struct Saved {
+      float* p[2] = {nullptr, nullptr};
+      ~Saved() {
+        for (float* q : p)
+          if (q) (void)hipFree(q);
       }
-      const bool full = e->halo_full_next;
-      const int cands[3] = {1, 2, 4};
-      float fastest[3] = {1e30f, 1e30f, 1e30f};
-      for (int round = 0; round < 3; ++round)
-        for (int c = 0; c < 3; ++c) {
-          e->mixed_nseg = cands[c];
-          engine_stage(e, 2, 0, full);   // warm up
-          HIP_TRY(hipEventRecord(e->ev0, e->stream));
-          for (int r = 0; r < 3; ++r) engine_stage(e, 2, 0, full);
-          HIP_TRY(hipEventRecord(e->ev1, e->stream));
-          HIP_TRY(hipEventSynchronize(e->ev1));
-          float ms = 0;
-          HIP_TRY(hipEventElapsedTime(&ms, e->ev0, e->ev1));
-          e->Uf = live[0];
-          e->Uf2 = live[1];
-          for (int a = 0; a < 2; ++a)
-            HIP_TRY(
-                hipMemcpyAsync(live[a], saved.p[a], bytes, hipMemcpyDeviceToDevice, e->stream));
-          fastest[c] = std::min(fastest[c], ms);
-        }
-      HIP_TRY(hipStreamSynchronize(e->stream));
-      int bn = cands[0];
-      float best = fastest[0];
-      for (int c = 1; c < 3; ++c)
-        if (fastest[c] < best) {
-          best = fastest[c];
-          bn = cands[c];
-        }
-      known = e->nseg_by_class.emplace(cls, bn).first;
+    } saved;
+    float* const live[2] = {e->Uf, e->Uf2};
+    for (int a = 0; a < 2; ++a) {
+      HIP_TRY(hipMalloc((void**)&saved.p[a], bytes));
+      HIP_TRY(hipMemcpyAsync(saved.p[a], live[a], bytes, hipMemcpyDeviceToDevice, e->stream));
     }
-    if (e->mixed_nseg != known->second) e->graph_valid = false;
-    e->mixed_nseg = known->second;
-    e->tuned_class = cls;
-    e->flux_tuned = true;
+    const bool full = e->halo_full_next;
+    const int cands[3] = {1, 2, 4};
+    float fastest[3] = {1e30f, 1e30f, 1e30f};
+    for (int round = 0; round < 3; ++round)
+      for (int c = 0; c < 3; ++c) {
+        e->mixed_nseg = cands[c];
+        e->tuned_class = size_class(e);   // (the candidate, not the rule)
+        engine_stage(e, 2, 0, full);   // warm up
+        HIP_TRY(hipEventRecord(e->ev0, e->stream));
+        for (int r = 0; r < 3; ++r) engine_stage(e, 2, 0, full);
+        HIP_TRY(hipEventRecord(e->ev1, e->stream));
+        HIP_TRY(hipEventSynchronize(e->ev1));
+        float ms = 0;
+        HIP_TRY(hipEventElapsedTime(&ms, e->ev0, e->ev1));
+        e->Uf = live[0];
+        e->Uf2 = live[1];
+        for (int a = 0; a < 2; ++a)
+          HIP_TRY(
+              hipMemcpyAsync(live[a], saved.p[a], bytes, hipMemcpyDeviceToDevice, e->stream));
+        fastest[c] = std::min(fastest[c], ms);
+      }
+    HIP_TRY(hipStreamSynchronize(e->stream));
+    int bn = cands[0];
+    float best = fastest[0];
+    for (int c = 1; c < 3; ++c)
+      if (fastest[c] < best) {
+        best = fastest[c];
+        bn = cands[c];
+      }
+    e->mixed_nseg = bn;
+    e->graph_valid = false;
+    e->tuned_class = size_class(e);
     if (variant) *variant = 2;
     if (nseg) *nseg = e->mixed_nseg;
     return 0;

@@ -7,7 +7,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <map>
 #include <string>
 #include <vector>
 
@@ -160,12 +159,11 @@ struct Engine {
   // stage reads back) only when set: captured steps clear it for all but
   // their last inner iteration.
   bool push_aux = true;
-  // Mixed path: runs per cube of the flux kernel (1, 2 or 4); the autotuner
-  // picks it per size class of the resident pool (log2 of its cubes) and
-  // keeps each class's pick.
+  // Mixed path: runs per cube of the flux kernel when pinned with set_flux, or
+  // found by the autotuner for size class tuned_class of the resident pool
+  // (log2 of its cubes); otherwise they follow the resident cubes by rule.
   int mixed_nseg = 1;
   int tuned_class = -1;
-  std::map<int, int> nseg_by_class;
   bool flux_tuned = false;
   bool flux_pinned = false;    // chosen with set_flux: no re-tuning
   // Cubes whose IB fill needs more LDS slots than this take the in-place
@@ -250,8 +248,7 @@ int engine_sync(Engine* e, std::string& err);
 // and keeps the fastest.  Returns the chosen (variant, nseg) through the
 // pointers.
 int engine_autotune(Engine* e, int* variant, int* nseg, std::string& err);
-// Tunes only when no choice was made yet, or (mixed path, choice not pinned
-// with set_flux) when the pool's size class has changed since the last tuning.
+// Selects the FP64 kernel when no choice was made yet.
 int engine_maybe_tune(Engine* e, std::string& err);
 
 // Asynchronous PLOT3D output (bcm_output.cpp): queues the current inner

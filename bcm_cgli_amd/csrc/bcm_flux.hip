@@ -29,7 +29,8 @@ struct MarchArgs {
   double *Rku, *Res;
   PhysTab pt;
   double deltaT, deltaTau, e;
-  int nseg, RK, ncube;
+  Runs runs;
+  int RK, ncube;
   double *U1p1, *U1p2, *partials, *Uout;
   const HaloSrc* halo;
   const uint8_t* cube_mask;
@@ -91,17 +92,15 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
   __shared__ double fzb[6][16];                     // z-faces before k = 2: flux, pressure
   __shared__ int8_t fl[2][400];                     // flags of planes i, i+1
   __shared__ double red[WG / 64][8];                // PUSH, RK 3: norm sums of the waves
-  const int nseg = A.nseg, RK = A.RK;
-  // Workgroups go to the 8 XCDs in turn; the runs of one cube share planes
-  // and so go to one XCD's L2.
-  const int seg = blockIdx.x / 8 % nseg;
-  const int c = blockIdx.x / (8 * nseg) * 8 + blockIdx.x % 8 + 1;
+  const int RK = A.RK;
+  const RunOf run = run_of(A.runs, blockIdx.x);
+  const int c = run.cube, seg = run.seg;
   if (c >= A.ncube) return;
   const int cc = A.pt.cube_case[c];
   if (cc < 0) return;
   const DevPhys ph = A.pt.phys[cc];
   const double deltaT = A.deltaT, deltaTau = A.deltaTau, e = A.e;
-  const int len = 16 / nseg;
+  const int len = 16 / run.nseg;
   const int i0 = 2 + seg * len, i1 = i0 + len - 1;
   const double dx = A.cube_size[c] / 16;
   const double inv = 1. / dx;
@@ -694,9 +693,6 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
   }
 }
 
-// Workgroups for n cubes in nseg runs: whole groups of one per XCD.
-dim3 march_grid(int ncube, int nseg) { return dim3((ncube + 6) / 8 * 8 * nseg); }
-
 }  // namespace
 
 void launch_flux_march(hipStream_t s, double* U, const double* U1, const double* U1q,
@@ -704,12 +700,12 @@ void launch_flux_march(hipStream_t s, double* U, const double* U1, const double*
                        int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int nseg,
                        int RK, int fuse, double* U1p1, double* U1p2, double* partials) {
   if (ncube <= 1) return;
-  const MarchArgs a{U, U1, U1q, fws, cube_size, Rku, Res, pt, deltaT, deltaTau, e, nseg, RK, ncube,
-                    U1p1, U1p2, partials, nullptr, nullptr, nullptr};
+  const MarchArgs a{U, U1, U1q, fws, cube_size, Rku, Res, pt, deltaT, deltaTau, e, Runs{0, nseg}, RK,
+                    ncube, U1p1, U1p2, partials, nullptr, nullptr, nullptr};
   if (fuse && nseg == 1)
-    hipLaunchKernelGGL((k_flux_march<IN_PLACE, true>), march_grid(ncube, 1), dim3(WG), 0, s, a);
+    hipLaunchKernelGGL((k_flux_march<IN_PLACE, true>), run_grid(a.runs, ncube), dim3(WG), 0, s, a);
   else
-    hipLaunchKernelGGL((k_flux_march<FLUX_ONLY, true>), march_grid(ncube, nseg), dim3(WG), 0, s, a);
+    hipLaunchKernelGGL((k_flux_march<FLUX_ONLY, true>), run_grid(a.runs, ncube), dim3(WG), 0, s, a);
 }
 
 void launch_flux_push(hipStream_t s, const double* Uin, double* Uout, const HaloSrc* halo,
@@ -719,11 +715,12 @@ void launch_flux_push(hipStream_t s, const double* Uin, double* Uout, const Halo
                       double* U1p1, double* U1p2, double* partials, int aux, int nseg) {
   if (ncube <= 1) return;
   const MarchArgs a{const_cast<double*>(Uin), U1, U1q, fws, cube_size, Rku, Res, pt, deltaT,
-                    deltaTau, e, nseg, RK, ncube, U1p1, U1p2, partials, Uout, halo, cube_mask};
+                    deltaTau, e, runs_for(ncube, nseg), RK, ncube, U1p1, U1p2, partials, Uout,
+                    halo, cube_mask};
   if (aux)
-    hipLaunchKernelGGL((k_flux_march<PUSH, true>), march_grid(ncube, nseg), dim3(WG), 0, s, a);
+    hipLaunchKernelGGL((k_flux_march<PUSH, true>), run_grid(a.runs, ncube), dim3(WG), 0, s, a);
   else
-    hipLaunchKernelGGL((k_flux_march<PUSH, false>), march_grid(ncube, nseg), dim3(WG), 0, s, a);
+    hipLaunchKernelGGL((k_flux_march<PUSH, false>), run_grid(a.runs, ncube), dim3(WG), 0, s, a);
 }
 
 // Runs per cube of the pushing kernel.  The chip holds 512 of its workgroups

@@ -139,6 +139,27 @@ constexpr int ZBC_IN_FLUX = 64;
 __device__ inline double zbc_neg(double x, double) { return -x; }
 __device__ inline float zbc_neg(float x, double r3) { return (float)(-((double)x + r3) - r3); }
 
+// How a marching flux kernel divides cubes 1..n among workgroups: cubes 1..whole
+// (a multiple of 8) take one each, every other cube nseg runs of 16/nseg planes.
+struct Runs {
+  int whole, nseg;
+};
+struct RunOf {
+  int cube, seg, nseg;
+};
+// Workgroups go to the 8 XCDs in turn; the runs of one cube share planes and so
+// go to one XCD's L2.
+__device__ inline RunOf run_of(const Runs& r, int block) {
+  if (block < r.whole) return RunOf{block + 1, 0, 1};
+  const int b = block - r.whole;
+  return RunOf{r.whole + b / (8 * r.nseg) * 8 + b % 8 + 1, b / 8 % r.nseg, r.nseg};
+}
+// Whole groups of one cube per XCD.
+inline dim3 run_grid(const Runs& r, int ncube) {
+  return dim3(r.whole + (ncube - 1 - r.whole + 7) / 8 * 8 * r.nseg);
+}
+inline Runs runs_for(int ncube, int nseg) { return Runs{0, nseg}; }
+
 // Copies, with the threads of one workgroup, the ghost regions the domain BCs
 // of cube c write (mask bits 1 x-min, 2 x-max, 4 y-min, 8 y-max, 16 z-min,
 // 32 z-max) from Uin to Uout: x faces over j,k in [2,17], y faces over all i
@@ -306,14 +327,16 @@ int update_blocks(int ncube);
 // (updated fluid cells, other cells unchanged).  Cells of the two layers
 // next to a face with an equal-size neighbour (halo[c]) are also written into
 // that neighbour's ghost layers in Uout: the face part of the post-update
-// exchange.  nseg (1, 2 or 4) runs of 16/nseg planes per cube, one workgroup
-// each; results are bitwise the same for every nseg.  At RK 3,
-// MIXED_ROWS_PER_CUBE rows of 8 norm partials per cube.
+// exchange.  nseg (1, 2, 4, 8 or 16) runs of 16/nseg planes per cube, one
+// workgroup each; results are bitwise the same for every nseg.  At RK 3,
+// MIXED_ROWS_PER_CUBE rows of 8 norm partials per cube (one per plane).
 constexpr int MIXED_ROWS_PER_CUBE = 16;
 void launch_flux_mixed(hipStream_t s, const float* Uin, float* Uout, const HaloSrc* halo,
                        const uint8_t* cube_mask, const double* Bsrc, const int8_t* fws,
                        const double* cube_size, int ncube, PhysTab pt, double deltaT,
                        double deltaTau, double e, int RK, double* partials, int nseg);
+// Runs per cube for n resident cubes.
+int mixed_runs(int n);
 // dst[0..n) <- src[0..n).
 void launch_copy_f(hipStream_t s, const float* src, float* dst, size_t n);
 // U1q <- U1, U1 <- ref_state + U and Bsrc <- 3 ref_state - 4 U1 + U1q on

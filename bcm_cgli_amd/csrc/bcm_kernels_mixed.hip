@@ -37,44 +37,12 @@ namespace bcm {
 namespace {
 
 constexpr int WG = 256;
-// First lanes of the 16 that evaluate the y- and z-faces next to the ghost
-// layers (waves 1 and 2: wave 0 stages the plane's border cells and forms
-// their primitives, wave 3 forms the corner primitives).
-#ifndef BCM_MIXED_BND_Y
-#define BCM_MIXED_BND_Y 64
-#endif
-#ifndef BCM_MIXED_BND_Z
-#define BCM_MIXED_BND_Z 128
-#endif
-constexpr int BND_Y = BCM_MIXED_BND_Y, BND_Z = BCM_MIXED_BND_Z;
 constexpr float KGf = 1.4f;
 constexpr float KM1f = 0.4f;
 constexpr float IKM1f = 2.5f;          // 1/(K-1)
 constexpr float IRGf = 1.0f / 287.0f;  // 1/R
 constexpr float HEATf = 717.5f * 1.4f / 0.72f;   // Cv K / Pr
 constexpr double KM1d = 1.4 - 1;
-
-// x of the lane CTRL's data-parallel move selects (0 where it selects none),
-// both halves of a double moved alike.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ double dpp_d(double x) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, ROW_MASK, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, ROW_MASK, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-// Sum of x over the 64 lanes of the wave, complete in lane 63, in a fixed
-// order: prefix sums along each row of 16 lanes (row_shr 1, 2, 4, 8), then
-// row 0's total into row 1 and row 2's into row 3 (row_bcast 15), then the
-// first half's total into the second half (row_bcast 31).
-__device__ __forceinline__ double wave_sum(double x) {
-  x += dpp_d<0x111, 0xf>(x);
-  x += dpp_d<0x112, 0xf>(x);
-  x += dpp_d<0x114, 0xf>(x);
-  x += dpp_d<0x118, 0xf>(x);
-  x += dpp_d<0x142, 0xa>(x);
-  x += dpp_d<0x143, 0xc>(x);
-  return x;
-}
 
 __device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
@@ -136,8 +104,10 @@ __device__ __forceinline__ void side(const float (&d)[5], const RefF& rf, Side& 
 //   energy    du_d (E + P) + u0_d (dE + dP)
 // The dissipation is built from differences R - L as in the reference.  dP
 // returns the deviation of the face pressure average.
-__device__ __forceinline__ void roe_f(const float (&L)[5], const float (&R)[5], int d, float e,
-                                      const RefF& rf, float (&F)[5], float& dP) {
+// D is the face-normal axis; 3: the lane's own choice of y (ydir) or z.
+template <int D>
+__device__ __forceinline__ void roe_f(const float (&L)[5], const float (&R)[5], float e,
+                                      const RefF& rf, float (&F)[5], float& dP, bool ydir = false) {
   Side l, r;
   side(L, rf, l);
   side(R, rf, r);
@@ -150,12 +120,12 @@ __device__ __forceinline__ void roe_f(const float (&L)[5], const float (&R)[5], 
   const float H = (t5 * l.H + t6 * r.H) * it4;
   const float C = (H - 0.5f * VV) * KM1f;
   const float beta = fmaxr(VV * frcp(C), e);
-  const float un = d == 0 ? q[0] : (d == 1 ? q[1] : q[2]);
-  const float lun = d == 0 ? l.u[0] : (d == 1 ? l.u[1] : l.u[2]);
-  const float run = d == 0 ? r.u[0] : (d == 1 ? r.u[1] : r.u[2]);
-  const float ldu = d == 0 ? l.du[0] : (d == 1 ? l.du[1] : l.du[2]);
-  const float rdu = d == 0 ? r.du[0] : (d == 1 ? r.du[1] : r.du[2]);
-  const float u0n = d == 0 ? rf.u[0] : (d == 1 ? rf.u[1] : rf.u[2]);
+  const bool normal[3] = {D == 0, D == 3 ? ydir : D == 1, D == 3 ? !ydir : D == 2};
+  auto pick = [&](const float (&x)[3]) { return D == 0 ? x[0] : (normal[1] ? x[1] : x[2]); };
+  const float un = pick(q), lun = pick(l.u), run = pick(r.u), ldu = pick(l.du), rdu = pick(r.du);
+  const float u0n = pick(rf.u);
+  const float Ln = D == 0 ? L[1] : (normal[1] ? L[2] : L[3]);
+  const float Rn = D == 0 ? R[1] : (normal[1] ? R[2] : R[3]);
   const float temp = 0.5f * (1 + beta) * un;
   const float S = 0.5f * fsqrt(4 * beta * C + un * un * (1 - beta) * (1 - beta));
   const float iS = frcp(S);
@@ -167,12 +137,12 @@ __device__ __forceinline__ void roe_f(const float (&L)[5], const float (&R)[5], 
   const float deltaU = (S - temp3 - beta * an) * temp1 + tS * dun;
   const float deltaP = tS * dPr + (S - an + temp3) * rho * dun;
   const float dUr = deltaU * rho;
-  F[0] = 0.5f * ((L[d + 1] + R[d + 1]) - (an * (R[0] - L[0]) + dUr));
+  F[0] = 0.5f * ((Ln + Rn) - (an * (R[0] - L[0]) + dUr));
 #pragma unroll
   for (int m = 0; m < 3; ++m) {
-    const float fav = an * (R[m + 1] - L[m + 1]) + dUr * q[m] + (m == d ? deltaP : 0.f);
+    const float fav = an * (R[m + 1] - L[m + 1]) + dUr * q[m] + (normal[m] ? deltaP : 0.f);
     const float cen = (L[m + 1] * lun + rf.m[m] * ldu) + (R[m + 1] * run + rf.m[m] * rdu) +
-                      (m == d ? l.dP + r.dP : 0.f);
+                      (normal[m] ? l.dP + r.dP : 0.f);
     F[m + 1] = 0.5f * (cen - fav);
   }
   const float EPl = rf.E + rf.P + L[4] + l.dP, EPr = rf.E + rf.P + R[4] + r.dP;
@@ -231,7 +201,6 @@ __device__ __forceinline__ int order_bwd(int q, int fm2, int fm1, int fp1) {
 // (staged plane, primitive ring) put them on distinct LDS banks.
 constexpr int PRW = 20;           // row stride of the primitive ring
 constexpr int PR = 18 * PRW;      // primitive plane, j,k in [1,18]
-constexpr int NF = 17 * 16;       // faces of one axis in one plane
 constexpr int NFY = 4 * 80;       // y-face slots (17 rows of 16 in 4 blocks of 5 rows)
 __device__ __forceinline__ int ring_idx(int jj, int kk) { return (jj - 1) * PRW + (kk - 1); }
 // y-face between rows p and p+1 at k = kk (p = 1..17): block (p-1) % 4, row
@@ -239,672 +208,650 @@ __device__ __forceinline__ int ring_idx(int jj, int kk) { return (jj - 1) * PRW 
 __device__ __forceinline__ int fy_idx(int p, int kk) {
   return ((p - 1) & 3) * 80 + ((p - 1) >> 2) * 16 + (kk - 2);
 }
-// z-face between columns p and p+1 in row jj (jj = 2..17, p = 1..17).
-__device__ __forceinline__ int fz_idx(int jj, int p) {
-  return ((jj - 2) & 3) * 68 + ((jj - 2) >> 2) * 17 + (p - 1);
-}
-
-// Flux of the face between p and p+1 along axis D (1 or 2) of the staged
-// plane: base is the plane index of cell p.  Orders below 5 read cell p in
-// place of the cells p-2 and p+3 they do not use (which may lie beyond the
-// plane).
-template <int D>
-__device__ __forceinline__ void plane_face(const float (*cp)[400], int base, int order, float e,
-                                           const RefF& rf, float (&F)[5], float& dP) {
-  constexpr int s = D == 1 ? 20 : 1;
-  const ReconW rw = recon_weights(order);
-  const int o0 = order == 5 ? -2 * s : 0, o5 = order == 5 ? 3 * s : 0;
-  float L[5], R[5];
+// States of the face between cells p and p+1 of a line whose cell p-2+m holds
+// s(m, v): every order's weighted sum over the six cells (a lane's order may
+// differ from its neighbour's).  An order below 5 does not use p-2 and p+3.
+template <typename S>
+__device__ __forceinline__ void face_states(int order, S s, float (&L)[5], float (&R)[5]) {
+  const ReconW w = recon_weights(order);
 #pragma unroll
-  for (int v = 0; v < 5; ++v) {
-    const float* q = cp[v] + base;
-    recon(rw, q[o0], q[-s], q[0], q[s], q[2 * s], q[o5], L[v], R[v]);
-  }
-  roe_f(L, R, D, e, rf, F, dP);
+  for (int v = 0; v < 5; ++v)
+    recon(w, s(0, v), s(1, v), s(2, v), s(3, v), s(4, v), s(5, v), L[v], R[v]);
 }
 
-// Viscous flux through the face between cell P = (i+a0, j0, k0) and P + e_D
-// (Flux.cpp:1946-2272, forward-face formulas of P): one evaluation serves
-// both adjacent cells.  ring holds deviations of u, v, w, T of planes i-1..i+1
-// (slot = plane & 3, j,k in [1,18]).  L receives the x, y, z stress and the
+// The same along a line of the staged plane, st floats apart; base is cell p.
+// Orders below 5 read cell p in place of the cells they do not use (which may
+// lie beyond the plane).
+__device__ __forceinline__ void plane_states(const float* cp, int base, int st, int order,
+                                             float (&L)[5], float (&R)[5]) {
+  const int o0 = order == 5 ? -2 * st : 0, o5 = order == 5 ? 3 * st : 0;
+  face_states(order, [&](int m, int v) {
+    return cp[v * 400 + base + (m == 0 ? o0 : m == 5 ? o5 : (m - 2) * st)];
+  }, L, R);
+}
+
+// Viscous flux through the face between cell P and P + e_D (Flux.cpp:1946-2272,
+// forward-face formulas of P): one evaluation serves both adjacent cells.  D as
+// for roe_f.  ring holds deviations of u, v, w, T; rm, r0 and rp are the ring
+// offsets of P in the plane before, its own and the next (rm unused for D = 0,
+// rp unused for the backward of nothing).  L receives the x, y, z stress and the
 // energy flux.
 template <int D>
-__device__ __forceinline__ void visc_face(const float (*ring)[4][PR], int i, int a0, int j0,
-                                          int k0, const RefF& rf, float inv, float iT0,
-                                          float muL, float sut, float (&L)[4]) {
-  constexpr int da = D == 0, dj = D == 1, dk = D == 2;
-  auto P = [&](int a, int jj, int kk, int m) -> float {
-    return ring[(i + a) & 3][m][ring_idx(jj, kk)];
-  };
+__device__ __forceinline__ void visc_face(const float (*ring)[3 * PR], int rm, int r0, int rp,
+                                          const RefF& rf, float inv, float iT0, float muL,
+                                          float sut, float (&L)[4], bool ydir = false) {
+  // Ring steps of the face normal and of the in-plane tangents.
+  const int sn = D == 1 ? PRW : D == 2 ? 1 : ydir ? PRW : 1;
   float me[4], fv[4];
 #pragma unroll
   for (int m = 0; m < 4; ++m) {
-    me[m] = P(a0, j0, k0, m);
-    fv[m] = P(a0 + da, j0 + dj, k0 + dk, m);
+    me[m] = ring[m][r0];
+    fv[m] = D == 0 ? ring[m][rp] : ring[m][r0 + sn];
   }
   const float Tf = rf.T + 0.5f * (me[3] + fv[3]);
   const float temp = Tf * iT0;
   const float mu = muL * temp * fsqrt(temp) * sut * frcp(Tf + 110.f);
-  float g[3][4];
+  const float q = 0.25f * inv;
+  float gn[4], gx[4], gy[4], gz[4];   // gradients along the normal and the axes
 #pragma unroll
-  for (int tt = 0; tt < 3; ++tt) {
-    if (tt == D) {
-#pragma unroll
-      for (int m = 0; m < 4; ++m) g[tt][m] = (fv[m] - me[m]) * inv;
+  for (int m = 0; m < 4; ++m) {
+    const float* a = ring[m];
+    gn[m] = (fv[m] - me[m]) * inv;
+    if (D == 0) {
+      gx[m] = gn[m];
+      gy[m] = (a[r0 + PRW] + a[rp + PRW] - a[r0 - PRW] - a[rp - PRW]) * q;
+      gz[m] = (a[r0 + 1] + a[rp + 1] - a[r0 - 1] - a[rp - 1]) * q;
     } else {
-      const int ta = tt == 0, tj = tt == 1, tk = tt == 2;
-#pragma unroll
-      for (int m = 0; m < 4; ++m)
-        g[tt][m] = (P(a0 + ta, j0 + tj, k0 + tk, m) + P(a0 + ta + da, j0 + tj + dj, k0 + tk + dk, m) -
-                    P(a0 - ta, j0 - tj, k0 - tk, m) - P(a0 - ta + da, j0 - tj + dj, k0 - tk + dk, m)) *
-                   (0.25f * inv);
+      gx[m] = (a[rp] + a[rp + sn] - a[rm] - a[rm + sn]) * q;
+      // The other in-plane axis.
+      const int so = D == 1 ? 1 : D == 2 ? PRW : ydir ? 1 : PRW;
+      const float go = (a[r0 + so] + a[r0 + sn + so] - a[r0 - so] - a[r0 + sn - so]) * q;
+      if (D == 3) {
+        gy[m] = ydir ? gn[m] : go;
+        gz[m] = ydir ? go : gn[m];
+      } else {
+        gy[m] = D == 1 ? gn[m] : go;
+        gz[m] = D == 1 ? go : gn[m];
+      }
     }
   }
   const float uf = rf.u[0] + 0.5f * (me[0] + fv[0]), vf = rf.u[1] + 0.5f * (me[1] + fv[1]),
               wf = rf.u[2] + 0.5f * (me[2] + fv[2]);
-  const float div = g[0][0] + g[1][1] + g[2][2];
+  const float div = gx[0] + gy[1] + gz[2];
+  const bool normal[3] = {D == 0, D == 3 ? ydir : D == 1, D == 3 ? !ydir : D == 2};
+  // d/dm of the normal velocity, m = x, y, z.
+  const float nx = D == 0 ? gx[0] : (normal[1] ? gx[1] : gx[2]);
+  const float ny = D == 0 ? gy[0] : (normal[1] ? gy[1] : gy[2]);
+  const float nz = D == 0 ? gz[0] : (normal[1] ? gz[1] : gz[2]);
+  const float gd[3] = {nx, ny, nz};
 #pragma unroll
-  for (int m = 0; m < 3; ++m)
-    L[m] = (m == D) ? mu * (2 * g[D][D] - (2.0f / 3.0f) * div) : mu * (g[m][D] + g[D][m]);
-  L[3] = uf * L[0] + vf * L[1] + wf * L[2] + mu * HEATf * g[D][3];
-}
-
-// y-face (D = 1) between (p, kk) and (p + 1, kk), or z-face (D = 2) between
-// (jj, p) and (jj, p + 1), of staged plane i: inviscid flux into fy / fz (face
-// slot fy_idx(p, kk), or fz_idx(jj, p); fz also keeps the face pressure
-// average) and viscous flux into vy / vz.  Face p = 1 lies between the first
-// ghost layer and the first interior cell.
-template <int D>
-__device__ __forceinline__ void yz_face(const float (*cp)[400], const int8_t* fl,
-                                        const float (*ring)[4][PR], int i, int a, int p,
-                                        float e, const RefF& rf, float inv, float iT0, float muL,
-                                        float sut, float* fo, float* vo) {
-  constexpr int W = D == 1 ? NFY : NF;   // row length of the face arrays
-  constexpr int s = D == 1 ? 20 : 1;
-  const int base = D == 1 ? p * 20 + a : a * 20 + p;
-  const int8_t* fb = fl + base;
-  const int o = p >= 2 ? order_fwd(p, fb[-s], fb[s], fb[2 * s])
-                       : order_bwd(2, fb[-s], fb[0], fb[2 * s]);
-  float F[5], dP, Lv[4];
-  plane_face<D>(cp, base, o, e, rf, F, dP);
-  if (D == 1)
-    visc_face<1>(ring, i, 0, p, a, rf, inv, iT0, muL, sut, Lv);
-  else
-    visc_face<2>(ring, i, 0, a, p, rf, inv, iT0, muL, sut, Lv);
-  const int g = D == 1 ? fy_idx(p, a) : fz_idx(a, p);
-#pragma unroll
-  for (int v = 0; v < 5; ++v) fo[v * W + g] = F[v];
-  if (D == 2) fo[5 * W + g] = dP;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) vo[v * W + g] = Lv[v];
-}
-
-// Border cells of a 20x20 plane (j or k in {0,1,18,19}): 144 of them.  (The
-// edge rows are formed arithmetically: a table indexed by lane would live in
-// memory.)
-__device__ __forceinline__ int edge4(int e) { return e < 2 ? e : e + 16; }
-__device__ __forceinline__ int border20(int t) {
-  if (t < 80) return edge4(t / 20) * 20 + t % 20;
-  const int u = t - 80;
-  return (2 + u / 4) * 20 + edge4(u % 4);
-}
-// Border cells of the 18x18 primitive plane (j or k in {1,18}): 68 of them,
-// as (j,k) in padded-plane numbering.
-__device__ __forceinline__ int border18(int t) {
-  if (t < 18) return 1 * 20 + (1 + t);
-  if (t < 36) return 18 * 20 + (1 + t - 18);
-  if (t < 52) return (2 + t - 36) * 20 + 1;
-  return (2 + t - 52) * 20 + 18;
-}
-// The border lanes holding the two face ghost cells each corner of the plane
-// averages, in corner order (1,1), (1,18), (18,1), (18,18): (1,2) and (2,1),
-// (1,17) and (2,18), (18,2) and (17,1), (18,17) and (17,18).  Returns the
-// lane's slot 0..7, or -1.
-__device__ __forceinline__ int corner_source_slot(int t) {
-  switch (t) {
-    case 1: return 0;
-    case 36: return 1;
-    case 16: return 2;
-    case 52: return 3;
-    case 19: return 4;
-    case 51: return 5;
-    case 34: return 6;
-    case 67: return 7;
-    default: return -1;
+  for (int m = 0; m < 3; ++m) {
+    const float dia = 2 * gn[m] - (2.0f / 3.0f) * div, off = gn[m] + gd[m];
+    L[m] = mu * (D == 3 ? (normal[m] ? dia : off) : m == D ? dia : off);
   }
+  L[3] = uf * L[0] + vf * L[1] + wf * L[2] + mu * HEATf * gn[3];
 }
 
-// Segmented march: with nseg > 1 each cube's interior planes 2..17 are split
-// into nseg runs of 16/nseg planes, one workgroup each (more workgroups when
-// few cubes are resident).  A run starting at i0 > 2 first executes one
-// prologue iteration at i0 - 1 that only forms the x-face i0 - 1/2 (inviscid
-// and viscous) the run carries into its first plane: the same loop body, and
-// so the same instructions and bits, as the unsegmented march computes it
-// with.  Norm partials are rows per (group of 4 planes, wave), 16 per cube,
-// summed in a fixed order, so every result is bitwise the same for every
-// nseg.
+// An address as a uniform base and a 32-bit byte offset per lane.
+template <typename T>
+__device__ __forceinline__ T& at_byte(T* base, unsigned off) {
+  using B = std::conditional_t<std::is_const_v<T>, const char, char>;
+  return *reinterpret_cast<T*>(reinterpret_cast<B*>(base) + off);
+}
 
+// One workgroup of 256 lanes marches through a run of a cube's i-planes, in two
+// phases per plane:
+//  1. the plane's 272 y-faces and 272 z-faces, inviscid and viscous, once each;
+//     meanwhile the next plane's conserved values go from memory straight into
+//     the other LDS buffer, and the lane's column cell three planes ahead and the
+//     border cells two planes ahead into registers;
+//  2. the primitives two planes ahead into the ring slot of the plane behind,
+//     the x-face i+1/2 from the lane's column (two planes behind and two ahead
+//     in registers, two in LDS), the differences, the residual, the increment,
+//     the update and its stores.
+//
+// Runs: with nseg > 1 each cube's interior planes 2..17 are split into nseg runs
+// of 16/nseg planes, one workgroup each (more workgroups when few cubes are
+// resident).  A run starting at i0 > 2 first executes one prologue iteration at
+// i0 - 1 that only forms the x-face i0 - 1/2 (inviscid and viscous) the run
+// carries into its first plane: the same loop body, and so the same instructions
+// and bits, as the unsegmented march computes it with.  Norm partials are one row
+// per plane, so every result is bitwise the same for every nseg.
+//
+// Bound: vector instructions, 1,655 per cell (62% of the issue rate over the
+// launch).  Two workgroups per CU: a third (46 KB of LDS, 168 registers with 25
+// spilled) gives the same rate, 624 us on 2,048 cubes against 555.  Against a
+// march that kept the whole column in registers, two face arrays more in LDS and
+// a boundary round per axis: 570 -> 555 us on 2,048 cubes, 51 -> 45 on 125.
 __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
     const float* __restrict__ U, float* __restrict__ Uout, const HaloSrc* __restrict__ halo,
     const uint8_t* __restrict__ cube_mask, const double* __restrict__ Bsrc,
     const int8_t* __restrict__ fws, const double* __restrict__ cube_size, PhysTab pt,
     double deltaT, double deltaTau, double e_d, int RK, double* __restrict__ partials,
-    int nseg) {
-  __shared__ float cp[2][5][400];     // conserved values of plane i (double-buffered)
-  __shared__ int8_t fl[2][400];       // flags of plane i
-  __shared__ float pr[4][4][PR];      // u, v, w, T of planes (ring of 4)
-  __shared__ float fy[5][NFY];
-  __shared__ float fz[6][NF];         // flux + face pressure average
-  __shared__ float vy[4][NFY];        // viscous fluxes of the y- and z-faces
-  __shared__ float vz[4][NF];
-  __shared__ float esrc[2][8][5];     // corner sources of interior planes (by parity)
+    Runs runs, int ncube) {
+  __shared__ __align__(16) float cp[2][5 * 400];   // conserved values of planes i, i+1
+  __shared__ int8_t fl[2][400];                    // flags of planes i, i+1
+  __shared__ float pr[4][3 * PR];                  // u, v, w, T of planes i-1..i+1
+  __shared__ float fy[9][NFY];                     // y-faces: flux, viscous flux
+  __shared__ float fzb[10][16];                    // z-faces before k = 2: flux, pressure, viscous
+  __shared__ double red[WG / 64][8];               // RK 3: norm sums of the waves
 
-  const int seg = blockIdx.x % nseg;
-  const int c = blockIdx.x / nseg + 1;
+  const RunOf run = run_of(runs, blockIdx.x);
+  const int c = run.cube, seg = run.seg;
+  if (c >= ncube) return;
   const int cc = pt.cube_case[c];
   if (cc < 0) return;
   const DevPhys ph = pt.phys[cc];
-  // Planes i0..i1 of this run; the march starts at `start` (a prologue
-  // iteration at i0 - 1 for runs after the first).
-  const int len = 16 / nseg;
+  // Planes i0..i1 of this run; the march starts at `start`.
+  const int len = 16 / run.nseg;
   const int i0 = 2 + seg * len, i1 = i0 + len - 1;
   const int start = i0 == 2 ? 2 : i0 - 1;
-  const int t = threadIdx.x;
-  const int j = 2 + (t >> 6) + 4 * ((t >> 4) & 3), k = (t & 15) + 2;
-  const int col = j * 20 + k;
-  // Border work goes to waves 0 and 3, whose face pass has no boundary
-  // round: of a staged plane's 144 border cells, s20a (wave 0: 0..63, wave 3:
-  // 64..127) and s20b (wave 3: 128..143); of a primitive plane's 68 border
-  // cells, s18 (wave 0: 0..63, wave 3: 64..67); -1 for none.  c20a, c20b and
-  // c18 are the cells.
-  const int s20a = t < 64 ? t : (t >= 192 ? t - 128 : -1);
-  const int s20b = t >= 196 && t < 212 ? t - 68 : -1;
-  const int s18 = t < 64 ? t : (t >= 192 && t < 196 ? t - 128 : -1);
-  const int c20a = border20(s20a < 0 ? 0 : s20a), c20b = border20(s20b < 0 ? 0 : s20b);
-  const int c18 = border18(s18 < 0 ? 0 : s18);
   const double dxd = cube_size[c] / 16;
   const float inv = (float)(1.0 / dxd), vol = (float)(dxd * dxd * dxd);
   const float e = (float)e_d;
   const RefF rf = make_ref(ph);
-  double uref[5];
-  ref_state(ph, uref);
   const float iT0 = (float)(1.0 / ph.T0), muL = (float)ph.mu_L;
   const float sut = (float)(ph.T0 + 110.);
   const double i2dT = 1.0 / (2 * deltaT);
   const float dT = (float)deltaT, dtau = (float)deltaTau;
   const float* __restrict__ Uc = U + (size_t)c * CUBE_STRIDE;
-  float* __restrict__ Oc = Uout + (size_t)c * CUBE_STRIDE;
   const HaloSrc hs = halo[c];
   const int8_t* __restrict__ Fc = fws + (size_t)c * PLANE;
   // ZBC_IN_FLUX faces: the z-ghost cells (k = 0, 1 or 18, 19) of the interior
-  // planes are read as the z-BC sets them, from the cell k = 2 (w negated) or
-  // 17 of the same row.  Prefetched border values take the redirected address
-  // at once and the negation when they are used.
+  // planes are taken as the z-BC sets them, from the cell k = 2 (w negated) or
+  // 17 of the same row.
   const int zm = cube_mask[c];
   const bool zlo = (zm & ZBC_IN_FLUX) != 0, zhi = (zm & (ZBC_IN_FLUX << 1)) != 0;
-  auto zsrc = [&](int cell, bool& neg) {
-    neg = false;
-    if (!(zlo || zhi)) return cell;
-    const int kk = cell % 20;
-    if (zlo && kk < 2 && cell >= 800 && cell < 7200) {
-      neg = true;
-      return cell - kk + 2;
-    }
-    if (zhi && kk > 17 && cell >= 800 && cell < 7200) return cell - kk + 17;
-    return cell;
-  };
-  const double r3 = uref[3];
-  const size_t gcol = (size_t)c * CUBE_STRIDE + col;
-  // Own column: w[m] = plane i-3+m, fw[m] = flag of plane i-2+m (plane -1,
-  // before the first ghost plane, is a placeholder no stencil uses).
-  // The leading plane of each (w[6], fw[4]) is loaded at the top of the
-  // iteration; its first use, the x-face, comes after the face pass.
-  float w[7][5];
-  int fw[5];
-#pragma unroll
-  for (int m = 0; m < 6; ++m)
-#pragma unroll
-    for (int v = 0; v < 5; ++v)
-      w[m][v] = start - 3 + m >= 0 ? Uc[v * PLANE + (start - 3 + m) * 400 + col] : 1.f;
-#pragma unroll
-  for (int m = 0; m < 4; ++m) fw[m] = Fc[(start - 2 + m) * 400 + col];
+  const double r3 = ph.rho0 * ph.W0;
 
-  // Deviations of the viscous block's primitives u, v, w and T = P/(rho R)
-  // from the reference state: dT = (dP - (P0/rho0) drho) / (rho R).
-  auto prims = [&](const float (&q)[5], float& u, float& v, float& ww, float& T) {
+  // The lane's cell, re-formed at the top of every plane iteration (below).
+  int t = threadIdx.x;
+  int j, k, col;
+  auto lane = [&] {
+    j = 2 + (t >> 6) + 4 * ((t >> 4) & 3);
+    k = (t & 15) + 2;
+    col = j * 20 + k;
+  };
+  lane();
+  // The wave whose lanes 0..31 evaluate the faces next to the first ghost
+  // layers (an extra round), and the one that forms the border primitives:
+  // another wave for every workgroup, so that each SIMD has its share.
+  const int wbnd = (blockIdx.x / 8) & 3, wbrd = wbnd ^ 2;
+
+  // Plane p's conserved values from memory straight into buffer p & 1: 500
+  // pieces of 16 bytes, piece q of a wave to the wave's LDS base (m0) + 16
+  // lane.  In asm, since the compiler would wait for the copy before the next
+  // read of any LDS array; wait_loads and a barrier stand between a copy and
+  // its readers.
+  auto stage = [&](int p) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const unsigned q = t + h * WG;
+      if (q < 500) {
+        const unsigned off = q / 100 * (4 * PLANE) + q % 100 * 16;
+        const unsigned dst = __builtin_amdgcn_readfirstlane(
+            (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)&cp[p & 1][0] +
+            16 * ((t & ~63) + h * WG));
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     :: "s"(dst), "v"(off), "s"(Uc + p * 400)
+                     : "memory");
+      }
+    }
+  };
+  auto wait_loads = [] { __builtin_amdgcn_s_waitcnt(0xF70); };   // vmcnt(0)
+  auto column = [&](int p, float (&q)[5]) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = at_byte(Uc + v * PLANE + p * 400, 4u * col);
+  };
+  // ZBC_IN_FLUX: the staged plane's z-ghost cells, 4 per row of 20.
+  auto fix_z = [&](int p) {
+    const int row = t >> 2, q = t & 3;
+    if (t >= 80 || !(q < 2 ? zlo : zhi)) return;
+    float* b = cp[p & 1] + row * 20;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      const float x = b[v * 400 + (q < 2 ? 2 : 17)];
+      b[v * 400 + (q < 2 ? q : q + 16)] = v == 3 && q < 2 ? zbc_neg(x, r3) : x;
+    }
+  };
+  // Deviations of the viscous block's primitives u, v, w and T = P/(rho R) of a
+  // cell from the reference state, into ring offset o:
+  // dT = (dP - (P0/rho0) drho) / (rho R).
+  auto put_prims = [&](int o, const float (&q)[5]) {
     Side sd;
     side(q, rf, sd);
-    u = sd.du[0];
-    v = sd.du[1];
-    ww = sd.du[2];
-    T = (sd.dP - rf.PoR * q[0]) * sd.ir * IRGf;
+    pr[0][o] = sd.du[0];
+    pr[1][o] = sd.du[1];
+    pr[2][o] = sd.du[2];
+    pr[3][o] = (sd.dP - rf.PoR * q[0]) * sd.ir * IRGf;
   };
-  // Primitive plane p into ring slot p & 3: the own cell from the column
-  // window (own holds plane p).
-  auto fill_own = [&](int p, const float (&own)[5]) {
-    float* dst = &pr[p & 3][0][0];
-    float u, v, ww, T;
-    prims(own, u, v, ww, T);
-    const int o = ring_idx(j, k);
-    dst[o] = u;
-    dst[PR + o] = v;
-    dst[2 * PR + o] = ww;
-    dst[3 * PR + o] = T;
-  };
-  // The border cells of primitive plane p from bq, their conserved values
-  // loaded beforehand.
-  auto fill_border = [&](int p, const float (&bq)[5]) {
-    float* dst = &pr[p & 3][0][0];
-    float u, v, ww, T;
-    if (s18 >= 0) {
-      const int cell = c18;
-      float q[5];
+  // Border cells of a primitive plane other than its corners: lane l of wave
+  // wbrd.  Their conserved values are loaded a phase before they are used.  In
+  // the ghost planes 1 and 18 they are edge ghost cells, the mean of two face
+  // ghost cells (loaded where they are used, once per cube each).
+  const int bl = t & 63, bm = (bl & 15) + 2;
+  const int bj = bl < 16 ? 1 : bl < 32 ? 18 : bm, bk = bl < 32 ? bm : bl < 48 ? 1 : 18;
+  const bool border = (t >> 6) == wbrd;
+  // A border cell of an interior plane as ZBC_IN_FLUX faces have it.
+  const bool blo = zlo && bk == 1, bhi = zhi && bk == 18;
+  const int bcell = bj * 20 + (blo ? 2 : bhi ? 17 : bk);
+  auto load_border = [&](int p, float (&q)[5]) {
+    if (border && p >= 2 && p <= 17)
 #pragma unroll
-      for (int m = 0; m < 5; ++m) q[m] = bq[m];
+      for (int v = 0; v < 5; ++v) q[v] = at_byte(Uc + v * PLANE + p * 400, 4u * bcell);
+  };
+  auto fill_border = [&](int p, int slot, float (&q)[5]) {
+    if (!border) return;
+    if (p == 1 || p == 18) {
       int ea, eb;
-      if (p == 1 || p == 18) {
-        // Ghost planes: the border cells other than the cube corners are
-        // edge ghost cells, the mean of two face ghost cells.
-        if (edge_sources(p, cell / 20, cell % 20, ea, eb)) {
-          bool na, nb;
-          ea = zsrc(ea, na);
-          eb = zsrc(eb, nb);
+      edge_sources(p, bj, bk, ea, eb);   // true: no corner among these cells
+      // eb lies in the interior plane 2 or 17, ea in the ghost plane.
+      if (blo || bhi) eb += blo ? 1 : -1;
 #pragma unroll
-          for (int m = 0; m < 5; ++m) {
-            const float x = Uc[m * PLANE + ea], y = Uc[m * PLANE + eb];
-            q[m] = 0.5f * ((m == 3 && na ? zbc_neg(x, r3) : x) + (m == 3 && nb ? zbc_neg(y, r3) : y));
-          }
-        }
-      } else {
-        if (zlo && cell % 20 == 1) q[3] = zbc_neg(q[3], r3);
-        // Interior planes: the sources of the plane's corners, edge ghost
-        // cells formed by corner_prims.
-        const int es = corner_source_slot(s18);
-        if (es >= 0) {
-#pragma unroll
-          for (int m = 0; m < 5; ++m) esrc[p & 1][es][m] = q[m];
-        }
+      for (int v = 0; v < 5; ++v) {
+        const float x = Uc[v * PLANE + ea], y = Uc[v * PLANE + eb];
+        q[v] = 0.5f * (x + (v == 3 && blo ? zbc_neg(y, r3) : y));
       }
-      prims(q, u, v, ww, T);
-      const int ob = ring_idx(cell / 20, cell % 20);
-      dst[ob] = u;
-      dst[PR + ob] = v;
-      dst[2 * PR + ob] = ww;
-      dst[3 * PR + ob] = T;
+    } else if (blo) {
+      q[3] = zbc_neg(q[3], r3);
     }
+    put_prims(slot + ring_idx(bj, bk), q);
   };
-  // The four corners of interior plane p are edge ghost cells: the mean of
-  // two face ghost cells each, as the pre-flux exchange's edge passes would
-  // leave them (no edge pass runs between the stage's face updates and this
-  // kernel).  Only the plane's own face pass reads them; four lanes with one
-  // face fewer to evaluate form them from the sources fill_border kept.
-  auto corner_prims = [&](int p) {
-    const int q4 = t - (WG - 4);
-    if (q4 < 0) return;
+  // The four corners of interior plane p, edge ghost cells that only the
+  // plane's own viscous faces read, from the staged plane.
+  auto fill_corners = [&](int p, int slot) {
+    const int l = t & 63;
+    if ((t >> 6) != (wbrd ^ 1) || l >= 4) return;
+    const float* b = cp[p & 1];
+    const int jj = l & 2 ? 18 : 1, kk = l & 1 ? 18 : 1, jn = l & 2 ? 17 : 2, kn = l & 1 ? 17 : 2;
+    const bool lo = zlo && kk == 1, hi = zhi && kk == 18;
     float q[5];
 #pragma unroll
-    for (int m = 0; m < 5; ++m) q[m] = 0.5f * (esrc[p & 1][2 * q4][m] + esrc[p & 1][2 * q4 + 1][m]);
-    float u, v, ww, T;
-    prims(q, u, v, ww, T);
-    const int o = ring_idx(q4 & 2 ? 18 : 1, q4 & 1 ? 18 : 1);
-    float* dst = &pr[p & 3][0][0];
-    dst[o] = u;
-    dst[PR + o] = v;
-    dst[2 * PR + o] = ww;
-    dst[3 * PR + o] = T;
+    for (int v = 0; v < 5; ++v) {
+      const float x = b[v * 400 + jj * 20 + kn], y = b[v * 400 + jn * 20 + (lo || hi ? kn : kk)];
+      q[v] = 0.5f * (x + (v == 3 && lo ? zbc_neg(y, r3) : y));
+    }
+    put_prims(slot + ring_idx(jj, kk), q);
   };
-  // Border values are loaded one iteration ahead of their use: bcp/bfl (and
-  // bcq/bfq) the border cells of a plane to stage, bpr those of a primitive
-  // plane.
-  auto load_b18 = [&](int p, float (&q)[5]) {
-    if (s18 >= 0 && p <= 19) {
-      bool neg;
-      const int src = zsrc(p * 400 + c18, neg);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) q[v] = Uc[v * PLANE + src];
-    }
+  int fo[2] = {0, 0};   // the lane's two flags of the plane to stage
+  auto load_flags = [&](int p) {
+    fo[0] = Fc[p * 400 + (unsigned)t];
+    if (t < 400 - WG) fo[1] = Fc[p * 400 + WG + (unsigned)t];
   };
-  auto load_b20 = [&](int p, float (&qa)[5], int& fa, float (&qb)[5], int& fb) {
-    if (p > 17) return;
-    bool neg;
-    if (s20a >= 0) {
-      const int src = zsrc(p * 400 + c20a, neg);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) qa[v] = Uc[v * PLANE + src];
-      fa = Fc[p * 400 + c20a];
-    }
-    if (s20b >= 0) {
-      const int src = zsrc(p * 400 + c20b, neg);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) qb[v] = Uc[v * PLANE + src];
-      fb = Fc[p * 400 + c20b];
-    }
+  auto store_flags = [&](int p) {
+    fl[p & 1][t] = (int8_t)fo[0];
+    if (t < 400 - WG) fl[p & 1][WG + t] = (int8_t)fo[1];
   };
-  // The border cells of plane p into its staging buffer.
-  auto stage_border = [&](int p, const float (&qa)[5], int fa, const float (&qb)[5], int fb) {
-    if (s20a >= 0) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v)
-        cp[p & 1][v][c20a] = v == 3 && zlo && c20a % 20 < 2 ? zbc_neg(qa[v], r3) : qa[v];
-      fl[p & 1][c20a] = (int8_t)fa;
-    }
-    if (s20b >= 0) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v)
-        cp[p & 1][v][c20b] = v == 3 && zlo && c20b % 20 < 2 ? zbc_neg(qb[v], r3) : qb[v];
-      fl[p & 1][c20b] = (int8_t)fb;
-    }
-  };
-  // Before the march: primitive planes start-1, start and the border of
-  // start+1; the border of the first staged plane.  In the march, iteration
-  // i stages plane i's own cells and forms plane i+1's own primitives before
-  // its face pass; during the face pass waves 0 and 3 stage the border of
-  // plane i+1 and form the border primitives of plane i+2.
-  float bcp[5] = {0, 0, 0, 0, 0}, bcq[5] = {0, 0, 0, 0, 0}, bpr[5] = {1, 0, 0, 0, 0};
-  int bfl = 0, bfq = 0;
-  load_b18(start - 1, bpr);
-  fill_own(start - 1, w[2]);
-  fill_border(start - 1, bpr);
-  load_b18(start, bpr);
-  fill_own(start, w[3]);
-  fill_border(start, bpr);
-  load_b18(start + 1, bpr);
-  fill_border(start + 1, bpr);
-  if (start >= i0) {
-    load_b20(start, bcp, bfl, bcq, bfq);
-    stage_border(start, bcp, bfl, bcq, bfq);
-  }
-  __syncthreads();
-  corner_prims(start);
-  load_b20(start + 1, bcp, bfl, bcq, bfq);
-  load_b18(start + 2, bpr);
 
-  float cF[5] = {0, 0, 0, 0, 0}, cdP = 0.f;
-  float cL[4] = {0, 0, 0, 0};   // viscous x-face flux carried from the previous plane
+  // ---- before the march: plane `start` staged, primitives of start-1, start
+  // and start+1, the column's registers ----
+  float p2[5], p1[5], n2[5];   // the lane's column cells of planes i-2, i-1, i+2
+  float bq[5] = {1, 0, 0, 0, 0};   // border cell of plane i+2
+  unsigned fb = 0;             // flags of planes i-2..i+2 equal to 1, bits 0..4
+  {
+    stage(start);
+    load_flags(start);
+    float own[2][5], b0[5] = {1, 0, 0, 0, 0}, b1[5] = {1, 0, 0, 0, 0}, b2[5] = {1, 0, 0, 0, 0};
+    column(start - 2, p2);
+    column(start - 1, p1);
+    column(start, own[0]);
+    column(start + 1, own[1]);
+    column(start + 2, n2);
+    load_border(start - 1, b0);
+    load_border(start, b1);
+    load_border(start + 1, b2);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) fb |= (Fc[(start - 2 + m) * 400 + (unsigned)col] == 1) << m;
+    const int o = ring_idx(j, k);
+    put_prims(o, p1);
+    put_prims(PR + o, own[0]);
+    put_prims(2 * PR + o, own[1]);
+    fill_border(start - 1, 0, b0);
+    fill_border(start, PR, b1);
+    fill_border(start + 1, 2 * PR, b2);
+    store_flags(start);
+    wait_loads();
+    __syncthreads();
+    // (Interior planes only: ghost planes' z-ghost cells are as the BCs left
+    // them, and no run starts there.)
+    if (zlo || zhi) fix_z(start);
+    fill_corners(start, PR);
+    __syncthreads();
+  }
+  float cF[5] = {0, 0, 0, 0, 0}, cdP = 0.f;   // x-face before plane i
+  float cL[4] = {0, 0, 0, 0};                 // and its viscous flux
   int corder = -1;
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+  int sl0 = 0, sl1 = PR, sl2 = 2 * PR;        // ring slots of planes i-1, i, i+1
 
 #pragma unroll 1
   for (int i = start; i <= i1; ++i) {
-    const int b = i & 1;
+    // The lane index passes through an empty asm statement, so the quantities
+    // derived from it are computed inside the iteration that uses them rather
+    // than held across it.
+    asm volatile("" : "+v"(t));
+    lane();
     const bool pro = i < i0;    // prologue: only the x-face i + 1/2
-    // Planes beyond the last ghost plane repeat it (a finite placeholder no
-    // stencil uses).
-#pragma unroll
-    for (int v = 0; v < 5; ++v) w[6][v] = Uc[v * PLANE + min(i + 3, 19) * 400 + col];
-    fw[4] = Fc[(i + 2) * 400 + col];
-    // ---- stage plane i's own cells, primitives of plane i+1's own cells ----
+    const float* __restrict__ cpi = cp[i & 1];
+    const int8_t* __restrict__ fli = fl[i & 1];
+    const int ro = ring_idx(j, k);
+
+    // ---- phase 1: y- and z-faces of plane i ----
+    stage(i + 1);
+    load_flags(i + 1);
+    float n3[5];
+    column(min(i + 3, 19), n3);   // (plane 20 is not used: order 3 or 1 there)
+    const int f2 = Fc[(i + 2) * 400 + (unsigned)col];
+    load_border(i + 2, bq);
+    // The viscous x-face before plane 2 (plane 1's ring slot is refilled in
+    // phase 2).
+    if (i == 2) visc_face<0>(pr, 0, sl0 + ro, sl1 + ro, rf, inv, iT0, muL, sut, cL);
+    float zF[5], dPzf, zL[4];
     if (!pro) {
+      const int8_t* f = fli + col;
+      float L[5], R[5], F[5], dP, Lv[4];
+      plane_states(cpi, col, 20, order_fwd(j, f[-20], f[20], f[40]), L, R);
+      roe_f<1>(L, R, e, rf, F, dP);
+      visc_face<1>(pr, sl0 + ro, sl1 + ro, sl2 + ro, rf, inv, iT0, muL, sut, Lv);
+      const int g = fy_idx(j, k);
 #pragma unroll
-      for (int v = 0; v < 5; ++v) cp[b][v][col] = w[3][v];
-      fl[b][col] = (int8_t)fw[2];
+      for (int v = 0; v < 5; ++v) fy[v][g] = F[v];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) fy[5 + v][g] = Lv[v];
+      plane_states(cpi, col, 1, order_fwd(k, f[-1], f[1], f[2]), L, R);
+      roe_f<2>(L, R, e, rf, zF, dPzf);
+      visc_face<2>(pr, sl0 + ro, sl1 + ro, sl2 + ro, rf, inv, iT0, muL, sut, zL);
+      // The 16 y-faces and 16 z-faces next to the first ghost layers.
+      if ((t >> 6) == wbnd && (t & 63) < 32) {
+        const bool ydir = t & 16;
+        const int a = (t & 15) + 2, st = ydir ? 20 : 1;
+        const int base = ydir ? 20 + a : a * 20 + 1;
+        const int rb = ydir ? ring_idx(1, a) : ring_idx(a, 1);
+        const int8_t* fa = fli + base;
+        plane_states(cpi, base, st, order_bwd(2, fa[-st], fa[0], fa[2 * st]), L, R);
+        roe_f<3>(L, R, e, rf, F, dP, ydir);
+        visc_face<3>(pr, sl0 + rb, sl1 + rb, sl2 + rb, rf, inv, iT0, muL, sut, Lv, ydir);
+        if (ydir) {
+          const int gb = fy_idx(1, a);
+#pragma unroll
+          for (int v = 0; v < 5; ++v) fy[v][gb] = F[v];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) fy[5 + v][gb] = Lv[v];
+        } else {
+#pragma unroll
+          for (int v = 0; v < 5; ++v) fzb[v][a - 2] = F[v];
+          fzb[5][a - 2] = dP;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) fzb[6 + v][a - 2] = Lv[v];
+        }
+      }
     }
-    fill_own(i + 1, w[4]);
-    // This cell's FP64 source constant Bv = 3 Uref - 4 U1 + U1q, first used
-    // in the residual after the face pass.
+    wait_loads();
+    __syncthreads();
+
+    // ---- phase 2 ----
+    if (RK == 3 && i > i0 && t < 8) {
+      double s = red[0][t];
+#pragma unroll
+      for (int w = 1; w < WG / 64; ++w) s += red[w][t];
+      partials[((size_t)(c - 1) * MIXED_ROWS_PER_CUBE + (i - 3)) * 8 + t] = s;
+    }
+    // This cell's FP64 source constant Bv = 3 Uref - 4 U1 + U1q, first used in
+    // the residual.
+    const size_t row = (size_t)c * CUBE_STRIDE + i * 400;
     double Bv[5] = {0, 0, 0, 0, 0};
     if (!pro) {
-      const size_t gb = gcol + (size_t)i * 400;
 #pragma unroll
-      for (int v = 0; v < 5; ++v) Bv[v] = Bsrc[gb + (size_t)v * PLANE];
+      for (int v = 0; v < 5; ++v) Bv[v] = at_byte(Bsrc + row + v * PLANE, 8u * col);
     }
-    __syncthreads();
-
-    // ---- y- and z-faces of plane i: 272 + 272 faces over 256 lanes ----
-    if (i + 1 <= 17) corner_prims(i + 1);
-    // Border work for later planes (waves 0 and 3), and its loads for the
-    // next iteration.  Plane i+1's staging buffer last held plane i-1, whose
-    // readers all passed this iteration's first barrier; ring slot i+2 last
-    // held plane i-2.
-    if (i + 1 <= i1) stage_border(i + 1, bcp, bfl, bcq, bfq);
-    if (i + 2 <= i1 + 1) fill_border(i + 2, bpr);
-    if (i + 2 <= i1) load_b20(i + 2, bcp, bfl, bcq, bfq);
-    if (i + 3 <= i1 + 1) load_b18(i + 3, bpr);
-    // Round 0: each lane the y-face above its cell; round 1: the z-face above
-    // it (every wave evaluates one face kind at a time); rounds 2 and 3: the
-    // 16 y-faces and the 16 z-faces between the first ghost layer and the
-    // first interior cells, on lanes of two different waves.  One face per
-    // loop iteration keeps the faces' working sets apart.
-#pragma unroll 1
-    for (int r = pro ? 4 : 0; r < 4; ++r) {
-      const bool bnd = r >= 2;
-      const int l0 = r == 2 ? BND_Y : BND_Z;
-      if (bnd && (t < l0 || t >= l0 + 16)) continue;
-      if ((r & 1) == 0)
-        yz_face<1>(cp[b], fl[b], pr, i, bnd ? t - l0 + 2 : k, bnd ? 1 : j, e, rf, inv, iT0, muL,
-                   sut, &fy[0][0], &vy[0][0]);
-      else
-        yz_face<2>(cp[b], fl[b], pr, i, bnd ? t - l0 + 2 : j, bnd ? 1 : k, e, rf, inv, iT0, muL,
-                   sut, &fz[0][0], &vz[0][0]);
+    // Primitives of plane i+2 into the ring slot of plane i-1, whose last
+    // readers were the viscous y- and z-faces of plane i.
+    store_flags(i + 1);
+    if (i + 2 <= i1 + 1) {
+      put_prims(sl0 + ro, n2);
+      fill_border(i + 2, sl0, bq);
     }
-    __syncthreads();
-
-    const int IF = fw[2];
+    if (i < i1) {
+      fill_corners(i + 1, sl2);
+      if (zlo || zhi) fix_z(i + 1);
+    }
+    float u[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) u[v] = cpi[v * 400 + col];
+    fb |= (unsigned)(f2 == 1) << 4;
+    const auto is = [&](int m) { return (int)(fb >> m & 1); };
     // ---- inviscid x: forward face from the column, backward carried ----
-    float Rx[5], Ry[5], Rz[5], dPxb, dPxf, dPzb, dPzf;
+    float Rx[5], px, pz;   // px, pz: face pressure differences
     {
-      // Column cells an order does not use hold finite values (placeholder
-      // planes beyond the cube repeat a loaded one).
-      const int of = order_fwd(i, fw[1], fw[3], fw[4]);
-      float L[5], R[5], Ff[5];
-      const ReconW rwf = recon_weights(of);
+      float n1[5];
+      const float* cpn = cp[~i & 1];
 #pragma unroll
-      for (int v = 0; v < 5; ++v)
-        recon(rwf, w[1][v], w[2][v], w[3][v], w[4][v], w[5][v], w[6][v], L[v], R[v]);
-      roe_f(L, R, 0, e, rf, Ff, dPxf);
-      const int ob = order_bwd(i, fw[0], fw[1], fw[3]);
-      if (pro) {
-      } else if (i != 2 && ob == corder) {
-        dPxb = cdP;
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Rx[v] = Ff[v] - cF[v];
-      } else {
-        float Fb[5];
-        const ReconW rwb = recon_weights(ob);
-#pragma unroll
-        for (int v = 0; v < 5; ++v)
-          recon(rwb, w[0][v], w[1][v], w[2][v], w[3][v], w[4][v], w[5][v], L[v], R[v]);
-        roe_f(L, R, 0, e, rf, Fb, dPxb);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Rx[v] = Ff[v] - Fb[v];
+      for (int v = 0; v < 5; ++v) n1[v] = cpn[v * 400 + col];
+      auto at = [&](int m, int v) {
+        return m == 0 ? p2[v] : m == 1 ? p1[v] : m == 2 ? u[v] : m == 3 ? n1[v] : m == 4 ? n2[v] : n3[v];
+      };
+      const int of = order_fwd(i, is(1), is(3), is(4));
+      float L[5], R[5], Ff[5], dPf;
+      face_states(of, at, L, R);
+      roe_f<0>(L, R, e, rf, Ff, dPf);
+      const int ob = order_bwd(i, is(0), is(1), is(3));
+      if (!pro && (i == 2 || ob != corder)) {
+        float q3[5];
+        column(max(i - 3, 0), q3);   // (plane -1 is not used: order 3 or 1)
+        face_states(ob, [&](int m, int v) { return m == 0 ? q3[v] : at(m - 1, v); }, L, R);
+        roe_f<0>(L, R, e, rf, cF, cdP);
       }
 #pragma unroll
-      for (int v = 0; v < 5; ++v) cF[v] = Ff[v];
-      cdP = dPxf;
+      for (int v = 0; v < 5; ++v) {
+        Rx[v] = Ff[v] - cF[v];
+        cF[v] = Ff[v];
+      }
+      px = dPf - cdP;
+      cdP = dPf;
       corder = of;
     }
-    const int8_t* fc = fl[b] + col;
-    // ---- inviscid y ----
-    if (!pro) {
-      const int fm2 = fc[-40], fm1 = fc[-20], fp1 = fc[20];
-      const int ff = fy_idx(j, k), fb = fy_idx(j - 1, k);
-      const int ob = order_bwd(j, fm2, fm1, fp1);
-      if (j == 2 || ob == order_fwd(j - 1, fm2, fc[0], fp1)) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Ry[v] = fy[v][ff] - fy[v][fb];
-      } else {
-        float Fb[5], dPu;
-        plane_face<1>(cp[b], col - 20, ob, e, rf, Fb, dPu);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Ry[v] = fy[v][ff] - Fb[v];
-      }
-    }
-    // ---- inviscid z ----
-    if (!pro) {
-      const int fm2 = fc[-2], fm1 = fc[-1], fp1 = fc[1];
-      const int ff = fz_idx(j, k);   // the backward face is ff - 1
-      const int ob = order_bwd(k, fm2, fm1, fp1);
-      dPzf = fz[5][ff];
-      if (k == 2 || ob == order_fwd(k - 1, fm2, fc[0], fp1)) {
-        dPzb = fz[5][ff - 1];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Rz[v] = fz[v][ff] - fz[v][ff - 1];
-      } else {
-        float Fb[5];
-        plane_face<2>(cp[b], col - 1, ob, e, rf, Fb, dPzb);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Rz[v] = fz[v][ff] - Fb[v];
-      }
-    }
-
-    // ---- viscous (Flux.cpp:1722-2279): x-face carried, y/z faces shared ----
     float vF[5] = {0, 0, 0, 0, 0};
     {
       float Lf[4];
-      visc_face<0>(pr, i, 0, j, k, rf, inv, iT0, muL, sut, Lf);
-      if (i == 2) visc_face<0>(pr, i, -1, j, k, rf, inv, iT0, muL, sut, cL);
-      if (!pro) {
-        const int fyf = fy_idx(j, k), fyb = fy_idx(j - 1, k), fzf = fz_idx(j, k);
+      visc_face<0>(pr, 0, sl1 + ro, sl2 + ro, rf, inv, iT0, muL, sut, Lf);
 #pragma unroll
-        for (int v = 1; v < 5; ++v)
-          vF[v] = ((Lf[v - 1] - cL[v - 1]) + (vy[v - 1][fyf] - vy[v - 1][fyb]) +
-                   (vz[v - 1][fzf] - vz[v - 1][fzf - 1])) * inv;
+      for (int v = 0; v < 4; ++v) {
+        vF[v + 1] = Lf[v] - cL[v];
+        cL[v] = Lf[v];
       }
-#pragma unroll
-      for (int v = 0; v < 4; ++v) cL[v] = Lf[v];
     }
     if (!pro) {
-
-    // ---- residual with the FP64 dual-time source ----
-    float u[5];
+      const int8_t* f = fli + col;
+      const int IF = f[0];
+      float Ry[5], Rz[5];
+      {
+        float Fb[5], dPu;
+        const int ff = fy_idx(j, k), fbk = fy_idx(j - 1, k);
+        const int ob = order_bwd(j, f[-40], f[-20], f[20]);
+        if (j == 2 || ob == order_fwd(j - 1, f[-40], f[0], f[20])) {
 #pragma unroll
-    for (int v = 0; v < 5; ++v) u[v] = w[3][v];
-    float Rk[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      const double Rp = -(3.0 * (double)u[v] + Bv[v]) * i2dT;
-      const float Rf = -(Rx[v] + Ry[v] + Rz[v]) * inv + (v == 0 ? 0.f : vF[v]);
-      Rk[v] = (float)(Rp + (double)Rf);
-    }
-
-    // ---- preconditioned increment (Flux.cpp:2295-2375) and RK update ----
-    float nv[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) nv[v] = u[v];
-    if (IF == 1) {
-      Side me;
-      side(w[3], rf, me);
-      const float U_ = me.u[0], V_ = me.u[1], W_ = me.u[2];
-      const float irho = me.ir;
-      const float VV = U_ * U_ + V_ * V_ + W_ * W_;
-      const float P = me.P;
-      const float C = KGf * P * irho;
-      const float T = P * irho;
-      const float H = 0.5f * VV + C * IKM1f;
-      const float beta = fmaxr(VV * frcp(C), e);
-      const float bm1 = beta - 1;
-      const float itemp = frcp(KGf * T * (2 * dT + 3 * dtau) * (2 * dT + 3 * beta * dtau));
-      const float temp2 = KM1f * bm1 * dT * dT;
-      const float temp3 = H - H * KGf - VV + KGf * (T + VV);
-      const float kTbt = 3 * KGf * T * beta * dtau;
-      const float a4 = 4 * temp2 * itemp;              // 4 temp2 / temp
-      const float b4 = 4 * temp3 * bm1 * dT * dT * itemp;
-      const float d11 = 2 * dT * (-2 * (-KM1f * (H - VV) - temp3 * beta) * dT + kTbt) * itemp;
-      const float dmm[3] = {
-          2 * dT * (2 * KGf * (T - U_ * U_ * bm1) * dT + 2 * U_ * U_ * bm1 * dT + kTbt) * itemp,
-          2 * dT * (2 * KGf * (T - V_ * V_ * bm1) * dT + 2 * V_ * V_ * bm1 * dT + kTbt) * itemp,
-          2 * dT * (2 * KGf * (T - W_ * W_ * bm1) * dT + 2 * W_ * W_ * bm1 * dT + kTbt) * itemp};
-      const float d55 = 2 * dT * (2 * H * KM1f * bm1 * dT + KGf * T * (2 * dT + 3 * beta * dtau)) * itemp;
-      const float vel[3] = {U_, V_, W_};
-      // Row 0: d11, -a4 U, -a4 V, -a4 W, a4.  Rows 1..3 (velocity m): b4 vm,
-      // -a4 vm vn off-diagonal, dmm on the diagonal, a4 vm.  Row 4: b4 H,
-      // -a4 H U, -a4 H V, -a4 H W, d55.
-      const float sv = U_ * Rk[1] + V_ * Rk[2] + W_ * Rk[3];
-      float out[5];
-      out[0] = dtau * (d11 * Rk[0] - a4 * sv + a4 * Rk[4]);
-#pragma unroll
-      for (int m = 0; m < 3; ++m)
-        out[m + 1] = dtau * (b4 * vel[m] * Rk[0] - a4 * vel[m] * (sv - vel[m] * Rk[m + 1]) +
-                             dmm[m] * Rk[m + 1] + a4 * vel[m] * Rk[4]);
-      out[4] = dtau * (b4 * H * Rk[0] - a4 * H * sv + d55 * Rk[4]);
-      float un[5];
-      if (RK == 1) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) un[v] = u[v] + out[v];
-      } else if (RK == 2) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) un[v] = 0.75f * u[v] + 0.25f * u[v] + 0.25f * out[v];
-      } else {
-#pragma unroll
-        for (int v = 0; v < 5; ++v)
-          un[v] = (1.0f / 3.0f) * u[v] + (2.0f / 3.0f) * u[v] + (2.0f / 3.0f) * out[v];
-      }
-#pragma unroll
-      for (int v = 0; v < 5; ++v) nv[v] = un[v];
-      if (RK == 3) {
-        // Change norms in FP64 (Flux.cpp:2530-2566).
-        double fo[5], fn[5];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) {
-          fo[v] = (double)u[v] + uref[v];
-          fn[v] = (double)un[v] + uref[v];
+          for (int v = 0; v < 5; ++v) Fb[v] = fy[v][fbk];
+        } else {
+          float L[5], R[5];
+          plane_states(cpi, col - 20, 20, ob, L, R);
+          roe_f<1>(L, R, e, rf, Fb, dPu);
         }
-        const double ro = fo[0], iro = 1.0 / ro;
-        const double uo = fo[1] * iro, vo = fo[2] * iro, wo = fo[3] * iro;
-        const double Po = (fo[4] - 0.5 * ro * (uo * uo + vo * vo + wo * wo)) * KM1d;
-        const double r = fn[0], ir = 1.0 / r;
-        const double uu = fn[1] * ir, vv = fn[2] * ir, ww = fn[3] * ir;
-        const double Pn = (fn[4] - 0.5 * r * (uu * uu + vv * vv + ww * ww)) * KM1d;
-        const double dTn = Pn * ir - Po * iro;
-        acc[0] += (Pn - Po) * (Pn - Po);
-        acc[1] += (uu - uo) * (uu - uo);
-        acc[2] += (vv - vo) * (vv - vo);
-        acc[3] += (ww - wo) * (ww - wo);
-        acc[4] += dTn * dTn;
+#pragma unroll
+        for (int v = 0; v < 5; ++v) Ry[v] = fy[v][ff] - Fb[v];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) vF[v + 1] += fy[5 + v][ff] - fy[5 + v][fbk];
       }
-    } else if (IF < 1 && RK == 3) {
-      // Force density of non-fluid cells (Flux.cpp:2395-2398), summed at RK 3.
-      acc[5] += (double)(-(-(dPxf - dPxb) * inv + vF[1]) * vol);
-      acc[6] += (double)(-(-(dPzf - dPzb) * inv + vF[3]) * vol);
-    }
-    // Every interior cell goes to Uout; cells next to a face with a
-    // neighbour also go to that neighbour's ghost layers.
-    {
-      const int o = i * 400 + col;
-      const int nx = i <= 3 ? hs.src[0] : (i >= 16 ? hs.src[1] : 0);
-      const int ny = j <= 3 ? hs.src[2] : (j >= 16 ? hs.src[3] : 0);
-      const int nz = k <= 3 ? hs.src[4] : (k >= 16 ? hs.src[5] : 0);
-      const int ox = o + (i <= 3 ? 16 * 400 : -16 * 400);
-      const int oy = o + (j <= 3 ? 16 * 20 : -16 * 20);
-      const int oz = o + (k <= 3 ? 16 : -16);
+      {
+        // The z-face behind comes from the lane behind in the row of 16, the
+        // first lane's from LDS.
+        float Fb[10];
+#pragma unroll
+        for (int v = 0; v < 10; ++v) {
+          const float x = v < 5 ? zF[v] : v == 5 ? dPzf : zL[v - 6];
+          Fb[v] = __int_as_float(__builtin_amdgcn_update_dpp(
+              __float_as_int(fzb[v][j - 2]), __float_as_int(x), 0x111, 0xf, 0xf, false));
+        }
+        const int ob = order_bwd(k, f[-2], f[-1], f[1]);
+        if (!(k == 2 || ob == order_fwd(k - 1, f[-2], f[0], f[1]))) {
+          float L[5], R[5], F[5];
+          plane_states(cpi, col - 1, 1, ob, L, R);
+          roe_f<2>(L, R, e, rf, F, Fb[5]);
+#pragma unroll
+          for (int v = 0; v < 5; ++v) Fb[v] = F[v];
+        }
+#pragma unroll
+        for (int v = 0; v < 5; ++v) Rz[v] = zF[v] - Fb[v];
+        pz = dPzf - Fb[5];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) vF[v + 1] = (vF[v + 1] + (zL[v] - Fb[6 + v])) * inv;
+      }
+
+      // ---- residual with the FP64 dual-time source ----
+      float Rk[5];
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
-        Oc[v * PLANE + o] = nv[v];
-        if (nx > 0) Uout[(size_t)nx * CUBE_STRIDE + v * PLANE + ox] = nv[v];
-        if (ny > 0) Uout[(size_t)ny * CUBE_STRIDE + v * PLANE + oy] = nv[v];
-        if (nz > 0) Uout[(size_t)nz * CUBE_STRIDE + v * PLANE + oz] = nv[v];
+        const double Rp = -(3.0 * (double)u[v] + Bv[v]) * i2dT;
+        const float Rf = -(Rx[v] + Ry[v] + Rz[v]) * inv + (v == 0 ? 0.f : vF[v]);
+        Rk[v] = (float)(Rp + (double)Rf);
       }
-    }
-    // Norm partials at the end of each group of 4 planes: one row per wave.
-    if (RK == 3 && ((i - 2) & 3) == 3) {
+
+      // ---- preconditioned increment (Flux.cpp:2295-2375) and RK update ----
+      double pn[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // the cell's norm and force terms
+      float nv[5];
 #pragma unroll
-      for (int m = 0; m < 7; ++m) acc[m] = wave_sum(acc[m]);
-      if ((t & 63) == 63) {
-        double* row =
-            partials + ((size_t)(c - 1) * MIXED_ROWS_PER_CUBE + ((i - 2) >> 2) * 4 + (t >> 6)) * 8;
+      for (int v = 0; v < 5; ++v) nv[v] = u[v];
+      if (IF == 1) {
+        Side me;
+        side(u, rf, me);
+        const float U_ = me.u[0], V_ = me.u[1], W_ = me.u[2];
+        const float irho = me.ir;
+        const float VV = U_ * U_ + V_ * V_ + W_ * W_;
+        const float P = me.P;
+        const float C = KGf * P * irho;
+        const float T = P * irho;
+        const float H = 0.5f * VV + C * IKM1f;
+        const float beta = fmaxr(VV * frcp(C), e);
+        const float bm1 = beta - 1;
+        const float itemp = frcp(KGf * T * (2 * dT + 3 * dtau) * (2 * dT + 3 * beta * dtau));
+        const float temp2 = KM1f * bm1 * dT * dT;
+        const float temp3 = H - H * KGf - VV + KGf * (T + VV);
+        const float kTbt = 3 * KGf * T * beta * dtau;
+        const float a4 = 4 * temp2 * itemp;              // 4 temp2 / temp
+        const float b4 = 4 * temp3 * bm1 * dT * dT * itemp;
+        const float d11 = 2 * dT * (-2 * (-KM1f * (H - VV) - temp3 * beta) * dT + kTbt) * itemp;
+        const float dmm[3] = {
+            2 * dT * (2 * KGf * (T - U_ * U_ * bm1) * dT + 2 * U_ * U_ * bm1 * dT + kTbt) * itemp,
+            2 * dT * (2 * KGf * (T - V_ * V_ * bm1) * dT + 2 * V_ * V_ * bm1 * dT + kTbt) * itemp,
+            2 * dT * (2 * KGf * (T - W_ * W_ * bm1) * dT + 2 * W_ * W_ * bm1 * dT + kTbt) * itemp};
+        const float d55 = 2 * dT * (2 * H * KM1f * bm1 * dT + KGf * T * (2 * dT + 3 * beta * dtau)) * itemp;
+        const float vel[3] = {U_, V_, W_};
+        // Row 0: d11, -a4 U, -a4 V, -a4 W, a4.  Rows 1..3 (velocity m): b4 vm,
+        // -a4 vm vn off-diagonal, dmm on the diagonal, a4 vm.  Row 4: b4 H,
+        // -a4 H U, -a4 H V, -a4 H W, d55.
+        const float sv = U_ * Rk[1] + V_ * Rk[2] + W_ * Rk[3];
+        float out[5];
+        out[0] = dtau * (d11 * Rk[0] - a4 * sv + a4 * Rk[4]);
 #pragma unroll
-        for (int m = 0; m < 7; ++m) row[m] = acc[m];
+        for (int m = 0; m < 3; ++m)
+          out[m + 1] = dtau * (b4 * vel[m] * Rk[0] - a4 * vel[m] * (sv - vel[m] * Rk[m + 1]) +
+                               dmm[m] * Rk[m + 1] + a4 * vel[m] * Rk[4]);
+        out[4] = dtau * (b4 * H * Rk[0] - a4 * H * sv + d55 * Rk[4]);
+        float un[5];
+        if (RK == 1) {
+#pragma unroll
+          for (int v = 0; v < 5; ++v) un[v] = u[v] + out[v];
+        } else if (RK == 2) {
+#pragma unroll
+          for (int v = 0; v < 5; ++v) un[v] = 0.75f * u[v] + 0.25f * u[v] + 0.25f * out[v];
+        } else {
+#pragma unroll
+          for (int v = 0; v < 5; ++v)
+            un[v] = (1.0f / 3.0f) * u[v] + (2.0f / 3.0f) * u[v] + (2.0f / 3.0f) * out[v];
+        }
+#pragma unroll
+        for (int v = 0; v < 5; ++v) nv[v] = un[v];
+        if (RK == 3) {
+          // Change norms in FP64 (Flux.cpp:2530-2566).
+          double uref[5], fo5[5], fn[5];
+          ref_state(ph, uref);
+#pragma unroll
+          for (int v = 0; v < 5; ++v) {
+            fo5[v] = (double)u[v] + uref[v];
+            fn[v] = (double)un[v] + uref[v];
+          }
+          const double ro5 = fo5[0], iro = 1.0 / ro5;
+          const double uo = fo5[1] * iro, vo = fo5[2] * iro, wo = fo5[3] * iro;
+          const double Po = (fo5[4] - 0.5 * ro5 * (uo * uo + vo * vo + wo * wo)) * KM1d;
+          const double r = fn[0], ir = 1.0 / r;
+          const double uu = fn[1] * ir, vv = fn[2] * ir, ww = fn[3] * ir;
+          const double Pn = (fn[4] - 0.5 * r * (uu * uu + vv * vv + ww * ww)) * KM1d;
+          const double dTn = Pn * ir - Po * iro;
+          pn[0] = (Pn - Po) * (Pn - Po);
+          pn[1] = (uu - uo) * (uu - uo);
+          pn[2] = (vv - vo) * (vv - vo);
+          pn[3] = (ww - wo) * (ww - wo);
+          pn[4] = dTn * dTn;
+        }
+      } else if (IF < 1 && RK == 3) {
+        // Force density of non-fluid cells (Flux.cpp:2395-2398), summed at RK 3.
+        pn[5] = (double)(-(-px * inv + vF[1]) * vol);
+        pn[6] = (double)(-(-pz * inv + vF[3]) * vol);
       }
+      // Every interior cell goes to Uout; cells next to a face with a
+      // neighbour also go to that neighbour's ghost layers.
+      {
+        const int nx = i <= 3 ? hs.src[0] : (i >= 16 ? hs.src[1] : 0);
+        const int ny = j <= 3 ? hs.src[2] : (j >= 16 ? hs.src[3] : 0);
+        const int nz = k <= 3 ? hs.src[4] : (k >= 16 ? hs.src[5] : 0);
+        const int o = i * 400 + col;
+        const int oy = o + (j <= 3 ? 16 * 20 : -16 * 20);
+        const int oz = o + (k <= 3 ? 16 : -16);
+        const size_t rx = (size_t)nx * CUBE_STRIDE + (i <= 3 ? i + 16 : i - 16) * 400;
 #pragma unroll
-      for (int m = 0; m < 7; ++m) acc[m] = 0.0;
-    }
+        for (int v = 0; v < 5; ++v) {
+          at_byte(Uout + row + v * PLANE, 4u * col) = nv[v];
+          if (nx > 0) at_byte(Uout + rx + v * PLANE, 4u * col) = nv[v];
+        }
+        if (ny > 0) {
+          float* O = Uout + (size_t)ny * CUBE_STRIDE + oy;
+#pragma unroll
+          for (int v = 0; v < 5; ++v) O[v * PLANE] = nv[v];
+        }
+        if (nz > 0) {
+          float* O = Uout + (size_t)nz * CUBE_STRIDE + oz;
+#pragma unroll
+          for (int v = 0; v < 5; ++v) O[v * PLANE] = nv[v];
+        }
+      }
+      if (RK == 3) {
+        const double s = wave_sum8(pn);
+        if ((t & 7) == 0) red[t >> 6][(t >> 3) & 7] = s;
+      }
     }  // !pro
 
-    // ---- advance the column window ----
+    // ---- advance the column, the flags and the ring ----
 #pragma unroll
-    for (int m = 0; m < 6; ++m)
+    for (int v = 0; v < 5; ++v) {
+      p2[v] = p1[v];
+      p1[v] = u[v];
+      n2[v] = n3[v];
+    }
+    fb >>= 1;
+    const int s = sl0;
+    sl0 = sl1;
+    sl1 = sl2;
+    sl2 = s;
+    __syncthreads();
+  }
+  if (RK == 3 && t < 8) {
+    double s = red[0][t];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) w[m][v] = w[m + 1][v];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) fw[m] = fw[m + 1];
+    for (int w = 1; w < WG / 64; ++w) s += red[w][t];
+    partials[((size_t)(c - 1) * MIXED_ROWS_PER_CUBE + (i1 - 2)) * 8 + t] = s;
   }
 
   // Ghost regions the domain BCs wrote this stage go to Uout as they are (no
   // neighbour writes them), so Uout holds them as an in-place update would.
-  if (seg == 0) {
-    const int bm = cube_mask[c];
-    if (bm) copy_bc_regions(U, Uout, c, bm, uref[3]);
-  }
+  if (seg == 0 && zm) copy_bc_regions(U, Uout, c, zm, r3);
 }
 
 __global__ __launch_bounds__(WG) void k_shift_mixed(const float* __restrict__ U,
@@ -991,10 +938,21 @@ void launch_flux_mixed(hipStream_t s, const float* Uin, float* Uout, const HaloS
                        const uint8_t* cube_mask, const double* Bsrc, const int8_t* fws,
                        const double* cube_size, int ncube, PhysTab pt, double deltaT,
                        double deltaTau, double e, int RK, double* partials, int nseg) {
-  if (ncube > 1)
-    hipLaunchKernelGGL(k_flux_mixed, dim3((ncube - 1) * nseg), dim3(WG), 0, s, Uin, Uout, halo,
-                       cube_mask, Bsrc, fws, cube_size, pt, deltaT, deltaTau, e, RK, partials,
-                       nseg);
+  if (ncube <= 1) return;
+  const Runs runs = runs_for(ncube, nseg);
+  hipLaunchKernelGGL(k_flux_mixed, run_grid(runs, ncube), dim3(WG), 0, s, Uin, Uout, halo,
+                     cube_mask, Bsrc, fws, cube_size, pt, deltaT, deltaTau, e, RK, partials, runs,
+                     ncube);
+}
+
+// Runs per cube of the mixed flux kernel; the chip holds 512 of its workgroups.
+// Most runs that fit at once to 128 cubes (8 cubes: 18 us in 16 runs, 112 in one;
+// 64: 28 in 8; 128: 45 in 4, 113 in one); above, a run's prologue stands against
+// the last wave of workgroups: 8 runs to 200 cubes (180: 68 us, 75 in 4), 4 to
+// 600 (343: 111, 128 in one; 512: 156, 159 in one), 2 to 1,600 (1,000: 279, 282
+// in one), then 1 (2,048: 552, 560 in 2).
+int mixed_runs(int n) {
+  return n <= 32 ? 16 : n <= 64 ? 8 : n <= 128 ? 4 : n <= 200 ? 8 : n <= 600 ? 4 : n <= 1600 ? 2 : 1;
 }
 
 void launch_copy_f(hipStream_t s, const float* src, float* dst, size_t n) {

@@ -16,10 +16,7 @@ LATTICES = [(1, 1, 1), (7, 1, 1), (5, 5, 4), (101, 1, 1), (10, 10, 7), (701, 1, 
 
 @pytest.mark.parametrize("dims", LATTICES, ids=lambda d: str(int(np.prod(d))))
 def test_runs_per_cube_bitwise(B, O, dims):
-    size = 1.0 / max(dims)
-    case = B.Case(B.case_params("tiny", lattice=dims, cube_size=size, ico_level=3,
-                                sphere_center=tuple(0.5 * d * size for d in dims),
-                                sphere_diameter=0.3 * min(dims) * size))
+    case = lattice_case(B, dims)
     e = B.Engine(0)
     try:
         e.load_case(case)
@@ -30,3 +27,35 @@ def test_runs_per_cube_bitwise(B, O, dims):
         assert er_close(h, ho)
     finally:
         e.close()
+
+
+def lattice_case(B, dims):
+    size = 1.0 / max(dims)
+    return B.Case(B.case_params("tiny", lattice=dims, cube_size=size, ico_level=3,
+                                sphere_center=tuple(0.5 * d * size for d in dims),
+                                sphere_diameter=0.3 * min(dims) * size))
+
+
+# 1, 32 | 33, 64 | 65, 128 | 129, 200 | 201, 600 | 601, 1,600 | 1,601 cubes
+@pytest.mark.parametrize("dims", [(1, 1, 1), (8, 4, 1), (11, 3, 1), (4, 4, 4), (13, 5, 1),
+                                  (8, 4, 4), (43, 3, 1), (8, 5, 5), (67, 3, 1), (10, 10, 6),
+                                  (601, 1, 1), (16, 10, 10), (1601, 1, 1)],
+                         ids=lambda d: str(int(np.prod(d))))
+def test_mixed_runs_by_rule_are_bitwise(B, dims):
+    # The runs the rule picks against a pinned count, on one case.
+    case = lattice_case(B, dims)
+    out = []
+    for pinned in (None, 1, 4):
+        e = B.Engine(0)
+        try:
+            e.alloc_pool(case.ncube - 1, 1, "mixed")
+            s = e.add_case(case)
+            if pinned:
+                e.set_flux(2, pinned, 0)
+            er = e.run(1, 1)[:, s, :]
+            out.append((e.case_state(s, "U1_"), er))
+        finally:
+            e.close()
+    for st, er in out[1:]:
+        assert np.array_equal(st.view(np.int64), out[0][0].view(np.int64))
+        assert np.array_equal(er.view(np.int64), out[0][1].view(np.int64))
