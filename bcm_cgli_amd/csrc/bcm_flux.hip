@@ -726,10 +726,10 @@ void launch_flux_push(hipStream_t s, const double* Uin, double* Uout, const Halo
 // Runs per cube of the pushing kernel.  The chip holds 512 of its workgroups
 // (two per CU), and a run costs one x-face pass and two primitive planes more,
 // about two thirds of a plane.  To 100 cubes a plane per run is fastest (8
-// cubes: 24 us, 166 in one run; 100: 77); to 700 four runs fill the last wave of
-// workgroups (128 cubes: 77 us, 168 in one run, 91 in 16; 512: 271, 294 in
-// one), then two (1,000 cubes: 499 us, 506 in one, 519 in four); from 1,100 on
-// the last wave matters little (2,048 cubes: 986 us, 1,004 in two).
-int push_runs(int n) { return n <= 100 ? 16 : n <= 700 ? 4 : n <= 1100 ? 2 : 1; }
+// cubes: 24 us, 166 in one run; 100: 77); to 560 four runs fill the last wave of
+// workgroups (128 cubes: 77 us, 168 in one run, 91 in 16; 512: 271, 283 in
+// one); above, one run with quartered last cubes (runs_for; 576: 286 us, 313 in
+// four; 1,000: 488, 495 in two).
+int push_runs(int n) { return n <= 100 ? 16 : n <= 560 ? 4 : 1; }
 
 }  // namespace bcm

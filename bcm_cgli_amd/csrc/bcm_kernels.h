@@ -158,7 +158,16 @@ __device__ inline RunOf run_of(const Runs& r, int block) {
 inline dim3 run_grid(const Runs& r, int ncube) {
   return dim3(r.whole + (ncube - 1 - r.whole + 7) / 8 * 8 * r.nseg);
 }
-inline Runs runs_for(int ncube, int nseg) { return Runs{0, nseg}; }
+// nseg runs per cube; with one run, the last 192 of more than 560 cubes take
+// four.  Workgroups of one CU fall out of step, and with whole cubes only the
+// last half cube's time finds half the slots empty; quarters fill them (FP64
+// 2,048 cubes 990 -> 975 us, 1,584: 799 -> 759, 800: 458 -> 400, 576: 364 -> 286;
+// mixed 552 -> 527, 454 -> 416, 256 -> 225, 216 -> 160).  128 to 256 cubes are alike;
+// 512 cost more prologues than they save.
+inline Runs runs_for(int ncube, int nseg) {
+  const int n = ncube - 1;
+  return nseg == 1 && n > 560 ? Runs{(n - 192) & ~7, 4} : Runs{0, nseg};
+}
 
 // Copies, with the threads of one workgroup, the ghost regions the domain BCs
 // of cube c write (mask bits 1 x-min, 2 x-max, 4 y-min, 8 y-max, 16 z-min,

@@ -949,10 +949,10 @@ void launch_flux_mixed(hipStream_t s, const float* Uin, float* Uout, const HaloS
 // Most runs that fit at once to 128 cubes (8 cubes: 18 us in 16 runs, 112 in one;
 // 64: 28 in 8; 128: 45 in 4, 113 in one); above, a run's prologue stands against
 // the last wave of workgroups: 8 runs to 200 cubes (180: 68 us, 75 in 4), 4 to
-// 600 (343: 111, 128 in one; 512: 156, 159 in one), 2 to 1,600 (1,000: 279, 282
-// in one), then 1 (2,048: 552, 560 in 2).
+// 560 (343: 111, 128 in one; 512: 156, 159 in one), then one with quartered last
+// cubes (runs_for; 576: 160, 183 in 4; 1,000: 273, 279 in 2).
 int mixed_runs(int n) {
-  return n <= 32 ? 16 : n <= 64 ? 8 : n <= 128 ? 4 : n <= 200 ? 8 : n <= 600 ? 4 : n <= 1600 ? 2 : 1;
+  return n <= 32 ? 16 : n <= 64 ? 8 : n <= 128 ? 4 : n <= 200 ? 8 : n <= 560 ? 4 : 1;
 }
 
 void launch_copy_f(hipStream_t s, const float* src, float* dst, size_t n) {
