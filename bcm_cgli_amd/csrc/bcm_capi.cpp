@@ -550,7 +550,7 @@ int bcm_engine_part(bcm_engine* h, int part, int RK) {
     case 0: engine_bc(e); break;
     case 1: engine_ghost(e); break;
     case 2: engine_interface(e); break;
-    case 3: engine_flux(e, RK); break;
+    case 3: engine_flux(e); break;
     case 4: engine_update(e, RK, 0); break;
     case 5: engine_shift(e); break;
     case 6: engine_stage(e, RK, 0, e->halo_full_next); e->halo_full_next = false; break;
@@ -610,7 +610,7 @@ int bcm_engine_time_part(bcm_engine* h, int part, int RK, int reps, double* ms) 
       case 0: engine_bc(e); break;
       case 1: engine_ghost(e); break;
       case 2: engine_interface(e); break;
-      case 3: engine_flux(e, RK); break;
+      case 3: engine_flux(e); break;
       case 4: engine_update(e, RK, 0); break;
       case 5: engine_shift(e); break;
       case 6: engine_stage(e, RK, 0); break;

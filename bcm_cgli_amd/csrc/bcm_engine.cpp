@@ -913,14 +913,13 @@ namespace {
 double* er_row(Engine* e, int er_slot) { return e->er_dev + (size_t)er_slot * e->max_cases * 8; }
 }  // namespace
 
-void engine_flux(Engine* e, int RK) {
+void engine_flux(Engine* e) {
   if (e->flux_variant == 0)
     launch_flux(e->stream, e->U, e->U1, e->U1q, e->fws, e->cube_size, e->Rku, e->Res, e->ncube,
                 e->pt(), e->deltaT, e->deltaTau, e->e);
   else
     launch_flux_march(e->stream, e->U, e->U1, e->U1q, e->fws, e->cube_size, e->Rku, e->Res,
-                      e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e, e->flux_nseg, RK, 0,
-                      e->U1p1, e->U1p2, e->partials);
+                      e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e, e->flux_nseg);
 }
 
 bool engine_fused(const Engine* e) {
@@ -962,15 +961,15 @@ void engine_flux_update(Engine* e, int RK, int er_slot) {
     return;
   }
   if (!engine_fused(e)) {
-    engine_flux(e, RK);
+    engine_flux(e);
     engine_update(e, RK, er_slot);
     return;
   }
-  launch_flux_march(e->stream, e->U, e->U1, e->U1q, e->fws, e->cube_size, e->Rku, e->Res,
-                    e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e, 1, RK, 1, e->U1p1, e->U1p2,
-                    e->partials);
+  const int rows = launch_flux_in_place(e->stream, e->U, e->U1, e->U1q, e->fws, e->cube_size,
+                                        e->Rku, e->Res, e->ncube, e->pt(), e->deltaT, e->deltaTau,
+                                        e->e, RK, e->U1p1, e->U1p2, e->partials);
   if (RK == 3)
-    launch_reduce(e->stream, e->partials, 1, e->case_desc, e->n_active, e->phys_dev,
+    launch_reduce(e->stream, e->partials, rows, e->case_desc, e->n_active, e->phys_dev,
                   er_row(e, er_slot));
 }
 

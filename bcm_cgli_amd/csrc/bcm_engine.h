@@ -217,7 +217,7 @@ void engine_bc(Engine* e);
 void engine_ghost(Engine* e);
 void engine_interface(Engine* e);
 void engine_halo_refresh(Engine* e);
-void engine_flux(Engine* e, int RK);
+void engine_flux(Engine* e);
 void engine_update(Engine* e, int RK, int er_slot);
 // Flux and RK update of one stage, fused into one kernel when the flux
 // choice allows it (marching kernel, one workgroup per cube).

@@ -278,7 +278,14 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
     }
     __syncthreads();
   }
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};   // IN_PLACE, RK 3: the lane's norm sums
+  // RK 3: totals of a plane's norm and force terms (lanes 0..7; waves in order).
+  auto plane_row = [&] {
+    double s = red[0][t];
+#pragma unroll
+    for (int w = 1; w < WG / 64; ++w) s += red[w][t];
+    return s;
+  };
+  double rows = 0;                         // IN_PLACE: sum of the planes' rows
   int sl0 = 0, sl1 = 1, sl2 = 2;           // ring slots of planes i-1, i, i+1
 
 #pragma unroll 1
@@ -337,12 +344,13 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
 
     // ---- phase 2: primitives of plane i+1, x-face, differences ----
     // One row of norm partials per plane, so the norms do not depend on the
-    // runs.
-    if (MODE == PUSH && RK == 3 && i > i0 && t < 8) {
-      double s = red[0][t];
-#pragma unroll
-      for (int w = 1; w < WG / 64; ++w) s += red[w][t];
-      A.partials[((size_t)(c - 1) * PUSH_ROWS_PER_CUBE + (i - 3)) * 8 + t] = s;
+    // runs; IN_PLACE adds a cube's rows in order, as k_fold_rows would.
+    if (MODE != FLUX_ONLY && RK == 3 && i > i0 && t < 8) {
+      const double s = plane_row();
+      if (MODE == PUSH)
+        A.partials[((size_t)(c - 1) * PUSH_ROWS_PER_CUBE + (i - 3)) * 8 + t] = s;
+      else
+        rows = i == i0 + 1 ? s : rows + s;
     }
     store_flags(i + 1);
     fill_prims(i + 1, sl2);
@@ -622,10 +630,6 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
 #pragma unroll
           for (int v = 0; v < 5; ++v) own(A.U, v) = nv[v];
         }
-        if (RK == 3) {
-#pragma unroll
-          for (int m = 0; m < 7; ++m) acc[m] += pn[m];
-        }
       } else {
         const int nx = i <= 3 ? hs.src[0] : (i >= 16 ? hs.src[1] : 0);
         const int ny = j <= 3 ? hs.src[2] : (j >= 16 ? hs.src[3] : 0);
@@ -649,10 +653,10 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
 #pragma unroll
           for (int v = 0; v < 5; ++v) O[v * PLANE] = nv[v];
         }
-        if (RK == 3) {
-          const double s = wave_sum8(pn);
-          if ((t & 7) == 0) red[t >> 6][(t >> 3) & 7] = s;
-        }
+      }
+      if (RK == 3) {
+        const double s = wave_sum8(pn);
+        if ((t & 7) == 0) red[t >> 6][(t >> 3) & 7] = s;
       }
     }
     // ---- advance the column, the flags and the ring ----
@@ -669,43 +673,47 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
     sl1 = sl2;
     sl2 = s;
   }
-  if constexpr (MODE == PUSH) {
-    if (RK == 3) {
-      __syncthreads();
-      if (t < 8) {
-        double s = red[0][t];
-#pragma unroll
-        for (int w = 1; w < WG / 64; ++w) s += red[w][t];
+  if (MODE != FLUX_ONLY && RK == 3) {
+    __syncthreads();
+    if (t < 8) {
+      const double s = plane_row();
+      if (MODE == PUSH)
         A.partials[((size_t)(c - 1) * PUSH_ROWS_PER_CUBE + (i1 - 2)) * 8 + t] = s;
-      }
-    }
-    // Ghost regions the domain BCs wrote go to Uout as they are.
-    if (zm && seg == 0) copy_bc_regions(A.U, A.Uout, c, zm, 0.0);
-  }
-  if constexpr (MODE == IN_PLACE) {
-    if (RK == 3) {
-      __shared__ double sh[(WG / 64) * 7];
-      block_sum<7>(acc, sh);
-      if (threadIdx.x == 0)
-#pragma unroll
-        for (int m = 0; m < 7; ++m) A.partials[(size_t)(c - 1) * 8 + m] = acc[m];
+      else
+        A.partials[(size_t)(c - 1) * 8 + t] = rows + s;
     }
   }
+  // Ghost regions the domain BCs wrote go to Uout as they are.
+  if (MODE == PUSH && zm && seg == 0) copy_bc_regions(A.U, A.Uout, c, zm, 0.0);
 }
 
 }  // namespace
 
 void launch_flux_march(hipStream_t s, double* U, const double* U1, const double* U1q,
                        const int8_t* fws, const double* cube_size, double* Rku, double* Res,
-                       int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int nseg,
-                       int RK, int fuse, double* U1p1, double* U1p2, double* partials) {
+                       int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int nseg) {
   if (ncube <= 1) return;
-  const MarchArgs a{U, U1, U1q, fws, cube_size, Rku, Res, pt, deltaT, deltaTau, e, Runs{0, nseg}, RK,
+  const MarchArgs a{U, U1, U1q, fws, cube_size, Rku, Res, pt, deltaT, deltaTau, e, Runs{0, nseg}, 1,
+                    ncube, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  hipLaunchKernelGGL((k_flux_march<FLUX_ONLY, true>), run_grid(a.runs, ncube), dim3(WG), 0, s, a);
+}
+
+int launch_flux_in_place(hipStream_t s, double* U, const double* U1, const double* U1q,
+                         const int8_t* fws, const double* cube_size, double* Rku, double* Res,
+                         int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int RK,
+                         double* U1p1, double* U1p2, double* partials) {
+  const int n = ncube - 1;
+  if (n <= IN_PLACE_SPLIT) {
+    launch_flux_march(s, U, U1, U1q, fws, cube_size, Rku, Res, ncube, pt, deltaT, deltaTau, e,
+                      push_runs(n));
+    launch_update(s, RK, U, U1p1, U1p2, Rku, Res, fws, ncube, pt.cube_case, partials,
+                  true);
+    return PUSH_ROWS_PER_CUBE;
+  }
+  const MarchArgs a{U, U1, U1q, fws, cube_size, Rku, Res, pt, deltaT, deltaTau, e, Runs{0, 1}, RK,
                     ncube, U1p1, U1p2, partials, nullptr, nullptr, nullptr};
-  if (fuse && nseg == 1)
-    hipLaunchKernelGGL((k_flux_march<IN_PLACE, true>), run_grid(a.runs, ncube), dim3(WG), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_flux_march<FLUX_ONLY, true>), run_grid(a.runs, ncube), dim3(WG), 0, s, a);
+  hipLaunchKernelGGL((k_flux_march<IN_PLACE, true>), run_grid(a.runs, ncube), dim3(WG), 0, s, a);
+  return 1;
 }
 
 void launch_flux_push(hipStream_t s, const double* Uin, double* Uout, const HaloSrc* halo,

@@ -282,13 +282,23 @@ void launch_flux(hipStream_t s, const double* U, const double* U1, const double*
                  const int8_t* fws, const double* cube_size, double* Rku, double* Res,
                  int ncube, PhysTab pt, double deltaT, double deltaTau, double e);
 // Marching variant of the flux kernel: one workgroup per cube segment
-// (nseg in {1, 2, 4, 8, 16} segments of the cube's 16 i-planes).  With
-// fuse != 0 and nseg == 1 it also applies the RK update in place and, at
-// RK 3, writes one row of 8 norm partials per cube (as k_update does per block).
+// (nseg in {1, 2, 4, 8, 16} segments of the cube's 16 i-planes).
 void launch_flux_march(hipStream_t s, double* U, const double* U1, const double* U1q,
                        const int8_t* fws, const double* cube_size, double* Rku, double* Res,
-                       int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int nseg,
-                       int RK, int fuse, double* U1p1, double* U1p2, double* partials);
+                       int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int nseg);
+// Flux and RK update of one stage in place, writing Rku, Res, U1p1 (RK1) and
+// U1p2 (RK2).  Returns the rows of 8 norm partials per cube that RK 3 writes: 1
+// from the marching kernel that updates as it goes (one run per cube, since a
+// run would read planes another has updated); 16 to IN_PLACE_SPLIT cubes, where
+// the flux runs in many runs and the update follows as a kernel of its own.  The
+// norms are bitwise the same either way (and those of launch_flux_push).  A
+// stage on 8 cubes takes 20 us split and 163 in one kernel, on 125 cubes 95 and
+// 193, on 294 200 and 258, on 512 340 and 300.
+int launch_flux_in_place(hipStream_t s, double* U, const double* U1, const double* U1q,
+                         const int8_t* fws, const double* cube_size, double* Rku, double* Res,
+                         int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int RK,
+                         double* U1p1, double* U1p2, double* partials);
+constexpr int IN_PLACE_SPLIT = 320;
 // Marching kernel with the update written to Uout, nseg (1, 2, 4, 8 or 16) runs
 // of 16/nseg planes per cube, one workgroup each, bitwise the same results for
 // every nseg: every interior cell, and the two layers next to each face with an
@@ -312,10 +322,10 @@ void launch_copy_d(hipStream_t s, const double* src, double* dst, size_t n);
 int div_selftest(unsigned long long seed, int n, unsigned long long* mismatches);
 void launch_update(hipStream_t s, int RK, double* U, double* U1p1, double* U1p2,
                    const double* Rku, const double* Res, const int8_t* fws, int ncube,
-                   const int* cube_case, double* partials);
+                   const int* cube_case, double* partials, bool body_only = false);
 // Norms er[0..7] of each case in cases[0..ncases): rows_per_cube partial rows
-// per cube (1 after the fused in-place FP64 kernel, 16 after k_update, the
-// pushing FP64 kernel and the mixed flux kernel; several rows are first summed in row order into each
+// per cube (as launch_flux_in_place says; 16 after k_update, the pushing FP64
+// kernel and the mixed flux kernel; several rows are first summed in row order into each
 // cube's first row); case d writes er[d.slot*8 .. d.slot*8+7].
 void launch_reduce(hipStream_t s, double* partials, int rows_per_cube, const CaseDesc* cases,
                    int ncases, const DevPhys* phys, double* er);

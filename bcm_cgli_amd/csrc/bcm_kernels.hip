@@ -311,7 +311,8 @@ __global__ __launch_bounds__(WG) void k_flux(const double* __restrict__ U,
 
 // RK stage update of fluid cells (Flux.cpp:2417-2599).  At RK3 each block
 // also writes its partial sums of the five change norms (:2530-2566) and of
-// the two force-density components (:2603-2625).
+// the two force-density components (:2603-2625; body_only: of the cells a flux
+// kernel just wrote, whatever the others hold).
 __global__ __launch_bounds__(WG) void k_update(int RK, double* __restrict__ U,
                                                double* __restrict__ U1p1,
                                                double* __restrict__ U1p2,
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(WG) void k_update(int RK, double* __restrict__ U,
                                                const double* __restrict__ Res,
                                                const int8_t* __restrict__ fws,
                                                const int* __restrict__ cube_case,
-                                               double* __restrict__ partials) {
+                                               double* __restrict__ partials, int body_only) {
   const int c = blockIdx.y + 1;
   if (cube_case[c] < 0) return;
   const int i = blockIdx.x + 2;
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(WG) void k_update(int RK, double* __restrict__ U,
       }
     return;
   }
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+  double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (fluid) {
     double u[5];
 #pragma unroll
@@ -375,14 +376,21 @@ __global__ __launch_bounds__(WG) void k_update(int RK, double* __restrict__ U,
     acc[3] = (wn - wo) * (wn - wo);
     acc[4] = (T - To) * (T - To);
   }
-  acc[5] = Res[b];
-  acc[6] = Res[b + PLANE];
-  __shared__ double sh[(WG / 64) * 7];
-  block_sum<7>(acc, sh);
-  if (threadIdx.x == 0) {
-    const size_t blk = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+  if (!body_only || fws[fidx(c, i, j, k)] < 1) {
+    acc[5] = Res[b];
+    acc[6] = Res[b + PLANE];
+  }
+  // The row the marching flux kernels write for this plane, bitwise.
+  __shared__ double red[WG / 64][8];
+  const int t = threadIdx.x;
+  const double s = wave_sum8(acc);
+  if ((t & 7) == 0) red[t >> 6][(t >> 3) & 7] = s;
+  __syncthreads();
+  if (t < 8) {
+    double r = red[0][t];
 #pragma unroll
-    for (int m = 0; m < 7; ++m) partials[blk * 8 + m] = acc[m];
+    for (int w = 1; w < WG / 64; ++w) r += red[w][t];
+    partials[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 8 + t] = r;
   }
 }
 
@@ -1342,10 +1350,10 @@ void launch_copy_d(hipStream_t s, const double* src, double* dst, size_t n) {
 
 void launch_update(hipStream_t s, int RK, double* U, double* U1p1, double* U1p2,
                    const double* Rku, const double* Res, const int8_t* fws, int ncube,
-                   const int* cube_case, double* partials) {
+                   const int* cube_case, double* partials, bool body_only) {
   if (ncube > 1)
     hipLaunchKernelGGL(k_update, dim3(16, ncube - 1), dim3(WG), 0, s, RK, U, U1p1, U1p2, Rku,
-                       Res, fws, cube_case, partials);
+                       Res, fws, cube_case, partials, body_only ? 1 : 0);
 }
 
 void launch_reduce(hipStream_t s, double* partials, int rows_per_cube, const CaseDesc* cases,

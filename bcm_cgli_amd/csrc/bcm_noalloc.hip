@@ -2,9 +2,8 @@
 // for callers that cannot call hipMalloc (code under HIP graph capture, tight
 // serving loops, harnesses that forbid allocation).
 //
-// The kernels are those of the drop-in BCM_Flux_XYZ_Viscous_Runge_kutta (the
-// marching flux kernel with the RK update fused in place, then the per-case
-// norm reduction at RK 3).  What that drop-in keeps in engine allocations --
+// The kernels are those of the drop-in BCM_Flux_XYZ_Viscous_Runge_kutta
+// (launch_flux_in_place, then the per-case norm reduction at RK 3).  What that drop-in keeps in engine allocations --
 // the per-cube norm partials, the cube-to-case map, the flow constants and
 // the case descriptor of the reduction -- lives here in one file-scope device
 // array, `scratch`, of fixed size.  Each device holds its own copy until the
@@ -24,7 +23,7 @@
 namespace bcm {
 namespace {
 
-// Layout of the scratch array (bytes): norm partials, 8 doubles per cube;
+// Layout of the scratch array (bytes): norm partials, rows of 8 doubles;
 // cube-to-case map, one int per cube slot (slot 0 included); the flow
 // constants and the reduction's case descriptor.
 constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -33,6 +32,8 @@ constexpr size_t CUBE_CASE_OFF = PARTIALS_OFF + (size_t)BCM_NOALLOC_MAX_CUBES * 
 constexpr size_t PHYS_OFF = align256(CUBE_CASE_OFF + (size_t)(BCM_NOALLOC_MAX_CUBES + 1) * sizeof(int));
 constexpr size_t DESC_OFF = PHYS_OFF + 128;
 constexpr size_t SCRATCH_BYTES = DESC_OFF + 128;
+static_assert((long long)IN_PLACE_SPLIT * PUSH_ROWS_PER_CUBE <= BCM_NOALLOC_MAX_CUBES,
+              "the norm partials of a split stage fit");
 static_assert(SCRATCH_BYTES == BCM_NOALLOC_SCRATCH_BYTES, "scratch size as declared");
 static_assert(sizeof(DevPhys) <= 128 && sizeof(CaseDesc) <= 128, "tables fit their slots");
 
@@ -125,10 +126,10 @@ extern "C" int bcm_flux_rk_noalloc(int ncube, int n_cubes_norm, int RK, double d
   double* partials = reinterpret_cast<double*>(s + PARTIALS_OFF);
   const PhysTab pt{reinterpret_cast<const DevPhys*>(s + PHYS_OFF),
                    reinterpret_cast<const int*>(s + CUBE_CASE_OFF)};
-  launch_flux_march(st, U1_, U1, U1q, FWS, cube_size, Rku1, Residual1, ncube, pt, deltaT, deltaTau,
-                    e, 1, RK, 1, U1p1, U1p2, partials);
+  const int rows = launch_flux_in_place(st, U1_, U1, U1q, FWS, cube_size, Rku1, Residual1, ncube, pt,
+                                        deltaT, deltaTau, e, RK, U1p1, U1p2, partials);
   if (RK == 3)
-    launch_reduce(st, partials, 1, reinterpret_cast<const CaseDesc*>(s + DESC_OFF), 1, pt.phys,
+    launch_reduce(st, partials, rows, reinterpret_cast<const CaseDesc*>(s + DESC_OFF), 1, pt.phys,
                   er);
   const hipError_t rc = hipGetLastError();
   if (rc != hipSuccess) {

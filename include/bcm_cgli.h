@@ -261,8 +261,8 @@ int bcm_engine_sync(bcm_engine* e);
 int bcm_engine_time_part(bcm_engine* e, int part, int RK, int reps, double* ms);
 /* Flux kernel choice: variant 0 (one workgroup per cell plane) or 1 (one
  * workgroup per cube segment marching along i, nseg in {1,2,4,8,16}); fuse 1
- * lets variant 1 with nseg 1 apply the RK update in the same kernel, in
- * place; fuse 2 (variant 1, nseg 1) writes the update and the face halos into
+ * lets variant 1 with nseg 1 apply the RK update in place (in the same kernel,
+ * on few cubes in one that follows); fuse 2 (variant 1, nseg 1) writes the update and the face halos into
  * a second copy of the iterate in engine stages, which then open with the
  * edge passes and BCs instead of closing with the halo exchange (that
  * kernel's runs per cube follow the number of resident cubes).  All choices

@@ -36,6 +36,30 @@ def lattice_case(B, dims):
                                 sphere_diameter=0.3 * min(dims) * size))
 
 
+# In place: 1, 100 | 101, 320 | 321 cubes (flux and update as two kernels | one).
+@pytest.mark.parametrize("dims", [(1, 1, 1), (5, 5, 4), (101, 1, 1), (8, 8, 5), (107, 3, 1)],
+                         ids=lambda d: str(int(np.prod(d))))
+def test_in_place_stages_bitwise(B, O, dims):
+    case = lattice_case(B, dims)
+    out = []
+    for fuse in (1, 2):
+        e = B.Engine(0)
+        try:
+            e.load_case(case)
+            e.set_flux(1, 1, fuse)
+            h = e.run(1, 2)
+            if fuse == 1:
+                orc = O.OracleRun(case, nthreads=16)
+                ho = orc.run(1, 2)
+                compare(e, orc, STATE)
+                assert er_close(h, ho)
+            out.append(h)
+        finally:
+            e.close()
+    # the norms do not depend on the kernel that formed them
+    assert np.array_equal(out[0].view(np.int64), out[1].view(np.int64))
+
+
 # 1, 32 | 33, 64 | 65, 128 | 129, 200 | 201, 560 | 561, 1,003 cubes
 @pytest.mark.parametrize("dims", [(1, 1, 1), (8, 4, 1), (11, 3, 1), (4, 4, 4), (13, 5, 1),
                                   (8, 4, 4), (43, 3, 1), (8, 5, 5), (67, 3, 1), (8, 10, 7),
