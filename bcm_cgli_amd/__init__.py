@@ -450,8 +450,8 @@ class Engine:
 
     def set_ghost_lds_limit(self, slots):
         """Cubes whose IB fill needs more LDS value slots than this take the
-        in-place schedule on memory (cases loaded or added afterwards); the
-        default 1536 is the kernel's LDS capacity.  A test hook."""
+        in-place schedule on memory (cases loaded or added afterwards); at most
+        1536, by default the kernel's capacity of 3072.  A test hook."""
         _check(_lib.bcm_engine_set_ghost_lds_limit(self._h, int(slots)))
 
     def ghost_stats(self):

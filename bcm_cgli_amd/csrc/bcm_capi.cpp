@@ -687,8 +687,8 @@ int bcm_selftest_division(unsigned long long seed, int n, unsigned long long* mi
 
 int bcm_engine_set_ghost_lds_limit(bcm_engine* h, int slots) {
   if (!h) return fail("null engine");
-  if (slots < 0 || slots > GHOST_LDS_SLOTS)
-    return fail("slot limit must be in 0.." + std::to_string(GHOST_LDS_SLOTS));
+  if (slots < 0 || slots > GHOST_LDS_HOOK_MAX)
+    return fail("slot limit must be in 0.." + std::to_string(GHOST_LDS_HOOK_MAX));
   h->e->ghost_slot_limit = slots;
   return 0;
 }

@@ -119,65 +119,59 @@ GhostSchedule build_ghost_schedule(const std::vector<GhostEntry>& ordered, int s
                 E.pj + (m == 2 || m == 4 || m == 6 || m == 7),
                 E.pk + (m == 3 || m == 5 || m == 6 || m == 7));
   };
-  std::vector<int> pos(8000), cur(8000), wlev(8000), rlev(8000);
+  std::vector<int> cur(8000), wlev(8000), rlev(8000), last(8000);
   for (auto& kv : by_cube) {
     const std::vector<int>& idx = kv.second;
     const int ne = (int)idx.size();
-    // Touched cells: written ghost cells first, then the other corners.
-    std::fill(pos.begin(), pos.end(), -1);
-    std::vector<int16_t> list;
     for (int a = 0; a < ne; ++a) {
       const GhostEntry& E = ordered[idx[a]];
-      const int g = cell(E.gi, E.gj, E.gk);
-      if (pos[g] < 0) {
-        pos[g] = (int)list.size();
-        list.push_back((int16_t)g);
-      }
+      last[cell(E.gi, E.gj, E.gk)] = a;
     }
-    const int nw = (int)list.size();
-    for (int a = 0; a < ne; ++a)
-      for (int m = 0; m < 8; ++m) {
-        const int ci = corner(ordered[idx[a]], m);
-        if (pos[ci] < 0) {
-          pos[ci] = (int)list.size();
-          list.push_back((int16_t)ci);
-        }
-      }
-    const int nt = (int)list.size();
+    // Renamed: entry a writes slot a and reads the slot holding the value the
+    // sequential fill would read (an earlier entry's, or that of a staged
+    // cell); only reads of earlier writes order the levels.
     std::vector<GhostEntry> ents(ne);
     std::vector<int> level(ne);
-    std::vector<int16_t> fin(nt);
+    std::vector<int16_t> list;
     int nlev = 0;
-    if (nt + ne <= std::min(slot_limit, GHOST_LDS_SLOTS)) {
-      // Renamed: entry a writes slot nt + a and reads the slot holding the
-      // value the sequential fill would read; only reads of earlier writes
-      // order the levels.
-      std::vector<int> slot_level(nt + ne, 0);
-      for (int n = 0; n < nt; ++n) cur[list[n]] = n;
-      for (int a = 0; a < ne; ++a) {
-        GhostEntry E = ordered[idx[a]];
-        int lv = 1;
-        for (int m = 0; m < 8; ++m) {
-          const int sl = cur[corner(E, m)];
-          E.lc[m] = (int16_t)sl;
-          lv = std::max(lv, slot_level[sl] + 1);
+    std::fill(cur.begin(), cur.end(), -1);
+    for (int a = 0; a < ne; ++a) {
+      GhostEntry E = ordered[idx[a]];
+      int lv = 1;
+      for (int m = 0; m < 8; ++m) {
+        const int ci = corner(E, m);
+        if (cur[ci] < 0) {
+          cur[ci] = ne + (int)list.size();
+          list.push_back((int16_t)ci);
         }
-        E.lg = (int16_t)(nt + a);
-        slot_level[nt + a] = lv;
-        cur[cell(E.gi, E.gj, E.gk)] = nt + a;
-        ents[a] = E;
-        level[a] = lv;
-        nlev = std::max(nlev, lv);
+        E.lc[m] = (int16_t)cur[ci];
+        if (cur[ci] < ne) lv = std::max(lv, level[cur[ci]] + 1);
       }
-      for (int n = 0; n < nt; ++n) fin[n] = (int16_t)cur[list[n]];
-      gs.max_slots = std::max(gs.max_slots, nt + ne);
+      const int g = cell(E.gi, E.gj, E.gk);
+      E.lg = (int16_t)a;
+      E.self = 8;
+      for (int m = 0; m < 8; ++m)
+        if (corner(E, m) == g) E.self = (int16_t)m;
+      gs.out.push_back((int16_t)(last[g] == a ? g : -1));
+      cur[g] = a;
+      ents[a] = E;
+      level[a] = lv;
+      nlev = std::max(nlev, lv);
+    }
+    GhostCube gc{kv.first, (int)gs.level_off.size(), 0, (int)gs.entries.size(), 0, ne,
+                 (int)gs.read.size(), (int)list.size()};
+    if (2 * ne + gc.nread <= std::min(slot_limit, GHOST_LDS_SLOTS)) {
+      gs.read.insert(gs.read.end(), list.begin(), list.end());
+      gs.max_slots = std::max(gs.max_slots, 2 * ne + gc.nread);
     } else {
       // In place: an entry also waits for earlier reads and writes of its
       // ghost cell.
+      gc.nread = -1;
+      nlev = 0;
       std::fill(wlev.begin(), wlev.end(), 0);
       std::fill(rlev.begin(), rlev.end(), 0);
       for (int a = 0; a < ne; ++a) {
-        GhostEntry E = ordered[idx[a]];
+        const GhostEntry& E = ents[a];
         int lv = 1;
         for (int m = 0; m < 8; ++m) lv = std::max(lv, wlev[corner(E, m)] + 1);
         const int g = cell(E.gi, E.gj, E.gk);
@@ -185,59 +179,46 @@ GhostSchedule build_ghost_schedule(const std::vector<GhostEntry>& ordered, int s
         lv = std::max(lv, wlev[g] + 1);
         wlev[g] = lv;
         for (int m = 0; m < 8; ++m) rlev[corner(E, m)] = std::max(rlev[corner(E, m)], lv);
-        for (int m = 0; m < 8; ++m) E.lc[m] = (int16_t)pos[corner(E, m)];
-        E.lg = (int16_t)pos[g];
-        ents[a] = E;
         level[a] = lv;
         nlev = std::max(nlev, lv);
       }
-      for (int n = 0; n < nt; ++n) fin[n] = (int16_t)n;
     }
-    gs.touched_off.push_back((int)gs.touched.size());
-    gs.touched_nw.push_back(nw);
-    gs.touched.insert(gs.touched.end(), list.begin(), list.end());
-    gs.touched_final.insert(gs.touched_final.end(), fin.begin(), fin.end());
-    gs.cube_level_off.push_back((int)gs.level_off.size());
+    gc.nlev = nlev;
     for (int lv = 1; lv <= nlev; ++lv) {
       gs.level_off.push_back((int)gs.entries.size());
       for (int a = 0; a < ne; ++a)
         if (level[a] == lv) gs.entries.push_back(ents[a]);
+      if (lv == 1) gc.n1 = (int)gs.entries.size() - gc.ent0;
     }
+    gs.cubes.push_back(gc);
     gs.max_levels = std::max(gs.max_levels, nlev);
   }
-  gs.cube_level_off.push_back((int)gs.level_off.size());
   gs.level_off.push_back((int)gs.entries.size());
-  gs.touched_off.push_back((int)gs.touched.size());
   return gs;
 }
 
 int ghost_upload(const GhostSchedule& gs, GhostDevice& d, std::string& err) {
   ghost_free(d);
   GhostEntry* ent;
-  int *clo, *lo, *toff, *tnw;
-  int16_t *tc, *tf;
+  GhostCube* cubes;
+  int* lo;
+  int16_t *rd, *out;
   if (dev_upload(&ent, gs.entries, err)) return 1;
   d.owned.push_back(ent);
-  if (dev_upload(&clo, gs.cube_level_off, err)) return 1;
-  d.owned.push_back(clo);
+  if (dev_upload(&cubes, gs.cubes, err)) return 1;
+  d.owned.push_back(cubes);
   if (dev_upload(&lo, gs.level_off, err)) return 1;
   d.owned.push_back(lo);
-  if (dev_upload(&tc, gs.touched, err)) return 1;
-  d.owned.push_back(tc);
-  if (dev_upload(&tf, gs.touched_final, err)) return 1;
-  d.owned.push_back(tf);
-  if (dev_upload(&toff, gs.touched_off, err)) return 1;
-  d.owned.push_back(toff);
-  if (dev_upload(&tnw, gs.touched_nw, err)) return 1;
-  d.owned.push_back(tnw);
+  if (dev_upload(&rd, gs.read, err)) return 1;
+  d.owned.push_back(rd);
+  if (dev_upload(&out, gs.out, err)) return 1;
+  d.owned.push_back(out);
   d.t.ent = ent;
-  d.t.cube_level_off = clo;
+  d.t.cubes = cubes;
   d.t.level_off = lo;
-  d.t.touched = tc;
-  d.t.touched_final = tf;
-  d.t.touched_off = toff;
-  d.t.touched_nw = tnw;
-  d.t.ncubes = (int)gs.cube_level_off.size() - 1;
+  d.t.read = rd;
+  d.t.out = out;
+  d.t.ncubes = (int)gs.cubes.size();
   d.t.max_slots = gs.max_slots;
   return 0;
 }
@@ -480,21 +461,22 @@ int rebuild_tables(Engine* e, std::string& err) {
       bm.push_back(tb.bc_masks[a]);
     }
     const int e0 = (int)gs.entries.size(), l0 = (int)gs.level_off.size();
-    const int t0 = (int)gs.touched.size();
+    const int r0 = (int)gs.read.size();
     for (GhostEntry E : tb.ghost.entries) {
       E.cube += off;
       gs.entries.push_back(E);
     }
     for (size_t a = 0; a + 1 < tb.ghost.level_off.size(); ++a)
       gs.level_off.push_back(tb.ghost.level_off[a] + e0);
-    for (size_t a = 0; a + 1 < tb.ghost.cube_level_off.size(); ++a) {
-      gs.cube_level_off.push_back(tb.ghost.cube_level_off[a] + l0);
-      gs.touched_off.push_back(tb.ghost.touched_off[a] + t0);
-      gs.touched_nw.push_back(tb.ghost.touched_nw[a]);
+    for (GhostCube g : tb.ghost.cubes) {
+      g.cube += off;
+      g.lev0 += l0;
+      g.ent0 += e0;
+      g.read0 += r0;
+      gs.cubes.push_back(g);
     }
-    gs.touched.insert(gs.touched.end(), tb.ghost.touched.begin(), tb.ghost.touched.end());
-    gs.touched_final.insert(gs.touched_final.end(), tb.ghost.touched_final.begin(),
-                            tb.ghost.touched_final.end());
+    gs.read.insert(gs.read.end(), tb.ghost.read.begin(), tb.ghost.read.end());
+    gs.out.insert(gs.out.end(), tb.ghost.out.begin(), tb.ghost.out.end());
     gs.max_levels = std::max(gs.max_levels, tb.ghost.max_levels);
     gs.max_slots = std::max(gs.max_slots, tb.ghost.max_slots);
     for (int2 pr : tb.halo_pairs) pairs.push_back(make_int2(pr.x + off * PLANE, pr.y + off * PLANE));
@@ -505,9 +487,7 @@ int rebuild_tables(Engine* e, std::string& err) {
     }
     desc.push_back(CaseDesc{cs.first, tb.n, tb.mpi_ncube, s});
   }
-  gs.cube_level_off.push_back((int)gs.level_off.size());
   gs.level_off.push_back((int)gs.entries.size());
-  gs.touched_off.push_back((int)gs.touched.size());
   std::vector<uint8_t> cube_mask(e->cap, 0);
   for (size_t a = 0; a < bc.size(); ++a) cube_mask[bc[a]] = bm[a];
   {
@@ -539,7 +519,7 @@ int rebuild_tables(Engine* e, std::string& err) {
   e->ncube = top;
   e->n_active = (int)order.size();
   e->n_bc = (int)bc.size();
-  e->n_ghost_cubes = (int)gs.cube_level_off.size() - 1;
+  e->n_ghost_cubes = (int)gs.cubes.size();
   e->n_ghost_entries = (int)gs.entries.size();
   e->ghost_levels = gs.max_levels;
   e->n_halo_pairs = (int)pairs.size();
@@ -578,22 +558,22 @@ int rebuild_tables(Engine* e, std::string& err) {
     }
     // One item per cube: IB cubes first (their fills are the longest chains),
     // then the other listed cubes.
-    std::vector<int> gidx(top, -1);
-    const int ng = (int)gs.cube_level_off.size() - 1;
-    for (int g = 0; g < ng; ++g) {
-      if (gs.cube_level_off[g] == gs.cube_level_off[g + 1]) continue;
-      const int c = gs.entries[gs.level_off[gs.cube_level_off[g]]].cube;
-      if (gidx[c] >= 0) {
+    std::vector<char> filled(top, 0);
+    std::vector<OpenItem> items;
+    for (const GhostCube& g : gs.cubes) {
+      if (filled[g.cube]) {
         err = "a cube appears twice in the IB fill schedule";
         return 1;
       }
-      gidx[c] = g;
+      filled[g.cube] = 1;
+      items.push_back(OpenItem{mark[g.cube], cube_mask[g.cube], e->cube_case_host[g.cube], g});
     }
-    std::vector<int2> items;
-    for (int c = 1; c < top; ++c)
-      if (gidx[c] >= 0) items.push_back(make_int2(mark[c] ? (mark[c] == 2 ? c : -c) : 0, gidx[c]));
-    for (int c = 1; c < top; ++c)
-      if (gidx[c] < 0 && mark[c]) items.push_back(make_int2(mark[c] == 2 ? c : -c, -1));
+    for (int c = 1; c < top; ++c) {
+      if (filled[c] || !mark[c]) continue;
+      GhostCube g{};
+      g.cube = c;
+      items.push_back(OpenItem{mark[c], cube_mask[c], e->cube_case_host[c], g});
+    }
     e->n_open_items = (int)items.size();
     if (dev_upload(&e->open_items, items, err)) return 1;
   }
@@ -901,7 +881,7 @@ namespace {
 template <typename T>
 void push_stage_open(Engine* e, T* U, bool full_pre_halo) {
   launch_halo_ml(e->stream, U, e->ml, e->n_ml, e->pt());
-  launch_open(e->stream, U, e->open_items, e->n_open_items, e->bc_mask_cube, e->ghost.t, e->pt());
+  launch_open(e->stream, U, e->open_items, e->n_open_items, e->ghost.t, e->phys_dev);
   if (full_pre_halo)
     engine_interface(e);
   else

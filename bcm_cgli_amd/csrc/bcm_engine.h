@@ -20,12 +20,10 @@ void set_last_error(const std::string& m);
 
 struct GhostSchedule {
   std::vector<GhostEntry> entries;   // grouped per cube, level-major within the cube
-  std::vector<int> cube_level_off;   // per ghost cube: first level index (+1 sentinel)
   std::vector<int> level_off;        // per level: first entry index (+1 sentinel)
-  std::vector<int16_t> touched;      // per ghost cube: written ghost cells, then other corners
-  std::vector<int16_t> touched_final;// slot of each written cell's last value
-  std::vector<int> touched_off;      // per ghost cube: first touched cell (+1 sentinel)
-  std::vector<int> touched_nw;       // per ghost cube: written cells
+  std::vector<GhostCube> cubes;
+  std::vector<int16_t> read;         // per ghost cube: cells its LDS fill stages
+  std::vector<int16_t> out;          // per entry slot: cell it stores to memory, or -1
   int max_levels = 0;
   int max_slots = 0;
 };
@@ -136,7 +134,7 @@ struct Engine {
   // touches an edge cell); -c: the k-edge cells the z-BC copies, then BCs
   // (other boundary cubes); 0: none.  Elsewhere only the pushing flux kernels
   // read edge cells, and they form them themselves.
-  int2* open_items = nullptr;
+  OpenItem* open_items = nullptr;
   int n_open_items = 0;
   // Set when an inner iterate was replaced from outside (state upload, new
   // case): the next pre-flux exchange must then be the full one.

@@ -80,34 +80,53 @@ struct CaseDesc {
 };
 
 // One IB ghost-fill entry in level order (see the ghost schedule in the engine).
-struct GhostEntry {
+struct alignas(16) GhostEntry {
+  double w[8];
+  int16_t lc[8], lg;                // LDS slots read for the corners and written
+  int16_t self;                     // corner that is the ghost cell itself (8: none)
   int cube;
   int16_t gi, gj, gk, pi, pj, pk;   // ghost cell and interpolation base corner
-  int16_t lc[8], lg;                // LDS slots read for the corners and written
-  double w[8];
 };
 
-// IB fill of one cube in LDS: value slots for the cells its entries touch
-// plus one slot per entry; a cube needing more slots works on memory.
-constexpr int GHOST_LDS_SLOTS = 1536;
+// IB fill of one cube in LDS: two value slots per entry (primitives for later
+// levels, conserved values for memory) and one per cell that an entry reads
+// before any entry has written it; a cube needing more slots works on memory.
+// 3072 slots of five doubles are 120 KB of the 160 KB of a CU; a whole body
+// inside one cube needs about 1000 to 2100.
+constexpr int GHOST_LDS_SLOTS = 3072;
+// Largest limit the diagnostic hook accepts.
+constexpr int GHOST_LDS_HOOK_MAX = 1536;
 
-// Device tables of the IB fill: entries grouped per cube and level, and per
-// cube the list of cells its entries touch (written ghost cells first).
-// In LDS (slots <= GHOST_LDS_SLOTS) every entry writes a slot of its own and
-// reads the slots of the values the sequential fill would read, so levels
-// follow read-after-write dependencies only; touched_final names the slot
-// holding each written cell's last value.  On memory the fill is in place
+// IB fill of one cube: its levels, entries and the cells it reads.
+struct GhostCube {
+  int cube;
+  int lev0, nlev;     // levels lev0 .. lev0+nlev-1 (nlev 0: no fill)
+  int ent0, n1, ne;   // first entry, entries of the first level, all entries
+  int read0, nread;   // staged cells; nread -1: the fill works on memory
+};
+
+// Device tables of the IB fill: entries grouped per cube and level.  In LDS
+// every entry writes a slot of its own (its index within the cube) and reads
+// the slots of the values the sequential fill would read, so levels follow
+// read-after-write dependencies only; the cells it reads as memory holds them
+// are staged in the slots after the entries'.  On memory the fill is in place
 // and levels also order writes after earlier reads and writes of a cell.
 struct GhostTables {
   const GhostEntry* ent = nullptr;
-  const int* cube_level_off = nullptr;   // per cube: first level (+1 sentinel)
-  const int* level_off = nullptr;        // per level: first entry (+1 sentinel)
-  const int16_t* touched = nullptr;      // cells i*400 + j*20 + k
-  const int16_t* touched_final = nullptr;// slot of the last value of each written cell
-  const int* touched_off = nullptr;      // per cube: first touched cell (+1 sentinel)
-  const int* touched_nw = nullptr;       // per cube: written cells at the head of its list
+  const GhostCube* cubes = nullptr;
+  const int* level_off = nullptr;   // per level: first entry (+1 sentinel)
+  const int16_t* read = nullptr;    // staged cells i*400 + j*20 + k
+  const int16_t* out = nullptr;     // per LDS slot of an entry: its ghost cell
+                                    // (-1: a later entry writes the cell)
   int ncubes = 0;
   int max_slots = 0;
+};
+
+// One cube's work at the opening of a stage: its edge passes (edges 0 none, 1
+// the edge cells its BCs read, 2 all), its BCs (mask) and its IB fill.
+struct OpenItem {
+  int edges, mask, slot;
+  GhostCube g;
 };
 
 // Source cubes for the six face halos of a cube (0 = no equal-size neighbour).
@@ -268,10 +287,10 @@ void launch_edge_list(hipStream_t s, float* U, const int* list, int n);
 // Opening of a pushed stage in one launch: per item (x: edge/BC entry as
 // above or 0, y: IB ghost-table index or -1) a cube's edge passes and BCs,
 // then its IB fill.
-void launch_open(hipStream_t s, double* U, const int2* items, int n, const uint8_t* cube_mask,
-                 const GhostTables& g, PhysTab pt);
-void launch_open(hipStream_t s, float* U, const int2* items, int n, const uint8_t* cube_mask,
-                 const GhostTables& g, PhysTab pt);
+void launch_open(hipStream_t s, double* U, const OpenItem* items, int n, const GhostTables& g,
+                 const DevPhys* phys);
+void launch_open(hipStream_t s, float* U, const OpenItem* items, int n, const GhostTables& g,
+                 const DevPhys* phys);
 // Edge passes of every cube.
 void launch_edge(hipStream_t s, double* U, int ncube, const int* cube_case);
 void launch_edge(hipStream_t s, float* U, int ncube, const int* cube_case);

@@ -37,6 +37,10 @@ template <typename T> struct OffOf;
 template <> struct OffOf<double> { using type = NoOff; };
 template <> struct OffOf<float> { using type = RefOff; };
 
+template <typename T> struct Vec2;
+template <> struct Vec2<double> { using type = double2; };
+template <> struct Vec2<float> { using type = float2; };
+
 // Inviscid flux difference of one cell along axis D (Flux.cpp:367-806 for Z):
 // upwind-biased face states of 5th, 3rd or 1st order depending on the cell
 // position and the neighbour flags, then the two face fluxes.
@@ -443,130 +447,223 @@ __global__ __launch_bounds__(WG) void k_reduce(const double* __restrict__ partia
 }
 
 // ---------------------------------------------------------------------------
-// Domain boundary conditions of one cube per block: X (BCM_X_boundary_condition
-// .cpp:43-118), then Y (BCM_Y_boundary_condition.cpp:36-80), then Z
-// (BCM_Z_boundary_condition.cpp:42-92).  mask bits: 1 x-min, 2 x-max, 4 y-min,
-// 8 y-max, 16 z-min, 32 z-max.
-// In each of the three phases the cells read (the layers next to the ghost
-// layers) and the cells written (the ghost layers) are disjoint, so every
-// lane issues all its loads of a phase before its first store: one memory
-// round trip per phase instead of one per value.
+// Edge passes and domain boundary conditions of one cube by the calling
+// workgroup (OPEN_WG lanes): edge-ghost averaging (Interface.cpp:5640-5732)
+// where asked for, then X (BCM_X_boundary_condition.cpp:43-118), Y
+// (BCM_Y_boundary_condition.cpp:36-80) and Z (BCM_Z_boundary_condition.cpp:42-92).
+// m bits: 1 x-min, 2 x-max, 4 y-min, 8 y-max, 16 z-min, 32 z-max.
+//
+// Pass by pass each of the six would read what the one before wrote: a chain
+// of up to six memory round trips for a few kilobytes.  Every cell written
+// has a closed form in the state before the first pass (a copy of a copy is a
+// copy of the first source, an edge mean's sources are face ghost cells or
+// such means), so all cells are loaded, one barrier passes, and all are
+// stored; a cell that a later pass overwrites is not stored by the earlier
+// one.  1024 lanes leave at most one cell of each pass to a lane.  A cube with
+// three BC faces and all edge passes 6 us, pass by pass 9.5; the opening of
+// 2,048 cubes in FP64 (872 with BCs) 28 us, with 256 lanes pass by pass 43.
+// edges 0: no edge passes; 1: only the k-edge cells the z-BC copies (four of
+// the cells of the plane k = 2 or 17); 2: all.
+constexpr int OPEN_WG = 1024;
 template <typename T>
-__device__ __forceinline__ void bc_cube(T* __restrict__ U, int c, int m, PhysTab pt) {
-  const DevPhys ph = pt.phys[pt.cube_case[c]];
+__device__ __forceinline__ void edge_bc_cube(T* __restrict__ U, int c, int edges, int m,
+                                             const DevPhys& ph) {
+  using T2 = typename Vec2<T>::type;
   const typename OffOf<T>::type F(ph);
   const int t = threadIdx.x;
-  {
-    const int j = (t >> 4) + 2, k = (t & 15) + 2;
-    T lo[5], hi[5];
+  T* const Uc = U + (size_t)c * CUBE_STRIDE;
+  auto at = [](int v, int i, int j, int k) { return v * PLANE + i * 400 + j * 20 + k; };
+  // Nearest interior index of 1 (2) or 18 (17).
+  auto near = [](int q) { return q == 1 ? 2 : 17; };
+  // x-min inflow state from the interior state next to it, as stored.
+  auto inflow = [&](const T (&q)[5], T (&o)[5]) {
+    const double rho = F.ld(q, 0, 0);
+    const double uu = F.ld(q, 1, 1) / rho;
+    const double vv = F.ld(q, 2, 2) / rho;
+    const double ww = F.ld(q, 3, 3) / rho;
+    double VV = uu * uu + vv * vv + ww * ww;
+    const double P = (F.ld(q, 4, 4) - 0.5 * rho * VV) * KM1;
+    VV = ph.Uin * ph.Uin + ph.V0 * ph.V0 + ph.W0 * ph.W0;
+    const double E = P / KM1 + 0.5 * rho * VV;
+    o[0] = q[0];
+    F.st(o, 1, 1, rho * ph.Uin);
+    F.st(o, 2, 2, rho * ph.V0);
+    F.st(o, 3, 3, rho * ph.W0);
+    F.st(o, 4, 4, E);
+  };
+  // Source row i of a BC copy along x, and whether it passes the inflow.
+  auto x_source = [&](int i, bool& in) {
+    in = i < 2 && (m & 1);
+    return in ? 2 : (i > 17 && (m & 2) ? 17 : i);
+  };
+
+  // X: (j, k) of side t / 256 (the other half of the lanes has none).
+  const int xs = t >> 8, xj = ((t >> 4) & 15) + 2, xk = (t & 15) + 2;
+  const bool dx = xs < 2 && (m & (1 << xs));
+  T x[5];
+  if (dx)
+#pragma unroll
+    for (int v = 0; v < 5; ++v) x[v] = Uc[at(v, xs ? 17 : 2, xj, xk)];
+
+  // Y: (i, k), i = 0..19, of side t / 512.
+  const int side = t >> 9, w = t & 511;
+  const int yi = w >> 4, yk = (w & 15) + 2;
+  const bool dy = w < 320 && (m & (4 << side));
+  bool yin = false;
+  T y[5];
+  if (dy) {
+    const int i = x_source(yi, yin);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) y[v] = Uc[at(v, i, side ? 17 : 2, yk)];
+  }
+
+  // Z: (i, j) of side t / 512.  Interior planes of a face marked ZBC_IN_FLUX
+  // get their z-BC from the flux kernel.
+  const int zi = w / 20, zj = w % 20, zk = side ? 17 : 2;
+  bool dz = w < 400 && (m & (16 << side)) &&
+            !(zi >= 2 && zi <= 17 && (m & (ZBC_IN_FLUX << side)));
+  bool zin = false;
+  T z[5];
+  if (dz) {
+    // Where the Y-BC wrote the source plane its own source, where that (or
+    // the cell itself) is in a row of the X-BC the source of that.  A k-edge
+    // cell is copied by the lane that forms it.
+    const int j = zj < 2 && (m & 4) ? 2 : (zj > 17 && (m & 8) ? 17 : zj);
+    int i = zi;
+    if (j >= 2 && j <= 17) i = x_source(zi, zin);
+    dz = !(edges != 0 && (i == 1 || i == 18) && (j == 1 || j == 18));
+    if (dz)
+#pragma unroll
+      for (int v = 0; v < 5; ++v) z[v] = Uc[at(v, i, j, zk)];
+  }
+
+  // Edges: item t of 320 per axis (lines of 16 cells, 4 edges, 5 variables),
+  // then the 8 corners x 5 variables, each the mean of the j-edge and the
+  // i-edge cell next to it.  With edges 1 the k-edge cells next to a z-BC.
+  bool de = false, corner = false;
+  int dst = 0, zcopy = 0, ev = 0;   // zcopy 1 (2): z-min (z-max) copies the cell
+  T ea, eb, ec;
+  if (edges == 2 && t < 1000) {
+    de = true;
+    corner = t >= 960;
+    const int A = t / 320, u = corner ? t - 960 : t % 320;
+    const int e = u & 3, v = corner ? (u >> 2) % 5 : (u >> 2) % 5, q = (u >> 2) / 5;
+    const int lo = e & 1 ? 18 : 1, hi = e & 2 ? 18 : 1;
+    int i, j, k;
+    if (corner)
+      i = lo, j = hi, k = q ? 18 : 1;
+    else if (A == 0)
+      i = q + 2, j = lo, k = hi;
+    else if (A == 1)
+      i = hi, j = q + 2, k = lo;
+    else
+      i = hi, j = lo, k = q + 2;
+    dst = at(v, i, j, k);
+    ev = v;
+    if (corner) {
+      // j-edge (i, near j, k) from ea and ec, i-edge (near i, j, k) from eb
+      // and ec.
+      ea = Uc[at(v, i, near(j), near(k))];
+      eb = Uc[at(v, near(i), j, near(k))];
+      ec = Uc[at(v, near(i), near(j), k)];
+    } else if (A == 0) {
+      ea = Uc[at(v, i, j, near(k))];
+      eb = Uc[at(v, i, near(j), k)];
+    } else if (A == 1) {
+      ea = Uc[at(v, i, j, near(k))];
+      eb = Uc[at(v, near(i), j, k)];
+    } else {
+      ea = Uc[at(v, i, near(j), k)];
+      eb = Uc[at(v, near(i), j, k)];
+    }
+    // Cells the BCs overwrite.
+    const bool zinner = i >= 2 && i <= 17;
+    if (!corner && A == 2) {
+      de = !((j == 1 && (m & 4)) || (j == 18 && (m & 8)));
+      zcopy = k == 2 && (m & 16) ? 1 : (k == 17 && (m & 32) ? 2 : 0);
+    } else {
+      de = !((k == 1 && (m & 16) && !(zinner && (m & ZBC_IN_FLUX))) ||
+             (k == 18 && (m & 32) && !(zinner && (m & (ZBC_IN_FLUX << 1)))));
+    }
+  } else if (edges == 1 && t < 40) {
+    const int zs = t / 20, cell = (t / 5) % 4, v = t % 5;
+    const int i = cell & 1 ? 18 : 1, j = cell & 2 ? 18 : 1, k = zs ? 17 : 2;
+    de = (m & (16 << zs)) && !((j == 1 && (m & 4)) || (j == 18 && (m & 8)));
+    if (de) {
+      dst = at(v, i, j, k);
+      ev = v;
+      zcopy = 1 + zs;
+      ea = Uc[at(v, i, near(j), k)];
+      eb = Uc[at(v, near(i), j, k)];
+    }
+  }
+  __syncthreads();   // all loads have returned
+
+  if (de) {
+    if (corner) {
+      ea = 0.5 * (ea + ec);
+      eb = 0.5 * (eb + ec);
+    }
+    const T x = 0.5 * (ea + eb);
+    Uc[dst] = x;
+    if (zcopy) {
+      // dst is the k = 2 (17) cell; its z ghost cells are k = 0, 1 (18, 19).
+      T o = x;
+      if (zcopy == 1 && ev == 3) F.st(&o, 0, 3, -F.ld(&o, 0, 3));
+      T2 q;
+      q.x = q.y = o;
+      *reinterpret_cast<T2*>(Uc + dst + (zcopy == 1 ? -2 : 1)) = q;
+    }
+  }
+  if (dx) {
+    T o[5];
+    if (xs)
+#pragma unroll
+      for (int v = 0; v < 5; ++v) o[v] = x[v];
+    else
+      inflow(x, o);
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
-      if (m & 1) lo[v] = U[sidx(c, v, 2, j, k)];
-      if (m & 2) hi[v] = U[sidx(c, v, 17, j, k)];
-    }
-    if (m & 1) {
-      const double rho = F.ld(lo, 0, 0);
-      const double uu = F.ld(lo, 1, 1) / rho;
-      const double vv = F.ld(lo, 2, 2) / rho;
-      const double ww = F.ld(lo, 3, 3) / rho;
-      double VV = uu * uu + vv * vv + ww * ww;
-      const double P = (F.ld(lo, 4, 4) - 0.5 * rho * VV) * KM1;
-      VV = ph.Uin * ph.Uin + ph.V0 * ph.V0 + ph.W0 * ph.W0;
-      const double E = P / KM1 + 0.5 * rho * VV;
-      for (int i = 0; i < 2; ++i) {
-        U[sidx(c, 0, i, j, k)] = lo[0];
-        F.st(U, sidx(c, 1, i, j, k), 1, rho * ph.Uin);
-        F.st(U, sidx(c, 2, i, j, k), 2, rho * ph.V0);
-        F.st(U, sidx(c, 3, i, j, k), 3, rho * ph.W0);
-        F.st(U, sidx(c, 4, i, j, k), 4, E);
-      }
-    }
-    if (m & 2)
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        U[sidx(c, v, 18, j, k)] = hi[v];
-        U[sidx(c, v, 19, j, k)] = hi[v];
-      }
-  }
-  __syncthreads();
-  {
-    // Rows (i, k) of the y-faces, i = 0..19: w = t and t + 256 (w < 320).
-    T lo[2][5], hi[2][5];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int w = t + h * WG, i = w >> 4, k = (w & 15) + 2;
-      if (w < 20 * 16)
-#pragma unroll
-        for (int v = 0; v < 5; ++v) {
-          if (m & 4) lo[h][v] = U[sidx(c, v, i, 2, k)];
-          if (m & 8) hi[h][v] = U[sidx(c, v, i, 17, k)];
-        }
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int w = t + h * WG, i = w >> 4, k = (w & 15) + 2;
-      if (w < 20 * 16)
-#pragma unroll
-        for (int v = 0; v < 5; ++v) {
-          if (m & 4) {
-            U[sidx(c, v, i, 1, k)] = lo[h][v];
-            U[sidx(c, v, i, 0, k)] = lo[h][v];
-          }
-          if (m & 8) {
-            U[sidx(c, v, i, 18, k)] = hi[h][v];
-            U[sidx(c, v, i, 19, k)] = hi[h][v];
-          }
-        }
+      Uc[at(v, xs ? 18 : 0, xj, xk)] = o[v];
+      Uc[at(v, xs ? 19 : 1, xj, xk)] = o[v];
     }
   }
-  __syncthreads();
-  {
-    // Rows (i, j) of the z-faces: w = t and t + 256 (w < 400).  Interior
-    // planes of a face marked ZBC_IN_FLUX get their z-BC from the flux
-    // kernel.
-    T lo[2][5], hi[2][5];
-    bool dlo[2], dhi[2];
+  if (dy) {
+    T o[5];
+    if (yin)
+      inflow(y, o);
+    else
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int w = t + h * WG, i = w / 20, j = w % 20;
-      const bool inner = i >= 2 && i <= 17;
-      dlo[h] = w < 400 && (m & 16) && !(inner && (m & ZBC_IN_FLUX));
-      dhi[h] = w < 400 && (m & 32) && !(inner && (m & (ZBC_IN_FLUX << 1)));
+      for (int v = 0; v < 5; ++v) o[v] = y[v];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        if (dlo[h]) lo[h][v] = U[sidx(c, v, i, j, 2)];
-        if (dhi[h]) hi[h][v] = U[sidx(c, v, i, j, 17)];
-      }
+    for (int v = 0; v < 5; ++v) {
+      Uc[at(v, yi, side ? 18 : 0, yk)] = o[v];
+      Uc[at(v, yi, side ? 19 : 1, yk)] = o[v];
     }
+  }
+  if (dz) {
+    T o[5];
+    if (zin)
+      inflow(z, o);
+    else
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int w = t + h * WG, i = w / 20, j = w % 20;
-      if (dlo[h])
+      for (int v = 0; v < 5; ++v) o[v] = z[v];
+    if (!side) F.st(o, 3, 3, -F.ld(o, 3, 3));
 #pragma unroll
-        for (int v = 0; v < 5; ++v) {
-          if (v == 3) {
-            const double y = -F.ld(lo[h], 3, 3);
-            F.st(U, sidx(c, v, i, j, 1), 3, y);
-            F.st(U, sidx(c, v, i, j, 0), 3, y);
-          } else {
-            U[sidx(c, v, i, j, 1)] = lo[h][v];
-            U[sidx(c, v, i, j, 0)] = lo[h][v];
-          }
-        }
-      if (dhi[h])
-#pragma unroll
-        for (int v = 0; v < 5; ++v) {
-          U[sidx(c, v, i, j, 18)] = hi[h][v];
-          U[sidx(c, v, i, j, 19)] = hi[h][v];
-        }
+    for (int v = 0; v < 5; ++v) {
+      // Both ghost cells at once: rows are a multiple of two values long.
+      T2 q;
+      q.x = q.y = o[v];
+      *reinterpret_cast<T2*>(Uc + at(v, zi, zj, side ? 18 : 0)) = q;
     }
   }
 }
 
 template <typename T>
-__global__ __launch_bounds__(WG) void k_bc(T* __restrict__ U, const int* __restrict__ cubes,
-                                           const uint8_t* __restrict__ masks, PhysTab pt) {
-  bc_cube(U, cubes[blockIdx.x], masks[blockIdx.x], pt);
+__global__ __launch_bounds__(OPEN_WG) void k_bc(T* __restrict__ U, const int* __restrict__ cubes,
+                                                const uint8_t* __restrict__ masks, PhysTab pt) {
+  const int c = cubes[blockIdx.x];
+  edge_bc_cube(U, c, 0, masks[blockIdx.x], pt.phys[pt.cube_case[c]]);
 }
 
 // ---------------------------------------------------------------------------
@@ -576,298 +673,276 @@ __global__ __launch_bounds__(WG) void k_bc(T* __restrict__ U, const int* __restr
 // the host (an entry's level is above every earlier entry it reads from or
 // whose corners it overwrites), so all entries of one level run in parallel
 // and levels are separated by workgroup barriers.  Interpolation corners
-// always lie in the ghost cell's own padded cube.  The cells a cube's entries
-// touch are staged in LDS as FP64 conserved values (full states), every level
-// runs out of LDS with one value slot per entry (see GhostTables), and the
-// last value of each written ghost cell goes back to memory once; a cube
-// needing more than lds_cap slots works on memory in place.  A value written
-// to LDS is rounded as storage would round it, so both ways give the same
-// results.
+// always lie in the ghost cell's own padded cube.
+//
+// The fill is a chain of latencies (one entry's arithmetic per level, table
+// and state loads before it), so all that can be is taken out of the chain.
+// A corner's density, velocity and pressure depend on its cell alone: they
+// are formed once per staged cell, at the load, and once per entry for the
+// levels above, and a level only reads and combines them, eight lanes to an
+// entry.  A cube's tables start from one record; the next level's entries and
+// the bounds of the one after load during a level, whose barrier leaves memory
+// operations in flight; ghost cells go back to memory once, at the end.  A
+// level takes 0.9 us with few entries and 2.3 with 126 (2.2 us when each
+// entry formed its corners' primitives in one lane and every level waited for
+// its table loads), the whole fill of a sphere inside one cube (7 levels) 12
+// us of 18, of a body on 7 cubes with one of 2040 slots 16 of 75 (then on
+// memory, beyond 1536 slots).
+// A value is rounded to storage precision before a later level reads it, as
+// memory would round it, so the fill on memory (cubes of more slots than
+// GHOST_LDS_SLOTS) gives the same results.
 
-// IB fill of ghost-table cube g by the calling workgroup; gsm holds
-// [5][lds_cap] doubles.
-// The fields of a GhostEntry the fill reads, loaded one by one so that a copy
-// held across a level stays in registers.
+// What the fill in LDS reads of an entry: the weights, the corners' slots (two
+// to a word), and its own slot with the corner that is the ghost cell.
 struct GhostEntryR {
-  int16_t gi, gj, gk, pi, pj, pk, lg;
-  int16_t lc[8];
   double w[8];
+  int lc[4], lg_self;
+  __device__ int slot(int m) const { return (m & 1 ? lc[m / 2] >> 16 : lc[m / 2] & 0xffff); }
 };
 __device__ __forceinline__ GhostEntryR load_entry(const GhostEntry* p) {
   GhostEntryR r;
-  r.gi = p->gi;
-  r.gj = p->gj;
-  r.gk = p->gk;
-  r.pi = p->pi;
-  r.pj = p->pj;
-  r.pk = p->pk;
-  r.lg = p->lg;
+  const int* q = reinterpret_cast<const int*>(p->lc);
 #pragma unroll
-  for (int m = 0; m < 8; ++m) {
-    r.lc[m] = p->lc[m];
-    r.w[m] = p->w[m];
-  }
+  for (int m = 0; m < 8; ++m) r.w[m] = p->w[m];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) r.lc[m] = q[m];
+  r.lg_self = q[4];
   return r;
 }
 
-template <typename T>
-__device__ __forceinline__ void ghost_cube(T* __restrict__ U, const GhostTables& gt, int g,
-                                           int lds_cap, PhysTab pt, double* gsm) {
-  const int l0 = gt.cube_level_off[g], l1 = gt.cube_level_off[g + 1];
-  if (l0 == l1) return;
-  const int c = gt.ent[gt.level_off[l0]].cube;
-  const DevPhys ph = pt.phys[pt.cube_case[c]];
-  const typename OffOf<T>::type F(ph);
-  const double rho0 = ph.rho0, P0 = ph.P0;
-  const int t0 = gt.touched_off[g];
-  const int nt = gt.touched_off[g + 1] - t0;
-  const int ne = gt.level_off[l1] - gt.level_off[l0];
-  const bool lds = nt + ne <= lds_cap;
-  if (lds) {
-    // Up to six cells per lane: the loads of two cells are issued together.
-    for (int n = threadIdx.x; n < nt; n += 2 * WG) {
-      const int n2 = n + WG;
-      const size_t o = (size_t)c * CUBE_STRIDE + gt.touched[t0 + n];
-      const size_t o2 = (size_t)c * CUBE_STRIDE + gt.touched[t0 + (n2 < nt ? n2 : n)];
-      double a[5], a2[5];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        a[v] = F.ld(U, o + (size_t)v * PLANE, v);
-        a2[v] = F.ld(U, o2 + (size_t)v * PLANE, v);
-      }
-#pragma unroll
-      for (int v = 0; v < 5; ++v) gsm[v * lds_cap + n] = a[v];
-      if (n2 < nt) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) gsm[v * lds_cap + n2] = a2[v];
-      }
-    }
-    __syncthreads();
+// Density, velocity and pressure of a conserved state.
+template <typename OFF>
+__device__ __forceinline__ void corner_prim(const double (&q)[5], double (&p)[5]) {
+  const double r = q[0];
+  p[0] = r;
+  if constexpr (OFF::exact) {
+    p[1] = q[1] / r;
+    p[2] = q[2] / r;
+    p[3] = q[3] / r;
+  } else {
+    // One reciprocal per corner instead of three divisions.
+    const double ir = 1.0 / r;
+    p[1] = q[1] * ir;
+    p[2] = q[2] * ir;
+    p[3] = q[3] * ir;
   }
-  // Density, velocity and pressure of one interpolation corner.
-  auto corner_prim = [&](const double (&q)[5], double& r, double& u, double& v, double& w,
-                         double& p) {
-    r = q[0];
-    if constexpr (OffOf<T>::type::exact) {
-      u = q[1] / r;
-      v = q[2] / r;
-      w = q[3] / r;
-    } else {
-      // One reciprocal per corner instead of three divisions.
-      const double ir = 1.0 / r;
-      u = q[1] * ir;
-      v = q[2] * ir;
-      w = q[3] * ir;
+  const double VV = p[1] * p[1] + p[2] * p[2] + p[3] * p[3];
+  p[4] = (q[4] - 0.5 * r * VV) * KM1;
+}
+
+// Conserved state of a ghost cell, by eight lanes that all return it: lane
+// r < 5 of them interpolates quantity r (density, velocity, pressure) from the
+// corners' values x with the weights w; s is the corner that is the ghost cell
+// itself (8: none).
+__device__ __forceinline__ void ghost_state(const double (&w)[8], const double (&x)[8], int s,
+                                            double rho0, double P0, double (&o)[5]) {
+  const int r = threadIdx.x & 7;
+  const bool scalar = r == 0 || r >= 4, self = s < 8;
+  const double off = r == 0 ? rho0 : (r >= 4 ? P0 : 0.0);
+  // Sums over all corners and over those but s, each in corner order.
+  // (Subtracting an offset of zero changes no value.)
+  double all = 0, but = 0, ws = 0, xs = 0;
+#pragma unroll
+  for (int m = 0; m < 8; ++m) {
+    const double y = w[m] * (x[m] - off);
+    all = m == 0 ? y : all + y;
+    but = m == 0 ? y : (m == 1 && s == 0 ? y : (m == s ? but : but + y));
+    ws = m == s ? w[m] : ws;
+    xs = m == s ? x[m] : xs;
+  }
+  double z;
+  if (self) {
+    // The ghost cell is an interpolation corner (:192-449).
+    const double qt = but / ((scalar ? 1 : 2) - ws);
+    z = scalar ? (ws > 0.9999 ? xs : qt + off) : qt;
+  } else {
+    z = scalar ? all + off : all;
+  }
+  const int l0 = threadIdx.x & 56;
+  const double rho = __shfl(z, l0), uu = __shfl(z, l0 + 1), vv = __shfl(z, l0 + 2),
+               ww = __shfl(z, l0 + 3), P = __shfl(z, l0 + 4);
+  const double VV = uu * uu + vv * vv + ww * ww;
+  o[0] = rho;
+  if (self) {
+    o[1] = rho * uu;
+    o[2] = rho * vv;
+    o[3] = rho * ww;
+    o[4] = P / KM1 + 0.5 * rho * VV;
+  } else {
+    o[1] = 0.5 * rho * uu;
+    o[2] = 0.5 * rho * vv;
+    o[3] = 0.5 * rho * ww;
+    o[4] = P / KM1 + 0.5 * rho * 0.25 * VV;
+  }
+}
+// The r-th of five values, by selection (values, as a reference to an array
+// would become an index into memory).
+__device__ __forceinline__ double pick(double a0, double a1, double a2, double a3, double a4,
+                                       int r) {
+  const double x = r == 1 ? a1 : a0, y = r == 3 ? a3 : a2;
+  return r > 3 ? a4 : (r > 1 ? y : x);
+}
+
+// Eight lanes share an entry.  Entry of a lane in a level of n entries
+// starting at e (a lane without one loads the level's first, which it does
+// not use).
+constexpr int GHOST_PASS = OPEN_WG / 8;
+__device__ __forceinline__ int entry_of(int e, int n) {
+  const int q = threadIdx.x / 8;
+  return e + (q < n ? q : 0);
+}
+
+// What a lane can load of a cube's fill before the state it reads is final:
+// its first staged cell (the last one where it has none), its entry of the
+// first level, and the ghost cell it stores (-1: none).
+struct GhostFirst {
+  int cell, out;
+  GhostEntryR E;
+};
+__device__ __forceinline__ void ghost_first(const GhostTables& gt, const GhostCube& g,
+                                            GhostFirst& f) {
+  if (g.nread < 0) return;
+  const int t = threadIdx.x;
+  f.cell = gt.read[g.read0 + (t < g.nread ? t : g.nread - 1)];
+  f.out = gt.out[g.ent0 + (t < g.ne ? t : 0)];
+  f.E = load_entry(gt.ent + entry_of(g.ent0, g.n1));
+}
+
+// Barrier for values exchanged through LDS: unlike __syncthreads it leaves
+// loads and stores of memory in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// IB fill of one cube in LDS by the calling workgroup.  prim holds the
+// primitives of slot n in prim[v * cap + n]; the conserved values of entry a
+// follow in cons[v * ne + a].
+template <typename T>
+__device__ __forceinline__ void ghost_lds(T* __restrict__ U, const GhostTables& gt,
+                                          const GhostCube& g, const GhostFirst& f,
+                                          const DevPhys& ph, double* gsm) {
+  using OFF = typename OffOf<T>::type;
+  const OFF F(ph);
+  const int t = threadIdx.x;
+  const size_t base = (size_t)g.cube * CUBE_STRIDE;
+  const int cap = g.ne + g.nread;
+  double* prim = gsm;
+  double* cons = gsm + 5 * cap;
+  for (int n = t; n < g.nread; n += OPEN_WG) {
+    const int cell = n < OPEN_WG ? f.cell : gt.read[g.read0 + n];
+    double a[5], p[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) a[v] = F.ld(U, base + (size_t)v * PLANE + cell, v);
+    corner_prim<OFF>(a, p);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) prim[v * cap + g.ne + n] = p[v];
+  }
+  lds_barrier();
+  // The value of an entry goes to LDS conserved for the store to memory and
+  // as primitives for the levels above.
+  const int r = t & 7, rv = r < 5 ? r : 4;
+  auto fill_entry = [&](const GhostEntryR& E) {
+    double x[8], o[5], p[5];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) x[m] = prim[rv * cap + E.slot(m)];
+    ghost_state(E.w, x, E.lg_self >> 16, ph.rho0, ph.P0, o);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) o[v] = F.rt(o[v], v);
+    corner_prim<OFF>(o, p);
+    const int lg = E.lg_self & 0xffff;
+    if (r < 5) {
+      cons[r * g.ne + lg] = pick(o[0], o[1], o[2], o[3], o[4], r);
+      prim[r * cap + lg] = pick(p[0], p[1], p[2], p[3], p[4], r);
     }
-    const double VV = u * u + v * v + w * w;
-    p = (q[4] - 0.5 * r * VV) * KM1;
   };
-  // One entry from its corners' primitives: into its slot (LDS) or its ghost
-  // cell (memory).
-  auto combine = [&](const GhostEntryR& E, const double (&rc)[8], const double (&uc)[8],
-                     const double (&vc)[8], const double (&wc)[8], const double (&pc)[8]) {
-    double rho = E.w[0] * (rc[0] - rho0), P = E.w[0] * (pc[0] - P0);
-    double uu = E.w[0] * uc[0], vv = E.w[0] * vc[0], ww = E.w[0] * wc[0];
+  // Levels run one after the other, each taking one entry's latency.  The
+  // lane's entry of the next level is loaded while the current one is
+  // computed, the bounds of the level after that as well.
+  const int end = g.lev0 + g.nlev;
+  GhostEntryR Enext = f.E;
+  int e0 = g.ent0, e1 = g.ent0 + g.n1;
+  int e2 = gt.level_off[min(g.lev0 + 2, end)];
+  for (int lv = g.lev0; lv < end; ++lv) {
+    const GhostEntryR E = Enext;
+    const int e3 = gt.level_off[min(lv + 3, end)];
+    if (e1 < e2) Enext = load_entry(gt.ent + entry_of(e1, e2 - e1));
+    if (e0 + t / 8 < e1) fill_entry(E);
+    for (int n = e0 + t / 8 + GHOST_PASS; n < e1; n += GHOST_PASS) fill_entry(load_entry(gt.ent + n));
+    lds_barrier();
+    e0 = e1;
+    e1 = e2;
+    e2 = e3;
+  }
+  // The last value of each ghost cell goes back to memory.
+  for (int a = t; a < g.ne; a += OPEN_WG) {
+    const int cell = a < OPEN_WG ? f.out : gt.out[g.ent0 + a];
+    if (cell < 0) continue;
 #pragma unroll
-    for (int m = 1; m < 8; ++m) {
-      rho = rho + E.w[m] * (rc[m] - rho0);
-      P = P + E.w[m] * (pc[m] - P0);
-      uu = uu + E.w[m] * uc[m];
-      vv = vv + E.w[m] * vc[m];
-      ww = ww + E.w[m] * wc[m];
-    }
-    rho = rho + rho0;
-    P = P + P0;
-    double VV = uu * uu + vv * vv + ww * ww;
-    double o0 = rho, o1 = 0.5 * rho * uu, o2 = 0.5 * rho * vv, o3 = 0.5 * rho * ww;
-    double o4 = P / KM1 + 0.5 * rho * 0.25 * VV;
-    // The ghost cell may itself be an interpolation corner (:192-449).
-    const int di = E.gi - E.pi, dj = E.gj - E.pj, dk = E.gk - E.pk;
-    if (di >= 0 && di <= 1 && dj >= 0 && dj <= 1 && dk >= 0 && dk <= 1) {
-      const int s = di && dj && dk ? 7
-                    : (dj && dk ? 6 : (di && dk ? 5 : (di && dj ? 4 : (dk ? 3 : (dj ? 2 : (di ? 1 : 0))))));
-      // Corner s's weight and values, selected without indexing by s (which
-      // would put the arrays in memory).
-      double ws = 0, rs = 0, ps = 0;
+    for (int v = 0; v < 5; ++v) F.st(U, base + (size_t)v * PLANE + cell, v, cons[v * g.ne + a]);
+  }
+}
+
+// IB fill of one cube in place on memory: lane m of an entry's eight forms
+// corner m's primitives.
+template <typename T>
+__device__ __forceinline__ void ghost_memory(T* __restrict__ U, const GhostTables& gt,
+                                             const GhostCube& g, const DevPhys& ph) {
+  using OFF = typename OffOf<T>::type;
+  const OFF F(ph);
+  const size_t base = (size_t)g.cube * CUBE_STRIDE;
+  const int r = threadIdx.x & 7, l0 = threadIdx.x & 56;
+  for (int lv = g.lev0; lv < g.lev0 + g.nlev; ++lv) {
+    const int e1 = gt.level_off[lv + 1];
+    for (int n = gt.level_off[lv] + threadIdx.x / 8; n < e1; n += GHOST_PASS) {
+      const GhostEntry& E = gt.ent[n];
+      const int a = (r == 1 || r == 4 || r == 5 || r == 7);
+      const int bq = (r == 2 || r == 4 || r == 6 || r == 7);
+      const int cq = (r == 3 || r == 5 || r == 6 || r == 7);
+      const size_t at = base + (E.pi + a) * 400 + (E.pj + bq) * 20 + (E.pk + cq);
+      double q[5], p[5], w[8], x[8], o[5];
 #pragma unroll
-      for (int m = 0; m < 8; ++m)
-        if (m == s) {
-          ws = E.w[m];
-          rs = rc[m];
-          ps = pc[m];
-        }
-      if (ws > 0.9999) {
-        rho = rs;
-        P = ps;
-      } else {
-        double sr = 0, sp = 0;
-        bool first = true;
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-          if (m == s) continue;
-          if (first) {
-            sr = E.w[m] * (rc[m] - rho0);
-            sp = E.w[m] * (pc[m] - P0);
-            first = false;
-          } else {
-            sr = sr + E.w[m] * (rc[m] - rho0);
-            sp = sp + E.w[m] * (pc[m] - P0);
-          }
-        }
-        rho = sr / (1 - ws) + rho0;
-        P = sp / (1 - ws) + P0;
-      }
-      double su = 0, sv = 0, sw = 0;
-      bool first = true;
+      for (int v = 0; v < 5; ++v) q[v] = F.ld(U, at + (size_t)v * PLANE, v);
+      corner_prim<OFF>(q, p);
 #pragma unroll
       for (int m = 0; m < 8; ++m) {
-        if (m == s) continue;
-        if (first) {
-          su = E.w[m] * uc[m];
-          sv = E.w[m] * vc[m];
-          sw = E.w[m] * wc[m];
-          first = false;
-        } else {
-          su = su + E.w[m] * uc[m];
-          sv = sv + E.w[m] * vc[m];
-          sw = sw + E.w[m] * wc[m];
+        w[m] = E.w[m];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+          const double y = __shfl(p[v], l0 + m);
+          x[m] = v == 0 || r == v ? y : (v == 4 && r > 4 ? y : x[m]);
         }
       }
-      uu = su / (2 - ws);
-      vv = sv / (2 - ws);
-      ww = sw / (2 - ws);
-      VV = uu * uu + vv * vv + ww * ww;
-      o0 = rho;
-      o1 = rho * uu;
-      o2 = rho * vv;
-      o3 = rho * ww;
-      o4 = P / KM1 + 0.5 * rho * VV;
-    }
-    const double out[5] = {o0, o1, o2, o3, o4};
-    if (lds) {
+      ghost_state(w, x, E.self, ph.rho0, ph.P0, o);
+      // Every corner has been read: the eight lanes are in one wave, and no
+      // other entry of the level reads or writes the cell.
+      const size_t go = base + E.gi * 400 + E.gj * 20 + E.gk;
+      if (r == 0)
 #pragma unroll
-      for (int v = 0; v < 5; ++v) gsm[v * lds_cap + E.lg] = F.rt(out[v], v);
-    } else {
-      const size_t go = sidx(c, 0, E.gi, E.gj, E.gk);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) F.st(U, go + (size_t)v * PLANE, v, out[v]);
-    }
-  };
-  // One entry by one lane: interpolation from the eight corners.
-  auto fill_entry = [&](const GhostEntryR& E) {
-    double rc[8], uc[8], vc[8], wc[8], pc[8];
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      const int a = (m == 1 || m == 4 || m == 5 || m == 7);
-      const int bq = (m == 2 || m == 4 || m == 6 || m == 7);
-      const int cq = (m == 3 || m == 5 || m == 6 || m == 7);
-      double q[5];
-      if (lds) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) q[v] = gsm[v * lds_cap + E.lc[m]];
-      } else {
-        const size_t o = sidx(c, 0, E.pi + a, E.pj + bq, E.pk + cq);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) q[v] = F.ld(U, o + (size_t)v * PLANE, v);
-      }
-      corner_prim(q, rc[m], uc[m], vc[m], wc[m], pc[m]);
-    }
-    combine(E, rc, uc, vc, wc, pc);
-  };
-  // Levels run one after the other, each taking one entry's latency.  A level
-  // of at most 64 (32) entries spreads each entry over 4 (8) lanes: they form
-  // its corners' primitives into LDS, and the entry's first lane combines them
-  // as one lane would.  The lane's entry (and corner slots) of the next level
-  // are loaded while the current one is computed; entries beyond the first
-  // 256 of a level load in place.  (A lane without an entry in a level loads
-  // entry 0 of the schedule, which it does not use.)
-  __shared__ double cpr[64 * 8 * 5];   // corner primitives [entry][corner][5]
-  const int t = threadIdx.x;
-  auto lanes_of = [&](int nl) { return !lds || nl > 64 ? 1 : (nl > 32 ? 4 : 8); };
-  // Entry of lane t in a level starting at e with nl entries.
-  auto entry_of = [&](int e, int nl) {
-    const int L = lanes_of(nl);
-    const int q = t / L;
-    return q < nl ? e + q : 0;
-  };
-  // Slots of the corners lane t forms in a level starting at e with nl
-  // entries (spread levels only; corners r*K and r*K+1 of entry q).
-  auto slots_of = [&](int e, int nl, int& s0, int& s1) {
-    const int L = lanes_of(nl);
-    s0 = s1 = 0;
-    if (L == 1) return;
-    const int q = t / L, r = t % L, K = 8 / L;
-    if (q >= nl) return;
-    s0 = gt.ent[e + q].lc[r * K];
-    if (K == 2) s1 = gt.ent[e + q].lc[r * K + 1];
-  };
-  int nl = gt.level_off[l0 + 1] - gt.level_off[l0];
-  GhostEntryR Enext = load_entry(gt.ent + entry_of(gt.level_off[l0], nl));
-  int sn0, sn1;
-  slots_of(gt.level_off[l0], nl, sn0, sn1);
-  for (int lv = l0; lv < l1; ++lv) {
-    const int e0 = gt.level_off[lv], e1 = gt.level_off[lv + 1];
-    nl = e1 - e0;
-    const int L = lanes_of(nl);
-    const GhostEntryR Ecur = Enext;
-    const int sc0 = sn0, sc1 = sn1;
-    if (lv + 1 < l1) {
-      const int nn = gt.level_off[lv + 2] - e1;
-      Enext = load_entry(gt.ent + entry_of(e1, nn));
-      slots_of(e1, nn, sn0, sn1);
-    }
-    if (L == 1) {
-      const int n0 = e0 + t;
-      if (n0 < e1) fill_entry(Ecur);
-      for (int n = n0 + WG; n < e1; n += WG) fill_entry(load_entry(gt.ent + n));
-    } else {
-      // Lane r of entry q forms corners r*K .. r*K+K-1 (the corner index only
-      // addresses memory, so the lanes of a wave run one instruction stream).
-      const int q = t / L, r = t % L, K = 8 / L;
-      if (q < nl) {
-        for (int kk = 0; kk < K; ++kk) {
-          const int m = r * K + kk, sl = kk == 0 ? sc0 : sc1;
-          double qv[5], pv[5];
-#pragma unroll
-          for (int v = 0; v < 5; ++v) qv[v] = gsm[v * lds_cap + sl];
-          corner_prim(qv, pv[0], pv[1], pv[2], pv[3], pv[4]);
-#pragma unroll
-          for (int v = 0; v < 5; ++v) cpr[(q * 8 + m) * 5 + v] = pv[v];
-        }
-      }
-      __syncthreads();
-      if (r == 0 && q < nl) {
-        double rc[8], uc[8], vc[8], wc[8], pc[8];
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-          const double* a = cpr + (q * 8 + m) * 5;
-          rc[m] = a[0];
-          uc[m] = a[1];
-          vc[m] = a[2];
-          wc[m] = a[3];
-          pc[m] = a[4];
-        }
-        combine(Ecur, rc, uc, vc, wc, pc);
-      }
+        for (int v = 0; v < 5; ++v) F.st(U, go + (size_t)v * PLANE, v, o[v]);
     }
     __syncthreads();
-  }
-  if (lds) {
-    const int nw = gt.touched_nw[g];
-    for (int n = threadIdx.x; n < nw; n += WG) {
-      const size_t o = (size_t)c * CUBE_STRIDE + gt.touched[t0 + n];
-      const int sl = gt.touched_final[t0 + n];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) F.st(U, o + (size_t)v * PLANE, v, gsm[v * lds_cap + sl]);
-    }
   }
 }
 
 template <typename T>
-__global__ __launch_bounds__(WG) void k_ghost(T* __restrict__ U, GhostTables gt, int lds_cap,
-                                              PhysTab pt) {
-  extern __shared__ double gsm[];   // [5][lds_cap]
-  ghost_cube(U, gt, blockIdx.x, lds_cap, pt, gsm);
+__device__ __forceinline__ void ghost_cube(T* __restrict__ U, const GhostTables& gt,
+                                           const GhostCube& g, GhostFirst& f, const DevPhys& ph,
+                                           double* gsm) {
+  if (g.nread >= 0)
+    ghost_lds(U, gt, g, f, ph, gsm);
+  else
+    ghost_memory(U, gt, g, ph);
+}
+
+template <typename T>
+__global__ __launch_bounds__(OPEN_WG) void k_ghost(T* __restrict__ U, GhostTables gt, PhysTab pt) {
+  extern __shared__ double gsm[];
+  const GhostCube g = gt.cubes[blockIdx.x];
+  GhostFirst f;
+  ghost_first(gt, g, f);
+  ghost_cube(U, gt, g, f, pt.phys[pt.cube_case[g.cube]], gsm);
 }
 
 // Edge-ghost averaging of one cube in the reference's three sequential passes
@@ -931,10 +1006,6 @@ __device__ __forceinline__ void edge_fill(T* __restrict__ U, int c) {
 // cube's edge-ghost averaging in the reference's three sequential passes
 // (:5640-5732).  Sources are interior layers, which nothing in this kernel
 // writes, so cubes proceed independently.
-template <typename T> struct Vec2;
-template <> struct Vec2<double> { using type = double2; };
-template <> struct Vec2<float> { using type = float2; };
-
 template <typename T>
 __global__ __launch_bounds__(WG) void k_halo_edge(T* __restrict__ U,
                                                   const HaloSrc* __restrict__ srcs,
@@ -1027,52 +1098,24 @@ __global__ __launch_bounds__(WG) void k_edge_list(T* __restrict__ U, const int* 
   edge_fill(U, list[blockIdx.x]);
 }
 
-// Stage start after a flux kernel that wrote its face halos into the
-// neighbours (flux_push), for one cube (entry c): the edge passes of the
-// post-update exchange (Interface.cpp:5640-5732), then the domain BCs of the
-// next stage.  Entry -c asks only for the edge cells the BCs read: the z-BC
-// (BCM_Z_boundary_condition.cpp:47-88) copies the plane k = 2 (or 17) whole,
-// four of whose cells are k-edges, each the mean of two face ghost cells
-// taken before the X- and Y-BCs overwrite them.
-template <typename T>
-__device__ __forceinline__ void edge_bc_cube(T* __restrict__ U, int entry,
-                                             const uint8_t* __restrict__ cube_mask, PhysTab pt) {
-  const int c = entry > 0 ? entry : -entry;
-  if (pt.cube_case[c] < 0) return;
-  const int m = cube_mask[c];
-  if (entry > 0) {
-    edge_fill(U, c);
-  } else if (threadIdx.x < 40) {
-    const int side = threadIdx.x / 20, cell = (threadIdx.x / 5) % 4, v = threadIdx.x % 5;
-    if (m & (side ? 32 : 16)) {
-      const int ii = cell & 1 ? 18 : 1, jj = cell & 2 ? 18 : 1, kk = side ? 17 : 2;
-      int a, b;
-      edge_sources(ii, jj, kk, a, b);
-      const size_t o = (size_t)c * CUBE_STRIDE + (size_t)v * PLANE;
-      U[o + ii * 400 + jj * 20 + kk] = 0.5 * (U[o + a] + U[o + b]);
-    }
-  }
-  if (m) {
-    __syncthreads();
-    bc_cube(U, c, m, pt);
-  }
-}
-
-// Opening of a pushed stage in one launch: per item, a cube's edge passes and
-// BCs (x: entry as for edge_bc_cube, 0 for none), then its IB fill (y: ghost
-// table index, -1 for none).  Both touch only the cube's own cells, so cubes
+// Opening of a stage after a flux kernel that wrote its face halos into the
+// neighbours (flux_push), in one launch: per item, a cube's edge passes of the
+// post-update exchange and the domain BCs of the next stage, then its IB fill.  Both touch only the cube's own cells, so cubes
 // proceed independently, each in the reference's order.
 template <typename T>
-__global__ __launch_bounds__(WG) void k_open(T* __restrict__ U, const int2* __restrict__ items,
-                                             const uint8_t* __restrict__ cube_mask,
-                                             GhostTables gt, int lds_cap, PhysTab pt) {
-  extern __shared__ double gsm[];   // [5][lds_cap]
-  const int2 it = items[blockIdx.x];
-  if (it.x != 0) edge_bc_cube(U, it.x, cube_mask, pt);
-  if (it.y >= 0) {
-    __syncthreads();
-    ghost_cube(U, gt, it.y, lds_cap, pt, gsm);
-  }
+__global__ __launch_bounds__(OPEN_WG) void k_open(T* __restrict__ U, const OpenItem* __restrict__ items,
+                                             GhostTables gt,
+                                             const DevPhys* __restrict__ phys) {
+  extern __shared__ double gsm[];
+  const OpenItem it = items[blockIdx.x];
+  const DevPhys ph = phys[it.slot];
+  if (it.edges) edge_bc_cube(U, it.g.cube, it.edges, it.mask, ph);
+  if (it.g.nlev == 0) return;
+  // The fill's tables load while the stores above complete.
+  GhostFirst f;
+  ghost_first(gt, it.g, f);
+  if (it.edges) __syncthreads();
+  ghost_cube(U, gt, it.g, f, ph, gsm);
 }
 
 // Two-level faces (BCM_Interface.cpp:1790-2600 for x, :2651-3470 for y,
@@ -1177,7 +1220,7 @@ int update_blocks(int ncube) { return 16 * (ncube - 1); }
 
 template <typename T>
 void launch_bc_t(hipStream_t s, T* U, const int* cubes, const uint8_t* masks, int n, PhysTab pt) {
-  if (n > 0) hipLaunchKernelGGL(k_bc<T>, dim3(n), dim3(WG), 0, s, U, cubes, masks, pt);
+  if (n > 0) hipLaunchKernelGGL(k_bc<T>, dim3(n), dim3(OPEN_WG), 0, s, U, cubes, masks, pt);
 }
 void launch_bc(hipStream_t s, double* U, const int* cubes, const uint8_t* masks, int n,
                PhysTab pt) {
@@ -1191,9 +1234,8 @@ void launch_bc(hipStream_t s, float* U, const int* cubes, const uint8_t* masks, 
 template <typename T>
 void launch_ghost_t(hipStream_t s, T* U, const GhostTables& g, PhysTab pt) {
   if (g.ncubes <= 0) return;
-  const int cap = g.max_slots < GHOST_LDS_SLOTS ? g.max_slots : GHOST_LDS_SLOTS;
-  const size_t shmem = (size_t)(cap > 0 ? cap : 1) * 5 * sizeof(double);
-  hipLaunchKernelGGL(k_ghost<T>, dim3(g.ncubes), dim3(WG), shmem, s, U, g, cap, pt);
+  const size_t shmem = (size_t)g.max_slots * 5 * sizeof(double);
+  hipLaunchKernelGGL(k_ghost<T>, dim3(g.ncubes), dim3(OPEN_WG), shmem, s, U, g, pt);
 }
 void launch_ghost(hipStream_t s, double* U, const GhostTables& g, PhysTab pt) {
   launch_ghost_t(s, U, g, pt);
@@ -1203,20 +1245,19 @@ void launch_ghost(hipStream_t s, float* U, const GhostTables& g, PhysTab pt) {
 }
 
 template <typename T>
-void launch_open_t(hipStream_t s, T* U, const int2* items, int n, const uint8_t* cube_mask,
-                   const GhostTables& g, PhysTab pt) {
+void launch_open_t(hipStream_t s, T* U, const OpenItem* items, int n, const GhostTables& g,
+                   const DevPhys* phys) {
   if (n <= 0) return;
-  const int cap = g.max_slots < GHOST_LDS_SLOTS ? g.max_slots : GHOST_LDS_SLOTS;
-  const size_t shmem = (size_t)(cap > 0 ? cap : 1) * 5 * sizeof(double);
-  hipLaunchKernelGGL(k_open<T>, dim3(n), dim3(WG), shmem, s, U, items, cube_mask, g, cap, pt);
+  const size_t shmem = (size_t)g.max_slots * 5 * sizeof(double);
+  hipLaunchKernelGGL(k_open<T>, dim3(n), dim3(OPEN_WG), shmem, s, U, items, g, phys);
 }
-void launch_open(hipStream_t s, double* U, const int2* items, int n, const uint8_t* cube_mask,
-                 const GhostTables& g, PhysTab pt) {
-  launch_open_t(s, U, items, n, cube_mask, g, pt);
+void launch_open(hipStream_t s, double* U, const OpenItem* items, int n, const GhostTables& g,
+                 const DevPhys* phys) {
+  launch_open_t(s, U, items, n, g, phys);
 }
-void launch_open(hipStream_t s, float* U, const int2* items, int n, const uint8_t* cube_mask,
-                 const GhostTables& g, PhysTab pt) {
-  launch_open_t(s, U, items, n, cube_mask, g, pt);
+void launch_open(hipStream_t s, float* U, const OpenItem* items, int n, const GhostTables& g,
+                 const DevPhys* phys) {
+  launch_open_t(s, U, items, n, g, phys);
 }
 
 template <typename T>

@@ -278,7 +278,7 @@ int bcm_engine_autotune(bcm_engine* e, int* out3);
 /* Ghost schedule statistics: entries, cubes with entries, maximum levels. */
 int bcm_engine_ghost_stats(bcm_engine* e, int* stats3);
 /* The IB fill of a cube runs out of LDS when its value slots fit the limit
- * (at most 1536, the default), else in place on memory; a lower limit,
+ * (0..1536; 3072 unless set), else in place on memory; a lower limit,
  * applied to cases loaded or added afterwards, puts more cubes on the memory
  * schedule (bitwise the same results).  Not a reference interface: a test
  * and diagnostic hook. */

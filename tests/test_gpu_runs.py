@@ -83,3 +83,35 @@ def test_mixed_runs_by_rule_are_bitwise(B, dims):
     for st, er in out[1:]:
         assert np.array_equal(st.view(np.int64), out[0][0].view(np.int64))
         assert np.array_equal(er.view(np.int64), out[0][1].view(np.int64))
+
+
+# Stage opening: IB cubes with BCs on three faces and entries at their edge
+# cells; levels of more entries than one pass takes, in more than 1536 slots.
+@pytest.mark.parametrize("dims", [(2, 2, 1), (2, 2, 2), (5, 5, 5)],
+                         ids=lambda d: str(int(np.prod(d))))
+def test_stage_opening_bitwise(B, O, dims):
+    size = 1.0 / max(dims)
+    case = B.Case(B.case_params("cfg2", lattice=dims, cube_size=size,
+                                sphere_center=tuple(0.5 * d * size for d in dims),
+                                sphere_diameter=0.25 * min(dims) * size))
+    e = B.Engine(0)
+    try:
+        e.load_case(case)
+        h = e.run(1, 2)
+        orc = O.OracleRun(case, nthreads=16)
+        ho = orc.run(1, 2)
+        compare(e, orc, STATE)
+        assert er_close(h, ho)
+        # mixed: the fill in LDS against the fill on memory
+        out = []
+        for limit in (None, 0):
+            if limit is not None:
+                e.set_ghost_lds_limit(limit)
+            e.alloc_pool(case.ncube - 1, 1, "mixed")
+            s = e.add_case(case)
+            er = e.run(1, 2)
+            out.append((e.case_state(s, "U1_"), er))
+        for a, b in zip(*out):
+            assert np.array_equal(a.view(np.int64), b.view(np.int64))
+    finally:
+        e.close()
