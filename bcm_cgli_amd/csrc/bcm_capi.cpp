@@ -603,7 +603,7 @@ int bcm_engine_time_part(bcm_engine* h, int part, int RK, int reps, double* ms) 
   // The pushing stage kernel is timed as the inner iterations of a step run
   // it, without the stores of Rku1, U1p1, U1p2 and Residual1 that only a
   // step's last inner iteration makes.
-  e->push_aux = part != 9;
+  e->push_aux = part != 9 ? PushAux::ALL : PushAux::NONE;
   if (hipEventRecord(e->ev0, e->stream) != hipSuccess) return fail("event record failed");
   for (int r = 0; r < reps; ++r) {
     switch (part) {
@@ -617,10 +617,10 @@ int bcm_engine_time_part(bcm_engine* h, int part, int RK, int reps, double* ms) 
       case 7: engine_flux_update(e, RK, 0); break;
       case 8: engine_halo_refresh(e); break;
       case 9: engine_flux_push(e, RK, 0); break;
-      default: e->push_aux = true; return fail("unknown part");
+      default: e->push_aux = PushAux::ALL; return fail("unknown part");
     }
   }
-  e->push_aux = true;
+  e->push_aux = PushAux::ALL;
   if (hipEventRecord(e->ev1, e->stream) != hipSuccess) return fail("event record failed");
   if (hipEventSynchronize(e->ev1) != hipSuccess) return fail("event wait failed");
   float t = 0;

@@ -58,7 +58,8 @@ void free_graph(Engine* e) {
 // Tables of the resident cases (rebuilt whenever a case comes or goes).
 void free_tables(Engine* e) {
   void* ptrs[] = {e->bc_cubes,     e->bc_masks, e->halo,     e->halo_pairs,
-                  e->case_desc,    e->bc_mask_cube, e->ml, e->edge_list, e->open_items};
+                  e->case_desc,    e->bc_mask_cube, e->ml, e->edge_list, e->open_items,
+                  e->halo_pairs_off, e->ml_ib};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   ghost_free(e->ghost);
@@ -67,11 +68,14 @@ void free_tables(Engine* e) {
   e->bc_mask_cube = nullptr;
   e->halo = nullptr;
   e->halo_pairs = nullptr;
+  e->halo_pairs_off = nullptr;
+  e->ml_ib = nullptr;
   e->case_desc = nullptr;
   e->ml = nullptr;
   e->edge_list = nullptr;
   e->open_items = nullptr;
-  e->n_halo_pairs = e->n_bc = e->n_ghost_cubes = e->n_ghost_entries = e->n_ml = 0;
+  e->n_halo_pairs = e->n_bc = e->n_ghost_cubes = e->n_ghost_entries = e->n_ml =
+      e->n_ml_ib = 0;
   e->n_edge_list = e->n_open_items = 0;
 }
 
@@ -526,6 +530,31 @@ int rebuild_tables(Engine* e, std::string& err) {
   e->n_ml = (int)ml.size();
   if (dev_upload(&e->ml, ml, err)) return 1;
   {
+    // (pairs come by destination cube within a case, cases in pool order)
+    std::vector<int> poff(top + 1, 0);
+    for (const int2& pr : pairs) ++poff[pr.y / PLANE + 1];
+    for (int c = 0; c < top; ++c) poff[c + 1] += poff[c];
+    if (dev_upload(&e->halo_pairs_off, poff, err)) return 1;
+    std::vector<std::vector<const GhostEntry*>> ib(ml.empty() ? 0 : top);
+    if (!ml.empty())
+      for (const GhostEntry& E : gs.entries) ib[E.cube].push_back(&E);
+    std::vector<MlTaskDev> again;
+    for (const MlTaskDev& t : ml) {
+      // Layers along the face's axis (of the source at least those read).
+      auto hit = [&](int cube, int lo, int hi) {
+        for (const GhostEntry* E : ib[cube]) {
+          const int q = t.axis == 0 ? E->gi : t.axis == 1 ? E->gj : E->gk;
+          if (q >= lo && q <= hi) return true;
+        }
+        return false;
+      };
+      if (hit(t.src, t.hi ? 2 : 14, t.hi ? 5 : 17) || hit(t.dst, t.hi ? 18 : 0, t.hi ? 19 : 1))
+        again.push_back(t);
+    }
+    e->n_ml_ib = (int)again.size();
+    if (dev_upload(&e->ml_ib, again, err)) return 1;
+  }
+  {
     std::vector<char> mark(top, 0);
     for (int c : bc) mark[c] = 1;
     for (const int2& pr : pairs) mark[pr.y / PLANE] = 1;
@@ -856,28 +885,27 @@ namespace {
 // two-level faces, whose restrictions read small cubes' cells near the face,
 // then the edge passes of the cubes whose face ghosts changed since the
 // stage's opening edge pass (elsewhere they would give the same values).
-// Before a halo-pushing flux kernel (which forms the edge cells it reads)
-// the edge passes are left out.
 template <typename T>
-void halo_refresh(Engine* e, T* U, bool edges) {
+void halo_refresh(Engine* e, T* U) {
   launch_halo_pairs(e->stream, U, e->halo_pairs, e->n_halo_pairs);
   launch_halo_ml(e->stream, U, e->ml, e->n_ml, e->pt());
-  if (edges) launch_edge_list(e->stream, U, e->edge_list, e->n_edge_list);
+  launch_edge_list(e->stream, U, e->edge_list, e->n_edge_list);
 }
 }  // namespace
 
 void engine_halo_refresh(Engine* e) {
   if (e->prec == 1)
-    halo_refresh(e, e->Uf, true);
+    halo_refresh(e, e->Uf);
   else
-    halo_refresh(e, e->U, true);
+    halo_refresh(e, e->U);
 }
 
 namespace {
 // Opening of a stage after a halo-pushing flux kernel: two-level faces, then
 // the edge passes and BCs of the cubes that need their edge cells in memory,
-// then the IB fill and the pre-flux exchange (full, or the refresh without
-// edge passes).
+// then the IB fill and the pre-flux exchange: the full one, or of the two-level
+// faces those that the fill changed.  The equal-size faces' IB ghost cells are
+// refreshed by the flux kernel, which also forms the edge cells it reads.
 template <typename T>
 void push_stage_open(Engine* e, T* U, bool full_pre_halo) {
   launch_halo_ml(e->stream, U, e->ml, e->n_ml, e->pt());
@@ -885,7 +913,7 @@ void push_stage_open(Engine* e, T* U, bool full_pre_halo) {
   if (full_pre_halo)
     engine_interface(e);
   else
-    halo_refresh(e, U, false);
+    launch_halo_ml(e->stream, U, e->ml_ib, e->n_ml_ib, e->pt());
 }
 }  // namespace
 
@@ -933,7 +961,7 @@ void engine_flux_update(Engine* e, int RK, int er_slot) {
   if (e->prec == 1) {
     launch_flux_mixed(e->stream, e->Uf, e->Uf2, e->halo, e->bc_mask_cube, e->Bsrc, e->fws,
                       e->cube_size, e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e, RK,
-                      e->partials, mixed_runs_now(e));
+                      e->partials, e->ib_refresh(), mixed_runs_now(e));
     std::swap(e->Uf, e->Uf2);
     if (RK == 3)
       launch_reduce(e->stream, e->partials, MIXED_ROWS_PER_CUBE, e->case_desc, e->n_active,
@@ -1063,7 +1091,7 @@ void engine_flux_push(Engine* e, int RK, int er_slot) {
   }
   launch_flux_push(e->stream, e->U, e->U2, e->halo, e->bc_mask_cube, e->U1, e->U1q, e->fws,
                    e->cube_size, e->Rku, e->Res, e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e,
-                   RK, e->U1p1, e->U1p2, e->partials, e->push_aux ? 1 : 0,
+                   RK, e->U1p1, e->U1p2, e->partials, e->push_aux, e->ib_refresh(),
                    push_runs(resident_cubes(e)));
   std::swap(e->U, e->U2);
   if (RK == 3)
@@ -1120,10 +1148,10 @@ void enqueue_step(Engine* e, int n_inner, bool full_first) {
   // Residual1, which no stage reads back: the step ends with the arrays the
   // reference leaves.
   for (int it = 0; it < n_inner; ++it) {
-    e->push_aux = it == n_inner - 1;
+    e->push_aux = it == n_inner - 1 ? PushAux::STEP_END : PushAux::NONE;
     for (int RK = 1; RK <= 3; ++RK) engine_stage(e, RK, it, full_first && it == 0 && RK == 1);
   }
-  e->push_aux = true;
+  e->push_aux = PushAux::ALL;
   engine_shift(e);
   // An odd number of flux kernels that swap copies: bring the iterate back to
   // the copy the step started from, so that every replay of a captured step
@@ -1264,7 +1292,9 @@ int engine_run_converge(Engine* e, int n_steps, int max_inner, double tol, doubl
     const bool full = e->halo_full_next;
     e->halo_full_next = false;
     for (int it = 1; running > 0; ++it) {
+      e->push_aux = PushAux::STEP_END;   // (any iteration may be the last)
       for (int RK = 1; RK <= 3; ++RK) engine_stage(e, RK, 0, full && it == 1 && RK == 1);
+      e->push_aux = PushAux::ALL;
       HIP_TRY(hipMemcpyAsync(e->er_host, e->er_dev, row * sizeof(double), hipMemcpyDeviceToHost,
                              e->stream));
       HIP_TRY(hipStreamSynchronize(e->stream));

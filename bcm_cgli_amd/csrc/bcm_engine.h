@@ -85,6 +85,7 @@ struct Engine {
   int* cube_case = nullptr;           // [cap]
   CaseDesc* case_desc = nullptr;      // [n_active], ordered by first cube
   PhysTab pt() const { return PhysTab{phys_dev, cube_case}; }
+  IbRefresh ib_refresh() const { return IbRefresh{halo_pairs, halo_pairs_off}; }
 
   // Arithmetic of the pool: 0 plain FP64 (bitwise the reference), 1 mixed
   // (FP32 inner iterate and stage arithmetic, FP64 time levels, source and norms).
@@ -118,22 +119,26 @@ struct Engine {
   // Pre-flux halo refresh: (source, destination) cells of the IB ghost cells
   // that lie in a neighbour's gather source layers.
   int2* halo_pairs = nullptr;
+  int* halo_pairs_off = nullptr;   // first pair of each destination cube
   int n_halo_pairs = 0;
   // Two-level faces of all resident cases, refreshed after the equal-size
   // faces and before the edge passes wherever an exchange runs.
   MlTaskDev* ml = nullptr;
   int n_ml = 0;
+  // Those of them that the pre-flux refresh repeats: an IB ghost cell lies in
+  // the cells the task reads or writes.
+  MlTaskDev* ml_ib = nullptr;
+  int n_ml_ib = 0;
   // Cubes whose face ghosts can change between a stage's opening edge pass
   // and its pre-flux exchange (BC, IB-refresh and two-level destinations):
   // the pre-flux edge pass covers only these.
   int* edge_list = nullptr;
   int n_edge_list = 0;
   // Opening of a stage after a flux kernel that pushed its face halos, one
-  // item per cube that needs one: (edge entry, ghost-table index or -1), IB
-  // cubes first.  Edge entry c: all edge passes, then BCs (the cube's IB fill
-  // touches an edge cell); -c: the k-edge cells the z-BC copies, then BCs
-  // (other boundary cubes); 0: none.  Elsewhere only the pushing flux kernels
-  // read edge cells, and they form them themselves.
+  // item per cube that needs one, IB cubes first (their fills are the longest
+  // chains).  All edge passes where the cube's IB fill touches an edge cell, in
+  // other boundary cubes the k-edge cells the z-BC copies.  Elsewhere only the
+  // pushing flux kernels read edge cells, and they form them themselves.
   OpenItem* open_items = nullptr;
   int n_open_items = 0;
   // Set when an inner iterate was replaced from outside (state upload, new
@@ -153,10 +158,10 @@ struct Engine {
   // into the other copy of the iterate (engine stages only; the stage pieces
   // and drop-ins keep the in-place kernels).
   bool flux_push = true;
-  // The pushing FP64 kernel stores Rku1, U1p1, U1p2 and Residual1 (which no
-  // stage reads back) only when set: captured steps clear it for all but
-  // their last inner iteration.
-  bool push_aux = true;
+  // What the pushing FP64 kernel stores of Rku1, U1p1, U1p2 and Residual1,
+  // which no stage reads back: a step asks for them in its last inner
+  // iteration, a single stage stores them all.
+  PushAux push_aux = PushAux::ALL;
   // Mixed path: runs per cube of the flux kernel when pinned with set_flux, or
   // found by the autotuner for size class tuned_class of the resident pool
   // (log2 of its cubes); otherwise they follow the resident cubes by rule.

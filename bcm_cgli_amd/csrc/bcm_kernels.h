@@ -230,6 +230,35 @@ __device__ inline void copy_bc_regions(const T* __restrict__ Uin, T* __restrict_
   }
 }
 
+// IB ghost cells that lie in the source layers of a neighbour, which the
+// pre-flux exchange refreshes in its face layers: cell pairs sorted by
+// destination cube, (source, destination) flat cells, cube * 8000 + cell, those
+// of cube c at off[c] .. off[c + 1] - 1.
+struct IbRefresh {
+  const int2* pairs = nullptr;
+  const int* off = nullptr;
+};
+// The refresh of cube c by a workgroup of the pushing flux kernel, before its
+// first read of the cube: in a launch of its own it took 5 us per stage, a
+// tenth of a stage on 8 cubes.  Sources are interior cells, which that kernel
+// writes in the other copy only; the runs of a cube store the same values.
+template <typename T>
+__device__ inline void refresh_cube(T* __restrict__ U, const IbRefresh& r, int c) {
+  const int q0 = r.off[c], q1 = r.off[c + 1];
+  if (q0 == q1) return;
+  for (int q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
+    const int2 pr = r.pairs[q];
+    const size_t so = (size_t)(pr.x / PLANE) * CUBE_STRIDE + pr.x % PLANE;
+    const size_t dd = (size_t)(pr.y / PLANE) * CUBE_STRIDE + pr.y % PLANE;
+    T x[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) x[v] = U[so + (size_t)v * PLANE];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) U[dd + (size_t)v * PLANE] = x[v];
+  }
+  __syncthreads();
+}
+
 // Sums eight doubles over the 64 lanes of a wave in a fixed order; every lane
 // returns the total of x[lane >> 3].  Halving the values kept at each exchange
 // (lane halves, rows of 16, halves of a row) takes 10 additions where eight
@@ -322,16 +351,19 @@ constexpr int IN_PLACE_SPLIT = 320;
 // of 16/nseg planes per cube, one workgroup each, bitwise the same results for
 // every nseg: every interior cell, and the two layers next to each face with an
 // equal-size neighbour (halo[c]) into that neighbour's ghost layers in Uout.
-// With aux != 0 it writes Rku, Res, U1p1 (RK1) and U1p2 (RK2) bitwise as the
-// in-place fused kernel does (nothing reads them back during stages); at RK 3
+// With PushAux::ALL it writes Rku, Res, U1p1 (RK1) and U1p2 (RK2) bitwise as the
+// in-place fused kernel does (nothing reads them back during stages), with
+// STEP_END Rku and Res at RK 3 only, with NONE none of them; at RK 3
 // PUSH_ROWS_PER_CUBE rows of 8 norm partials per cube (one per plane) either way.
 // Ghost regions the domain BCs wrote (cube_mask) are copied from Uin to Uout.
 constexpr int PUSH_ROWS_PER_CUBE = 16;
-void launch_flux_push(hipStream_t s, const double* Uin, double* Uout, const HaloSrc* halo,
+enum class PushAux { NONE, STEP_END, ALL };
+void launch_flux_push(hipStream_t s, double* Uin, double* Uout, const HaloSrc* halo,
                       const uint8_t* cube_mask, const double* U1, const double* U1q,
                       const int8_t* fws, const double* cube_size, double* Rku, double* Res,
                       int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int RK,
-                      double* U1p1, double* U1p2, double* partials, int aux, int nseg);
+                      double* U1p1, double* U1p2, double* partials, PushAux aux, IbRefresh ib,
+                      int nseg);
 // Runs per cube of the pushing FP64 kernel for n resident cubes.
 int push_runs(int n);
 void launch_copy_d(hipStream_t s, const double* src, double* dst, size_t n);
@@ -369,10 +401,10 @@ int update_blocks(int ncube);
 // workgroup each; results are bitwise the same for every nseg.  At RK 3,
 // MIXED_ROWS_PER_CUBE rows of 8 norm partials per cube (one per plane).
 constexpr int MIXED_ROWS_PER_CUBE = 16;
-void launch_flux_mixed(hipStream_t s, const float* Uin, float* Uout, const HaloSrc* halo,
+void launch_flux_mixed(hipStream_t s, float* Uin, float* Uout, const HaloSrc* halo,
                        const uint8_t* cube_mask, const double* Bsrc, const int8_t* fws,
                        const double* cube_size, int ncube, PhysTab pt, double deltaT,
-                       double deltaTau, double e, int RK, double* partials, int nseg);
+                       double deltaTau, double e, int RK, double* partials, IbRefresh ib, int nseg);
 // Runs per cube for n resident cubes.
 int mixed_runs(int n);
 // dst[0..n) <- src[0..n).

@@ -324,11 +324,11 @@ __device__ __forceinline__ T& at_byte(T* base, unsigned off) {
 // march that kept the whole column in registers, two face arrays more in LDS and
 // a boundary round per axis: 570 -> 555 us on 2,048 cubes, 51 -> 45 on 125.
 __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
-    const float* __restrict__ U, float* __restrict__ Uout, const HaloSrc* __restrict__ halo,
+    float* __restrict__ U, float* __restrict__ Uout, const HaloSrc* __restrict__ halo,
     const uint8_t* __restrict__ cube_mask, const double* __restrict__ Bsrc,
     const int8_t* __restrict__ fws, const double* __restrict__ cube_size, PhysTab pt,
     double deltaT, double deltaTau, double e_d, int RK, double* __restrict__ partials,
-    Runs runs, int ncube) {
+    IbRefresh ib, Runs runs, int ncube) {
   __shared__ __align__(16) float cp[2][5 * 400];   // conserved values of planes i, i+1
   __shared__ int8_t fl[2][400];                    // flags of planes i, i+1
   __shared__ float pr[4][3 * PR];                  // u, v, w, T of planes i-1..i+1
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
   const float sut = (float)(ph.T0 + 110.);
   const double i2dT = 1.0 / (2 * deltaT);
   const float dT = (float)deltaT, dtau = (float)deltaTau;
-  const float* __restrict__ Uc = U + (size_t)c * CUBE_STRIDE;
+  const float* Uc = U + (size_t)c * CUBE_STRIDE;
   const HaloSrc hs = halo[c];
   const int8_t* __restrict__ Fc = fws + (size_t)c * PLANE;
   // ZBC_IN_FLUX faces: the z-ghost cells (k = 0, 1 or 18, 19) of the interior
@@ -363,6 +363,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
   const int zm = cube_mask[c];
   const bool zlo = (zm & ZBC_IN_FLUX) != 0, zhi = (zm & (ZBC_IN_FLUX << 1)) != 0;
   const double r3 = ph.rho0 * ph.W0;
+  refresh_cube(U, ib, c);
 
   // The lane's cell, re-formed at the top of every plane iteration (below).
   int t = threadIdx.x;
@@ -934,15 +935,15 @@ __global__ __launch_bounds__(WG) void k_soa_to_aos_f(const float* __restrict__ s
 
 }  // namespace
 
-void launch_flux_mixed(hipStream_t s, const float* Uin, float* Uout, const HaloSrc* halo,
+void launch_flux_mixed(hipStream_t s, float* Uin, float* Uout, const HaloSrc* halo,
                        const uint8_t* cube_mask, const double* Bsrc, const int8_t* fws,
                        const double* cube_size, int ncube, PhysTab pt, double deltaT,
-                       double deltaTau, double e, int RK, double* partials, int nseg) {
+                       double deltaTau, double e, int RK, double* partials, IbRefresh ib, int nseg) {
   if (ncube <= 1) return;
   const Runs runs = runs_for(ncube, nseg);
   hipLaunchKernelGGL(k_flux_mixed, run_grid(runs, ncube), dim3(WG), 0, s, Uin, Uout, halo,
-                     cube_mask, Bsrc, fws, cube_size, pt, deltaT, deltaTau, e, RK, partials, runs,
-                     ncube);
+                     cube_mask, Bsrc, fws, cube_size, pt, deltaT, deltaTau, e, RK, partials, ib,
+                     runs, ncube);
 }
 
 // Runs per cube of the mixed flux kernel; the chip holds 512 of its workgroups.
