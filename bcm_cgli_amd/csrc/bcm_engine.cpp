@@ -959,12 +959,13 @@ int mixed_runs_now(const Engine* e) {
 
 void engine_flux_update(Engine* e, int RK, int er_slot) {
   if (e->prec == 1) {
-    launch_flux_mixed(e->stream, e->Uf, e->Uf2, e->halo, e->bc_mask_cube, e->Bsrc, e->fws,
-                      e->cube_size, e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e, RK,
-                      e->partials, e->ib_refresh(), mixed_runs_now(e));
+    const int single = launch_flux_mixed(
+        e->stream, e->Uf, e->Uf2, e->halo, e->bc_mask_cube, e->Bsrc, e->fws, e->cube_size,
+        e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e, RK, e->partials, e->ib_refresh(),
+        mixed_runs_now(e));
     std::swap(e->Uf, e->Uf2);
     if (RK == 3)
-      launch_reduce(e->stream, e->partials, MIXED_ROWS_PER_CUBE, e->case_desc, e->n_active,
+      launch_reduce(e->stream, e->partials, MIXED_ROWS_PER_CUBE, single, e->case_desc, e->n_active,
                     e->phys_dev, er_row(e, er_slot));
     return;
   }
@@ -977,7 +978,8 @@ void engine_flux_update(Engine* e, int RK, int er_slot) {
                                         e->Rku, e->Res, e->ncube, e->pt(), e->deltaT, e->deltaTau,
                                         e->e, RK, e->U1p1, e->U1p2, e->partials);
   if (RK == 3)
-    launch_reduce(e->stream, e->partials, rows, e->case_desc, e->n_active, e->phys_dev,
+    launch_reduce(e->stream, e->partials, rows, rows == 1 ? e->ncube - 1 : 0, e->case_desc,
+                  e->n_active, e->phys_dev,
                   er_row(e, er_slot));
 }
 
@@ -1073,7 +1075,7 @@ void engine_update(Engine* e, int RK, int er_slot) {
   launch_update(e->stream, RK, e->U, e->U1p1, e->U1p2, e->Rku, e->Res, e->fws, e->ncube,
                 e->cube_case, e->partials);
   if (RK == 3)
-    launch_reduce(e->stream, e->partials, 16, e->case_desc, e->n_active, e->phys_dev,
+    launch_reduce(e->stream, e->partials, 16, 0, e->case_desc, e->n_active, e->phys_dev,
                   er_row(e, er_slot));
 }
 
@@ -1089,14 +1091,15 @@ void engine_flux_push(Engine* e, int RK, int er_slot) {
     engine_flux_update(e, RK, er_slot);
     return;
   }
-  launch_flux_push(e->stream, e->U, e->U2, e->halo, e->bc_mask_cube, e->U1, e->U1q, e->fws,
+  const int single =
+      launch_flux_push(e->stream, e->U, e->U2, e->halo, e->bc_mask_cube, e->U1, e->U1q, e->fws,
                    e->cube_size, e->Rku, e->Res, e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e,
                    RK, e->U1p1, e->U1p2, e->partials, e->push_aux, e->ib_refresh(),
                    push_runs(resident_cubes(e)));
   std::swap(e->U, e->U2);
   if (RK == 3)
-    launch_reduce(e->stream, e->partials, PUSH_ROWS_PER_CUBE, e->case_desc, e->n_active, e->phys_dev,
-                  er_row(e, er_slot));
+    launch_reduce(e->stream, e->partials, PUSH_ROWS_PER_CUBE, single, e->case_desc, e->n_active,
+                  e->phys_dev, er_row(e, er_slot));
 }
 
 void engine_stage(Engine* e, int RK, int er_slot, bool full_pre_halo) {

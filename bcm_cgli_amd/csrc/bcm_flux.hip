@@ -95,7 +95,8 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
   __shared__ double fy[5][NFY];
   __shared__ double fzb[6][16];                     // z-faces before k = 2: flux, pressure
   __shared__ int8_t fl[2][400];                     // flags of planes i, i+1
-  __shared__ double red[WG / 64][8];                // PUSH, RK 3: norm sums of the waves
+  __shared__ double red[WG / 64][8];                // RK 3: norm sums of the waves
+  __shared__ double tot[8];                         // and of the cube's planes
   const int RK = A.RK;
   const RunOf run = run_of(A.runs, blockIdx.x);
   const int c = run.cube, seg = run.seg;
@@ -290,7 +291,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
     for (int w = 1; w < WG / 64; ++w) s += red[w][t];
     return s;
   };
-  double rows = 0;                         // IN_PLACE: sum of the planes' rows
+  const bool single = MODE == IN_PLACE || run.nseg == 1;   // one row per cube
   int sl0 = 0, sl1 = 1, sl2 = 2;           // ring slots of planes i-1, i, i+1
 
 #pragma unroll 1
@@ -349,13 +350,13 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
 
     // ---- phase 2: primitives of plane i+1, x-face, differences ----
     // One row of norm partials per plane, so the norms do not depend on the
-    // runs; IN_PLACE adds a cube's rows in order, as k_fold_rows would.
+    // runs; a whole cube's rows are added here, in the order k_reduce would.
     if (MODE != FLUX_ONLY && RK == 3 && i > i0 && t < 8) {
       const double s = plane_row();
-      if (MODE == PUSH)
-        A.partials[((size_t)(c - 1) * PUSH_ROWS_PER_CUBE + (i - 3)) * 8 + t] = s;
+      if (single)
+        tot[t] = i == i0 + 1 ? s : tot[t] + s;
       else
-        rows = i == i0 + 1 ? s : rows + s;
+        A.partials[((size_t)(c - 1) * PUSH_ROWS_PER_CUBE + (i - 3)) * 8 + t] = s;
     }
     store_flags(i + 1);
     fill_prims(i + 1, sl2);
@@ -682,10 +683,11 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
     __syncthreads();
     if (t < 8) {
       const double s = plane_row();
-      if (MODE == PUSH)
-        A.partials[((size_t)(c - 1) * PUSH_ROWS_PER_CUBE + (i1 - 2)) * 8 + t] = s;
+      const size_t row = (size_t)(c - 1) * (MODE == IN_PLACE ? 1 : PUSH_ROWS_PER_CUBE);
+      if (single)
+        A.partials[row * 8 + t] = tot[t] + s;
       else
-        A.partials[(size_t)(c - 1) * 8 + t] = rows + s;
+        A.partials[(row + i1 - 2) * 8 + t] = s;
     }
   }
   // Ghost regions the domain BCs wrote go to Uout as they are.
@@ -721,13 +723,13 @@ int launch_flux_in_place(hipStream_t s, double* U, const double* U1, const doubl
   return 1;
 }
 
-void launch_flux_push(hipStream_t s, double* Uin, double* Uout, const HaloSrc* halo,
+int launch_flux_push(hipStream_t s, double* Uin, double* Uout, const HaloSrc* halo,
                       const uint8_t* cube_mask, const double* U1, const double* U1q,
                       const int8_t* fws, const double* cube_size, double* Rku, double* Res,
                       int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int RK,
                       double* U1p1, double* U1p2, double* partials, PushAux aux, IbRefresh ib,
                       int nseg) {
-  if (ncube <= 1) return;
+  if (ncube <= 1) return 0;
   const MarchArgs a{Uin, U1, U1q, fws, cube_size, Rku, Res, pt, deltaT, deltaTau, e,
                     runs_for(ncube, nseg), RK, ncube, U1p1, U1p2, partials, Uout, halo, cube_mask,
                     ib, aux == PushAux::ALL || RK == 3};
@@ -735,6 +737,7 @@ void launch_flux_push(hipStream_t s, double* Uin, double* Uout, const HaloSrc* h
     hipLaunchKernelGGL((k_flux_march<PUSH, true>), run_grid(a.runs, ncube), dim3(WG), 0, s, a);
   else
     hipLaunchKernelGGL((k_flux_march<PUSH, false>), run_grid(a.runs, ncube), dim3(WG), 0, s, a);
+  return single_rows(a.runs, ncube);
 }
 
 // Runs per cube of the pushing kernel.  The chip holds 512 of its workgroups

@@ -151,28 +151,6 @@ __device__ __forceinline__ void roe_flux(const double (&L)[5], const double (&R)
   dP = 0.5 * (lP + rP);
 }
 
-// Block sum of NS doubles per lane in a fixed tree order; lane 0 returns the totals.
-template <int NS>
-__device__ __forceinline__ void block_sum(double (&x)[NS], double* sh) {
-#pragma unroll
-  for (int m = 0; m < NS; ++m)
-    for (int off = 32; off > 0; off >>= 1) x[m] += __shfl_down(x[m], off, 64);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0)
-#pragma unroll
-    for (int m = 0; m < NS; ++m) sh[wave * NS + m] = x[m];
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int nw = blockDim.x >> 6;
-#pragma unroll
-    for (int m = 0; m < NS; ++m) {
-      double s = sh[m];
-      for (int w = 1; w < nw; ++w) s += sh[w * NS + m];
-      x[m] = s;
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Face-based formulation of the same flux (used by k_flux_march).
 //

@@ -188,6 +188,10 @@ inline Runs runs_for(int ncube, int nseg) {
   return nseg == 1 && n > 560 ? Runs{(n - 192) & ~7, 4} : Runs{0, nseg};
 }
 
+// Leading cubes of the pool that one workgroup marches whole: it sums their
+// planes' norm rows into one.
+inline int single_rows(const Runs& r, int ncube) { return r.nseg == 1 ? ncube - 1 : r.whole; }
+
 // Copies, with the threads of one workgroup, the ghost regions the domain BCs
 // of cube c write (mask bits 1 x-min, 2 x-max, 4 y-min, 8 y-max, 16 z-min,
 // 32 z-max) from Uin to Uout: x faces over j,k in [2,17], y faces over all i
@@ -353,12 +357,13 @@ constexpr int IN_PLACE_SPLIT = 320;
 // equal-size neighbour (halo[c]) into that neighbour's ghost layers in Uout.
 // With PushAux::ALL it writes Rku, Res, U1p1 (RK1) and U1p2 (RK2) bitwise as the
 // in-place fused kernel does (nothing reads them back during stages), with
-// STEP_END Rku and Res at RK 3 only, with NONE none of them; at RK 3
-// PUSH_ROWS_PER_CUBE rows of 8 norm partials per cube (one per plane) either way.
+// STEP_END Rku and Res at RK 3 only, with NONE none of them.  At RK 3 one row
+// of 8 norm partials per plane, PUSH_ROWS_PER_CUBE to a cube; the leading cubes
+// marched whole, whose number it returns, have their sum in the first.
 // Ghost regions the domain BCs wrote (cube_mask) are copied from Uin to Uout.
 constexpr int PUSH_ROWS_PER_CUBE = 16;
 enum class PushAux { NONE, STEP_END, ALL };
-void launch_flux_push(hipStream_t s, double* Uin, double* Uout, const HaloSrc* halo,
+int launch_flux_push(hipStream_t s, double* Uin, double* Uout, const HaloSrc* halo,
                       const uint8_t* cube_mask, const double* U1, const double* U1q,
                       const int8_t* fws, const double* cube_size, double* Rku, double* Res,
                       int ncube, PhysTab pt, double deltaT, double deltaTau, double e, int RK,
@@ -374,12 +379,11 @@ int div_selftest(unsigned long long seed, int n, unsigned long long* mismatches)
 void launch_update(hipStream_t s, int RK, double* U, double* U1p1, double* U1p2,
                    const double* Rku, const double* Res, const int8_t* fws, int ncube,
                    const int* cube_case, double* partials, bool body_only = false);
-// Norms er[0..7] of each case in cases[0..ncases): rows_per_cube partial rows
-// per cube (as launch_flux_in_place says; 16 after k_update, the pushing FP64
-// kernel and the mixed flux kernel; several rows are first summed in row order into each
-// cube's first row); case d writes er[d.slot*8 .. d.slot*8+7].
-void launch_reduce(hipStream_t s, double* partials, int rows_per_cube, const CaseDesc* cases,
-                   int ncases, const DevPhys* phys, double* er);
+// Norms er[0..7] of each case in cases[0..ncases) from partial rows, stride per
+// cube (1 or 16), of which the pool's first `single` cubes use one; case d
+// writes er[d.slot*8 .. d.slot*8+7].
+void launch_reduce(hipStream_t s, const double* partials, int stride, int single,
+                   const CaseDesc* cases, int ncases, const DevPhys* phys, double* er);
 void launch_shift(hipStream_t s, const double* U, double* U1, double* U1q, int ncube,
                   const int* cube_case);
 // AoS <-> SoA transposes of ncube whole cubes (cube 0 of both arrays included).
@@ -398,10 +402,10 @@ int update_blocks(int ncube);
 // next to a face with an equal-size neighbour (halo[c]) are also written into
 // that neighbour's ghost layers in Uout: the face part of the post-update
 // exchange.  nseg (1, 2, 4, 8 or 16) runs of 16/nseg planes per cube, one
-// workgroup each; results are bitwise the same for every nseg.  At RK 3,
-// MIXED_ROWS_PER_CUBE rows of 8 norm partials per cube (one per plane).
+// workgroup each; results are bitwise the same for every nseg.  Norm rows at
+// RK 3, and the return value, as launch_flux_push has them.
 constexpr int MIXED_ROWS_PER_CUBE = 16;
-void launch_flux_mixed(hipStream_t s, float* Uin, float* Uout, const HaloSrc* halo,
+int launch_flux_mixed(hipStream_t s, float* Uin, float* Uout, const HaloSrc* halo,
                        const uint8_t* cube_mask, const double* Bsrc, const int8_t* fws,
                        const double* cube_size, int ncube, PhysTab pt, double deltaT,
                        double deltaTau, double e, int RK, double* partials, IbRefresh ib, int nseg);

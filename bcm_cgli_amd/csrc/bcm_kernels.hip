@@ -398,54 +398,56 @@ __global__ __launch_bounds__(WG) void k_update(int RK, double* __restrict__ U,
   }
 }
 
-// With several partial rows per cube, each cube's rows are first summed in
-// row order into its first row, one thread per cube (blockIdx.y: case).
-__global__ __launch_bounds__(WG) void k_fold_rows(double* __restrict__ partials,
-                                                  int rows_per_cube,
-                                                  const CaseDesc* __restrict__ cases) {
-  const CaseDesc cd = cases[blockIdx.y];
-  for (int q = blockIdx.x * WG + threadIdx.x; q < cd.n; q += gridDim.x * WG) {
-    double* r = partials + (size_t)(cd.first - 1 + q) * rows_per_cube * 8;
-    double acc[7];
-#pragma unroll
-    for (int m = 0; m < 7; ++m) acc[m] = r[m];
-    for (int b = 1; b < rows_per_cube; ++b)
-#pragma unroll
-      for (int m = 0; m < 7; ++m) acc[m] += r[b * 8 + m];
-#pragma unroll
-    for (int m = 0; m < 7; ++m) r[m] = acc[m];
-  }
-}
-
-// Final norm reduction (Flux.cpp:2627-2652 at one rank): er[1..7] of one
-// case per block from one partial row per cube (every stride-th row).  The
-// rows of a case are summed in an order fixed relative to the case's first
-// cube, so a case gives the same bits alone and next to other cases.
-__global__ __launch_bounds__(WG) void k_reduce(const double* __restrict__ partials,
-                                               int stride,
-                                               const CaseDesc* __restrict__ cases,
-                                               const DevPhys* __restrict__ phys,
-                                               double* __restrict__ er_all) {
+// Final norm reduction (Flux.cpp:2627-2652 at one rank): er[1..7] of one case
+// per block from its cubes' rows of 8 partial sums, stride rows apart: 16 rows
+// per cube (one per plane), already summed into the first for the pool's first
+// `single` cubes.  Eight lanes read a row; a cube's rows are summed in order,
+// then the cubes in an order fixed relative to the case's first cube, so a case
+// gives the same bits alone and next to other cases, in any number of runs.
+//
+// Bound: one CU's loads for one large case (2,048 cubes: 14 us, 21 when every
+// cube had 16 rows, folded by a kernel of its own), latencies for a small one (8
+// cubes: 4.6 us, 9 in two kernels).
+constexpr int REDUCE_WG = 1024;
+__global__ __launch_bounds__(REDUCE_WG) void k_reduce(const double* __restrict__ partials,
+                                                      int stride, int single,
+                                                      const CaseDesc* __restrict__ cases,
+                                                      const DevPhys* __restrict__ phys,
+                                                      double* __restrict__ er_all) {
+  __shared__ double sh[REDUCE_WG / 64][8];
   const CaseDesc cd = cases[blockIdx.x];
   const DevPhys ph = phys[cd.slot];
-  const double* rows = partials + (size_t)(cd.first - 1) * stride * 8;
-  const int nrows = cd.n;
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-  for (int bi = threadIdx.x; bi < nrows; bi += WG)
+  const int t = threadIdx.x;
+  const double* rows = partials + (size_t)(cd.first - 1) * stride * 8 + (t & 7);
+  double acc = 0;
+  for (int q = t / 8; q < cd.n; q += REDUCE_WG / 8) {
+    const double* r = rows + (size_t)q * stride * 8;
+    double s = r[0];
+    if (cd.first + q > single) {
+      double x[15];
 #pragma unroll
-    for (int m = 0; m < 7; ++m) acc[m] += rows[(size_t)bi * stride * 8 + m];
-  __shared__ double sh[(WG / 64) * 7];
-  block_sum<7>(acc, sh);
-  if (threadIdx.x == 0) {
+      for (int b = 0; b < 15; ++b) x[b] = r[(b + 1) * 8];
+#pragma unroll
+      for (int b = 0; b < 15; ++b) s += x[b];
+    }
+    acc += s;
+  }
+#pragma unroll
+  for (int off = 32; off >= 8; off >>= 1) acc += __shfl_down(acc, off, 64);
+  if ((t & 63) < 8) sh[t >> 6][t & 7] = acc;
+  __syncthreads();
+  if (t < 7) {
+    double s = sh[0][t];
+#pragma unroll
+    for (int w = 1; w < REDUCE_WG / 64; ++w) s += sh[w][t];
     double* er = er_all + (size_t)cd.slot * 8;
     const double DN = 1. / (cd.mpi_ncube * 16 * 16 * 16);
-    er[0] = 0;
-    for (int m = 0; m < 5; ++m) er[m + 1] = sqrt(acc[m]) * DN;
-    er[6] = acc[5] / (0.5 * ph.rho0 * ph.U0 * ph.U0 * 2.602);
-    er[7] = acc[6] / (0.5 * ph.rho0 * ph.U0 * ph.U0 * 2.602);
+    if (t == 0) er[0] = 0;
+    er[t + 1] = t < 5 ? sqrt(s) * DN : s / (0.5 * ph.rho0 * ph.U0 * ph.U0 * 2.602);
   }
 }
 
+// ---------------------------------------------------------------------------
 // ---------------------------------------------------------------------------
 // Edge passes and domain boundary conditions of one cube by the calling
 // workgroup (OPEN_WG lanes): edge-ghost averaging (Interface.cpp:5640-5732)
@@ -1397,14 +1399,11 @@ void launch_update(hipStream_t s, int RK, double* U, double* U1p1, double* U1p2,
                        Res, fws, cube_case, partials, body_only ? 1 : 0);
 }
 
-void launch_reduce(hipStream_t s, double* partials, int rows_per_cube, const CaseDesc* cases,
-                   int ncases, const DevPhys* phys, double* er) {
-  if (ncases <= 0) return;
-  if (rows_per_cube > 1)
-    hipLaunchKernelGGL(k_fold_rows, dim3(8, ncases), dim3(WG), 0, s, partials, rows_per_cube,
-                       cases);
-  hipLaunchKernelGGL(k_reduce, dim3(ncases), dim3(WG), 0, s, partials, rows_per_cube, cases, phys,
-                     er);
+void launch_reduce(hipStream_t s, const double* partials, int stride, int single,
+                   const CaseDesc* cases, int ncases, const DevPhys* phys, double* er) {
+  if (ncases > 0)
+    hipLaunchKernelGGL(k_reduce, dim3(ncases), dim3(REDUCE_WG), 0, s, partials, stride, single,
+                       cases, phys, er);
 }
 
 void launch_shift(hipStream_t s, const double* U, double* U1, double* U1q, int ncube,

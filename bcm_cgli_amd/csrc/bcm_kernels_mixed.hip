@@ -335,6 +335,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
   __shared__ float fy[9][NFY];                     // y-faces: flux, viscous flux
   __shared__ float fzb[10][16];                    // z-faces before k = 2: flux, pressure, viscous
   __shared__ double red[WG / 64][8];               // RK 3: norm sums of the waves
+  __shared__ double tot[8];                        // and, of a whole cube, of its planes
 
   const RunOf run = run_of(runs, blockIdx.x);
   const int c = run.cube, seg = run.seg;
@@ -594,7 +595,10 @@ __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
       double s = red[0][t];
 #pragma unroll
       for (int w = 1; w < WG / 64; ++w) s += red[w][t];
-      partials[((size_t)(c - 1) * MIXED_ROWS_PER_CUBE + (i - 3)) * 8 + t] = s;
+      if (run.nseg == 1)   // (in the order k_reduce adds rows)
+        tot[t] = i == i0 + 1 ? s : tot[t] + s;
+      else
+        partials[((size_t)(c - 1) * MIXED_ROWS_PER_CUBE + (i - 3)) * 8 + t] = s;
     }
     // This cell's FP64 source constant Bv = 3 Uref - 4 U1 + U1q, first used in
     // the residual.
@@ -847,7 +851,11 @@ __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
     double s = red[0][t];
 #pragma unroll
     for (int w = 1; w < WG / 64; ++w) s += red[w][t];
-    partials[((size_t)(c - 1) * MIXED_ROWS_PER_CUBE + (i1 - 2)) * 8 + t] = s;
+    const size_t row = (size_t)(c - 1) * MIXED_ROWS_PER_CUBE;
+    if (run.nseg == 1)
+      partials[row * 8 + t] = tot[t] + s;
+    else
+      partials[(row + i1 - 2) * 8 + t] = s;
   }
 
   // Ghost regions the domain BCs wrote this stage go to Uout as they are (no
@@ -935,15 +943,16 @@ __global__ __launch_bounds__(WG) void k_soa_to_aos_f(const float* __restrict__ s
 
 }  // namespace
 
-void launch_flux_mixed(hipStream_t s, float* Uin, float* Uout, const HaloSrc* halo,
+int launch_flux_mixed(hipStream_t s, float* Uin, float* Uout, const HaloSrc* halo,
                        const uint8_t* cube_mask, const double* Bsrc, const int8_t* fws,
                        const double* cube_size, int ncube, PhysTab pt, double deltaT,
                        double deltaTau, double e, int RK, double* partials, IbRefresh ib, int nseg) {
-  if (ncube <= 1) return;
+  if (ncube <= 1) return 0;
   const Runs runs = runs_for(ncube, nseg);
   hipLaunchKernelGGL(k_flux_mixed, run_grid(runs, ncube), dim3(WG), 0, s, Uin, Uout, halo,
                      cube_mask, Bsrc, fws, cube_size, pt, deltaT, deltaTau, e, RK, partials, ib,
                      runs, ncube);
+  return single_rows(runs, ncube);
 }
 
 // Runs per cube of the mixed flux kernel; the chip holds 512 of its workgroups.

@@ -129,8 +129,8 @@ extern "C" int bcm_flux_rk_noalloc(int ncube, int n_cubes_norm, int RK, double d
   const int rows = launch_flux_in_place(st, U1_, U1, U1q, FWS, cube_size, Rku1, Residual1, ncube, pt,
                                         deltaT, deltaTau, e, RK, U1p1, U1p2, partials);
   if (RK == 3)
-    launch_reduce(st, partials, rows, reinterpret_cast<const CaseDesc*>(s + DESC_OFF), 1, pt.phys,
-                  er);
+    launch_reduce(st, partials, rows, rows == 1 ? ncube - 1 : 0,
+                  reinterpret_cast<const CaseDesc*>(s + DESC_OFF), 1, pt.phys, er);
   const hipError_t rc = hipGetLastError();
   if (rc != hipSuccess) {
     set_last_error(std::string("bcm_flux_rk_noalloc: launch failed: ") + hipGetErrorString(rc));
