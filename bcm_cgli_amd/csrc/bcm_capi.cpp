@@ -559,6 +559,7 @@ int bcm_engine_part(bcm_engine* h, int part, int RK) {
     case 9: engine_flux_push(e, RK, 0); break;
     default: return fail("unknown part");
   }
+  engine_carry_bc(e);
   std::string err;
   if (engine_sync(e, err)) return fail(err);
   return 0;
@@ -621,7 +622,9 @@ int bcm_engine_time_part(bcm_engine* h, int part, int RK, int reps, double* ms) 
     }
   }
   e->push_aux = PushAux::ALL;
-  if (hipEventRecord(e->ev1, e->stream) != hipSuccess) return fail("event record failed");
+  const bool recorded = hipEventRecord(e->ev1, e->stream) == hipSuccess;
+  engine_carry_bc(e);
+  if (!recorded) return fail("event record failed");
   if (hipEventSynchronize(e->ev1) != hipSuccess) return fail("event wait failed");
   float t = 0;
   if (hipEventElapsedTime(&t, e->ev0, e->ev1) != hipSuccess) return fail("event timing failed");

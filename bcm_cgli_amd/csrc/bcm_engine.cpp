@@ -99,6 +99,7 @@ void free_case(Engine* e) {
   e->phys_dev = nullptr;
   e->cube_case = nullptr;
   e->er_slots = 0;
+  e->bc_behind = false;
   e->ncube = 0;
   e->cap = 0;
   e->n_active = 0;
@@ -906,10 +907,12 @@ namespace {
 // then the IB fill and the pre-flux exchange: the full one, or of the two-level
 // faces those that the fill changed.  The equal-size faces' IB ghost cells are
 // refreshed by the flux kernel, which also forms the edge cells it reads.
+// `other` is the other copy of the iterate.
 template <typename T>
-void push_stage_open(Engine* e, T* U, bool full_pre_halo) {
+void push_stage_open(Engine* e, T* U, const T* other, bool full_pre_halo) {
   launch_halo_ml(e->stream, U, e->ml, e->n_ml, e->pt());
-  launch_open(e->stream, U, e->open_items, e->n_open_items, e->ghost.t, e->phys_dev);
+  launch_open(e->stream, U, e->bc_behind ? other : U, e->open_items, e->n_open_items, e->ghost.t,
+              e->phys_dev);
   if (full_pre_halo)
     engine_interface(e);
   else
@@ -955,18 +958,43 @@ int mixed_runs_now(const Engine* e) {
   if (e->flux_pinned || e->tuned_class == size_class(e)) return e->mixed_nseg;
   return mixed_runs(resident_cubes(e));
 }
+
+// The pushing flux kernel of the pool's precision and its norms; swaps the
+// copies of the iterate.
+void push_flux(Engine* e, int RK, int er_slot) {
+  int single;
+  if (e->prec == 1) {
+    single = launch_flux_mixed(e->stream, e->Uf, e->Uf2, e->halo, e->bc_mask_cube, e->Bsrc, e->fws,
+                               e->cube_size, e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e, RK,
+                               e->partials, e->ib_refresh(), mixed_runs_now(e));
+    std::swap(e->Uf, e->Uf2);
+  } else {
+    single = launch_flux_push(e->stream, e->U, e->U2, e->halo, e->bc_mask_cube, e->U1, e->U1q,
+                              e->fws, e->cube_size, e->Rku, e->Res, e->ncube, e->pt(), e->deltaT,
+                              e->deltaTau, e->e, RK, e->U1p1, e->U1p2, e->partials, e->push_aux,
+                              e->ib_refresh(), push_runs(resident_cubes(e)));
+    std::swap(e->U, e->U2);
+  }
+  e->bc_behind = true;
+  static_assert(MIXED_ROWS_PER_CUBE == PUSH_ROWS_PER_CUBE, "one layout of the norm rows");
+  if (RK == 3)
+    launch_reduce(e->stream, e->partials, PUSH_ROWS_PER_CUBE, single, e->case_desc, e->n_active,
+                  e->phys_dev, er_row(e, er_slot));
+}
 }  // namespace
+
+void engine_carry_bc(Engine* e) {
+  if (!e->bc_behind) return;
+  if (e->prec == 1)
+    launch_carry_bc(e->stream, e->Uf2, e->Uf, e->bc_cubes, e->n_bc, e->bc_mask_cube, e->pt());
+  else
+    launch_carry_bc(e->stream, e->U2, e->U, e->bc_cubes, e->n_bc, e->bc_mask_cube, e->pt());
+  e->bc_behind = false;
+}
 
 void engine_flux_update(Engine* e, int RK, int er_slot) {
   if (e->prec == 1) {
-    const int single = launch_flux_mixed(
-        e->stream, e->Uf, e->Uf2, e->halo, e->bc_mask_cube, e->Bsrc, e->fws, e->cube_size,
-        e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e, RK, e->partials, e->ib_refresh(),
-        mixed_runs_now(e));
-    std::swap(e->Uf, e->Uf2);
-    if (RK == 3)
-      launch_reduce(e->stream, e->partials, MIXED_ROWS_PER_CUBE, single, e->case_desc, e->n_active,
-                    e->phys_dev, er_row(e, er_slot));
+    push_flux(e, RK, er_slot);
     return;
   }
   if (!engine_fused(e)) {
@@ -1034,6 +1062,7 @@ int engine_autotune(Engine* e, int* variant, int* nseg, std::string& err) {
         HIP_TRY(hipEventElapsedTime(&ms, e->ev0, e->ev1));
         e->Uf = live[0];
         e->Uf2 = live[1];
+        e->bc_behind = false;
         for (int a = 0; a < 2; ++a)
           HIP_TRY(
               hipMemcpyAsync(live[a], saved.p[a], bytes, hipMemcpyDeviceToDevice, e->stream));
@@ -1086,35 +1115,19 @@ void engine_shift(Engine* e) {
     launch_shift(e->stream, e->U, e->U1, e->U1q, e->ncube, e->cube_case);
 }
 
-void engine_flux_push(Engine* e, int RK, int er_slot) {
-  if (e->prec == 1) {
-    engine_flux_update(e, RK, er_slot);
-    return;
-  }
-  const int single =
-      launch_flux_push(e->stream, e->U, e->U2, e->halo, e->bc_mask_cube, e->U1, e->U1q, e->fws,
-                   e->cube_size, e->Rku, e->Res, e->ncube, e->pt(), e->deltaT, e->deltaTau, e->e,
-                   RK, e->U1p1, e->U1p2, e->partials, e->push_aux, e->ib_refresh(),
-                   push_runs(resident_cubes(e)));
-  std::swap(e->U, e->U2);
-  if (RK == 3)
-    launch_reduce(e->stream, e->partials, PUSH_ROWS_PER_CUBE, single, e->case_desc, e->n_active,
-                  e->phys_dev, er_row(e, er_slot));
-}
+void engine_flux_push(Engine* e, int RK, int er_slot) { push_flux(e, RK, er_slot); }
 
 void engine_stage(Engine* e, int RK, int er_slot, bool full_pre_halo) {
-  if (e->prec == 1) {
+  if (e->prec == 1 || e->flux_push) {
     // The previous flux kernel wrote the equal-size face halos; the
     // two-level faces and, where needed, the edge passes of that exchange and
     // this stage's BCs open the stage (all idempotent when no interior cell
     // changed, as at the start of a run).
-    push_stage_open(e, e->Uf, full_pre_halo);
-    engine_flux_update(e, RK, er_slot);
-    return;
-  }
-  if (e->flux_push) {
-    push_stage_open(e, e->U, full_pre_halo);
-    engine_flux_push(e, RK, er_slot);
+    if (e->prec == 1)
+      push_stage_open(e, e->Uf, e->Uf2, full_pre_halo);
+    else
+      push_stage_open(e, e->U, e->U2, full_pre_halo);
+    push_flux(e, RK, er_slot);
     return;
   }
   engine_bc(e);
@@ -1155,6 +1168,7 @@ void enqueue_step(Engine* e, int n_inner, bool full_first) {
     for (int RK = 1; RK <= 3; ++RK) engine_stage(e, RK, it, full_first && it == 0 && RK == 1);
   }
   e->push_aux = PushAux::ALL;
+  engine_carry_bc(e);
   engine_shift(e);
   // An odd number of flux kernels that swap copies: bring the iterate back to
   // the copy the step started from, so that every replay of a captured step
@@ -1324,6 +1338,7 @@ int engine_run_converge(Engine* e, int n_steps, int max_inner, double tol, doubl
         // Cases that end their inner loop while others go on: shift them now
         // and keep their iterate aside until the step ends; their cubes keep
         // being computed with the rest, and the results are discarded.
+        engine_carry_bc(e);
         complete_exchange(e);
         for (int c : ended) {
           shift_case(e, e->cases[c]);
@@ -1332,6 +1347,7 @@ int engine_run_converge(Engine* e, int n_steps, int max_inner, double tol, doubl
         }
       }
     }
+    engine_carry_bc(e);
     if (stashed.empty()) {
       engine_shift(e);
     } else {

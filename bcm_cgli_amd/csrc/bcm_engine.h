@@ -141,6 +141,10 @@ struct Engine {
   // pushing flux kernels read edge cells, and they form them themselves.
   OpenItem* open_items = nullptr;
   int n_open_items = 0;
+  // A pushing flux kernel ran since the BCs did: the ghost regions they write
+  // are in the other copy of the iterate.  The next stage's opening reads them
+  // there; engine_carry_bc brings them over where stages end.
+  bool bc_behind = false;
   // Set when an inner iterate was replaced from outside (state upload, new
   // case): the next pre-flux exchange must then be the full one.
   bool halo_full_next = false;
@@ -228,7 +232,11 @@ void engine_flux_update(Engine* e, int RK, int er_slot);
 bool engine_fused(const Engine* e);
 // Flux and update of one stage written to the other copy of the iterate with
 // the face halos (the form stages use when flux_push is set); swaps copies.
+// The ghost regions the BCs wrote stay behind (also with engine_flux_update and
+// engine_stage where they push): the caller ends its sequence of stages with
+// engine_carry_bc, so that no interface call returns without them.
 void engine_flux_push(Engine* e, int RK, int er_slot);
+void engine_carry_bc(Engine* e);
 void engine_shift(Engine* e);
 void engine_stage(Engine* e, int RK, int er_slot, bool full_pre_halo = false);
 // n_steps physical steps of n_inner inner iterations for every resident case.

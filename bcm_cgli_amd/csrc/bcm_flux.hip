@@ -690,8 +690,6 @@ __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
         A.partials[(row + i1 - 2) * 8 + t] = s;
     }
   }
-  // Ghost regions the domain BCs wrote go to Uout as they are.
-  if (MODE == PUSH && zm && seg == 0) copy_bc_regions(A.U, A.Uout, c, zm, 0.0);
 }
 
 }  // namespace

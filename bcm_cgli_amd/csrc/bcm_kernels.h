@@ -320,10 +320,15 @@ void launch_edge_list(hipStream_t s, float* U, const int* list, int n);
 // Opening of a pushed stage in one launch: per item (x: edge/BC entry as
 // above or 0, y: IB ghost-table index or -1) a cube's edge passes and BCs,
 // then its IB fill.
-void launch_open(hipStream_t s, double* U, const OpenItem* items, int n, const GhostTables& g,
-                 const DevPhys* phys);
-void launch_open(hipStream_t s, float* U, const OpenItem* items, int n, const GhostTables& g,
-                 const DevPhys* phys);
+void launch_open(hipStream_t s, double* U, const double* before, const OpenItem* items, int n,
+                 const GhostTables& g, const DevPhys* phys);
+void launch_open(hipStream_t s, float* U, const float* before, const OpenItem* items, int n,
+                 const GhostTables& g, const DevPhys* phys);
+// Ghost regions the BCs wrote of the listed cubes, from Uin to Uout.
+void launch_carry_bc(hipStream_t s, const double* Uin, double* Uout, const int* cubes, int n,
+                     const uint8_t* cube_mask, PhysTab pt);
+void launch_carry_bc(hipStream_t s, const float* Uin, float* Uout, const int* cubes, int n,
+                     const uint8_t* cube_mask, PhysTab pt);
 // Edge passes of every cube.
 void launch_edge(hipStream_t s, double* U, int ncube, const int* cube_case);
 void launch_edge(hipStream_t s, float* U, int ncube, const int* cube_case);
@@ -360,7 +365,7 @@ constexpr int IN_PLACE_SPLIT = 320;
 // STEP_END Rku and Res at RK 3 only, with NONE none of them.  At RK 3 one row
 // of 8 norm partials per plane, PUSH_ROWS_PER_CUBE to a cube; the leading cubes
 // marched whole, whose number it returns, have their sum in the first.
-// Ghost regions the domain BCs wrote (cube_mask) are copied from Uin to Uout.
+// Ghost regions the domain BCs wrote (cube_mask) stay in Uin (launch_carry_bc).
 constexpr int PUSH_ROWS_PER_CUBE = 16;
 enum class PushAux { NONE, STEP_END, ALL };
 int launch_flux_push(hipStream_t s, double* Uin, double* Uout, const HaloSrc* halo,

@@ -465,18 +465,28 @@ __global__ __launch_bounds__(REDUCE_WG) void k_reduce(const double* __restrict__
 // three BC faces and all edge passes 6 us, pass by pass 9.5; the opening of
 // 2,048 cubes in FP64 (872 with BCs) 28 us, with 256 lanes pass by pass 43.
 // edges 0: no edge passes; 1: only the k-edge cells the z-BC copies (four of
-// the cells of the plane k = 2 or 17); 2: all.
+// the cells of the plane k = 2 or 17); 2: all.  The edge passes belong to the
+// exchange after the last update, so where they read face ghost cells that the
+// BCs write they read the previous stage's: from `before`, the copy of the
+// iterate that holds them (U itself where no pushing flux kernel ran since).
 constexpr int OPEN_WG = 1024;
 template <typename T>
-__device__ __forceinline__ void edge_bc_cube(T* __restrict__ U, int c, int edges, int m,
+__device__ __forceinline__ void edge_bc_cube(T* U, const T* before, int c, int edges, int m,
                                              const DevPhys& ph) {
   using T2 = typename Vec2<T>::type;
   const typename OffOf<T>::type F(ph);
   const int t = threadIdx.x;
   T* const Uc = U + (size_t)c * CUBE_STRIDE;
+  const T* const Bc = before + (size_t)c * CUBE_STRIDE;
   auto at = [](int v, int i, int j, int k) { return v * PLANE + i * 400 + j * 20 + k; };
   // Nearest interior index of 1 (2) or 18 (17).
   auto near = [](int q) { return q == 1 ? 2 : 17; };
+  // Face ghost cell as the last exchange's edge passes read it.
+  auto face = [&](int v, int i, int j, int k) {
+    const bool bc = (i == 1 && (m & 1)) || (i == 18 && (m & 2)) || (j == 1 && (m & 4)) ||
+                    (j == 18 && (m & 8)) || (k == 1 && (m & 16)) || (k == 18 && (m & 32));
+    return (bc ? Bc : Uc)[at(v, i, j, k)];
+  };
   // x-min inflow state from the interior state next to it, as stored.
   auto inflow = [&](const T (&q)[5], T (&o)[5]) {
     const double rho = F.ld(q, 0, 0);
@@ -565,18 +575,18 @@ __device__ __forceinline__ void edge_bc_cube(T* __restrict__ U, int c, int edges
     if (corner) {
       // j-edge (i, near j, k) from ea and ec, i-edge (near i, j, k) from eb
       // and ec.
-      ea = Uc[at(v, i, near(j), near(k))];
-      eb = Uc[at(v, near(i), j, near(k))];
-      ec = Uc[at(v, near(i), near(j), k)];
+      ea = face(v, i, near(j), near(k));
+      eb = face(v, near(i), j, near(k));
+      ec = face(v, near(i), near(j), k);
     } else if (A == 0) {
-      ea = Uc[at(v, i, j, near(k))];
-      eb = Uc[at(v, i, near(j), k)];
+      ea = face(v, i, j, near(k));
+      eb = face(v, i, near(j), k);
     } else if (A == 1) {
-      ea = Uc[at(v, i, j, near(k))];
-      eb = Uc[at(v, near(i), j, k)];
+      ea = face(v, i, j, near(k));
+      eb = face(v, near(i), j, k);
     } else {
-      ea = Uc[at(v, i, near(j), k)];
-      eb = Uc[at(v, near(i), j, k)];
+      ea = face(v, i, near(j), k);
+      eb = face(v, near(i), j, k);
     }
     // Cells the BCs overwrite.
     const bool zinner = i >= 2 && i <= 17;
@@ -595,8 +605,8 @@ __device__ __forceinline__ void edge_bc_cube(T* __restrict__ U, int c, int edges
       dst = at(v, i, j, k);
       ev = v;
       zcopy = 1 + zs;
-      ea = Uc[at(v, i, near(j), k)];
-      eb = Uc[at(v, near(i), j, k)];
+      ea = face(v, i, near(j), k);
+      eb = face(v, near(i), j, k);
     }
   }
   __syncthreads();   // all loads have returned
@@ -665,7 +675,23 @@ template <typename T>
 __global__ __launch_bounds__(OPEN_WG) void k_bc(T* __restrict__ U, const int* __restrict__ cubes,
                                                 const uint8_t* __restrict__ masks, PhysTab pt) {
   const int c = cubes[blockIdx.x];
-  edge_bc_cube(U, c, 0, masks[blockIdx.x], pt.phys[pt.cube_case[c]]);
+  edge_bc_cube<T>(U, U, c, 0, masks[blockIdx.x], pt.phys[pt.cube_case[c]]);
+}
+
+// Ghost regions the BCs wrote, from the copy of the iterate that a pushing flux
+// kernel read to the one it wrote, which no BC pass has seen: one boundary cube
+// per workgroup, once per step.  (When each flux kernel copied them in its last
+// lines, a stage's took 24.6 us instead of 19.1 on 8 cubes in FP64 and 529 instead
+// of 493 on 2,048 mixed.)
+template <typename T>
+__global__ __launch_bounds__(OPEN_WG) void k_carry_bc(const T* __restrict__ Uin,
+                                                      T* __restrict__ Uout,
+                                                      const int* __restrict__ cubes,
+                                                      const uint8_t* __restrict__ cube_mask,
+                                                      PhysTab pt) {
+  const int c = cubes[blockIdx.x];
+  const DevPhys ph = pt.phys[pt.cube_case[c]];
+  copy_bc_regions(Uin, Uout, c, cube_mask[c], ph.rho0 * ph.W0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1105,13 +1131,14 @@ __global__ __launch_bounds__(WG) void k_edge_list(T* __restrict__ U, const int* 
 // post-update exchange and the domain BCs of the next stage, then its IB fill.  Both touch only the cube's own cells, so cubes
 // proceed independently, each in the reference's order.
 template <typename T>
-__global__ __launch_bounds__(OPEN_WG) void k_open(T* __restrict__ U, const OpenItem* __restrict__ items,
-                                             GhostTables gt,
-                                             const DevPhys* __restrict__ phys) {
+__global__ __launch_bounds__(OPEN_WG) void k_open(T* U, const T* before,
+                                                  const OpenItem* __restrict__ items,
+                                                  GhostTables gt,
+                                                  const DevPhys* __restrict__ phys) {
   extern __shared__ double gsm[];
   const OpenItem it = items[blockIdx.x];
   const DevPhys ph = phys[it.slot];
-  if (it.edges) edge_bc_cube(U, it.g.cube, it.edges, it.mask, ph);
+  if (it.edges) edge_bc_cube(U, before, it.g.cube, it.edges, it.mask, ph);
   if (it.g.nlev == 0) return;
   // The fill's tables load while the stores above complete.
   GhostFirst f;
@@ -1247,19 +1274,36 @@ void launch_ghost(hipStream_t s, float* U, const GhostTables& g, PhysTab pt) {
 }
 
 template <typename T>
-void launch_open_t(hipStream_t s, T* U, const OpenItem* items, int n, const GhostTables& g,
-                   const DevPhys* phys) {
+void launch_open_t(hipStream_t s, T* U, const T* before, const OpenItem* items, int n,
+                   const GhostTables& g, const DevPhys* phys) {
   if (n <= 0) return;
   const size_t shmem = (size_t)g.max_slots * 5 * sizeof(double);
-  hipLaunchKernelGGL(k_open<T>, dim3(n), dim3(OPEN_WG), shmem, s, U, items, g, phys);
+  hipLaunchKernelGGL(k_open<T>, dim3(n), dim3(OPEN_WG), shmem, s, U, before, items, g,
+                     phys);
 }
-void launch_open(hipStream_t s, double* U, const OpenItem* items, int n, const GhostTables& g,
-                 const DevPhys* phys) {
-  launch_open_t(s, U, items, n, g, phys);
+void launch_open(hipStream_t s, double* U, const double* before, const OpenItem* items, int n,
+                 const GhostTables& g, const DevPhys* phys) {
+  launch_open_t(s, U, before, items, n, g, phys);
 }
-void launch_open(hipStream_t s, float* U, const OpenItem* items, int n, const GhostTables& g,
-                 const DevPhys* phys) {
-  launch_open_t(s, U, items, n, g, phys);
+void launch_open(hipStream_t s, float* U, const float* before, const OpenItem* items, int n,
+                 const GhostTables& g, const DevPhys* phys) {
+  launch_open_t(s, U, before, items, n, g, phys);
+}
+
+template <typename T>
+void launch_carry_bc_t(hipStream_t s, const T* Uin, T* Uout, const int* cubes, int n,
+                       const uint8_t* cube_mask, PhysTab pt) {
+  if (n > 0)
+    hipLaunchKernelGGL(k_carry_bc<T>, dim3(n), dim3(OPEN_WG), 0, s, Uin, Uout, cubes, cube_mask,
+                       pt);
+}
+void launch_carry_bc(hipStream_t s, const double* Uin, double* Uout, const int* cubes, int n,
+                     const uint8_t* cube_mask, PhysTab pt) {
+  launch_carry_bc_t(s, Uin, Uout, cubes, n, cube_mask, pt);
+}
+void launch_carry_bc(hipStream_t s, const float* Uin, float* Uout, const int* cubes, int n,
+                     const uint8_t* cube_mask, PhysTab pt) {
+  launch_carry_bc_t(s, Uin, Uout, cubes, n, cube_mask, pt);
 }
 
 template <typename T>

@@ -857,10 +857,6 @@ __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
     else
       partials[(row + i1 - 2) * 8 + t] = s;
   }
-
-  // Ghost regions the domain BCs wrote this stage go to Uout as they are (no
-  // neighbour writes them), so Uout holds them as an in-place update would.
-  if (seg == 0 && zm) copy_bc_regions(U, Uout, c, zm, r3);
 }
 
 __global__ __launch_bounds__(WG) void k_shift_mixed(const float* __restrict__ U,

@@ -115,3 +115,23 @@ def test_stage_opening_bitwise(B, O, dims):
             assert np.array_equal(a.view(np.int64), b.view(np.int64))
     finally:
         e.close()
+
+
+# Single stages that write the other copy of the iterate: each leaves the ghost
+# regions of the domain BCs where the next one and a reader find them.
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 2, 2), (3, 1, 2)],
+                         ids=lambda d: "x".join(map(str, d)))
+def test_single_pushing_stages_bitwise(B, O, dims):
+    case = lattice_case(B, dims)
+    e = B.Engine(0)
+    try:
+        e.load_case(case)
+        e.set_flux(1, 1, 2)
+        orc = O.OracleRun(case, nthreads=16)
+        for RK in (1, 2, 3, 1):
+            e.part("stage", RK)
+            e.part("interface")
+            orc.stage(RK)
+            compare(e, orc, ("U1_",))
+    finally:
+        e.close()
