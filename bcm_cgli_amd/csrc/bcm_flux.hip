@@ -740,11 +740,17 @@ int launch_flux_push(hipStream_t s, double* Uin, double* Uout, const HaloSrc* ha
 
 // Runs per cube of the pushing kernel.  The chip holds 512 of its workgroups
 // (two per CU), and a run costs one x-face pass and two primitive planes more,
-// about two thirds of a plane.  To 100 cubes a plane per run is fastest (8
-// cubes: 24 us, 166 in one run; 100: 77); to 560 four runs fill the last wave of
-// workgroups (128 cubes: 77 us, 168 in one run, 91 in 16; 512: 271, 283 in
-// one); above, one run with quartered last cubes (runs_for; 576: 286 us, 313 in
-// four; 1,000: 488, 495 in two).
-int push_runs(int n) { return n <= 100 ? 16 : n <= 560 ? 4 : 1; }
+// about two thirds of a plane.  The most runs that fit at once to 64 cubes (8
+// cubes: 19 us in 16 runs, 161 in one; 64: 43 in 8, 45 in 16); a plane per run to
+// 90, where 8 runs would leave a second, nearly empty wave (80: 54, 59 in 8);
+// again what fits at once to 128 (100: 68 in 4, 69 in 16; 128: 73, 99 in 2); then
+// the last wave's share against the prologues: 8 runs to 240 (216: 117, 127 in
+// 4), 4 to 370 (294: 158, 166 in 8, 185 in 2), 2 to 560 (384: 193, 197 in 4; 512:
+// 256, 262 in 4), above one run with quartered last cubes (runs_for; 576: 284,
+// 299 in 2; 1,000: 479, 487 in one without them).
+int push_runs(int n) {
+  return n <= 48 ? 16 : n <= 64 ? 8 : n <= 90 ? 16 : n <= 128 ? 4 : n <= 240 ? 8 : n <= 370 ? 4
+       : n <= 560 ? 2 : 1;
+}
 
 }  // namespace bcm

@@ -180,8 +180,8 @@ inline dim3 run_grid(const Runs& r, int ncube) {
 // nseg runs per cube; with one run, the last 192 of more than 560 cubes take
 // four.  Workgroups of one CU fall out of step, and with whole cubes only the
 // last half cube's time finds half the slots empty; quarters fill them (FP64
-// 2,048 cubes 990 -> 975 us, 1,584: 799 -> 759, 800: 458 -> 400, 576: 364 -> 286;
-// mixed 552 -> 527, 454 -> 416, 256 -> 225, 216 -> 160).  128 to 256 cubes are alike;
+// 2,048 cubes 958 -> 947 us, 1,584: 779 -> 742, 800: 448 -> 386, 576: 362 -> 285;
+// mixed 519 -> 492, 435 -> 396, 245 -> 220, 206 -> 154).  128 to 256 cubes are alike;
 // 512 cost more prologues than they save.
 inline Runs runs_for(int ncube, int nseg) {
   const int n = ncube - 1;

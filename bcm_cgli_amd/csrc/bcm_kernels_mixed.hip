@@ -952,13 +952,14 @@ int launch_flux_mixed(hipStream_t s, float* Uin, float* Uout, const HaloSrc* hal
 }
 
 // Runs per cube of the mixed flux kernel; the chip holds 512 of its workgroups.
-// Most runs that fit at once to 128 cubes (8 cubes: 18 us in 16 runs, 112 in one;
-// 64: 28 in 8; 128: 45 in 4, 113 in one); above, a run's prologue stands against
-// the last wave of workgroups: 8 runs to 200 cubes (180: 68 us, 75 in 4), 4 to
-// 560 (343: 111, 128 in one; 512: 156, 159 in one), then one with quartered last
-// cubes (runs_for; 576: 160, 183 in 4; 1,000: 273, 279 in 2).
+// Most runs that fit at once to 128 cubes (8 cubes: 14 us in 16 runs, 106 in one;
+// 64: 28 in 8; 128: 46 in 4, 112 in one); above, a run's prologue stands against
+// the last wave of workgroups: 8 runs to 200 cubes (180: 62 us, 66 in 4), 4 to
+// 370 (343: 104, 112 in 2), 2 to 560 (512: 146, 150 in 4, 154 in one), then one
+// with quartered last cubes (runs_for; 576: 154, 171 in 2; 1,000: 254, 271 in 2).
 int mixed_runs(int n) {
-  return n <= 32 ? 16 : n <= 64 ? 8 : n <= 128 ? 4 : n <= 200 ? 8 : n <= 560 ? 4 : 1;
+  return n <= 32 ? 16 : n <= 64 ? 8 : n <= 128 ? 4 : n <= 200 ? 8 : n <= 370 ? 4 : n <= 560 ? 2
+       : 1;
 }
 
 void launch_copy_f(hipStream_t s, const float* src, float* dst, size_t n) {

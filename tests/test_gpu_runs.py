@@ -9,9 +9,11 @@ from test_gpu_parity import STATE, compare, er_close
 
 pytestmark = pytest.mark.gpu
 
-# 1, 7, 100 | 101, 560 | 561, 800 cubes (whole and ragged groups of 8; from 561 on
-# the last 192 cubes in four runs)
-LATTICES = [(1, 1, 1), (7, 1, 1), (5, 5, 4), (101, 1, 1), (8, 10, 7), (187, 3, 1), (10, 10, 8)]
+# 1, 7, 48 | 49, 64 | 65, 90 | 91, 128 | 129, 240 | 241, 370 | 371, 560 | 561, 800
+# cubes (whole and ragged groups of 8; from 561 on the last 192 cubes in four runs)
+LATTICES = [(1, 1, 1), (7, 1, 1), (4, 4, 3), (7, 7, 1), (4, 4, 4), (13, 5, 1), (6, 5, 3), (13, 7, 1),
+            (8, 4, 4), (43, 3, 1), (8, 6, 5), (241, 1, 1), (37, 5, 2), (53, 7, 1), (8, 10, 7),
+            (187, 3, 1), (10, 10, 8)]
 
 
 @pytest.mark.parametrize("dims", LATTICES, ids=lambda d: str(int(np.prod(d))))
@@ -60,10 +62,10 @@ def test_in_place_stages_bitwise(B, O, dims):
     assert np.array_equal(out[0].view(np.int64), out[1].view(np.int64))
 
 
-# 1, 32 | 33, 64 | 65, 128 | 129, 200 | 201, 560 | 561, 1,003 cubes
+# 1, 32 | 33, 64 | 65, 128 | 129, 200 | 201, 370 | 371, 560 | 561, 1,003 cubes
 @pytest.mark.parametrize("dims", [(1, 1, 1), (8, 4, 1), (11, 3, 1), (4, 4, 4), (13, 5, 1),
-                                  (8, 4, 4), (43, 3, 1), (8, 5, 5), (67, 3, 1), (8, 10, 7),
-                                  (187, 3, 1), (59, 17, 1)],
+                                  (8, 4, 4), (43, 3, 1), (8, 5, 5), (67, 3, 1), (37, 5, 2),
+                                  (53, 7, 1), (8, 10, 7), (187, 3, 1), (59, 17, 1)],
                          ids=lambda d: str(int(np.prod(d))))
 def test_mixed_runs_by_rule_are_bitwise(B, dims):
     # The runs the rule picks against a pinned count, on one case.
