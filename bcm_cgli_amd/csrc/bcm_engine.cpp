@@ -59,7 +59,7 @@ void free_graph(Engine* e) {
 void free_tables(Engine* e) {
   void* ptrs[] = {e->bc_cubes,     e->bc_masks, e->halo,     e->halo_pairs,
                   e->case_desc,    e->bc_mask_cube, e->ml, e->edge_list, e->open_items,
-                  e->halo_pairs_off, e->ml_ib};
+                  e->halo_pairs_off, e->ml_ib, e->open_edges};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   ghost_free(e->ghost);
@@ -70,6 +70,7 @@ void free_tables(Engine* e) {
   e->halo_pairs = nullptr;
   e->halo_pairs_off = nullptr;
   e->ml_ib = nullptr;
+  e->open_edges = nullptr;
   e->case_desc = nullptr;
   e->ml = nullptr;
   e->edge_list = nullptr;
@@ -157,6 +158,10 @@ GhostSchedule build_ghost_schedule(const std::vector<GhostEntry>& ordered, int s
       E.self = 8;
       for (int m = 0; m < 8; ++m)
         if (corner(E, m) == g) E.self = (int16_t)m;
+      if (E.self < 8) {
+        std::rotate(E.w + E.self, E.w + E.self + 1, E.w + 8);
+        std::rotate(E.lc + E.self, E.lc + E.self + 1, E.lc + 8);
+      }
       gs.out.push_back((int16_t)(last[g] == a ? g : -1));
       cur[g] = a;
       ents[a] = E;
@@ -567,16 +572,31 @@ int rebuild_tables(Engine* e, std::string& err) {
     if (dev_upload(&e->edge_list, list, err)) return 1;
   }
   {
-    // 2: the IB fill touches an edge cell (all edge passes), 1: boundary cube
-    // only (the edge cells its BCs read).
-    std::vector<char> mark(top, 0);
-    for (int c : bc) mark[c] = 1;
-    for (const GhostEntry& E : gs.entries) {
-      bool touch = edge_cell(E.gi, E.gj, E.gk);
-      for (int d = 0; d < 8; ++d)
-        touch = touch || edge_cell(E.pi + (d & 1), E.pj + ((d >> 1) & 1), E.pk + ((d >> 2) & 1));
-      if (touch) mark[E.cube] = 2;
-    }
+    // Edge cells to form per cube.
+    std::vector<std::vector<int16_t>> edges(top);
+    for (int c : bc)
+      for (int i : {1, 18})
+        for (int j : {1, 18}) {
+          if (cube_mask[c] & 16) edges[c].push_back((int16_t)(i * 400 + j * 20 + 2));
+          if (cube_mask[c] & 32) edges[c].push_back((int16_t)(i * 400 + j * 20 + 17));
+        }
+    for (const GhostEntry& E : gs.entries)
+      for (int d = 0; d < 8; ++d) {
+        const int i = E.pi + (d & 1), j = E.pj + ((d >> 1) & 1), k = E.pk + ((d >> 2) & 1);
+        // (Cells of the outer ghost layer are not among the passes'.)
+        auto in = [](int q) { return q >= 1 && q <= 18; };
+        if (edge_cell(i, j, k) && in(i) && in(j) && in(k))
+          edges[E.cube].push_back((int16_t)(i * 400 + j * 20 + k));
+      }
+    std::vector<int16_t> list;
+    auto item = [&](int c, const GhostCube& g) {
+      std::vector<int16_t>& e_ = edges[c];
+      std::sort(e_.begin(), e_.end());
+      e_.erase(std::unique(e_.begin(), e_.end()), e_.end());
+      const int e0 = (int)list.size();
+      list.insert(list.end(), e_.begin(), e_.end());
+      return OpenItem{e0, (int)e_.size(), cube_mask[c], e->cube_case_host[c], g};
+    };
     // The refresh copies land on face ghost cells, which the flux kernels
     // read from memory; an edge destination would be skipped by them.
     for (const int2& pr : pairs) {
@@ -596,16 +616,16 @@ int rebuild_tables(Engine* e, std::string& err) {
         return 1;
       }
       filled[g.cube] = 1;
-      items.push_back(OpenItem{mark[g.cube], cube_mask[g.cube], e->cube_case_host[g.cube], g});
+      items.push_back(item(g.cube, g));
     }
     for (int c = 1; c < top; ++c) {
-      if (filled[c] || !mark[c]) continue;
+      if (filled[c] || !cube_mask[c]) continue;
       GhostCube g{};
       g.cube = c;
-      items.push_back(OpenItem{mark[c], cube_mask[c], e->cube_case_host[c], g});
+      items.push_back(item(c, g));
     }
     e->n_open_items = (int)items.size();
-    if (dev_upload(&e->open_items, items, err)) return 1;
+    if (dev_upload(&e->open_items, items, err) || dev_upload(&e->open_edges, list, err)) return 1;
   }
   if (dev_upload(&e->bc_cubes, bc, err) || dev_upload(&e->bc_masks, bm, err) ||
       ghost_upload(gs, e->ghost, err) || dev_upload(&e->halo, hs, err) ||
@@ -911,8 +931,8 @@ namespace {
 template <typename T>
 void push_stage_open(Engine* e, T* U, const T* other, bool full_pre_halo) {
   launch_halo_ml(e->stream, U, e->ml, e->n_ml, e->pt());
-  launch_open(e->stream, U, e->bc_behind ? other : U, e->open_items, e->n_open_items, e->ghost.t,
-              e->phys_dev);
+  launch_open(e->stream, U, e->bc_behind ? other : U, e->open_items, e->n_open_items,
+              e->open_edges, e->ghost.t, e->phys_dev);
   if (full_pre_halo)
     engine_interface(e);
   else

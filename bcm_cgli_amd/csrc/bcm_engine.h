@@ -136,10 +136,11 @@ struct Engine {
   int n_edge_list = 0;
   // Opening of a stage after a flux kernel that pushed its face halos, one
   // item per cube that needs one, IB cubes first (their fills are the longest
-  // chains).  All edge passes where the cube's IB fill touches an edge cell, in
-  // other boundary cubes the k-edge cells the z-BC copies.  Elsewhere only the
-  // pushing flux kernels read edge cells, and they form them themselves.
+  // chains), and the edge ghost cells (flat i*400 + j*20 + k) it forms: those
+  // the z-BC copies or the IB fill reads.  Elsewhere only the pushing flux
+  // kernels read edge cells, and they form them themselves.
   OpenItem* open_items = nullptr;
+  int16_t* open_edges = nullptr;
   int n_open_items = 0;
   // A pushing flux kernel ran since the BCs did: the ghost regions they write
   // are in the other copy of the iterate.  The next stage's opening reads them

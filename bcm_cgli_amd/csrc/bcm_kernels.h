@@ -80,6 +80,9 @@ struct CaseDesc {
 };
 
 // One IB ghost-fill entry in level order (see the ghost schedule in the engine).
+// Where the ghost cell itself is a corner its weights and slots come with that
+// corner last, the others in their order: the interpolation without it is then
+// the sum of the first seven.
 struct alignas(16) GhostEntry {
   double w[8];
   int16_t lc[8], lg;                // LDS slots read for the corners and written
@@ -122,10 +125,10 @@ struct GhostTables {
   int max_slots = 0;
 };
 
-// One cube's work at the opening of a stage: its edge passes (edges 0 none, 1
-// the edge cells its BCs read, 2 all), its BCs (mask) and its IB fill.
+// One cube's work at the opening of a stage: edge ghost cells edge0 ..
+// edge0 + nedge - 1 of the list, its BCs (mask) and its IB fill.
 struct OpenItem {
-  int edges, mask, slot;
+  int edge0, nedge, mask, slot;
   GhostCube g;
 };
 
@@ -321,9 +324,9 @@ void launch_edge_list(hipStream_t s, float* U, const int* list, int n);
 // above or 0, y: IB ghost-table index or -1) a cube's edge passes and BCs,
 // then its IB fill.
 void launch_open(hipStream_t s, double* U, const double* before, const OpenItem* items, int n,
-                 const GhostTables& g, const DevPhys* phys);
+                 const int16_t* edges, const GhostTables& g, const DevPhys* phys);
 void launch_open(hipStream_t s, float* U, const float* before, const OpenItem* items, int n,
-                 const GhostTables& g, const DevPhys* phys);
+                 const int16_t* edges, const GhostTables& g, const DevPhys* phys);
 // Ghost regions the BCs wrote of the listed cubes, from Uin to Uout.
 void launch_carry_bc(hipStream_t s, const double* Uin, double* Uout, const int* cubes, int n,
                      const uint8_t* cube_mask, PhysTab pt);

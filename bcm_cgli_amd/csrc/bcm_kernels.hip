@@ -462,17 +462,18 @@ __global__ __launch_bounds__(REDUCE_WG) void k_reduce(const double* __restrict__
 // such means), so all cells are loaded, one barrier passes, and all are
 // stored; a cell that a later pass overwrites is not stored by the earlier
 // one.  1024 lanes leave at most one cell of each pass to a lane.  A cube with
-// three BC faces and all edge passes 6 us, pass by pass 9.5; the opening of
-// 2,048 cubes in FP64 (872 with BCs) 28 us, with 256 lanes pass by pass 43.
-// edges 0: no edge passes; 1: only the k-edge cells the z-BC copies (four of
-// the cells of the plane k = 2 or 17); 2: all.  The edge passes belong to the
-// exchange after the last update, so where they read face ghost cells that the
-// BCs write they read the previous stage's: from `before`, the copy of the
-// iterate that holds them (U itself where no pushing flux kernel ran since).
+// three BC faces 6 us, pass by pass 9.5; the opening of 2,048 cubes (872 with
+// BCs) in FP64 28 us, with 256 lanes pass by pass 43.
+// Of the edge passes only the listed cells are formed: those the z-BC copies
+// (four of the plane k = 2 or 17 of such a face; listed wherever there is one)
+// and those the IB fill reads.  The passes belong to the exchange after the last
+// update, so where they read face ghost cells that the BCs write they read the
+// previous stage's: from `before`, the copy of the iterate that holds them (U
+// itself where no pushing flux kernel ran since).
 constexpr int OPEN_WG = 1024;
 template <typename T>
-__device__ __forceinline__ void edge_bc_cube(T* U, const T* before, int c, int edges, int m,
-                                             const DevPhys& ph) {
+__device__ __forceinline__ void edge_bc_cube(T* U, const T* before, int c, const int16_t* edges,
+                                             int nedge, int m, const DevPhys& ph) {
   using T2 = typename Vec2<T>::type;
   const typename OffOf<T>::type F(ph);
   const int t = threadIdx.x;
@@ -481,6 +482,8 @@ __device__ __forceinline__ void edge_bc_cube(T* U, const T* before, int c, int e
   auto at = [](int v, int i, int j, int k) { return v * PLANE + i * 400 + j * 20 + k; };
   // Nearest interior index of 1 (2) or 18 (17).
   auto near = [](int q) { return q == 1 ? 2 : 17; };
+  bool de = t < 5 * nedge;
+  const int ecell = de ? edges[t / 5] : 0, ev = t % 5;
   // Face ghost cell as the last exchange's edge passes read it.
   auto face = [&](int v, int i, int j, int k) {
     const bool bc = (i == 1 && (m & 1)) || (i == 18 && (m & 2)) || (j == 1 && (m & 4)) ||
@@ -543,70 +546,41 @@ __device__ __forceinline__ void edge_bc_cube(T* U, const T* before, int c, int e
     const int j = zj < 2 && (m & 4) ? 2 : (zj > 17 && (m & 8) ? 17 : zj);
     int i = zi;
     if (j >= 2 && j <= 17) i = x_source(zi, zin);
-    dz = !(edges != 0 && (i == 1 || i == 18) && (j == 1 || j == 18));
+    dz = !(nedge > 0 && (i == 1 || i == 18) && (j == 1 || j == 18));
     if (dz)
 #pragma unroll
       for (int v = 0; v < 5; ++v) z[v] = Uc[at(v, i, j, zk)];
   }
 
-  // Edges: item t of 320 per axis (lines of 16 cells, 4 edges, 5 variables),
-  // then the 8 corners x 5 variables, each the mean of the j-edge and the
-  // i-edge cell next to it.  With edges 1 the k-edge cells next to a z-BC.
-  bool de = false, corner = false;
-  int dst = 0, zcopy = 0, ev = 0;   // zcopy 1 (2): z-min (z-max) copies the cell
+  // Edges: a listed cell's variable t % 5 by lane t (at most 200 cells), the
+  // mean of two face ghost cells, or at a cube corner of the j-edge and the
+  // i-edge cell next to it.
+  bool corner = false;
+  int zcopy = 0;   // 1 (2): z-min (z-max) copies the cell
   T ea, eb, ec;
-  if (edges == 2 && t < 1000) {
-    de = true;
-    corner = t >= 960;
-    const int A = t / 320, u = corner ? t - 960 : t % 320;
-    const int e = u & 3, v = corner ? (u >> 2) % 5 : (u >> 2) % 5, q = (u >> 2) / 5;
-    const int lo = e & 1 ? 18 : 1, hi = e & 2 ? 18 : 1;
-    int i, j, k;
-    if (corner)
-      i = lo, j = hi, k = q ? 18 : 1;
-    else if (A == 0)
-      i = q + 2, j = lo, k = hi;
-    else if (A == 1)
-      i = hi, j = q + 2, k = lo;
-    else
-      i = hi, j = lo, k = q + 2;
-    dst = at(v, i, j, k);
-    ev = v;
+  if (de) {
+    const int i = ecell / 400, j = ecell / 20 % 20, k = ecell % 20;
+    const bool gi = i == 1 || i == 18, gj = j == 1 || j == 18, gk = k == 1 || k == 18;
+    corner = gi && gj && gk;
     if (corner) {
       // j-edge (i, near j, k) from ea and ec, i-edge (near i, j, k) from eb
       // and ec.
-      ea = face(v, i, near(j), near(k));
-      eb = face(v, near(i), j, near(k));
-      ec = face(v, near(i), near(j), k);
-    } else if (A == 0) {
-      ea = face(v, i, j, near(k));
-      eb = face(v, i, near(j), k);
-    } else if (A == 1) {
-      ea = face(v, i, j, near(k));
-      eb = face(v, near(i), j, k);
+      ea = face(ev, i, near(j), near(k));
+      eb = face(ev, near(i), j, near(k));
+      ec = face(ev, near(i), near(j), k);
     } else {
-      ea = face(v, i, near(j), k);
-      eb = face(v, near(i), j, k);
+      // (For each pair of ghost layers the cell one step in from either.)
+      ea = gk ? face(ev, i, j, near(k)) : face(ev, i, near(j), k);
+      eb = gi ? face(ev, near(i), j, k) : face(ev, i, near(j), k);
     }
     // Cells the BCs overwrite.
     const bool zinner = i >= 2 && i <= 17;
-    if (!corner && A == 2) {
+    if (!gk) {
       de = !((j == 1 && (m & 4)) || (j == 18 && (m & 8)));
       zcopy = k == 2 && (m & 16) ? 1 : (k == 17 && (m & 32) ? 2 : 0);
     } else {
       de = !((k == 1 && (m & 16) && !(zinner && (m & ZBC_IN_FLUX))) ||
              (k == 18 && (m & 32) && !(zinner && (m & (ZBC_IN_FLUX << 1)))));
-    }
-  } else if (edges == 1 && t < 40) {
-    const int zs = t / 20, cell = (t / 5) % 4, v = t % 5;
-    const int i = cell & 1 ? 18 : 1, j = cell & 2 ? 18 : 1, k = zs ? 17 : 2;
-    de = (m & (16 << zs)) && !((j == 1 && (m & 4)) || (j == 18 && (m & 8)));
-    if (de) {
-      dst = at(v, i, j, k);
-      ev = v;
-      zcopy = 1 + zs;
-      ea = face(v, i, near(j), k);
-      eb = face(v, near(i), j, k);
     }
   }
   __syncthreads();   // all loads have returned
@@ -617,6 +591,7 @@ __device__ __forceinline__ void edge_bc_cube(T* U, const T* before, int c, int e
       eb = 0.5 * (eb + ec);
     }
     const T x = 0.5 * (ea + eb);
+    const int dst = ev * PLANE + ecell;
     Uc[dst] = x;
     if (zcopy) {
       // dst is the k = 2 (17) cell; its z ghost cells are k = 0, 1 (18, 19).
@@ -675,7 +650,7 @@ template <typename T>
 __global__ __launch_bounds__(OPEN_WG) void k_bc(T* __restrict__ U, const int* __restrict__ cubes,
                                                 const uint8_t* __restrict__ masks, PhysTab pt) {
   const int c = cubes[blockIdx.x];
-  edge_bc_cube<T>(U, U, c, 0, masks[blockIdx.x], pt.phys[pt.cube_case[c]]);
+  edge_bc_cube<T>(U, U, c, nullptr, 0, masks[blockIdx.x], pt.phys[pt.cube_case[c]]);
 }
 
 // Ghost regions the BCs wrote, from the copy of the iterate that a pushing flux
@@ -711,10 +686,10 @@ __global__ __launch_bounds__(OPEN_WG) void k_carry_bc(const T* __restrict__ Uin,
 // entry.  A cube's tables start from one record; the next level's entries and
 // the bounds of the one after load during a level, whose barrier leaves memory
 // operations in flight; ghost cells go back to memory once, at the end.  A
-// level takes 0.9 us with few entries and 2.3 with 126 (2.2 us when each
-// entry formed its corners' primitives in one lane and every level waited for
-// its table loads), the whole fill of a sphere inside one cube (7 levels) 12
-// us of 18, of a body on 7 cubes with one of 2040 slots 16 of 75 (then on
+// level takes 0.85 us with few entries and 1.9 with 126 (2.2 us when each entry
+// formed its corners' primitives in one lane and every level waited for its
+// table loads), the opening of a stage with a sphere inside one cube (7 levels)
+// 11.5 us of 20, of a body on 7 cubes with one of 2040 slots 12.5 of 75 (then on
 // memory, beyond 1536 slots).
 // A value is rounded to storage precision before a later level reads it, as
 // memory would round it, so the fill on memory (cubes of more slots than
@@ -760,31 +735,25 @@ __device__ __forceinline__ void corner_prim(const double (&q)[5], double (&p)[5]
 
 // Conserved state of a ghost cell, by eight lanes that all return it: lane
 // r < 5 of them interpolates quantity r (density, velocity, pressure) from the
-// corners' values x with the weights w; s is the corner that is the ghost cell
-// itself (8: none).
-__device__ __forceinline__ void ghost_state(const double (&w)[8], const double (&x)[8], int s,
+// corners' values x with the weights w, in the order of a GhostEntry; self: the
+// last corner is the ghost cell.
+__device__ __forceinline__ void ghost_state(const double (&w)[8], const double (&x)[8], bool self,
                                             double rho0, double P0, double (&o)[5]) {
   const int r = threadIdx.x & 7;
-  const bool scalar = r == 0 || r >= 4, self = s < 8;
+  const bool scalar = r == 0 || r >= 4;
   const double off = r == 0 ? rho0 : (r >= 4 ? P0 : 0.0);
-  // Sums over all corners and over those but s, each in corner order.
   // (Subtracting an offset of zero changes no value.)
-  double all = 0, but = 0, ws = 0, xs = 0;
+  double s = w[0] * (x[0] - off);
 #pragma unroll
-  for (int m = 0; m < 8; ++m) {
-    const double y = w[m] * (x[m] - off);
-    all = m == 0 ? y : all + y;
-    but = m == 0 ? y : (m == 1 && s == 0 ? y : (m == s ? but : but + y));
-    ws = m == s ? w[m] : ws;
-    xs = m == s ? x[m] : xs;
-  }
+  for (int m = 1; m < 7; ++m) s = s + w[m] * (x[m] - off);
   double z;
   if (self) {
     // The ghost cell is an interpolation corner (:192-449).
-    const double qt = but / ((scalar ? 1 : 2) - ws);
-    z = scalar ? (ws > 0.9999 ? xs : qt + off) : qt;
+    const double qt = s / ((scalar ? 1 : 2) - w[7]);
+    z = scalar ? (w[7] > 0.9999 ? x[7] : qt + off) : qt;
   } else {
-    z = scalar ? all + off : all;
+    s = s + w[7] * (x[7] - off);
+    z = scalar ? s + off : s;
   }
   const int l0 = threadIdx.x & 56;
   const double rho = __shfl(z, l0), uu = __shfl(z, l0 + 1), vv = __shfl(z, l0 + 2),
@@ -875,7 +844,7 @@ __device__ __forceinline__ void ghost_lds(T* __restrict__ U, const GhostTables& 
     double x[8], o[5], p[5];
 #pragma unroll
     for (int m = 0; m < 8; ++m) x[m] = prim[rv * cap + E.slot(m)];
-    ghost_state(E.w, x, E.lg_self >> 16, ph.rho0, ph.P0, o);
+    ghost_state(E.w, x, (E.lg_self >> 16) < 8, ph.rho0, ph.P0, o);
 #pragma unroll
     for (int v = 0; v < 5; ++v) o[v] = F.rt(o[v], v);
     corner_prim<OFF>(o, p);
@@ -912,8 +881,8 @@ __device__ __forceinline__ void ghost_lds(T* __restrict__ U, const GhostTables& 
   }
 }
 
-// IB fill of one cube in place on memory: lane m of an entry's eight forms
-// corner m's primitives.
+// IB fill of one cube in place on memory: an entry's eight lanes form a corner's
+// primitives each.
 template <typename T>
 __device__ __forceinline__ void ghost_memory(T* __restrict__ U, const GhostTables& gt,
                                              const GhostCube& g, const DevPhys& ph) {
@@ -925,9 +894,11 @@ __device__ __forceinline__ void ghost_memory(T* __restrict__ U, const GhostTable
     const int e1 = gt.level_off[lv + 1];
     for (int n = gt.level_off[lv] + threadIdx.x / 8; n < e1; n += GHOST_PASS) {
       const GhostEntry& E = gt.ent[n];
-      const int a = (r == 1 || r == 4 || r == 5 || r == 7);
-      const int bq = (r == 2 || r == 4 || r == 6 || r == 7);
-      const int cq = (r == 3 || r == 5 || r == 6 || r == 7);
+      // Corner of the entry's r-th weight.
+      const int m = E.self > 7 ? r : r == 7 ? E.self : r + (r >= E.self);
+      const int a = (m == 1 || m == 4 || m == 5 || m == 7);
+      const int bq = (m == 2 || m == 4 || m == 6 || m == 7);
+      const int cq = (m == 3 || m == 5 || m == 6 || m == 7);
       const size_t at = base + (E.pi + a) * 400 + (E.pj + bq) * 20 + (E.pk + cq);
       double q[5], p[5], w[8], x[8], o[5];
 #pragma unroll
@@ -942,7 +913,7 @@ __device__ __forceinline__ void ghost_memory(T* __restrict__ U, const GhostTable
           x[m] = v == 0 || r == v ? y : (v == 4 && r > 4 ? y : x[m]);
         }
       }
-      ghost_state(w, x, E.self, ph.rho0, ph.P0, o);
+      ghost_state(w, x, E.self < 8, ph.rho0, ph.P0, o);
       // Every corner has been read: the eight lanes are in one wave, and no
       // other entry of the level reads or writes the cell.
       const size_t go = base + E.gi * 400 + E.gj * 20 + E.gk;
@@ -1133,17 +1104,19 @@ __global__ __launch_bounds__(WG) void k_edge_list(T* __restrict__ U, const int* 
 template <typename T>
 __global__ __launch_bounds__(OPEN_WG) void k_open(T* U, const T* before,
                                                   const OpenItem* __restrict__ items,
+                                                  const int16_t* __restrict__ edges,
                                                   GhostTables gt,
                                                   const DevPhys* __restrict__ phys) {
   extern __shared__ double gsm[];
   const OpenItem it = items[blockIdx.x];
   const DevPhys ph = phys[it.slot];
-  if (it.edges) edge_bc_cube(U, before, it.g.cube, it.edges, it.mask, ph);
+  const bool shell = it.mask || it.nedge;
+  if (shell) edge_bc_cube(U, before, it.g.cube, edges + it.edge0, it.nedge, it.mask, ph);
   if (it.g.nlev == 0) return;
   // The fill's tables load while the stores above complete.
   GhostFirst f;
   ghost_first(gt, it.g, f);
-  if (it.edges) __syncthreads();
+  if (shell) __syncthreads();
   ghost_cube(U, gt, it.g, f, ph, gsm);
 }
 
@@ -1275,19 +1248,19 @@ void launch_ghost(hipStream_t s, float* U, const GhostTables& g, PhysTab pt) {
 
 template <typename T>
 void launch_open_t(hipStream_t s, T* U, const T* before, const OpenItem* items, int n,
-                   const GhostTables& g, const DevPhys* phys) {
+                   const int16_t* edges, const GhostTables& g, const DevPhys* phys) {
   if (n <= 0) return;
   const size_t shmem = (size_t)g.max_slots * 5 * sizeof(double);
-  hipLaunchKernelGGL(k_open<T>, dim3(n), dim3(OPEN_WG), shmem, s, U, before, items, g,
-                     phys);
+  hipLaunchKernelGGL(k_open<T>, dim3(n), dim3(OPEN_WG), shmem, s, U, before, items,
+                     edges, g, phys);
 }
 void launch_open(hipStream_t s, double* U, const double* before, const OpenItem* items, int n,
-                 const GhostTables& g, const DevPhys* phys) {
-  launch_open_t(s, U, before, items, n, g, phys);
+                 const int16_t* edges, const GhostTables& g, const DevPhys* phys) {
+  launch_open_t(s, U, before, items, n, edges, g, phys);
 }
 void launch_open(hipStream_t s, float* U, const float* before, const OpenItem* items, int n,
-                 const GhostTables& g, const DevPhys* phys) {
-  launch_open_t(s, U, before, items, n, g, phys);
+                 const int16_t* edges, const GhostTables& g, const DevPhys* phys) {
+  launch_open_t(s, U, before, items, n, edges, g, phys);
 }
 
 template <typename T>
