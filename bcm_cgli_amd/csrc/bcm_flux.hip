@@ -87,7 +87,8 @@ __device__ __forceinline__ T& at_byte(T* base, unsigned off) {
 // give two workgroups per CU.  Against a march that loaded the plane's and the
 // column's cells in the iteration that uses them, with three barriers and one
 // boundary round per axis: 1,252 -> 1,004 us on 2,048 cubes (PUSH), 1,487 ->
-// 1,072 (IN_PLACE).
+// 1,072 (IN_PLACE).  (PUSH 947 with quartered last cubes and without the copy of
+// the BC regions.)
 template <March MODE, bool AUX>
 __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
   __shared__ __align__(16) double cp[2][5 * 400];   // conserved values of planes i, i+1

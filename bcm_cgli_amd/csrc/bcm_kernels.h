@@ -316,13 +316,10 @@ void launch_halo_pairs(hipStream_t s, float* U, const int2* pairs, int npairs);
 // Edge passes of the listed cubes.
 void launch_edge_list(hipStream_t s, double* U, const int* list, int n);
 void launch_edge_list(hipStream_t s, float* U, const int* list, int n);
-// Edge passes of the n listed cubes (entry c; entry -c: only the k-edge cells
-// the z-BC reads), then the domain BCs of those that are boundary cubes
-// (cube_mask[c]: the k_bc side bits of pool cube c, 0 for none).  Used after
-// a flux kernel that wrote the face halos itself.
-// Opening of a pushed stage in one launch: per item (x: edge/BC entry as
-// above or 0, y: IB ghost-table index or -1) a cube's edge passes and BCs,
-// then its IB fill.
+// Opening of a stage after a flux kernel that wrote the face halos itself, in one
+// launch: per item the listed edge cells and the domain BCs, then the IB fill.
+// `before` holds the ghost regions the previous stage's BCs wrote: the other copy
+// of the iterate, or U where they were carried over.
 void launch_open(hipStream_t s, double* U, const double* before, const OpenItem* items, int n,
                  const int16_t* edges, const GhostTables& g, const DevPhys* phys);
 void launch_open(hipStream_t s, float* U, const float* before, const OpenItem* items, int n,

@@ -16,11 +16,8 @@
 // operation order is free here, so divisions become reciprocal multiplies and
 // square roots the hardware approximations.
 //
-// Kernel shape: one workgroup of 256 lanes per cube, lane (j,k), marching
-// along i.  Each lane keeps its own i-column of conserved values (planes
-// i-3..i+3) and flags (i-2..i+2) in registers for the x-stencils; the plane
-// being processed is staged in LDS for the y- and z-stencils; primitives of
-// three planes sit in an LDS ring for the viscous terms.  The kernel reads
+// Kernel shape: one workgroup of 256 lanes per cube or run of its planes, a lane
+// per (j,k), marching along i (k_flux_mixed below).  The kernel reads
 // one copy of the iterate and writes the other, so each cell's RK update is
 // stored as soon as it is computed: no stage increment array, no RK scratch
 // arrays; the two layers next to a face with a neighbour are written into
@@ -233,9 +230,8 @@ __device__ __forceinline__ void plane_states(const float* cp, int base, int st, 
 // Viscous flux through the face between cell P and P + e_D (Flux.cpp:1946-2272,
 // forward-face formulas of P): one evaluation serves both adjacent cells.  D as
 // for roe_f.  ring holds deviations of u, v, w, T; rm, r0 and rp are the ring
-// offsets of P in the plane before, its own and the next (rm unused for D = 0,
-// rp unused for the backward of nothing).  L receives the x, y, z stress and the
-// energy flux.
+// offsets of P in the plane before, its own and the next (rm unused for D = 0).
+// L receives the x, y, z stress and the energy flux.
 template <int D>
 __device__ __forceinline__ void visc_face(const float (*ring)[3 * PR], int rm, int r0, int rp,
                                           const RefF& rf, float inv, float iT0, float muL,
@@ -322,7 +318,9 @@ __device__ __forceinline__ T& at_byte(T* base, unsigned off) {
 // launch).  Two workgroups per CU: a third (46 KB of LDS, 168 registers with 25
 // spilled) gives the same rate, 624 us on 2,048 cubes against 555.  Against a
 // march that kept the whole column in registers, two face arrays more in LDS and
-// a boundary round per axis: 570 -> 555 us on 2,048 cubes, 51 -> 45 on 125.
+// a boundary round per axis: 570 -> 555 us on 2,048 cubes, 51 -> 45 on 125.  (476
+// and 43 with what followed: quartered last cubes, BC regions carried by a kernel
+// of their own, another schedule.)
 __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
     float* __restrict__ U, float* __restrict__ Uout, const HaloSrc* __restrict__ halo,
     const uint8_t* __restrict__ cube_mask, const double* __restrict__ Bsrc,
