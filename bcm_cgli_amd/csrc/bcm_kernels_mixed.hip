@@ -536,6 +536,17 @@ __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
     const int ro = ring_idx(j, k);
 
     // ---- phase 1: y- and z-faces of plane i ----
+    // The row of the plane before, from the waves' sums: after the barrier that
+    // closed that plane, before the one ahead of this plane's sums.
+    if (RK == 3 && i > i0 && t < 8) {
+      double s = red[0][t];
+#pragma unroll
+      for (int w = 1; w < WG / 64; ++w) s += red[w][t];
+      if (run.nseg == 1)   // (in the order k_reduce adds rows)
+        tot[t] = i == i0 + 1 ? s : tot[t] + s;
+      else
+        partials[((size_t)(c - 1) * MIXED_ROWS_PER_CUBE + (i - 3)) * 8 + t] = s;
+    }
     stage(i + 1);
     load_flags(i + 1);
     float n3[5];
@@ -589,15 +600,6 @@ __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
     __syncthreads();
 
     // ---- phase 2 ----
-    if (RK == 3 && i > i0 && t < 8) {
-      double s = red[0][t];
-#pragma unroll
-      for (int w = 1; w < WG / 64; ++w) s += red[w][t];
-      if (run.nseg == 1)   // (in the order k_reduce adds rows)
-        tot[t] = i == i0 + 1 ? s : tot[t] + s;
-      else
-        partials[((size_t)(c - 1) * MIXED_ROWS_PER_CUBE + (i - 3)) * 8 + t] = s;
-    }
     // This cell's FP64 source constant Bv = 3 Uref - 4 U1 + U1q, first used in
     // the residual.
     const size_t row = (size_t)c * CUBE_STRIDE + i * 400;
