@@ -942,6 +942,11 @@ void push_stage_open(Engine* e, T* U, const T* other, bool full_pre_halo) {
 
 namespace {
 double* er_row(Engine* e, int er_slot) { return e->er_dev + (size_t)er_slot * e->max_cases * 8; }
+
+// The current copy of the iterate.
+const void* iterate(const Engine* e) {
+  return e->prec == 1 ? static_cast<const void*>(e->Uf) : e->U;
+}
 }  // namespace
 
 void engine_flux(Engine* e) {
@@ -1214,8 +1219,11 @@ int engine_run(Engine* e, int n_steps, int n_inner, double* er_hist, bool use_gr
   }
   if (ensure_er(e, n_inner, err)) return 1;
   if (engine_maybe_tune(e, err)) return 1;
-  if (use_graph && (!e->graph_valid || e->graph_inner != n_inner)) {
+  // (A single stage may have left the iterate in the other copy.)
+  if (use_graph &&
+      (!e->graph_valid || e->graph_inner != n_inner || e->graph_iterate != iterate(e))) {
     free_graph(e);
+    e->graph_iterate = iterate(e);
     HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
     enqueue_step(e, n_inner, false);
     HIP_TRY(hipStreamEndCapture(e->stream, &e->graph));

@@ -185,6 +185,7 @@ struct Engine {
   hipGraphExec_t graph_exec = nullptr;
   hipGraph_t graph = nullptr;
   int graph_inner = 0;
+  const void* graph_iterate = nullptr;   // copy of the iterate the captured step starts from
 };
 
 // Bytes of device memory per pool cube for a precision (0 FP64, 1 mixed).
