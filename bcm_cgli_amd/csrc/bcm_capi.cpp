@@ -605,6 +605,7 @@ int bcm_engine_time_part(bcm_engine* h, int part, int RK, int reps, double* ms) 
   // it, without the stores of Rku1, U1p1, U1p2 and Residual1 that only a
   // step's last inner iteration makes.
   e->push_aux = part != 9 ? PushAux::ALL : PushAux::NONE;
+  if (part == 9 || (part == 7 && e->prec == 1)) engine_share_bc(e);
   if (hipEventRecord(e->ev0, e->stream) != hipSuccess) return fail("event record failed");
   for (int r = 0; r < reps; ++r) {
     switch (part) {

@@ -1017,6 +1017,13 @@ void engine_carry_bc(Engine* e) {
   e->bc_behind = false;
 }
 
+void engine_share_bc(Engine* e) {
+  if (e->prec == 1)
+    launch_carry_bc(e->stream, e->Uf, e->Uf2, e->bc_cubes, e->n_bc, e->bc_mask_cube, e->pt());
+  else
+    launch_carry_bc(e->stream, e->U, e->U2, e->bc_cubes, e->n_bc, e->bc_mask_cube, e->pt());
+}
+
 void engine_flux_update(Engine* e, int RK, int er_slot) {
   if (e->prec == 1) {
     push_flux(e, RK, er_slot);

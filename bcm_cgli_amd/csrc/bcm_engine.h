@@ -239,6 +239,10 @@ bool engine_fused(const Engine* e);
 // engine_carry_bc, so that no interface call returns without them.
 void engine_flux_push(Engine* e, int RK, int er_slot);
 void engine_carry_bc(Engine* e);
+// The same regions of the current copy into the other one, before several pushing
+// kernels with no stage opening between them: each then finds the regions in the
+// copy it reads.
+void engine_share_bc(Engine* e);
 void engine_shift(Engine* e);
 void engine_stage(Engine* e, int RK, int er_slot, bool full_pre_halo = false);
 // n_steps physical steps of n_inner inner iterations for every resident case.

@@ -53,3 +53,26 @@ def test_captured_steps_continue_from_a_part(B, precision, part, n_inner):
     finally:
         graph.close()
         eager.close()
+
+
+@pytest.mark.parametrize("reps", [1, 2, 3, 4])
+@pytest.mark.parametrize("precision,part", [("fp64", "flux_push"), ("mixed", "flux_push"),
+                                            ("mixed", "flux_update")])
+def test_repeated_pushing_kernel_carries_the_bc_regions(B, precision, part, reps):
+    # The kernel several times with no stage opening in between: each reads the
+    # ghost regions of the domain BCs, and the last leaves them in the iterate.
+    case = B.Case(B.case_params("tiny"))
+    timed, single = pool(B, case, precision), pool(B, case, precision)
+    try:
+        for e in (timed, single):
+            e.run(1, 2)   # (an even number of kernels: the copies differ)
+        timed.time_part(part, RK=2, reps=reps)
+        for _ in range(reps):
+            single.part(part, 2)
+        same(timed, single, ("U1_",))
+        for e in (timed, single):
+            e.run(1, 1)
+        same(timed, single, STATE[precision])
+    finally:
+        timed.close()
+        single.close()
