@@ -40,12 +40,16 @@ namespace {
 // The engine's chunks, or null when they cannot be had.
 HostChunks* host_chunks(Engine* e) {
   if (e->chunks) return e->chunks;
+  const bool clean = hipPeekAtLastError() == hipSuccess;
   e->chunks = new (std::nothrow) HostChunks();
   if (!e->chunks) return nullptr;
   bool ok = hipHostMalloc((void**)&e->chunks->pin, 2 * THREADS * CHUNK) == hipSuccess;
   for (hipEvent_t& ev : e->chunks->ready)
     ok = ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
-  if (!ok) engine_chunks_free(e);
+  if (!ok) {
+    engine_chunks_free(e);
+    if (clean) (void)hipGetLastError();   // (no error but the allocation's)
+  }
   return e->chunks;
 }
 
@@ -63,7 +67,6 @@ void engine_chunks_free(Engine* e) {
 hipError_t engine_to_host(Engine* e, void* dst, const void* src, size_t bytes) {
   HostChunks* h = bytes < DIRECT_BELOW ? nullptr : host_chunks(e);
   if (!h) {
-    (void)hipGetLastError();
     const hipError_t rc = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, e->stream);
     return rc != hipSuccess ? rc : hipStreamSynchronize(e->stream);
   }

@@ -785,6 +785,17 @@ int engine_load_case(Engine* e, const Case& cs, std::string& err) {
   return 0;
 }
 
+namespace {
+// Whether a launch succeeded, as far as it can be told: an error that was pending
+// before stays for the next call that looks for one.
+template <typename F>
+bool launched(F launch) {
+  const bool clean = hipPeekAtLastError() == hipSuccess;
+  launch();
+  return !clean || hipPeekAtLastError() == hipSuccess;
+}
+}  // namespace
+
 int engine_case_state(Engine* e, int slot, int which, double* aos, bool upload,
                       std::string& err) {
   if (slot < 0 || slot >= e->max_cases || !e->cases[slot].active) {
@@ -824,10 +835,16 @@ int engine_case_state(Engine* e, int slot, int which, double* aos, bool upload,
   } else {
     double ref[5];
     ref_state(S.tb.ph, ref);
-    if (f32)
-      launch_soa_to_aos_f(e->stream, dstf, e->staging, (int)n, ref);
-    else
-      launch_soa_to_aos(e->stream, dst, e->staging, (int)n);
+    const bool ok = launched([&] {
+      if (f32)
+        launch_soa_to_aos_f(e->stream, dstf, e->staging, (int)n, ref);
+      else
+        launch_soa_to_aos(e->stream, dst, e->staging, (int)n);
+    });
+    if (!ok) {
+      err = "the state's layout conversion could not be launched";
+      return 1;
+    }
     HIP_TRY(engine_to_host(e, aos + CUBE_STRIDE, e->staging, n * cube_bytes));
     memset(aos, 0, cube_bytes);
   }
@@ -855,7 +872,7 @@ int engine_download_state(Engine* e, int which, double* aos) {
   if (e->prec != 0) return 1;
   double* d = state_ptr(e, which);
   if (!d) return 1;
-  launch_soa_to_aos(e->stream, d, e->staging, e->ncube);
+  if (!launched([&] { launch_soa_to_aos(e->stream, d, e->staging, e->ncube); })) return 1;
   return engine_to_host(e, aos, e->staging, pool_bytes(e)) == hipSuccess ? 0 : 1;
 }
 
