@@ -394,7 +394,7 @@ __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
             16 * ((t & ~63) + h * WG));
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                      :: "s"(dst), "v"(off), "s"(Uc + p * 400)
-                     : "memory");
+                     : "memory", "m0");
       }
     }
   };

@@ -1,5 +1,6 @@
-"""CPU check of the marching kernels' source: what a wave writes to LDS for the
-others is read only after a workgroup barrier."""
+"""CPU checks of the marching kernels' source: what a wave writes to LDS for the
+others is read only after a workgroup barrier, and inline assembly declares the
+LDS base register that it writes."""
 import os
 import re
 
@@ -43,3 +44,15 @@ def test_norm_sums_of_the_waves_cross_a_barrier(name, loop):
             assert not {"write", "read"} <= stretch, events
             stretch = set()
         stretch.add(ev)
+
+
+@pytest.mark.parametrize("name", ["bcm_flux.hip", "bcm_kernels_mixed.hip"])
+def test_inline_assembly_declares_m0(name):
+    text = source(name)
+    writers = 0
+    for m in re.finditer(r"asm volatile\((.*?)\);", text, re.S):
+        if re.search(r"s_mov_b32 m0", m.group(1)):
+            writers += 1
+            clobbers = m.group(1).rsplit(":", 1)[1]
+            assert '"m0"' in clobbers and '"memory"' in clobbers, m.group(0)
+    assert writers
