@@ -450,8 +450,9 @@ class Engine:
 
     def set_ghost_lds_limit(self, slots):
         """Cubes whose IB fill needs more LDS value slots than this take the
-        in-place schedule on memory (cases loaded or added afterwards); at most
-        1536, by default the kernel's capacity of 3072.  A test hook."""
+        in-place schedule on memory (cases loaded or added afterwards); 1536,
+        the largest, stands for the default, the kernel's capacity of 3072.  A
+        test hook."""
         _check(_lib.bcm_engine_set_ghost_lds_limit(self._h, int(slots)))
 
     def ghost_stats(self):

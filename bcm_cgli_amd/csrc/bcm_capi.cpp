@@ -693,7 +693,7 @@ int bcm_engine_set_ghost_lds_limit(bcm_engine* h, int slots) {
   if (!h) return fail("null engine");
   if (slots < 0 || slots > GHOST_LDS_HOOK_MAX)
     return fail("slot limit must be in 0.." + std::to_string(GHOST_LDS_HOOK_MAX));
-  h->e->ghost_slot_limit = slots;
+  h->e->ghost_slot_limit = slots == GHOST_LDS_HOOK_MAX ? GHOST_LDS_SLOTS : slots;
   return 0;
 }
 

@@ -97,7 +97,8 @@ struct alignas(16) GhostEntry {
 // 3072 slots of five doubles are 120 KB of the 160 KB of a CU; a whole body
 // inside one cube needs about 1000 to 2100.
 constexpr int GHOST_LDS_SLOTS = 3072;
-// Largest limit the diagnostic hook accepts.
+// Largest limit the diagnostic hook accepts; it stands for no limit but the
+// kernel's (a caller that lowered the limit takes that back with it).
 constexpr int GHOST_LDS_HOOK_MAX = 1536;
 
 // IB fill of one cube: its levels, entries and the cells it reads.

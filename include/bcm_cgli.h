@@ -278,10 +278,10 @@ int bcm_engine_autotune(bcm_engine* e, int* out3);
 /* Ghost schedule statistics: entries, cubes with entries, maximum levels. */
 int bcm_engine_ghost_stats(bcm_engine* e, int* stats3);
 /* The IB fill of a cube runs out of LDS when its value slots fit the limit
- * (0..1536; 3072 unless set), else in place on memory; a lower limit,
- * applied to cases loaded or added afterwards, puts more cubes on the memory
- * schedule (bitwise the same results).  Not a reference interface: a test
- * and diagnostic hook. */
+ * (0..1536, 1536 standing for the default, the kernel's capacity of 3072), else
+ * in place on memory; a lower limit, applied to cases loaded or added
+ * afterwards, puts more cubes on the memory schedule (bitwise the same
+ * results).  Not a reference interface: a test and diagnostic hook. */
 int bcm_engine_set_ghost_lds_limit(bcm_engine* e, int slots);
 /* The FP64 kernels divide and take square roots without range scaling, and
  * divide several numerators by one denominator with the denominator's part of
