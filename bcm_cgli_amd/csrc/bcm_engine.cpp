@@ -1076,12 +1076,14 @@ int engine_autotune(Engine* e, int* variant, int* nseg, std::string& err) {
     return 1;
   }
   if (e->prec == 1) {
-    // The mixed flux kernel in 1, 2 or 4 runs per cube (bitwise the same
-    // results), each timed as one whole RK stage on the resident cases; the
-    // iterate the stages write is restored.  The candidates are timed in three
-    // interleaved rounds and each keeps its fastest round, so a clock ramp at
-    // the start favours none of them.  The choice holds for this size class of
-    // the pool; a run on another takes the rule's.
+    // The mixed flux kernel in the rule's runs per cube and in the counts that
+    // can be pinned, 1, 2 and 4 (bitwise the same results), each timed as one
+    // whole RK stage on the resident cases; the iterate the stages write is
+    // restored.  The candidates are timed in three interleaved rounds and each
+    // keeps its fastest round, so a clock ramp at the start favours none of them.
+    // The choice holds for this size class of the pool; a run on another takes
+    // the rule's, as does this one where the rule's 8 or 16 runs are the fastest
+    // (8 cubes, a stage: 23 us in 16 runs, 47 in 4).
     const size_t bytes = (size_t)e->ncube * CUBE_STRIDE * sizeof(float);
     struct Saved {
       float* p[2] = {nullptr, nullptr};
@@ -1096,10 +1098,11 @@ int engine_autotune(Engine* e, int* variant, int* nseg, std::string& err) {
       HIP_TRY(hipMemcpyAsync(saved.p[a], live[a], bytes, hipMemcpyDeviceToDevice, e->stream));
     }
     const bool full = e->halo_full_next;
-    const int cands[3] = {1, 2, 4};
-    float fastest[3] = {1e30f, 1e30f, 1e30f};
+    const int cands[4] = {1, 2, 4, mixed_runs(resident_cubes(e))};
+    const int ncand = cands[3] > 4 ? 4 : 3;   // (else the rule's is among the others)
+    float fastest[4] = {1e30f, 1e30f, 1e30f, 1e30f};
     for (int round = 0; round < 3; ++round)
-      for (int c = 0; c < 3; ++c) {
+      for (int c = 0; c < ncand; ++c) {
         e->mixed_nseg = cands[c];
         e->tuned_class = size_class(e);   // (the candidate, not the rule)
         engine_stage(e, 2, 0, full);   // warm up
@@ -1127,7 +1130,7 @@ int engine_autotune(Engine* e, int* variant, int* nseg, std::string& err) {
       }
     e->mixed_nseg = bn;
     e->graph_valid = false;
-    e->tuned_class = size_class(e);
+    e->tuned_class = ncand == 4 && fastest[3] <= best ? -1 : size_class(e);
     if (variant) *variant = 2;
     if (nseg) *nseg = e->mixed_nseg;
     return 0;

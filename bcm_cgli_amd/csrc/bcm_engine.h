@@ -260,10 +260,10 @@ int engine_run(Engine* e, int n_steps, int n_inner, double* er_hist, bool use_gr
 int engine_run_converge(Engine* e, int n_steps, int max_inner, double tol, double* E, int* iters,
                         double* er_hist, std::string& err);
 int engine_sync(Engine* e, std::string& err);
-// FP64: selects the pushing flux kernel.  Mixed: times one RK stage for every
-// number of runs per cube on the resident cases (state restored afterwards)
-// and keeps the fastest.  Returns the chosen (variant, nseg) through the
-// pointers.
+// FP64: selects the pushing flux kernel.  Mixed: times one RK stage in the rule's
+// runs per cube and in 1, 2 and 4 on the resident cases (state restored
+// afterwards) and keeps the fastest.  Returns (variant, nseg) through the
+// pointers, nseg the fastest of those that can be pinned.
 int engine_autotune(Engine* e, int* variant, int* nseg, std::string& err);
 // Selects the FP64 kernel when no choice was made yet.
 int engine_maybe_tune(Engine* e, std::string& err);

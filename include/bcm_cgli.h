@@ -269,11 +269,12 @@ int bcm_engine_time_part(bcm_engine* e, int part, int RK, int reps, double* ms);
  * give bitwise the same state arrays.  Setting a choice disables tuning. */
 int bcm_engine_set_flux(bcm_engine* e, int variant, int nseg, int fuse);
 /* Selects the fastest flux choice, as the first bcm_engine_run does otherwise:
- * FP64 variant 1, fuse 2; mixed, unlike a run's own rule (runs per cube by the
- * number of resident cubes), the fastest of nseg 1, 2 and 4, each timed as one
- * whole RK stage on the resident cases (the state is restored), until the
- * pool's size class changes.  out3 (may be null) receives {variant, nseg,
- * fuse}. */
+ * FP64 variant 1, fuse 2; mixed, instead of a run's own rule alone (runs per
+ * cube by the number of resident cubes), the fastest of the rule's number and
+ * nseg 1, 2 and 4, each timed as one whole RK stage on the resident cases (the
+ * state is restored), until the pool's size class changes.  out3 (may be null)
+ * receives {variant, nseg, fuse}, nseg the fastest that bcm_engine_set_flux can
+ * pin, also where the rule's 8 or 16 runs are kept. */
 int bcm_engine_autotune(bcm_engine* e, int* out3);
 /* Ghost schedule statistics: entries, cubes with entries, maximum levels. */
 int bcm_engine_ghost_stats(bcm_engine* e, int* stats3);
