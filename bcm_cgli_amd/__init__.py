@@ -242,8 +242,9 @@ FORCE_AREA = 2.602
 
 
 def selftest_division(n, seed=1):
-    """Quotients (of 4 * n on random operands) whose bits differ between the
-    FP64 kernels' shared-denominator division and plain division."""
+    """Quotients and roots (of 4 * n and n, random and at the ends of their range)
+    whose bits differ between the FP64 kernels' division without range scaling
+    and their square root, and plain division and sqrt on the device."""
     out = ctypes.c_ulonglong(0)
     _check(load_library().bcm_selftest_division(int(seed), int(n), ctypes.byref(out)))
     return int(out.value)

@@ -37,12 +37,19 @@ __device__ __forceinline__ double rmax(double a, double b) { return (a > b) ? a 
 // quotient's part (div_sh) is the product a r, its exact remainder, one
 // correction and the fixup that sets zeros, infinities, NaN and signs.
 // Several quotients share one denominator's part.  The bits are those of a / b
-// unless a nonzero numerator is below 2^-969 in magnitude (its remainder is
-// then subnormal) or the denominator's reciprocal is out of range, states no
-// flow reaches; k_div_selftest compares.  Against the scaled form: one
-// instruction less per quotient (4), two less per denominator, no wait
-// between a flag's producer and its consumer (with root below, the pushing
-// flux kernel 1,345 -> 1,252 us on 2,048 cubes).
+// where the numerator is zero or at least 2^-969 in magnitude (below, its
+// remainder is subnormal), the denominator and its reciprocal are normal numbers,
+// and the quotient, if not zero, is normal and below 2^1023 (above, the product
+// a r may overflow to infinity and the correction give NaN where the quotient is
+// finite).  One correction does not suffice where r is not the rounded
+// reciprocal, which a step from below cannot reach for a significand of all ones;
+// there the hardware's estimate is that value, and the step keeps it.
+// k_div_selftest compares at random, at such significands and near these limits.
+// No flow reaches them: the smallest momenta are those at the front of a
+// disturbance that spreads through a uniform field, above 1e-120 on rows of 24 to
+// 120 cubes.  Against the scaled form: one instruction less per quotient (4), two
+// less per denominator, no wait between a flag's producer and its consumer (with
+// root below, the pushing flux kernel 1,345 -> 1,252 us on 2,048 cubes).
 struct DivBy {
   double b, r;   // denominator and its reciprocal
 };

@@ -1354,18 +1354,29 @@ __global__ __launch_bounds__(WG) void k_copy_d(const double* __restrict__ src,
 
 namespace {
 // DivBy/div_sh against a / b and root against sqrt: per thread one denominator
-// and four numerators
-// from a seeded hash (random signs, significands and exponents in
-// [-126, 126]; about one numerator in 16 is a signed zero).
+// and four numerators from a seeded hash, with random signs; about one numerator
+// in 16 is a signed zero.  Of four threads one each takes
+//   0: random significands, exponents in [-126, 126];
+//   1: significands next to 1, 1.5 and 2 (all ones), the same exponents;
+//   2: numerators next to the smallest division is right for, 2^-969 to 2^-965,
+//      over denominators in 2^-24 to 2^24, half of either with significands as in
+//      1, and roots of 2^-767 to 2^-763;
+//   3: numerators and denominators of exponents in [-480, 480].
 __device__ __forceinline__ unsigned long long mix64(unsigned long long x) {
   x += 0x9e3779b97f4a7c15ull;
   x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
   x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
   return x ^ (x >> 31);
 }
-__device__ __forceinline__ double test_value(unsigned long long r) {
-  const double m = 1.0 + (double)(r >> 12) * 0x1p-52;
-  const double v = ldexp(m, (int)((r >> 1) % 253) - 126);
+// A value with exponent in [lo, lo + n) from the bits of r; ends: its significand
+// at most 3 units off 1, 1.5 or 2.
+__device__ __forceinline__ double test_value(unsigned long long r, int lo, int n, bool ends) {
+  long long m = (long long)(r >> 12);
+  if (ends) {
+    const int at = (int)(m % 3), by = (int)(m / 3 % 4);
+    m = at == 0 ? by : at == 1 ? (1ll << 51) - 2 + by : (1ll << 52) - 1 - by;
+  }
+  const double v = ldexp(1.0 + (double)m * 0x1p-52, lo + (int)((r >> 1) % n));
   return (r & 1) ? -v : v;
 }
 __global__ __launch_bounds__(WG) void k_div_selftest(unsigned long long seed, int n,
@@ -1373,11 +1384,20 @@ __global__ __launch_bounds__(WG) void k_div_selftest(unsigned long long seed, in
   const int g = blockIdx.x * WG + threadIdx.x;
   if (g >= n) return;
   const unsigned long long base = mix64(seed ^ ((unsigned long long)g << 20));
-  const double b = test_value(mix64(base));
+  const int kind = g & 3;
+  auto ends = [&](unsigned long long r) { return kind == 1 || (kind == 2 && (r >> 32 & 1)); };
+  auto den = [&](unsigned long long r) {
+    return kind < 2 ? test_value(r, -126, 253, ends(r))
+                    : kind == 2 ? test_value(r, -24, 49, ends(r)) : test_value(r, -480, 961, false);
+  };
+  auto num = [&](unsigned long long r) {
+    return kind == 2 ? test_value(r, -969, 5, ends(r)) : den(r);
+  };
+  const double b = den(mix64(base));
   double a[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    a[k] = test_value(mix64(base + 1 + k));
+    a[k] = num(mix64(base + 1 + k));
     if ((mix64(base + 10 + k) & 15) == 0) a[k] = (k & 1) ? -0.0 : 0.0;
   }
   const DivBy d = div_by(b);
@@ -1385,7 +1405,9 @@ __global__ __launch_bounds__(WG) void k_div_selftest(unsigned long long seed, in
 #pragma unroll
   for (int k = 0; k < 4; ++k)
     nb += __double_as_longlong(div_sh(d, a[k])) != __double_as_longlong(a[k] / b);
-  nb += __double_as_longlong(root(fabs(a[0]))) != __double_as_longlong(sqrt(fabs(a[0])));
+  const unsigned long long q = mix64(base + 5);
+  const double x = fabs(kind == 2 ? test_value(q, -767, 5, ends(q)) : a[0]);
+  nb += __double_as_longlong(root(x)) != __double_as_longlong(sqrt(x));
   if (nb) atomicAdd(bad, nb);
 }
 }  // namespace

@@ -287,8 +287,10 @@ int bcm_engine_set_ghost_lds_limit(bcm_engine* e, int slots);
 /* The FP64 kernels divide and take square roots without range scaling, and
  * divide several numerators by one denominator with the denominator's part of
  * the correctly rounded division formed once.  This runs n threads of four
- * such quotients and one root on random operands against plain division and
- * sqrt on the current device; *mismatches receives the number of results
+ * such quotients and one root on random operands, on significands next to 1, 1.5
+ * and 2 and near the smallest operands they are right for (numerators of 2^-969,
+ * roots of 2^-767; zero apart) against plain division and sqrt on the current
+ * device; *mismatches receives the number of results
  * whose bits differ (0 expected).  Not a reference interface: a self-test. */
 int bcm_selftest_division(unsigned long long seed, int n, unsigned long long* mismatches);
 
