@@ -546,16 +546,16 @@ int rebuild_tables(Engine* e, std::string& err) {
       for (const GhostEntry& E : gs.entries) ib[E.cube].push_back(&E);
     std::vector<MlTaskDev> again;
     for (const MlTaskDev& t : ml) {
-      // Layers along the face's axis (of the source at least those read).
-      auto hit = [&](int cube, int lo, int hi) {
-        for (const GhostEntry* E : ib[cube]) {
-          const int q = t.axis == 0 ? E->gi : t.axis == 1 ? E->gj : E->gk;
-          if (q >= lo && q <= hi) return true;
+      // An IB ghost cell in the source's layers along the face's axis (at least
+      // those read).  The layers written are ghost layers, where none lies.
+      const int lo = t.hi ? 2 : 14, hi = t.hi ? 5 : 17;
+      for (const GhostEntry* E : ib[t.src]) {
+        const int q = t.axis == 0 ? E->gi : t.axis == 1 ? E->gj : E->gk;
+        if (q >= lo && q <= hi) {
+          again.push_back(t);
+          break;
         }
-        return false;
-      };
-      if (hit(t.src, t.hi ? 2 : 14, t.hi ? 5 : 17) || hit(t.dst, t.hi ? 18 : 0, t.hi ? 19 : 1))
-        again.push_back(t);
+      }
     }
     e->n_ml_ib = (int)again.size();
     if (dev_upload(&e->ml_ib, again, err)) return 1;

@@ -126,7 +126,7 @@ struct Engine {
   MlTaskDev* ml = nullptr;
   int n_ml = 0;
   // Those of them that the pre-flux refresh repeats: an IB ghost cell lies in
-  // the cells the task reads or writes.
+  // the cells the task reads.
   MlTaskDev* ml_ib = nullptr;
   int n_ml_ib = 0;
   // Cubes whose face ghosts can change between a stage's opening edge pass
