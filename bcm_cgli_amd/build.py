@@ -43,7 +43,7 @@ HIP_HOST = ("bcm_engine.cpp", "bcm_download.cpp", "bcm_output.cpp", "bcm_capi.cp
 # The mixed-precision kernels carry no bitwise contract with the reference:
 # they let the compiler fuse multiply-adds.  Their marching kernel runs at two
 # waves per SIMD whatever its registers (up to 256): the scheduler that goes for
-# instruction parallelism uses 226 of them instead of 205 and takes 476 us on
+# instruction parallelism uses 227 of them instead of 205 and takes 476 us on
 # 2,048 cubes instead of 494 (max-ilp: 482).  The FP64 one, at 253, gains nothing
 # (954 us with max-ilp, 950 without).
 PER_FILE_FLAGS = {"bcm_kernels_mixed.hip": ["-ffp-contract=fast", "-mllvm",

@@ -1139,8 +1139,8 @@ int engine_autotune(Engine* e, int* variant, int* nseg, std::string& err) {
   // copy of the iterate, whose runs per cube follow the resident cubes
   // (push_runs).  The in-place kernels stay selectable with set_flux and serve
   // the stage pieces and drop-ins; as whole stages they are slower at every
-  // size (flux kernel 1,072 against 1,004 us on 2,048 cubes, 161 against 24 on
-  // 8, and the exchange they need afterwards).
+  // size (flux kernel 1,072 against 1,004 us on 2,048 cubes; flux and update 20
+  // against 19 on 8, in two launches; and the exchange they need afterwards).
   e->flux_variant = 1;
   e->flux_nseg = 1;
   e->flux_fuse = true;

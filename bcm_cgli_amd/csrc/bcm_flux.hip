@@ -83,12 +83,13 @@ __device__ __forceinline__ T& at_byte(T* base, unsigned off) {
 // Runs: a run's first plane needs the x-face before it (evaluated before the
 // march) and two primitive planes; nothing else is done twice.
 //
-// Bound: vector instructions, about 3,000 per cell; 253 VGPRs and 76 KB of LDS
-// give two workgroups per CU.  Against a march that loaded the plane's and the
+// Bound: vector instructions, 2,797 per cell (68% of the issue rate); 253 VGPRs
+// and 76 KB of LDS give two workgroups per CU.  Against a march that loaded the plane's and the
 // column's cells in the iteration that uses them, with three barriers and one
 // boundary round per axis: 1,252 -> 1,004 us on 2,048 cubes (PUSH), 1,487 ->
 // 1,072 (IN_PLACE).  (PUSH 947 with quartered last cubes and without the copy of
-// the BC regions.)
+// the BC regions.  These are bursts of some hundred launches; runs of seconds
+// take 960 to 1,080.)
 template <March MODE, bool AUX>
 __global__ __launch_bounds__(WG, 2) void k_flux_march(const MarchArgs A) {
   __shared__ __align__(16) double cp[2][5 * 400];   // conserved values of planes i, i+1

@@ -314,13 +314,14 @@ __device__ __forceinline__ T& at_byte(T* base, unsigned off) {
 // and bits, as the unsegmented march computes it with.  Norm partials are one row
 // per plane, so every result is bitwise the same for every nseg.
 //
-// Bound: vector instructions, 1,655 per cell (62% of the issue rate over the
+// Bound: vector instructions, 1,654 per cell (70% of the issue rate over the
 // launch).  Two workgroups per CU: a third (46 KB of LDS, 168 registers with 25
 // spilled) gives the same rate, 624 us on 2,048 cubes against 555.  Against a
 // march that kept the whole column in registers, two face arrays more in LDS and
 // a boundary round per axis: 570 -> 555 us on 2,048 cubes, 51 -> 45 on 125.  (476
 // and 43 with what followed: quartered last cubes, BC regions carried by a kernel
-// of their own, another schedule.)
+// of their own, another schedule.  Bursts of some hundred launches; runs of seconds
+// take 500 to 520 on 2,048.)
 __global__ __launch_bounds__(WG, 2) void k_flux_mixed(
     float* __restrict__ U, float* __restrict__ Uout, const HaloSrc* __restrict__ halo,
     const uint8_t* __restrict__ cube_mask, const double* __restrict__ Bsrc,
